@@ -197,6 +197,9 @@ void launch_splat8(bool additive, int variant, const uint32_t *items, uint32_t n
 // optional): the staged lists are min(n, *dn) (n, i1 are capacities).
 constexpr int kStageLoad = 8;  // a list's groups of 4 entries: a multiple of kStageLoad
 constexpr int kStageQ = 4;     // groups per block of q_c (48 floats: 3 channels x 16)
+// Groups behind the last list's operands that the chains' loads may run into
+// (read ahead, never applied).
+constexpr uint32_t kStagePad = 512;
 uint64_t stage_floats(bool additive, uint64_t groups);
 uint64_t stage_q_floats(bool additive, uint64_t groups);
 void launch_stage_base(const uint32_t *items, uint32_t n, uint32_t *cbase, uint32_t *cbat,

@@ -1370,25 +1370,63 @@ __global__ __launch_bounds__(256) void k_stage_ops(SplatArgs a, const uint32_t *
 
 // The chains of the staged lists.  A wave applies channel c of list i to a
 // slice of kPix pixels of the block: workgroup (3 i + c) kS + h takes pixels
-// [h kPix, h kPix + kPix).  One load instruction brings kS consecutive groups
-// of a plane (lane part q: group g + q of the slice's pixels, 16 bytes per
-// lane), so the loads in flight per wave cover kS groups each; lanes
-// [0, kPix) run the chains and read the other parts' groups back through
-// LDS one step ahead.  A chain's wave is bound by its bytes in flight and
-// its serial operations, not by issue, so narrower slices (more waves per
-// list, fewer bytes per entry and wave) run a list faster: 8 pixels for
-// additive chains, 16 for ordered ones (whose three operand planes would not
-// fit the registers at 8).
+// [h kPix, h kPix + kPix).  One load brings kS consecutive groups of a plane
+// (lane part q: group g + q of the slice's pixels, 16 bytes per lane) straight
+// into a ring of kRing slots in LDS, so the loads in flight hold no registers;
+// lanes [0, kPix) run the chains and read the kS parts of a slot one step
+// ahead.  A chain's wave is bound by its own issue, a dependent operation
+// every 4.2 clocks and about as much per other instruction, so narrower slices
+// (more entries per load) run a list faster: 8 pixels for additive chains, 16
+// for ordered ones (three planes per entry).  With the loads in registers, the
+// copies at the end of each round waited for every load in flight (500k
+// ordered at 512^2, longest list 79.7k entries: 15.3 -> 9.8 ns per entry; 1M
+// additive at 800^2, 165k entries: 5.1 -> 4.5 ns, there bound by HBM traffic).
 template <int ADD> constexpr int chain_groups() { return ADD ? kStageLoad : kStageQ; }
 static_assert(kStageLoad % kStageQ == 0, "chain loads tile the padded groups");
+// slots of the ring (ordered: one of m1_c and one of m2 each)
+template <int ADD> constexpr int chain_ring() { return ADD ? 24 : 16; }
+static_assert(2 * chain_ring<1>() * chain_groups<1>() <= static_cast<int>(kStagePad) &&
+                  2 * chain_ring<0>() * chain_groups<0>() <= static_cast<int>(kStagePad),
+              "the chains' loads past a list stay inside the operands");
+
+// LDS byte address of a shared object.
+__device__ __forceinline__ uint32_t lds_address(const void *p) {
+  return static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
+      (const __attribute__((address_space(3))) void *)p));
+}
+
+// 16 (load_lds4: 4) bytes per lane from base + off into LDS at byte address lds +
+// 16 (4) lane.  Completion counts in vmcnt; the caller waits for it.
+__device__ __forceinline__ void load_lds16(uint32_t lds, const void *base, uint32_t off) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+               :
+               : "s"(lds), "v"(off), "s"(base)
+               : "memory", "m0");
+}
+__device__ __forceinline__ void load_lds4(uint32_t lds, const void *base, uint32_t off) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
+               :
+               : "s"(lds), "v"(off), "s"(base)
+               : "memory", "m0");
+}
+
 template <int ADD>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2))) void k_stage_chain(
+__global__ __launch_bounds__(64) void k_stage_chain(
     SplatArgs a, const uint32_t *items, uint32_t i0, const uint32_t *cbase,
     const float4 *__restrict__ ops, const float *__restrict__ qv, const uint32_t *dn) {
   constexpr int kS = chain_groups<ADD>(), kPix = 64 / kS;
   constexpr uint32_t P = stage_planes<ADD>();
-  constexpr int kR = ADD ? 32 : 10;  // steps in flight (ordered: three loads per step)
-  __shared__ float4 xs[3][64];
+  constexpr int kRing = chain_ring<ADD>();
+  constexpr int kPl = ADD ? 1 : 2;          // planes per slot
+  constexpr int kQs = ADD ? 1 : kRing / 4;  // q_c: blocks of 4 steps
+  static_assert(kRing % 4 == 0, "whole blocks of q_c per ring");
+  typedef float v4f __attribute__((ext_vector_type(4)));
+  // one LDS block at address 0
+  struct Lds {
+    v4f op[kRing][kPl][64];
+    float q[kQs][64];
+  };
+  __shared__ Lds L;
   const uint32_t i = i0 + blockIdx.x / (3u * kS);
   if (dn && i >= *dn) return;  // past the device count (uniform per workgroup)
   const uint32_t r3 = blockIdx.x % (3u * kS);
@@ -1409,120 +1447,103 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2))) void
   float *d = ug.pic + (static_cast<int64_t>(ug.x0s + lx) * ug.yres + (ug.y0s + ly)) * 3 + c;
   float l = 0.f;
   if (ug.accumulate == 2 && pix_in) l = *d;  // a later chunk: continue the chain
-  // l is in its register before the operand loads are issued: a load still
-  // in flight at the loop would make the compiler wait for every load there
+  // l is in its register before the operand loads are issued
   asm volatile("" : "+v"(l));
-  // group g of plane c and this pixel: src[g * P * 64]; lane quarter qo reads g + qo
-  const float4 *src = ops + static_cast<size_t>(gb0) * P * 64u + static_cast<size_t>(c) * 64u + px;
-  const float4 *srcw = ops + static_cast<size_t>(gb0) * P * 64u + 3u * 64u + px;  // m2 (ordered)
-  // q_c of the entries of group g + qo (4 floats; the same for a part's lanes;
-  // ordered chains load kS = kStageQ groups, one block of q_c)
-  const float4 *qsrc = reinterpret_cast<const float4 *>(qv + static_cast<size_t>(gb0 / kStageQ) * 48u +
-                                                       static_cast<size_t>(c) * 16u) + qo;
-  auto at_load = [&](uint32_t g0) {  // groups [g0, g0 + kS), the last ones again past the list
-    return static_cast<size_t>(min<uint32_t>(g0, G - kS) + qo) * P * 64u;
+  // A load brings groups g .. g + kS - 1 of plane c for the slice's pixels:
+  // a wave-uniform base per plane, advanced by the scalar unit, and one lane
+  // offset (part qo: group g + qo).  Loads run up to 2 kRing steps past the
+  // list's end (kStagePad groups of slack behind the last list; never applied).
+  constexpr uint32_t kStep = kS * P * 1024u;  // bytes per load
+  const char *pw = reinterpret_cast<const char *>(ops + static_cast<size_t>(gb0) * P * 64u) + 3072u;
+  const char *pm = pw - 3072u + static_cast<uint32_t>(c) * 1024u;
+  // q_c of four loads (kStageQ groups each) per q load: lane = entry
+  const char *pq = reinterpret_cast<const char *>(qv + static_cast<size_t>(gb0 / kStageQ) * 48u +
+                                                  static_cast<size_t>(c) * 16u);
+  const uint32_t vo = (static_cast<uint32_t>(qo) * P * 64u + static_cast<uint32_t>(px)) * 16u;
+  const uint32_t vq = static_cast<uint32_t>(lane / 16) * 192u + static_cast<uint32_t>(lane % 16) * 4u;
+  const uint32_t lop = lds_address(&L.op[0][0][0]), lq = lds_address(&L.q[0][0]);
+  auto refill_q = [&](int b) {  // q_c of slots 4 b .. 4 b + 3
+    load_lds4(lq + static_cast<uint32_t>(b) * 256u, pq, vq);
+    pq += 4u * 192u;
   };
-  auto at_q = [&](uint32_t g0) {  // that load's q_c (48 floats per kStageQ groups)
-    return static_cast<size_t>(min<uint32_t>(g0, G - kS) / kStageQ) * 12u;
-  };
-  // one load's 4 kS entries for lanes [0, kPix): its own part, then the
-  // others read back through LDS
-  struct Q {
-    float4 v[kS];
-  };
-  auto exchange = [&](int slot, const float4 &v) {
-    xs[slot][lane] = v;
-    wave_sync();
-    Q r;
-    r.v[0] = v;
-#pragma unroll
-    for (int k = 1; k < kS; ++k) r.v[k] = xs[slot][pl + k * kPix];
-    return r;
-  };
-  struct Step {
-    Q m, w, q;  // ordered: m1_c, m2 and q_c (the same in every lane) of the load's entries
-  };
-  auto step_of = [&](const float4 &vm, const float4 &vw, const float4 &vq) {
-    Step st;
-    st.m = exchange(0, vm);
+  auto refill = [&](int r) {  // slot r: the next load
+    load_lds16(lop + static_cast<uint32_t>(r * kPl) * 1024u, pm, vo);
+    pm += kStep;
     if (!ADD) {
-      st.w = exchange(1, vw);
-      st.q = exchange(2, vq);
+      load_lds16(lop + static_cast<uint32_t>(r * kPl + 1) * 1024u, pw, vo);
+      pw += kStep;
     }
+  };
+  struct Step {  // one load's 4 kS entries: m1_c (or t_c), m2 and q_c
+    v4f m[kS], w[ADD ? 1 : kS], q[ADD ? 1 : kS];
+  };
+  auto read = [&](int r) {  // slot r, once its loads have landed
+    // Loads complete in order.  Behind slot r's load at least those of the
+    // kRing - 2 slots refilled since are in flight; behind its q_c, loaded
+    // with the last slot of its four, those of kRing - 4.
+    asm volatile("s_waitcnt vmcnt(%0)" : : "n"(kPl * (kRing - (ADD ? 2 : 4))) : "memory");
+    Step st;
+#pragma unroll
+    for (int k = 0; k < kS; ++k) {
+      st.m[k] = L.op[r][0][pl + k * kPix];
+      if (!ADD) {
+        st.w[k] = L.op[r][kPl - 1][pl + k * kPix];
+        st.q[k] = *reinterpret_cast<const v4f *>(&L.q[r / 4][(r % 4) * 16 + 4 * k]);
+      }
+    }
+    asm volatile("" ::: "memory");
     return st;
   };
   auto apply = [&](const Step &st) {
-    if (ADD) {
 #pragma unroll
-      for (int k = 0; k < kS; ++k) {  // load part k: entries 4k .. 4k + 3
-        l = l + st.m.v[k].x;
-        l = l + st.m.v[k].y;
-        l = l + st.m.v[k].z;
-        l = l + st.m.v[k].w;
-      }
-    } else {
-#pragma unroll
-      for (int k = 0; k < kS; ++k) {
-        const float4 &m4 = st.m.v[k], &w4 = st.w.v[k], &q4 = st.q.v[k];
-        l = l + ((l - q4.x) * m4.x) * w4.x;
-        l = l + ((l - q4.y) * m4.y) * w4.y;
-        l = l + ((l - q4.z) * m4.z) * w4.z;
-        l = l + ((l - q4.w) * m4.w) * w4.w;
+    for (int k = 0; k < kS; ++k) {  // load part k: entries 4k .. 4k + 3
+      if (ADD) {
+        l = l + st.m[k].x;
+        l = l + st.m[k].y;
+        l = l + st.m[k].z;
+        l = l + st.m[k].w;
+      } else {
+        l = l + ((l - st.q[k].x) * st.m[k].x) * st.w[k].x;
+        l = l + ((l - st.q[k].y) * st.m[k].y) * st.w[k].y;
+        l = l + ((l - st.q[k].z) * st.m[k].z) * st.w[k].z;
+        l = l + ((l - st.q[k].w) * st.m[k].w) * st.w[k].w;
       }
     }
   };
-  float4 bm[kR], bw[ADD ? 1 : kR], bq[ADD ? 1 : kR];
+  if (!ADD)
 #pragma unroll
-  for (int r = 0; r < kR; ++r) {  // issued in the order they are consumed
-    const size_t o = at_load(r * kS);
-    bm[r] = src[o];
-    if (!ADD) {
-      bw[r] = srcw[o];
-      bq[r] = qsrc[at_q(r * kS)];
-    }
-    asm volatile("" ::: "memory");
-  }
-  // Software pipeline over the loads: step r of a round applies the entries
-  // of load r (exchanged a step earlier), exchanges load r + 1 meanwhile, and
-  // refills that load's registers with the groups kR loads further on.
-  Step cur = step_of(bm[0], bw[0], bq[0]);
-  asm volatile("" ::: "memory");
-  {
-    const size_t o = at_load(kR * kS);
-    bm[0] = src[o];
-    if (!ADD) {
-      bw[0] = srcw[o];
-      bq[0] = qsrc[at_q(kR * kS)];
-    }
-  }
-  // whole rounds first (every step applies: one straight-line block per
-  // round, a scheduling region per step, in which the exchange and the
-  // refill sit among the dependent additions), then the last, partial round
+    for (int b = 0; b < kQs; ++b) refill_q(b);
+#pragma unroll
+  for (int r = 0; r < kRing; ++r) refill(r);  // issued in the order they are consumed
+  Step cur = read(0);
+  // Software pipeline: step r starts the reads of slot r + 1, then applies the
+  // entries of slot r (read a step earlier: one wait for all of them, as they
+  // return in order), and then refills slot r.  Whole rounds first (every step
+  // applies: one straight-line block per round), then the last, partial round.
   auto round = [&](uint32_t g, bool whole) {
 #pragma unroll
-    for (int r = 0; r < kR; ++r) {
-      const int rn = (r + 1) % kR;
-      const uint32_t g0 = g + r * kS;
-      const Step nxt = step_of(bm[rn], bw[ADD ? 0 : rn], bq[ADD ? 0 : rn]);
-      if (whole || g0 < G) apply(cur);
+    for (int r = 0; r < kRing; ++r) {
+      const int rn = (r + 1) % kRing;
+      Step nxt = read(rn);
+      __builtin_amdgcn_sched_barrier(0);
+      if (whole || g + r * kS < G) {
+        asm volatile("" : "+v"(l) : "v"(ADD ? cur.m[kS - 1].w : cur.q[ADD ? 0 : kS - 1].w));
+        apply(cur);
+      }
       cur = nxt;
-      // the barriers order the exchange and sums before the refill (and the
-      // next exchange's LDS writes after these reads), keep the load from
-      // sinking to its use a round later, so kR loads stay in flight, and
-      // keep the scheduler from moving an exchange next to its use
+      // the sums stay ahead of the refill of their slot (and of the q_c of
+      // the four slots that end with it)
       asm volatile("" : "+v"(l) : : "memory");
       __builtin_amdgcn_sched_barrier(0);
-      const size_t o = at_load(g + (r + 1) * kS + kR * kS);
-      bm[rn] = src[o];
-      if (!ADD) {
-        bw[rn] = srcw[o];
-        bq[rn] = qsrc[at_q(g + (r + 1) * kS + kR * kS)];
-      }
+      if (!ADD && r % 4 == 3) refill_q(r / 4);
+      refill(r);
     }
   };
   uint32_t g = 0;
-  for (; g + kR * kS <= G; g += kR * kS) round(g, true);
+  for (; g + kRing * kS <= G; g += kRing * kS) round(g, true);
   if (g < G) round(g, false);
+  // no load is in flight into the LDS of an ended workgroup
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   if (a.trace && c == 0 && h == 0 && lane == 0) {
     uint64_t *tr = a.trace + 4 * static_cast<uint64_t>(i);
     tr[0] = t_start;
@@ -1634,11 +1655,11 @@ void launch_items_emit(const uint32_t *bin_off, uint32_t nunits, const SplatArgs
 }
 
 uint64_t stage_floats(bool additive, uint64_t groups) {
-  return groups * (additive ? 3u : 4u) * 256u;
+  return (groups + kStagePad) * (additive ? 3u : 4u) * 256u;
 }
 
 uint64_t stage_q_floats(bool additive, uint64_t groups) {
-  return additive ? 0 : groups / kStageQ * 48u;
+  return additive ? 0 : (groups + kStagePad) / kStageQ * 48u;
 }
 
 void launch_stage_base(const uint32_t *items, uint32_t n, uint32_t *cbase, uint32_t *cbat,
