@@ -103,19 +103,22 @@ typedef struct {
                                               of an additive pass is staged: its per-pixel
                                               terms are computed across the GPU first, then
                                               summed in list order by one wave per channel
-                                              (0 = auto: 8192, but none for a single view
-                                              with both passes in one chunk, whose additive
-                                              splat runs beside the ordered pass; < 0 =
-                                              never) */
+                                              and pixel column (0 = auto: from entries /
+                                              1300 or the longest list / 64 on, but none for
+                                              a single view with both passes in one chunk,
+                                              whose additive splat runs beside the ordered
+                                              pass, and none where the longest list is below
+                                              1536 entries; < 0 = never) */
   int32_t hip_stage_ordered;               /* hip_stage_ordered: the same for an ordered pass
                                               (per-pixel operands of the compositing update
                                               computed first; not when a particle's q_c is
                                               non-finite) (0 = auto: when the longest list
                                               x 216 reaches the pass's bin entries, the
-                                              lists from about the longest / 16 on; else,
-                                              when it x 432 does, the lists from entries /
-                                              432 on; else none; thresholds are levels
-                                              8192 x 2^(j/2); < 0 = never) */
+                                              lists from the longest / 16 or entries / 700
+                                              on; else, when it x 432 does, the lists from
+                                              entries / 432 on; else, and where the longest
+                                              list is below 512 entries, none; thresholds
+                                              are levels 256 x 2^(j/2); < 0 = never) */
 } splhip_params;
 
 /* SoA particle fields (device pointers), post particle_normalize:

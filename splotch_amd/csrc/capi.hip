@@ -647,17 +647,17 @@ void make_plan(splhip_ctx *c, int nj, const JobIn *jobs, int G, Plan &pl, hipStr
 // [4..5] work items, [6..7] heavy items, [8..11] bin entries as u64,
 // [12..13] region entries, [14] the ordered pass has a non-finite q,
 // [15] capacity overflow bits of a device-count render (bit p: pass p),
-// [16..47] lists from stage_level(stage_len, j) entries on, [48..79] their
-// groups of 4 entries (padded), j = 0..15 ([16 + 16 p + j]: pass p),
-// [80..81] the longest list, [82..89] a device-count render's long-list
+// from T_STAGE on the lists from stage_level(stage_len, j) entries on and from
+// T_SGRP on their groups of 4 entries (at most), kStageLevels per pass, then
+// the longest list of each pass and a device-count render's long-list
 // partition (4 per pass: staged, producer/consumer, both).
 enum {
   T_M = 0, T_E = 2, T_ITEMS = 4, T_HEAVY = 6, T_E64 = 8, T_E16 = 12, T_QBAD = 14, T_OVF = 15,
-  T_STAGE = 16, T_SGRP = 48, T_LMAX = 80, T_PART = 82, T_N = 90
+  T_STAGE = 16, T_SGRP = T_STAGE + 2 * kStageLevels, T_LMAX = T_SGRP + 2 * kStageLevels,
+  T_PART = T_LMAX + 2, T_N = T_PART + 8
 };
-constexpr int kTotalsWords = 128;  // the totals buffer, device and pinned host
+constexpr int kTotalsWords = 256;  // the totals buffer, device and pinned host
 static_assert(T_N <= kTotalsWords, "totals fit their buffers");
-static_assert(T_SGRP - T_STAGE == 2 * kStageLevels, "one level count per pass");
 
 // Project all jobs, then the compaction scan of each present pass and its job
 // offsets in pass order; one host sync reads the pass sizes and offsets.
@@ -864,30 +864,13 @@ struct Tuning {
   uint64_t chunk;  // most (block, particle) entries of one pass chunk
   uint32_t stage, stage_ord;  // lists from this length on are staged, additive / ordered
                               // pass (0xffffffff: none)
-  bool stage_ord_auto;        // ordered staging only for a pass bound by its longest list
+  StageMode mode[2];          // the staging length's rule, ordered / additive pass
 };
 
-// Staged operands of a pass (3 KiB per group of 4 entries additive, 4 KiB +
-// 48 B ordered); a pass whose staged lists need more renders them unstaged.
+// Staged operands of a pass: room for 3 KiB per group of 4 entries additive, 7
+// KiB ordered (what is written depends on the entries' coverage); of a pass
+// whose staged lists need more, fewer are staged (the longest).
 constexpr uint64_t kStageBudget = uint64_t(32) << 30;
-// Default ordered staging only for a pass bound by its longest list: one
-// whose longest list, at about 108 clocks per entry in a producer/consumer
-// workgroup, takes at least twice as long as the pass's entries at about 0.25
-// clocks each over all CUs (the 8x8 splat's VALU work), i.e. longest list x
-// kStageOrderedRatio >= entries.  A pass below keeps every CU's VALU busy for
-// about as long as its longest lists take, and the operand kernel's extra
-// VALU and HBM work would only slow it (16M particles at 2048^2: 837k-entry
-// list, 301M entries, 43.3-53.7 ms staged from 786432-393216 entries on
-// against 43.7 ms unstaged; 64 views: 65.6M ordered entries, 68.6 -> 48.1 ms;
-// 500k at 512^2: 121k-entry list, 1.3M entries, 6.21 -> 3.58 ms).
-constexpr uint64_t kStageOrderedRatio = 216;
-// Below that, a pass whose longest lists would still end after its other
-// entries (longest list x kStageOrderedCrit >= entries, at 108 / 0.25 clocks
-// per entry) stages only those: the lists from entries / kStageOrderedCrit
-// on (rounded down to a level), whose operands then compete least with the
-// rest (16M particles at 2048^2: 813k-entry list, 331M entries; the 4 lists
-// from 741376 on staged, 41.8 ms against 42.8 unstaged).
-constexpr uint64_t kStageOrderedCrit = 432;
 // Long lists left to the 8x8 splat that would outlast the pass, walked by
 // one wave at about 230 ns per entry against about 0.1 ns per entry of the
 // pass over all CUs (16M particles at 2048^2), are served by channel, three
@@ -901,11 +884,6 @@ constexpr uint32_t kSplitRatio = 2048;
 // batch: 34.9 ms with 64, 33.7 with 16, 34.1 with 4; the 1M / 800^2 frame and
 // the 500k ordered one within 1 % of each other.
 constexpr uint32_t kStagePhase1 = 16;
-// Default ordered staging threshold: about the longest list / 16 (the
-// 64-view batch: 40.4 ms staged from 65536 entries on, 43.9 from 8192; 500k
-// at 512^2, longest list 121k: 2.67 ms from 8192, 3.39 from 65536).
-constexpr uint64_t kStageOrderedSpan = 16;
-
 Tuning tuning_of(const splhip_params *prm) {
   Tuning t;
   t.variant = prm->hip_variant > 0 ? prm->hip_variant : 4;
@@ -922,16 +900,13 @@ Tuning tuning_of(const splhip_params *prm) {
   // pipeline with a host sync and a splat tail; offsets stay below 2^31
   t.chunk = prm->hip_chunk_entries > 0 ? static_cast<uint64_t>(prm->hip_chunk_entries)
                                        : (uint64_t(1) << 31) - (uint64_t(1) << 20);
-  // additive lists from 8192 entries on: a lane-per-pixel wave walks such a
-  // list at about 100 ns per entry
-  t.stage = prm->hip_stage < 0 ? 0xffffffffu
-            : prm->hip_stage > 0 ? static_cast<uint32_t>(prm->hip_stage) : 8192u;
-  // ordered lists from 8192 entries on (for a pass bound by its longest
-  // list, see kStageOrderedRatio)
-  t.stage_ord = prm->hip_stage_ordered < 0 ? 0xffffffffu
-                : prm->hip_stage_ordered > 0 ? static_cast<uint32_t>(prm->hip_stage_ordered)
-                                             : 8192u;
-  t.stage_ord_auto = prm->hip_stage_ordered == 0;
+  // by default from a level of 256 entries on (stage_rule)
+  auto stage = [&](int32_t key, int p, uint32_t &len) {
+    len = key < 0 ? 0xffffffffu : key > 0 ? static_cast<uint32_t>(key) : 256u;
+    t.mode[p] = key != 0 ? kStageGiven : p == 1 ? kStageAutoAdditive : kStageAutoOrdered;
+  };
+  stage(prm->hip_stage, 1, t.stage);
+  stage(prm->hip_stage_ordered, 0, t.stage_ord);
   return t;
 }
 
@@ -981,24 +956,26 @@ void stage_items_count(splhip_ctx *c, Plan &pl, int p, const Tuning &tn, uint32_
 
 // Item counts of pass p from c->h_tot read from tot + T_ITEMS on (T_N -
 // T_ITEMS words): work items; long lists (one item each, sorted first) = the
-// staged ones (when their operands fit kStageBudget, else none), then at
-// most heavy_max of the others from heavy_len on for the producer/consumer
-// kernel; the rest go to the 8x8 splat.  Ordered passes by default stage the lists from
-// stage_len << k entries on, k the least with stage_len << k >= the longest
-// list / kStageOrderedSpan: shorter lists are off the critical path, and
-// staging them costs more than the 8x8 splat does.
+// staged ones (from stage_rule's level on, raised until their operands fit
+// kStageBudget), then at most heavy_max of the others from heavy_len on for
+// the producer/consumer kernel; the rest go to the 8x8 splat.
 void take_items(splhip_ctx *c, Plan &pl, int p, const Tuning &tn) {
   const uint32_t *h = c->h_tot;
   pl.nitems[p] = pl.m[p] ? h[T_ITEMS - T_ITEMS + p] : 0u;
   const uint32_t nheavy_lists = pl.m[p] ? h[T_HEAVY - T_ITEMS + p] : 0u;
   const uint64_t lmax = h[T_LMAX - T_ITEMS + p];
   const uint32_t len0 = p == 1 ? tn.stage : tn.stage_ord;
-  const int j = stage_rule(len0, p == 0 && tn.stage_ord_auto, lmax, pl.etot[p],
-                           kStageOrderedSpan, kStageOrderedRatio, kStageOrderedCrit);
-  uint32_t ns = pl.m[p] && j >= 0 ? h[T_STAGE - T_ITEMS + kStageLevels * p + j] : 0u;
-  const uint64_t groups = j >= 0 ? h[T_SGRP - T_ITEMS + kStageLevels * p + j] : 0u;
-  const uint64_t bytes = 4 * (stage_floats(p == 1, groups) + stage_q_floats(p == 1, groups));
-  if (bytes > kStageBudget) ns = 0;
+  const uint32_t *cnt = h + (T_STAGE - T_ITEMS + kStageLevels * p);
+  const uint32_t *grp = h + (T_SGRP - T_ITEMS + kStageLevels * p);
+  uint32_t ns = 0;
+  uint64_t groups = 0;
+  if (pl.m[p] && len0 != 0xffffffffu)
+    for (int j = stage_rule(len0, tn.mode[p], lmax, pl.etot[p]); j >= 0 && j < kStageLevels; ++j)
+      if (4 * stage_floats(p == 1, grp[j]) <= kStageBudget) {
+        ns = cnt[j];
+        groups = grp[j];
+        break;
+      }
   pl.nstage[p] = ns;
   pl.sgroups[p] = ns ? groups : 0;
   c->last_stage_n[p] = ns;
@@ -1012,10 +989,8 @@ void take_items(splhip_ctx *c, Plan &pl, int p, const Tuning &tn) {
   pl.nheavy[p] = std::min(ns + npc, pl.nitems[p]);
   // lists from min(stage length, heavy_len) entries on have one item each
   const uint32_t len0s = p == 1 ? tn.stage : tn.stage_ord;
-  const uint32_t nlong = !pl.m[p] ? 0u
-                         : len0s <= tn.heavy ? h[T_STAGE - T_ITEMS + kStageLevels * p]
-                                             : nheavy_lists;
-  pl.nsplit[p] = pl.m[p] ? split_lists(len0s, h + (T_STAGE - T_ITEMS + kStageLevels * p),
+  const uint32_t nlong = !pl.m[p] ? 0u : len0s <= tn.heavy ? cnt[0] : nheavy_lists;
+  pl.nsplit[p] = pl.m[p] ? split_lists(len0s, cnt,
                                        std::min(nlong, pl.nitems[p]), pl.nheavy[p], pl.etot[p],
                                        kSplitRatio)
                          : 0u;
@@ -1060,15 +1035,12 @@ void stage_splat(splhip_ctx *c, Plan &pl, int p, const Tuning &tn, hipStream_t s
     pa.lmax = pl.tot + T_LMAX + p;
     pa.etot = reinterpret_cast<const uint64_t *>(pl.tot + T_E64 + 2 * p);
     pa.len0 = pl.nstage[p] ? (p == 1 ? tn.stage : tn.stage_ord) : 0xffffffffu;
-    pa.ordered_auto = p == 0 && tn.stage_ord_auto;
+    pa.mode = tn.mode[p];
     pa.ns_cap = pl.nstage[p];
     pa.groups_cap = pl.sgroups[p];
     pa.heavy_max = tn.heavy == 0xffffffffu ? 0u : tn.heavy_max;
     pa.heavy_len = tn.heavy;
-    pa.span = static_cast<uint32_t>(kStageOrderedSpan);
-    pa.ratio = static_cast<uint32_t>(kStageOrderedRatio);
     pa.split = kSplitRatio;
-    pa.crit = static_cast<uint32_t>(kStageOrderedCrit);
     launch_partition(pa, part, s);
     dc.items = pl.tot + T_ITEMS + p;
     dc.heavy = part + 2;
@@ -1118,11 +1090,16 @@ void stage_splat(splhip_ctx *c, Plan &pl, int p, const Tuning &tn, hipStream_t s
       // the operand kernel and then the chains on a third stream, beside the
       // normal items
       const bool add = p == 1;
-      uint32_t *cb = ws.get_as<uint32_t>(pslot(p, P_SBASE), nstage + 1);
+      uint32_t *cb = ws.get_as<uint32_t>(pslot(p, P_SBASE), nstage + 3);
+      uint32_t *nrows = cb + nstage + 1;
       uint32_t *cbt = ws.get_as<uint32_t>(pslot(p, P_SBAT), nstage + 1);
       float4 *ops = ws.get_as<float4>(pslot(p, P_SOPS), stage_floats(add, pl.sgroups[p]) / 4);
-      float *qv = add ? nullptr
-                      : ws.get_as<float>(pslot(p, P_SQ), stage_q_floats(add, pl.sgroups[p]));
+      const uint64_t stride = stage_stride(pl.sgroups[p]);
+      const uint64_t nbat = stage_batches(pl.sgroups[p], nstage);
+      uint64_t *masks = ws.get_as<uint64_t>(pslot(p, P_SMASK), nbat * 64);
+      uint32_t *rows = ws.get_as<uint32_t>(pslot(p, P_SROWS), nbat * 16);
+      uint32_t *gofs = ws.get_as<uint32_t>(pslot(p, P_SGOFS), nbat * 16);
+      Workspace &tmp = wt ? *wt : ws;
       // the kStagePhase1 longest lists first: their chains start after their
       // own operands; the other lists' operands and chains follow on a fourth
       // stream, beside those chains
@@ -1131,17 +1108,27 @@ void stage_splat(splhip_ctx *c, Plan &pl, int p, const Tuning &tn, hipStream_t s
       hip_check(hipEventRecord(X.fork3, s), "record fork");
       hip_check(hipStreamWaitEvent(X.aux3, X.fork3, 0), "wait fork");
       mark(c, p == 0 ? 11 : 12, true, X.aux3);
-      launch_stage_base(items, nstage, cb, cbt, sa, X.aux3, part);
-      launch_stage_ops(add, items, 0, n1, pl.sgroups[p], cb, cbt, ops, qv, sa, X.aux3, part);
+      launch_stage_base(items, nstage, n1, cb, cbt, nrows, sa, X.aux3, part);
+      // the scans' temporaries are the pass's own: phase 2's runs after phase 1's
+      auto operands = [&](uint32_t i0, uint32_t i1, uint32_t phase, hipStream_t q) {
+        uint32_t *r = rows + phase * nbat * 8, *g = gofs + phase * nbat * 8;
+        launch_stage_rows(items, i0, i1, nbat, cbt, masks, r, sa, q, part);
+        scan_u32(r, g, static_cast<int64_t>(nbat * 8), nullptr, tmp, q, 0, nrows + phase);
+        launch_stage_ops(add, items, i0, i1, nbat, cb, cbt, masks, r, g, ops, stride, sa, q, part);
+      };
+      auto chains = [&](uint32_t i0, uint32_t i1, uint32_t phase, hipStream_t q) {
+        launch_stage_chain(add, items, i0, i1, cb, cbt, rows + phase * nbat * 8,
+                           gofs + phase * nbat * 8, ops, stride, sa, q, part);
+      };
+      operands(0, n1, 0, X.aux3);
       if (n1 < nstage) {
         hip_check(hipEventRecord(X.fork4, X.aux3), "record fork");
         hip_check(hipStreamWaitEvent(X.aux4, X.fork4, 0), "wait fork");
-        launch_stage_ops(add, items, n1, nstage, pl.sgroups[p], cb, cbt, ops, qv, sa, X.aux4,
-                         part);
-        launch_stage_chain(add, items, n1, nstage, cb, ops, qv, sa, X.aux4, part);
+        operands(n1, nstage, 1, X.aux4);
+        chains(n1, nstage, 1, X.aux4);
         hip_check(hipEventRecord(X.join4, X.aux4), "record join");
       }
-      launch_stage_chain(add, items, 0, n1, cb, ops, qv, sa, X.aux3, part);
+      chains(0, n1, 0, X.aux3);
       mark(c, p == 0 ? 11 : 12, false, X.aux3);
       hip_check(hipEventRecord(X.join3, X.aux3), "record join");
     }
@@ -1852,8 +1839,8 @@ int capture_reserve(splhip_ctx *c, int nj, const JobIn *jobs, float headroom, hi
       rv->ns_cap[p] = static_cast<uint32_t>(std::min(
           static_cast<double>(c->last_stage_n[p]) * headroom + 16.0, 1048576.0));
       const double g = static_cast<double>(c->last_stage_groups[p]) * headroom + 1024.0;
-      const uint64_t gc = static_cast<uint64_t>(g / kStageLoad + 1) * kStageLoad;
-      if (4 * (stage_floats(p == 1, gc) + stage_q_floats(p == 1, gc)) <= kStageBudget) {
+      const uint64_t gc = static_cast<uint64_t>(g);
+      if (4 * stage_floats(p == 1, gc) <= kStageBudget) {
         rv->groups_cap[p] = gc;
       } else {
         rv->ns_cap[p] = 0;

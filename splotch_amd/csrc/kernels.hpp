@@ -147,7 +147,7 @@ void launch_unpack_records(const char *stage, int64_t n, int64_t C, int ncol, fl
 
 // Staging thresholds: level j = 0..kStageLevels-1 of a base length sl is
 // sl * 2^(j/2) (odd levels times 181/128, about sqrt 2, rounded down).
-constexpr int kStageLevels = 16;
+constexpr int kStageLevels = 26;
 __host__ __device__ inline uint64_t stage_level(uint32_t sl, int j) {
   const uint64_t b = static_cast<uint64_t>(sl) << (j >> 1);
   return (j & 1) ? (b * 181u) >> 7 : b;
@@ -157,8 +157,7 @@ __host__ __device__ inline uint64_t stage_level(uint32_t sl, int j) {
 // channel 3 = all), heaviest first.  heavy_cnt (device, optional): incremented
 // once per unit whose list reaches a.heavy_len (one item); stage_cnt /
 // stage_grp (optional, [kStageLevels] each): [j] once per unit whose list
-// reaches stage_level(a.stage_len, j), and by its groups of 4 entries (padded
-// to whole chain loads); lmax (optional): the longest list of a unit with
+// reaches stage_level(a.stage_len, j), and by its groups of 4 entries (at most); lmax (optional): the longest list of a unit with
 // items.
 void launch_items_count(const uint32_t *bin_off, uint32_t nunits, const SplatArgs &a,
                         int ordered, uint32_t split, uint32_t *cnt, uint32_t *heavy_cnt,
@@ -188,32 +187,43 @@ struct ItemCounts {
 void launch_splat8(bool additive, int variant, const uint32_t *items, uint32_t nitems,
                    const SplatArgs &a, hipStream_t s, const ItemCounts &dc = ItemCounts{},
                    int ppw = 0, uint32_t nsplit = 0);
-// Staged lists (splat8.hip), the first n items of a pass (groups: their
-// groups of 4 entries, padded): list offsets into cbase / cbat ([n + 1] each);
-// then, for lists [i0, i1), the per-pixel operands into ops (stage_floats
-// floats for all n) and, ordered, the entries' q_c into qv (stage_q_floats
-// floats), and the chains, one wave per list, channel and pixel slice (8
-// pixels additive, 16 ordered), which write the lists' blocks.  dn (device,
-// optional): the staged lists are min(n, *dn) (n, i1 are capacities).
-constexpr int kStageLoad = 8;  // a list's groups of 4 entries: a multiple of kStageLoad
-constexpr int kStageQ = 4;     // groups per block of q_c (48 floats: 3 channels x 16)
-// Groups behind the last list's operands that the chains' loads may run into
+// Staged lists (splat8.hip), the first n items of a pass (groups: an upper
+// bound of their groups of 4 entries): list offsets into cbase / cbat ([n + 1]
+// each); then, for lists [i0, i1) (called in two phases, [0, n1) and [n1, n)),
+// each pixel's coverage per batch of 64 entries (masks) and the row counts of
+// each batch and pixel column (rows), their scan (gofs; nrows[0] / nrows[1]
+// counts on the device), the operands of the covering entries (ops:
+// stage_floats floats in planes of stage_stride groups of 8 pixels), and the
+// chains, one wave per list, channel and pixel column, which write the lists'
+// blocks.  batches: stage_batches(groups, n), the room of masks (64 each) and
+// of each phase's rows and gofs (8 each).  dn (device, optional): the staged
+// lists are min(n, *dn) (n, i1 are capacities).
+// Groups behind a plane's last stream that the chains' loads may run into
 // (read ahead, never applied).
 constexpr uint32_t kStagePad = 512;
 uint64_t stage_floats(bool additive, uint64_t groups);
-uint64_t stage_q_floats(bool additive, uint64_t groups);
-void launch_stage_base(const uint32_t *items, uint32_t n, uint32_t *cbase, uint32_t *cbat,
-                       const SplatArgs &a, hipStream_t s, const uint32_t *dn = nullptr);
+uint64_t stage_stride(uint64_t groups);
+uint64_t stage_batches(uint64_t groups, uint32_t n);
+void launch_stage_base(const uint32_t *items, uint32_t n, uint32_t n1, uint32_t *cbase,
+                       uint32_t *cbat, uint32_t *nrows, const SplatArgs &a, hipStream_t s,
+                       const uint32_t *dn = nullptr);
+void launch_stage_rows(const uint32_t *items, uint32_t i0, uint32_t i1, uint64_t batches,
+                       const uint32_t *cbat, uint64_t *masks, uint32_t *rows, const SplatArgs &a,
+                       hipStream_t s, const uint32_t *dn = nullptr);
 void launch_stage_ops(bool additive, const uint32_t *items, uint32_t i0, uint32_t i1,
-                      uint64_t groups, const uint32_t *cbase, const uint32_t *cbat, float4 *ops,
-                      float *qv, const SplatArgs &a, hipStream_t s,
+                      uint64_t batches, const uint32_t *cbase, const uint32_t *cbat,
+                      const uint64_t *masks, const uint32_t *rows, const uint32_t *gofs,
+                      float4 *ops, uint64_t stride, const SplatArgs &a, hipStream_t s,
                       const uint32_t *dn = nullptr);
 void launch_stage_chain(bool additive, const uint32_t *items, uint32_t i0, uint32_t i1,
-                        const uint32_t *cbase, const float4 *ops, const float *qv,
+                        const uint32_t *cbase, const uint32_t *cbat, const uint32_t *rows,
+                        const uint32_t *gofs, const float4 *ops, uint64_t stride,
                         const SplatArgs &a, hipStream_t s, const uint32_t *dn = nullptr);
+// How a pass's staging length is chosen (stage_rule).
+enum StageMode { kStageGiven, kStageAutoAdditive, kStageAutoOrdered };
 // Device-count partition of a pass's long lists (one thread), as the host
 // does it with exact counts (stage_rule): the staged lists stage_cnt[j] at
-// the rule's level j (none past ns_cap or groups_cap), then at most heavy_max
+// the rule's level j (raised until they fit ns_cap and groups_cap), then at most heavy_max
 // of the other lists from heavy_len on (the count heavy_cnt).  out[0] staged,
 // out[1] producer/consumer, out[2] both, out[3] the first of the other long
 // lists (one item each: from min(len0, heavy_len) entries on), which the 8x8
@@ -222,12 +232,12 @@ struct PartitionArgs {
   const uint32_t *stage_cnt, *stage_grp, *heavy_cnt, *lmax;
   const uint64_t *etot;
   uint32_t len0;  // 0xffffffff: no staging
-  int ordered_auto;
+  StageMode mode;
   uint32_t ns_cap;
   uint64_t groups_cap;
   uint32_t heavy_max;  // 0: no producer/consumer workgroups
   uint32_t heavy_len;  // lists from this length on go to producer/consumer workgroups
-  uint32_t span, ratio, crit, split;
+  uint32_t split;
 };
 // The long lists after the first nheavy items that the 8x8 splat serves by
 // channel: those from the greatest level of len0 with level * split <= etot
@@ -242,24 +252,44 @@ __host__ __device__ inline uint32_t split_lists(uint32_t len0, const uint32_t *c
   const uint32_t n = count[j] < nlong ? count[j] : nlong;
   return n > nheavy ? n - nheavy : 0u;
 }
-// The staging level of a pass: 0, or for an ordered pass by default (auto)
-// - when lmax * ratio >= etot (bound by its longest lists): the least level
-//   with level * span >= lmax,
-// - else when lmax * crit >= etot (its longest lists would end after the
-//   rest): the greatest level with level * crit <= etot (none when even the
-//   top level is below etot / crit),
-// - else none (-1).
-__host__ __device__ inline int stage_rule(uint32_t len0, bool ordered_auto, uint64_t lmax,
-                                          uint64_t etot, uint32_t span, uint32_t ratio,
-                                          uint32_t crit) {
-  if (!ordered_auto) return 0;
+// The staging level of a pass (-1: none): level 0 with a given length, else by
+// the pass's entries and its longest list.  A staged entry costs the GPU about
+// 1.5 times an entry of the 8x8 splat, whose lone wave walks a list at about
+// 75 (additive) or 200 (ordered; by channel about 100) ns per entry against
+// 0.1 ns per entry of the pass over all CUs.  So lists are staged from the
+// length on whose walk would outlast the pass, and not below a share of the
+// longest list, whose chain bounds the pass anyway:
+//   additive  from entries / 1300 (rounded down to a level) or the longest
+//             list / 64 on (1M at 800^2, 5.2M entries, longest 165k: 1.23 ms
+//             from 4096, 1.32 from 8192, 1.36 from 1024; 2M at 512^2: 2.35 ms
+//             from 4096, 2.41 from 512)
+//   ordered   from entries / 700 (rounded down) or the longest list / 16 on,
+//             where the longest list bounds the pass: longest x 216 >= entries
+//             (1.33M at 1279 x 719, 6.1M entries, longest 41k: 2.20 ms from
+//             4096, 2.03 from 8192, 2.26 from 11585; 500k at 512^2, 1.5M
+//             entries, longest 80k: 3.12 ms from 5793, 4.22 from 8192); else,
+//             where it would still end after the rest in a producer/consumer
+//             workgroup (108 clocks per entry against 0.25 per entry of the
+//             pass: longest x 432 >= entries), the lists from entries / 432 on
+//             (rounded down; 16M at 2048^2, 331M entries, longest 813k: 41.8
+//             ms against 42.8 unstaged), whose operands compete least with
+//             the rest; else none
+// and none where the longest list is short: its walk costs less than the
+// staged kernels' launches (20k ordered at 257 x 193, longest 1345 entries:
+// 0.54 ms staged, 0.67 not).
+__host__ __device__ inline int stage_rule(uint32_t len0, StageMode mode, uint64_t lmax,
+                                          uint64_t etot) {
+  if (mode == kStageGiven) return 0;
+  const bool add = mode == kStageAutoAdditive;
+  if (lmax < (add ? 1536u : 512u)) return -1;
   int j = 0;
-  if (lmax * ratio >= etot) {
-    while (j < kStageLevels - 1 && stage_level(len0, j) * span < lmax) ++j;
+  if (add || lmax * 216u >= etot) {
+    while (j < kStageLevels - 1 && stage_level(len0, j) * (add ? 64u : 16u) < lmax) ++j;
+    while (j < kStageLevels - 1 && stage_level(len0, j + 1) * (add ? 1300u : 700u) <= etot) ++j;
     return j;
   }
-  if (lmax * crit < etot || stage_level(len0, kStageLevels - 1) * crit < etot) return -1;
-  while (j < kStageLevels - 1 && stage_level(len0, j + 1) * crit <= etot) ++j;
+  if (lmax * 432u < etot || stage_level(len0, kStageLevels - 1) * 432u < etot) return -1;
+  while (j < kStageLevels - 1 && stage_level(len0, j + 1) * 432u <= etot) ++j;
   return j;
 }
 void launch_partition(const PartitionArgs &pa, uint32_t *out, hipStream_t s);

@@ -491,6 +491,59 @@ __device__ __forceinline__ void tabulate(const SplatArgs &a, const Rec &R, int l
   att_bound = nan ? __builtin_inff() : b1 * b2;
 }
 
+// The lane's particle R over the block at (bxo, byo) of the tile (tile frame):
+// tabulate's column masks (bit r: row byo + r of the column lies in the
+// footprint) ...
+__device__ __forceinline__ void column_masks(const SplatArgs &a, const Rec &R, int x0s, int y0s,
+                                             int w, int h, int bxo, int byo, uint32_t (&cm)[8]) {
+  const float rfacr = R.r * a.rfac;
+  const float posx = R.x - static_cast<float>(x0s), posy = R.y - static_cast<float>(y0s);
+  const int bx0 = max(cvt_i32(posx - rfacr + 1), 0), bx1 = min(cvt_i32(posx + rfacr + 1), w);
+  const int by0 = max(cvt_i32(posy - rfacr + 1), 0), by1 = min(cvt_i32(posy + rfacr + 1), h);
+  const float radsq = rfacr * rfacr;
+#pragma unroll
+  for (int c = 0; c < 8; ++c) {
+    const int x = bxo + c;
+    const float dxsq = (static_cast<float>(x) - posx) * (static_cast<float>(x) - posx);
+    const float dy = sqrtf(radsq - dxsq);
+    const int lo = max(by0, cvt_i32(posy - dy + 1));
+    const int hi = min(by1, cvt_i32(posy + dy + 1));
+    const int r0 = min(max(lo - byo, 0), 8), r1 = min(max(hi - byo, 0), 8);
+    // hi > lo first: a column outside the disc has hi = INT_MIN (NaN root)
+    cm[c] = (x >= bx0 && x < bx1 && hi > lo && r1 > r0)
+                ? (((1u << r1) - 1u) & ~((1u << r0) - 1u)) : 0u;
+  }
+}
+
+// ... and its Gaussian column and row factors (splotch_host.cc:596-607), for
+// every column and row of the block: outside the footprint they are not used.
+__device__ __forceinline__ void block_factors(const SplatArgs &a, const Rec &R, int lane, int x0s,
+                                              int y0s, int bxo, int byo, const float *s_tab,
+                                              float (*pre2)[kPad], float (*pre1)[kPad],
+                                              float expfac) {
+  const float posx = R.x - static_cast<float>(x0s), posy = R.y - static_cast<float>(y0s);
+  const float sigma = a.h2sigma * R.r;
+  const float stp = -1.f / (sigma * sigma);
+  float p[16], t1[16], t2[16];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const float dx = static_cast<float>(bxo + k) - posx, dy = static_cast<float>(byo + k) - posy;
+    p[k] = (stp * (dx * dx)) * expfac;
+    p[8 + k] = (stp * dy * dy) * expfac;
+    xop_reads(s_tab, p[k], t1[k], t2[k]);
+    xop_reads(s_tab, p[8 + k], t1[8 + k], t2[8 + k]);
+  }
+  // every read is used here, so that none is moved into a branch of the
+  // selects below
+#pragma unroll
+  for (int k = 0; k < 16; ++k) asm volatile("" : "+v"(t1[k]), "+v"(t2[k]));
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    pre2[k][lane] = xop_value(p[k], t1[k], t2[k]);
+    pre1[k][lane] = xop_value(p[8 + k], t1[8 + k], t2[8 + k]);
+  }
+}
+
 // Work items of a launch: items[0, n), or with device counts (dc: the pass's
 // item total and long-list total) the items after the first min(dc[1], cap)
 // (those go to the producer/consumer kernel).
@@ -1180,40 +1233,51 @@ __global__ __launch_bounds__(kPThreads) void k_splat_pc(SplatArgs a, const uint3
 // Staged long lists.  A long list's pixel chains are serial, and in a
 // lane-per-pixel wave (or a producer/consumer workgroup) the per-particle
 // table work, not the chain, sets their pace.  The staged path moves that
-// work off the chain: k_stage_ops (every CU) writes each staged list's
-// per-pixel operands to HBM, and k_stage_chain streams them back in list
-// order, one wave per list, channel and 16-pixel slice, which applies only
-// the chain's own operations (splotch_host.cc:615, 648-658):
-//   additive  l_c = l_c + t_c                 t_c = a_c * att
-//   ordered   l_c = l_c + ((l_c - q_c) * m1_c) * m2
-//             Taylor branch m1 = a, m2 = att; expm1 branch m1 = expm1(att a),
-//             m2 = 1 (x * 1 == x)
-// A pixel outside a particle's footprint gets t = +0, or m1 = m2 = 0 (l + +-0
-// == l: l starts at +0 and a float sum is -0 only if both terms are -0; for
-// finite records l - q stays finite, so (l - q) * 0 is a zero, and ordered
-// lists are staged only when every q_c of the pass is finite), so every
-// pixel sees the reference's sums and compositing, rounded as it rounds them.
+// work off the chain and drops what a pixel's chain does not need: for every
+// pixel only the entries whose footprint covers it, in list order.
+//   k_stage_rows  (every CU) per batch of 64 entries: each pixel's coverage as
+//                 a 64-bit mask, and each column's longest count of covering
+//                 entries ("rows"), whose scan places the operands
+//   k_stage_ops   (every CU) writes the rows' operands to HBM
+//   k_stage_chain one wave per list, channel and pixel column streams them back
+//                 and applies only the chain's own operations
+//                 (splotch_host.cc:615, 648-658):
+//     additive  l_c = l_c + t_c                 t_c = a_c * att
+//     ordered   l_c = l_c + ((l_c - q_c) * m1_c) * m2
+//               Taylor branch m1 = a, m2 = att; expm1 branch m1 =
+//               expm1(att a), m2 = 1 (x * 1 == x)
+// A pixel with fewer rows than its column gets t = +0, or q = m1 = m2 = 0, in
+// the rest (l + +-0 == l: l starts at +0 and a float sum is -0 only if both
+// terms are -0; l stays finite where every q_c of the pass is finite, and
+// ordered lists are staged only then), so every pixel sees the reference's
+// sums and compositing, rounded as it rounds them.
 //
-// Operand layout: the lists' entries in groups of 4, a list's groups padded
-// with zero operands to a multiple of kStageLoad (the groups of one load of
-// the chain kernel); list i owns groups [cbase[i], cbase[i+1]).  Group g of
-// plane c is 64 float4 (lane = pixel cx * 8 + cy, components = the group's 4
-// entries) at ops + (g * P + c) * 64, with P = 3 planes t_c (additive) or 4
-// (m1_0, m1_1, m1_2, m2; ordered).  Ordered lists also have q_c per entry:
-// qv[(g / kStageQ) * 48 + c * 16 + e] for entry e of the kStageQ groups
-// holding g.  A list's groups are padded to a multiple of kStageLoad.
+// Why rows: a long list of small particles covers a pixel with few of its
+// entries (1M particles at 800^2: 17-40 %), and both the chains' length and
+// the operands' HBM traffic shrink with the coverage.
+//
+// Layout: a stream per list and pixel column (8 pixels); its rows in groups
+// of 4 per batch, group g of plane c being 8 float4 (lane = pixel row,
+// components = the 4 rows) at ops + (c * stride + g) * 8, planes t_c
+// (additive) or m1_0..2, m2, q_0..2 (ordered).  Streams lie list after list,
+// column after column: group offsets gofs from the scan of the counts rows[],
+// both indexed 8 (batches of the lists before) + h * nb + b for batch b of
+// column h of a list of nb batches.  A list of n entries has at most
+// stage_groups(n) groups per column.
 __host__ __device__ constexpr uint32_t stage_groups(uint32_t len) {
-  return (len + 4 * kStageLoad - 1) / (4 * kStageLoad) * kStageLoad;
+  return (len + 31u) / 32u * 8u;
 }
 template <int ADD>
-constexpr uint32_t stage_planes() {
-  return ADD ? 3u : 4u;
+__host__ __device__ constexpr uint32_t stage_planes() {
+  return ADD ? 3u : 7u;
 }
 
-// List offsets of the staged items (one workgroup): cbase (groups of 4
-// entries) and cbat (batches of 64 entries), exclusive, totals at [n].
+// List offsets of the staged items (one workgroup): cbase (groups per column
+// at most) and cbat (batches of 64 entries), exclusive, totals at [n]; and the
+// counts of rows[] of lists [0, n1) and [n1, n).
 __global__ __launch_bounds__(256) void k_stage_base(SplatArgs a, const uint32_t *items,
-                                                    uint32_t n, uint32_t *cbase, uint32_t *cbat,
+                                                    uint32_t n, uint32_t n1, uint32_t *cbase,
+                                                    uint32_t *cbat, uint32_t *nrows,
                                                     const uint32_t *dn) {
   if (dn) n = min(n, *dn);
   __shared__ uint32_t s_g[256], s_b[256];
@@ -1253,32 +1317,20 @@ __global__ __launch_bounds__(256) void k_stage_base(SplatArgs a, const uint32_t 
   if (tid == 0) {
     cbase[n] = s_carry[0];
     cbat[n] = s_carry[1];
+    n1 = min(n1, n);
+    const uint32_t b1 = n1 < n ? cbat[n1] : s_carry[1];
+    nrows[0] = 8u * b1;
+    nrows[1] = 8u * (s_carry[1] - b1);
   }
 }
 
-// Operands of staged lists [i0, i1): their batches of 64 entries (cbat[i0]
-// to cbat[i1]) split evenly over the launch's waves, each wave walking a
-// contiguous run (phase A as the 8x8 splat's, then lane = pixel for the
-// batch's groups).
-template <int ADD>
-__global__ __launch_bounds__(256) void k_stage_ops(SplatArgs a, const uint32_t *items,
-                                                   uint32_t i0, uint32_t i1,
-                                                   const uint32_t *cbase, const uint32_t *cbat,
-                                                   float4 *ops, float *qv, const uint32_t *dn) {
-  constexpr uint32_t P = stage_planes<ADD>();
-  if (dn) i1 = min(i1, *dn);
-  if (i1 <= i0) return;  // the whole grid (device count)
-  // the chains wait for these operands: issue ahead of the 8x8 splat's waves
-  __builtin_amdgcn_s_setprio(3);
-  __shared__ float s_tab[2048];
-  __shared__ uint32_t s_col[4][8][kPad];
-  __shared__ float s_pre2[4][8][kPad];
-  __shared__ float s_pre1[4][8][kPad];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  for (int i = tid; i < 2048; i += 256) s_tab[i] = a.exptab[i];
-  __syncthreads();
+// A wave's run of consecutive batches of staged lists [i0, i1) (their batches
+// split evenly over the launch's waves): visit(i, b, gb) for batch b of list
+// i, the gb-th batch of all staged lists (all wave-uniform).
+template <class F>
+__device__ __forceinline__ void staged_batches(uint32_t i0, uint32_t i1, const uint32_t *cbat,
+                                               uint32_t w, uint32_t nw, F &&visit) {
   const uint32_t first = uniform(cbat[i0]), total = uniform(cbat[i1]) - first;
-  const uint32_t nw = gridDim.x * 4u, w = blockIdx.x * 4u + static_cast<uint32_t>(wave);
   const uint32_t span = (total + nw - 1) / nw;
   uint32_t gb = first + w * span;
   const uint32_t gend = first + min(total, w * span + span);
@@ -1290,104 +1342,180 @@ __global__ __launch_bounds__(256) void k_stage_ops(SplatArgs a, const uint32_t *
     if (uniform(cbat[mid]) <= gb) lo = mid;
     else hi = mid;
   }
-  uint32_t (*col)[kPad] = s_col[wave];
-  float(*pre2)[kPad] = s_pre2[wave];
-  float(*pre1)[kPad] = s_pre1[wave];
-  const float expfac = a.expfac, tl = a.taylorlimit;
-  const int cx = lane >> 3, cy = lane & 7;
   uint32_t i = lo, b = gb - uniform(cbat[lo]);
   for (; gb < gend; ++gb, ++b) {
     while (gb >= uniform(cbat[i + 1])) {  // next list (uniform)
       ++i;
       b = 0;
     }
+    visit(i, b, gb);
+  }
+}
+
+// Pixel coverage of the batches of staged lists [i0, i1): lane = entry builds
+// the 8 column masks of its footprint (tabulate's rule), lane = pixel gathers
+// its bit of the 64 entries.  masks[64 gb + pixel]; rows as described above,
+// counted from list i0 on.
+__global__ __launch_bounds__(256) void k_stage_rows(SplatArgs a, const uint32_t *items,
+                                                    uint32_t i0, uint32_t i1,
+                                                    const uint32_t *cbat, uint64_t *masks,
+                                                    uint32_t *rows, const uint32_t *dn) {
+  if (dn) i1 = min(i1, *dn);
+  if (i1 <= i0) return;  // the whole grid (device count)
+  __builtin_amdgcn_s_setprio(3);
+  // byte [column][entry]: bit r = row r of the block (16-byte rows, padded)
+  __shared__ __align__(16) uint8_t s_cb[4][8][80];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int cx = lane >> 3, cy = lane & 7;
+  uint8_t(*cb)[80] = s_cb[wave];
+  staged_batches(i0, i1, cbat, blockIdx.x * 4u + static_cast<uint32_t>(wave), gridDim.x * 4u,
+                 [&](uint32_t i, uint32_t b, uint32_t gb) {
     const uint32_t u = uniform(items[i]) >> 2;
     const UnitGeom ug = unit_geom_uniform(a, u);
     const uint32_t e0 = uniform(a.bin_off[u]), e1 = uniform(a.bin_off[u + 1]);
     const uint32_t base = e0 + 64u * b;
-    const int nb = static_cast<int>(uniform(min<uint32_t>(64u, e1 - base)));
-    const uint32_t g0 = uniform(cbase[i]) + 16u * b;  // the batch's first group
-    const int ng = static_cast<int>(stage_groups(nb));  // 64 entries: whole loads
-    float va0 = 0.f, va1 = 0.f, va2 = 0.f, vmx = 0.f;
-    float vq[3] = {0.f, 0.f, 0.f};
-    if (lane < nb) {
+    const int bxo = ug.gx * 8, byo = ug.gy * 8;
+    uint32_t cm[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (base + lane < e1) {
       const Rec R = a.recs[a.ent[base + lane]];
-      float ab;
-      tabulate<true>(a, R, lane, ug.x0s, ug.y0s, ug.w, ug.h, ug.gx * 8, ug.gy * 8, s_tab, col, pre2,
-                     pre1, expfac, ab);
-      va0 = -R.e0;
-      va1 = -R.e1;
-      va2 = -R.e2;
-      if (!ADD) {
-        const float gray = ug.grayabsorb;
-        vq[0] = R.e0 / (R.e0 + gray);
-        vq[1] = R.e1 / (R.e1 + gray);
-        vq[2] = R.e2 / (R.e2 + gray);
-        vmx = fmaxf(fabsf(va0), fmaxf(fabsf(va1), fabsf(va2)));
-      }
+      column_masks(a, R, ug.x0s, ug.y0s, ug.w, ug.h, bxo, byo, cm);
     }
-    if (!ADD && lane < ng * 4) {  // q_c per entry (0 past the list), lane = entry
-      float *qd = qv + (g0 / kStageQ + static_cast<uint32_t>(lane) / 16u) * 48u + lane % 16;
-      qd[0] = vq[0];
-      qd[16] = vq[1];
-      qd[32] = vq[2];
-    }
-    wave_sync();
-    float4 *dst = ops + static_cast<size_t>(g0) * P * 64u + lane;
-    for (int q = 0; q < ng; ++q) {
-      float t0[4], t1[4], t2[4], t3[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int k0 = 4 * q + j, k = min(k0, nb - 1);  // uniform; slots past the list are 0
-        const bool in = k0 < nb && ((col[cx][k] >> cy) & 1u);
-        const float at = pre1[cy][k] * pre2[cx][k];
-        const float a0 = lane_f(va0, k), a1 = lane_f(va1, k), a2 = lane_f(va2, k);
-        if (ADD) {
-          const float x0 = a0 * at, x1 = a1 * at, x2 = a2 * at;
-          t0[j] = in ? x0 : 0.f;
-          t1[j] = in ? x1 : 0.f;
-          t2[j] = in ? x2 : 0.f;
-        } else {
-          const bool tay = (lane_f(vmx, k) * at) < tl;
-          const float em0 = xexpm1_bf(s_tab, at * a0, expfac, tl);
-          const float em1 = xexpm1_bf(s_tab, at * a1, expfac, tl);
-          const float em2 = xexpm1_bf(s_tab, at * a2, expfac, tl);
-          t0[j] = in ? (tay ? a0 : em0) : 0.f;
-          t1[j] = in ? (tay ? a1 : em1) : 0.f;
-          t2[j] = in ? (tay ? a2 : em2) : 0.f;
-          t3[j] = in ? (tay ? at : 1.f) : 0.f;
-        }
+    for (int c = 0; c < 8; ++c) cb[c][lane] = static_cast<uint8_t>(cm[c]);
+    wave_sync();
+    // bit cy of the column's 64 bytes: four bytes at a time, their bits 0
+    // gathered by a multiplication (bytes 0..3 to bits 24..27)
+    uint32_t m[2] = {0, 0};
+    const uint4 *src = reinterpret_cast<const uint4 *>(&cb[cx][0]);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const uint4 v = src[q];
+      const uint32_t w4[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const uint32_t t = (w4[k] >> cy) & 0x01010101u;
+        m[q >> 1] |= ((t * 0x01020408u) >> 24) << (16 * (q & 1) + 4 * k);
       }
-      float4 *g = dst + static_cast<size_t>(q) * P * 64u;
-      g[0] = make_float4(t0[0], t0[1], t0[2], t0[3]);
-      g[64] = make_float4(t1[0], t1[1], t1[2], t1[3]);
-      g[128] = make_float4(t2[0], t2[1], t2[2], t2[3]);
-      if (!ADD) g[192] = make_float4(t3[0], t3[1], t3[2], t3[3]);
     }
     wave_sync();
-  }
+    masks[static_cast<size_t>(gb) * 64u + lane] =
+        static_cast<uint64_t>(m[0]) | (static_cast<uint64_t>(m[1]) << 32);
+    int n = __popc(m[0]) + __popc(m[1]);
+#pragma unroll
+    for (int d = 1; d < 8; d <<= 1) n = max(n, __shfl_xor(n, d, 64));
+    const uint32_t nb = (e1 - e0 + 63u) / 64u;
+    if (cy == 0)
+      rows[(uniform(cbat[i]) - uniform(cbat[i0])) * 8u + static_cast<uint32_t>(cx) * nb + b] =
+          static_cast<uint32_t>(n + 3) >> 2;
+  });
 }
 
-// The chains of the staged lists.  A wave applies channel c of list i to a
-// slice of kPix pixels of the block: workgroup (3 i + c) kS + h takes pixels
-// [h kPix, h kPix + kPix).  One load brings kS consecutive groups of a plane
-// (lane part q: group g + q of the slice's pixels, 16 bytes per lane) straight
+// Operands of staged lists [i0, i1): per batch lane = entry tabulates the
+// block's Gaussian factors and the entry's constants, then lane = pixel walks
+// its own covering entries (the bits of its mask), four rows at a time.
+// Bound by its LDS gathers (three or four per row, plus six table lookups for
+// an ordered one); only covering entries are computed and written.
+template <int ADD>
+__global__ __launch_bounds__(256) void k_stage_ops(SplatArgs a, const uint32_t *items,
+                                                   uint32_t i0, uint32_t i1,
+                                                   const uint32_t *cbase, const uint32_t *cbat,
+                                                   const uint64_t *masks, const uint32_t *rows,
+                                                   const uint32_t *gofs, float4 *ops,
+                                                   uint64_t stride, const uint32_t *dn) {
+  if (dn) i1 = min(i1, *dn);
+  if (i1 <= i0) return;  // the whole grid (device count)
+  // the chains wait for these operands: issue ahead of the 8x8 splat's waves
+  __builtin_amdgcn_s_setprio(3);
+  __shared__ float s_tab[2048];
+  __shared__ float s_pre2[4][8][kPad];
+  __shared__ float s_pre1[4][8][kPad];
+  __shared__ float4 s_a[4][64];  // (a0, a1, a2, max |a|)
+  __shared__ float4 s_q[4][ADD ? 1 : 64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  for (int i = tid; i < 2048; i += 256) s_tab[i] = a.exptab[i];
+  __syncthreads();
+  float(*pre2)[kPad] = s_pre2[wave];
+  float(*pre1)[kPad] = s_pre1[wave];
+  float4 *ca = s_a[wave], *cq = s_q[wave];
+  const float expfac = a.expfac, tl = a.taylorlimit;
+  const int cx = lane >> 3, cy = lane & 7;
+  float4 *phase = ops + static_cast<size_t>(uniform(cbase[i0])) * 64u;
+  staged_batches(i0, i1, cbat, blockIdx.x * 4u + static_cast<uint32_t>(wave), gridDim.x * 4u,
+                 [&](uint32_t i, uint32_t b, uint32_t gb) {
+    const uint32_t u = uniform(items[i]) >> 2;
+    const UnitGeom ug = unit_geom_uniform(a, u);
+    const uint32_t e0 = uniform(a.bin_off[u]), e1 = uniform(a.bin_off[u + 1]);
+    const uint32_t base = e0 + 64u * b, nb = (e1 - e0 + 63u) / 64u;
+    uint64_t M = masks[static_cast<size_t>(gb) * 64u + lane];
+    const uint32_t ri = (uniform(cbat[i]) - uniform(cbat[i0])) * 8u +
+                        static_cast<uint32_t>(cx) * nb + b;
+    const uint32_t ng = rows[ri];  // of the lane's column
+    float4 *dst = phase + static_cast<size_t>(gofs[ri]) * 8u + cy;
+    if (base + lane < e1) {
+      const Rec R = a.recs[a.ent[base + lane]];
+      block_factors(a, R, lane, ug.x0s, ug.y0s, ug.gx * 8, ug.gy * 8, s_tab, pre2, pre1, expfac);
+      const float a0 = -R.e0, a1 = -R.e1, a2 = -R.e2;
+      ca[lane] = make_float4(a0, a1, a2, fmaxf(fabsf(a0), fmaxf(fabsf(a1), fabsf(a2))));
+      if (!ADD) {
+        const float gray = ug.grayabsorb;
+        cq[lane] = make_float4(R.e0 / (R.e0 + gray), R.e1 / (R.e1 + gray), R.e2 / (R.e2 + gray),
+                               0.f);
+      }
+    }
+    wave_sync();
+    for (uint32_t j = 0; __ballot(M != 0) != 0; ++j) {
+      float o[stage_planes<ADD>()][4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const bool in = M != 0;
+        const int k = in ? __builtin_ctzll(M) : 0;  // slot 0 holds an entry of the batch
+        M &= M - 1;
+        const float at = pre1[cy][k] * pre2[cx][k];
+        const float4 c = ca[k];
+        if (ADD) {
+          o[0][r] = in ? c.x * at : 0.f;
+          o[1][r] = in ? c.y * at : 0.f;
+          o[2][r] = in ? c.z * at : 0.f;
+        } else {
+          const float4 q = cq[k];
+          const bool tay = (c.w * at) < tl;
+          const float em0 = xexpm1_bf(s_tab, at * c.x, expfac, tl);
+          const float em1 = xexpm1_bf(s_tab, at * c.y, expfac, tl);
+          const float em2 = xexpm1_bf(s_tab, at * c.z, expfac, tl);
+          o[0][r] = in ? (tay ? c.x : em0) : 0.f;
+          o[1][r] = in ? (tay ? c.y : em1) : 0.f;
+          o[2][r] = in ? (tay ? c.z : em2) : 0.f;
+          o[stage_planes<ADD>() - 4][r] = in ? (tay ? at : 1.f) : 0.f;
+          o[stage_planes<ADD>() - 3][r] = in ? q.x : 0.f;
+          o[stage_planes<ADD>() - 2][r] = in ? q.y : 0.f;
+          o[stage_planes<ADD>() - 1][r] = in ? q.z : 0.f;
+        }
+      }
+      if (j < ng) {
+#pragma unroll
+        for (uint32_t c = 0; c < stage_planes<ADD>(); ++c)
+          dst[(c * stride + j) * 8u] = make_float4(o[c][0], o[c][1], o[c][2], o[c][3]);
+      }
+    }
+    wave_sync();
+  });
+}
+
+// The chains of the staged lists.  A wave applies channel c of list i to
+// pixel column h: workgroup (3 i + c) 8 + h.  One load brings 8 consecutive
+// groups of a plane (32 rows, lane = group part * 8 + pixel, 1 KB) straight
 // into a ring of kRing slots in LDS, so the loads in flight hold no registers;
-// lanes [0, kPix) run the chains and read the kS parts of a slot one step
-// ahead.  A chain's wave is bound by its own issue, a dependent operation
-// every 4.2 clocks and about as much per other instruction, so narrower slices
-// (more entries per load) run a list faster: 8 pixels for additive chains, 16
-// for ordered ones (three planes per entry).  With the loads in registers, the
-// copies at the end of each round waited for every load in flight (500k
-// ordered at 512^2, longest list 79.7k entries: 15.3 -> 9.8 ns per entry; 1M
-// additive at 800^2, 165k entries: 5.1 -> 4.5 ns, there bound by HBM traffic).
-template <int ADD> constexpr int chain_groups() { return ADD ? kStageLoad : kStageQ; }
-static_assert(kStageLoad % kStageQ == 0, "chain loads tile the padded groups");
-// slots of the ring (ordered: one of m1_c and one of m2 each)
-template <int ADD> constexpr int chain_ring() { return ADD ? 24 : 16; }
-static_assert(2 * chain_ring<1>() * chain_groups<1>() <= static_cast<int>(kStagePad) &&
-                  2 * chain_ring<0>() * chain_groups<0>() <= static_cast<int>(kStagePad),
-              "the chains' loads past a list stay inside the operands");
+// lanes [0, 8) run the chains and read the 8 parts of a slot one step ahead.
+// A chain's wave is bound by its own issue: a dependent operation every 4.2
+// clocks and about as much per other instruction (18 per 32 rows additive, 35
+// ordered).  With the loads in registers, the copies at the end of each round
+// waited for every load in flight (500k ordered at 512^2, longest list 79.7k
+// entries: 15.3 -> 9.8 ns per entry).
+// slots of the ring (ordered: one each of m1_c, m2 and q_c)
+template <int ADD> constexpr int chain_ring() { return ADD ? 32 : 10; }
+static_assert(2 * chain_ring<1>() * 8 <= static_cast<int>(kStagePad) &&
+                  2 * chain_ring<0>() * 8 <= static_cast<int>(kStagePad),
+              "the chains' loads past a stream stay inside the operands");
 
 // LDS byte address of a shared object.
 __device__ __forceinline__ uint32_t lds_address(const void *p) {
@@ -1395,16 +1523,10 @@ __device__ __forceinline__ uint32_t lds_address(const void *p) {
       (const __attribute__((address_space(3))) void *)p));
 }
 
-// 16 (load_lds4: 4) bytes per lane from base + off into LDS at byte address lds +
-// 16 (4) lane.  Completion counts in vmcnt; the caller waits for it.
+// 16 bytes per lane from base + off into LDS at byte address lds + 16 lane.
+// Completion counts in vmcnt; the caller waits for it.
 __device__ __forceinline__ void load_lds16(uint32_t lds, const void *base, uint32_t off) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-               :
-               : "s"(lds), "v"(off), "s"(base)
-               : "memory", "m0");
-}
-__device__ __forceinline__ void load_lds4(uint32_t lds, const void *base, uint32_t off) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
                :
                : "s"(lds), "v"(off), "s"(base)
                : "memory", "m0");
@@ -1412,130 +1534,112 @@ __device__ __forceinline__ void load_lds4(uint32_t lds, const void *base, uint32
 
 template <int ADD>
 __global__ __launch_bounds__(64) void k_stage_chain(
-    SplatArgs a, const uint32_t *items, uint32_t i0, const uint32_t *cbase,
-    const float4 *__restrict__ ops, const float *__restrict__ qv, const uint32_t *dn) {
-  constexpr int kS = chain_groups<ADD>(), kPix = 64 / kS;
-  constexpr uint32_t P = stage_planes<ADD>();
+    SplatArgs a, const uint32_t *items, uint32_t i0, const uint32_t *cbase, const uint32_t *cbat,
+    const uint32_t *rows, const uint32_t *gofs, const float4 *ops, uint64_t stride,
+    const uint32_t *dn) {
+  constexpr int kS = 8;  // groups per load
   constexpr int kRing = chain_ring<ADD>();
-  constexpr int kPl = ADD ? 1 : 2;          // planes per slot
-  constexpr int kQs = ADD ? 1 : kRing / 4;  // q_c: blocks of 4 steps
-  static_assert(kRing % 4 == 0, "whole blocks of q_c per ring");
+  constexpr int kPl = ADD ? 1 : 3;  // planes per slot
+  static_assert(kPl * (kRing - 2) < 64, "vmcnt holds the loads in flight");
   typedef float v4f __attribute__((ext_vector_type(4)));
-  // one LDS block at address 0
-  struct Lds {
-    v4f op[kRing][kPl][64];
-    float q[kQs][64];
-  };
-  __shared__ Lds L;
-  const uint32_t i = i0 + blockIdx.x / (3u * kS);
+  __shared__ v4f ring[kRing][kPl][64];
+  const uint32_t i = i0 + blockIdx.x / 24u;
   if (dn && i >= *dn) return;  // past the device count (uniform per workgroup)
-  const uint32_t r3 = blockIdx.x % (3u * kS);
-  const int c = static_cast<int>(r3 / kS), h = static_cast<int>(r3 % kS);
-  const int lane = threadIdx.x, qo = lane / kPix, pl = lane % kPix;
-  const int px = h * kPix + pl;  // pixel cx * 8 + cy
+  const uint32_t r3 = blockIdx.x % 24u;
+  const int c = static_cast<int>(r3 >> 3), h = static_cast<int>(r3 & 7u);
+  const int lane = threadIdx.x, pl = lane & 7;
   const uint64_t t_start = a.trace ? __builtin_amdgcn_s_memrealtime() : 0;
   __builtin_amdgcn_s_setprio(3);
   const uint32_t u = uniform(items[i]) >> 2;
   const UnitGeom ug = unit_geom_uniform(a, u);
   const uint32_t len = uniform(a.bin_off[u + 1]) - uniform(a.bin_off[u]);
-  const uint32_t G = stage_groups(len);  // the list is not empty
-  const uint32_t gb0 = uniform(cbase[i]);
-  const int cx = px >> 3, cy = px & 7;
-  const int lx = ug.gx * 8 + cx, ly = ug.gy * 8 + cy;
-  const bool pix_in = lane < kPix && lx < min(ug.gx * 8 + 8, ug.w) &&
-                      ly < min(ug.gy * 8 + 8, ug.h);
+  // the stream: its first group and number of groups (the list is not empty)
+  const uint32_t nb = (len + 63u) / 64u;
+  const uint32_t r0 = (uniform(cbat[i]) - uniform(cbat[i0])) * 8u + static_cast<uint32_t>(h) * nb;
+  const uint32_t g0 = uniform(gofs[r0]);
+  const uint32_t G = uniform(gofs[r0 + nb - 1u]) + uniform(rows[r0 + nb - 1u]) - g0;
+  const int lx = ug.gx * 8 + h, ly = ug.gy * 8 + pl;
+  const bool pix_in = lane < 8 && lx < min(ug.gx * 8 + 8, ug.w) && ly < min(ug.gy * 8 + 8, ug.h);
   float *d = ug.pic + (static_cast<int64_t>(ug.x0s + lx) * ug.yres + (ug.y0s + ly)) * 3 + c;
   float l = 0.f;
   if (ug.accumulate == 2 && pix_in) l = *d;  // a later chunk: continue the chain
   // l is in its register before the operand loads are issued
   asm volatile("" : "+v"(l));
-  // A load brings groups g .. g + kS - 1 of plane c for the slice's pixels:
-  // a wave-uniform base per plane, advanced by the scalar unit, and one lane
-  // offset (part qo: group g + qo).  Loads run up to 2 kRing steps past the
-  // list's end (kStagePad groups of slack behind the last list; never applied).
-  constexpr uint32_t kStep = kS * P * 1024u;  // bytes per load
-  const char *pw = reinterpret_cast<const char *>(ops + static_cast<size_t>(gb0) * P * 64u) + 3072u;
-  const char *pm = pw - 3072u + static_cast<uint32_t>(c) * 1024u;
-  // q_c of four loads (kStageQ groups each) per q load: lane = entry
-  const char *pq = reinterpret_cast<const char *>(qv + static_cast<size_t>(gb0 / kStageQ) * 48u +
-                                                  static_cast<size_t>(c) * 16u);
-  const uint32_t vo = (static_cast<uint32_t>(qo) * P * 64u + static_cast<uint32_t>(px)) * 16u;
-  const uint32_t vq = static_cast<uint32_t>(lane / 16) * 192u + static_cast<uint32_t>(lane % 16) * 4u;
-  const uint32_t lop = lds_address(&L.op[0][0][0]), lq = lds_address(&L.q[0][0]);
-  auto refill_q = [&](int b) {  // q_c of slots 4 b .. 4 b + 3
-    load_lds4(lq + static_cast<uint32_t>(b) * 256u, pq, vq);
-    pq += 4u * 192u;
-  };
+  // A load: a wave-uniform base per plane, advanced by the scalar unit.  Loads
+  // run up to 2 kRing steps past the stream's end (kStagePad groups of slack
+  // behind the planes; never applied).
+  const char *pm = reinterpret_cast<const char *>(
+      ops + (static_cast<size_t>(uniform(cbase[i0])) * 8u + g0) * 8u);
+  const char *pw = pm + 3u * stride * 128u, *pq = pw + static_cast<uint64_t>(c + 1) * stride * 128u;
+  pm += static_cast<uint64_t>(c) * stride * 128u;
+  const uint32_t vo = static_cast<uint32_t>(lane) * 16u;
+  const uint32_t lds = lds_address(&ring[0][0][0]);
   auto refill = [&](int r) {  // slot r: the next load
-    load_lds16(lop + static_cast<uint32_t>(r * kPl) * 1024u, pm, vo);
-    pm += kStep;
+    const uint32_t at = lds + static_cast<uint32_t>(r * kPl) * 1024u;
+    load_lds16(at, pm, vo);
+    pm += 1024;
     if (!ADD) {
-      load_lds16(lop + static_cast<uint32_t>(r * kPl + 1) * 1024u, pw, vo);
-      pw += kStep;
+      load_lds16(at + 1024u, pw, vo);
+      load_lds16(at + 2048u, pq, vo);
+      pw += 1024;
+      pq += 1024;
     }
   };
-  struct Step {  // one load's 4 kS entries: m1_c (or t_c), m2 and q_c
+  struct Step {  // one load's 32 rows: m1_c (or t_c), m2 and q_c
     v4f m[kS], w[ADD ? 1 : kS], q[ADD ? 1 : kS];
   };
   auto read = [&](int r) {  // slot r, once its loads have landed
-    // Loads complete in order.  Behind slot r's load at least those of the
-    // kRing - 2 slots refilled since are in flight; behind its q_c, loaded
-    // with the last slot of its four, those of kRing - 4.
-    asm volatile("s_waitcnt vmcnt(%0)" : : "n"(kPl * (kRing - (ADD ? 2 : 4))) : "memory");
+    // loads complete in order, and behind slot r's at least those of kRing - 2
+    // other slots have been issued
+    asm volatile("s_waitcnt vmcnt(%0)" : : "n"(kPl * (kRing - 2)) : "memory");
     Step st;
 #pragma unroll
     for (int k = 0; k < kS; ++k) {
-      st.m[k] = L.op[r][0][pl + k * kPix];
+      st.m[k] = ring[r][0][pl + k * 8];
       if (!ADD) {
-        st.w[k] = L.op[r][kPl - 1][pl + k * kPix];
-        st.q[k] = *reinterpret_cast<const v4f *>(&L.q[r / 4][(r % 4) * 16 + 4 * k]);
+        st.w[k] = ring[r][kPl - 2][pl + k * 8];
+        st.q[k] = ring[r][kPl - 1][pl + k * 8];
       }
     }
     asm volatile("" ::: "memory");
     return st;
   };
-  auto apply = [&](const Step &st) {
-#pragma unroll
-    for (int k = 0; k < kS; ++k) {  // load part k: entries 4k .. 4k + 3
-      if (ADD) {
-        l = l + st.m[k].x;
-        l = l + st.m[k].y;
-        l = l + st.m[k].z;
-        l = l + st.m[k].w;
-      } else {
-        l = l + ((l - st.q[k].x) * st.m[k].x) * st.w[k].x;
-        l = l + ((l - st.q[k].y) * st.m[k].y) * st.w[k].y;
-        l = l + ((l - st.q[k].z) * st.m[k].z) * st.w[k].z;
-        l = l + ((l - st.q[k].w) * st.m[k].w) * st.w[k].w;
-      }
+  auto apply = [&](const Step &st, int k) {  // load part k: rows 4k .. 4k + 3
+    if (ADD) {
+      l = l + st.m[k].x;
+      l = l + st.m[k].y;
+      l = l + st.m[k].z;
+      l = l + st.m[k].w;
+    } else {
+      l = l + ((l - st.q[k].x) * st.m[k].x) * st.w[k].x;
+      l = l + ((l - st.q[k].y) * st.m[k].y) * st.w[k].y;
+      l = l + ((l - st.q[k].z) * st.m[k].z) * st.w[k].z;
+      l = l + ((l - st.q[k].w) * st.m[k].w) * st.w[k].w;
     }
   };
-  if (!ADD)
-#pragma unroll
-    for (int b = 0; b < kQs; ++b) refill_q(b);
 #pragma unroll
   for (int r = 0; r < kRing; ++r) refill(r);  // issued in the order they are consumed
   Step cur = read(0);
   // Software pipeline: step r starts the reads of slot r + 1, then applies the
-  // entries of slot r (read a step earlier: one wait for all of them, as they
-  // return in order), and then refills slot r.  Whole rounds first (every step
-  // applies: one straight-line block per round), then the last, partial round.
+  // rows of slot r (read a step earlier: one wait for all of them, as they
+  // return in order), and then refills slot r.  Whole rounds first (every
+  // group applies: one straight-line block per round), then the last,
+  // partial round.
   auto round = [&](uint32_t g, bool whole) {
 #pragma unroll
     for (int r = 0; r < kRing; ++r) {
-      const int rn = (r + 1) % kRing;
-      Step nxt = read(rn);
+      const uint32_t gr = g + static_cast<uint32_t>(r * kS);
+      if (!whole && gr >= G) break;
+      Step nxt = read((r + 1) % kRing);
       __builtin_amdgcn_sched_barrier(0);
-      if (whole || g + r * kS < G) {
-        asm volatile("" : "+v"(l) : "v"(ADD ? cur.m[kS - 1].w : cur.q[ADD ? 0 : kS - 1].w));
-        apply(cur);
-      }
+      asm volatile("" : "+v"(l) : "v"(ADD ? cur.m[kS - 1].w : cur.q[ADD ? 0 : kS - 1].w));
+#pragma unroll
+      for (int k = 0; k < kS; ++k)
+        if (whole || gr + static_cast<uint32_t>(k) < G) apply(cur, k);
       cur = nxt;
-      // the sums stay ahead of the refill of their slot (and of the q_c of
-      // the four slots that end with it)
+      // the sums stay ahead of the refill of their slot
       asm volatile("" : "+v"(l) : : "memory");
       __builtin_amdgcn_sched_barrier(0);
-      if (!ADD && r % 4 == 3) refill_q(r / 4);
       refill(r);
     }
   };
@@ -1592,20 +1696,42 @@ __global__ __launch_bounds__(256) void k_items_count(SplatArgs a, uint32_t nunit
                                                      uint32_t split, uint32_t *cnt,
                                                      uint32_t *heavy_cnt, uint32_t *stage_cnt,
                                                      uint32_t *stage_grp, uint32_t *lmax) {
+  // the block's counts in LDS, then one atomic per count (thousands of long
+  // lists would queue up on the same few words)
+  __shared__ uint32_t s_cnt[kStageLevels], s_grp[kStageLevels], s_heavy, s_lmax;
+  const int tid = threadIdx.x;
+  if (tid < kStageLevels) s_cnt[tid] = s_grp[tid] = 0;
+  if (tid == 0) s_heavy = s_lmax = 0;
+  __syncthreads();
   for (int64_t u = gtid(); u < nunits; u += gstride()) {
     uint32_t len;
     const uint32_t k = unit_items(a, static_cast<uint32_t>(u), ordered, split, len);
     cnt[u] = k;
-    if (heavy_cnt && k > 0 && len >= heavy_len_of(a)) atomicAdd(heavy_cnt, k);
+    if (k == 0) continue;
+    if (len >= heavy_len_of(a)) atomicAdd(&s_heavy, k);
     const uint32_t sl = stage_len_of(a);
-    if (stage_cnt && k > 0 && len >= sl) {  // counts per level of sl
-      for (int j = 0; j < kStageLevels; ++j) {
-        if (static_cast<uint64_t>(len) < stage_level(sl, j)) break;
-        atomicAdd(stage_cnt + j, 1u);
-        atomicAdd(stage_grp + j, stage_groups(len));
-      }
+    if (len >= sl) {  // counts per level of sl
+      int j = 0;
+      while (j < kStageLevels - 1 && static_cast<uint64_t>(len) >= stage_level(sl, j + 1)) ++j;
+      atomicAdd(&s_cnt[j], 1u);
+      atomicAdd(&s_grp[j], stage_groups(len));
     }
-    if (lmax && k > 0) atomicMax(lmax, len);
+    atomicMax(&s_lmax, len);
+  }
+  __syncthreads();
+  if (tid == 0) {
+    if (heavy_cnt && s_heavy) atomicAdd(heavy_cnt, s_heavy);
+    if (lmax && s_lmax) atomicMax(lmax, s_lmax);
+    // lists whose top level is j, to lists from level j on
+    for (int j = kStageLevels - 2; j >= 0; --j) {
+      s_cnt[j] += s_cnt[j + 1];
+      s_grp[j] += s_grp[j + 1];
+    }
+  }
+  __syncthreads();
+  if (stage_cnt && tid < kStageLevels && s_cnt[tid]) {
+    atomicAdd(stage_cnt + tid, s_cnt[tid]);
+    atomicAdd(stage_grp + tid, s_grp[tid]);
   }
 }
 
@@ -1654,24 +1780,25 @@ void launch_items_emit(const uint32_t *bin_off, uint32_t nunits, const SplatArgs
   hip_check(hipGetLastError(), "k_items_emit launch");
 }
 
+uint64_t stage_stride(uint64_t groups) { return 8u * groups + kStagePad; }
+
 uint64_t stage_floats(bool additive, uint64_t groups) {
-  return (groups + kStagePad) * (additive ? 3u : 4u) * 256u;
+  return (additive ? stage_planes<1>() : stage_planes<0>()) * stage_stride(groups) * 32u;
 }
 
-uint64_t stage_q_floats(bool additive, uint64_t groups) {
-  return additive ? 0 : (groups + kStagePad) / kStageQ * 48u;
-}
+uint64_t stage_batches(uint64_t groups, uint32_t n) { return groups / 16u + n; }
 
-void launch_stage_base(const uint32_t *items, uint32_t n, uint32_t *cbase, uint32_t *cbat,
-                       const SplatArgs &a, hipStream_t s, const uint32_t *dn) {
+void launch_stage_base(const uint32_t *items, uint32_t n, uint32_t n1, uint32_t *cbase,
+                       uint32_t *cbat, uint32_t *nrows, const SplatArgs &a, hipStream_t s,
+                       const uint32_t *dn) {
   if (n == 0) return;
-  k_stage_base<<<1, 256, 0, s>>>(a, items, n, cbase, cbat, dn);
+  k_stage_base<<<1, 256, 0, s>>>(a, items, n, n1, cbase, cbat, nrows, dn);
   hip_check(hipGetLastError(), "k_stage_base launch");
 }
 
 // Workgroups of kernel k (256 threads) resident at once on the current device.
 unsigned resident_grid(const void *k, int slot) {
-  static unsigned cache[2][16] = {};
+  static unsigned cache[3][16] = {};
   int dev = 0;
   hip_check(hipGetDevice(&dev), "get device");
   unsigned &r = cache[slot][dev & 15];
@@ -1684,43 +1811,64 @@ unsigned resident_grid(const void *k, int slot) {
   return r;
 }
 
-void launch_stage_ops(bool additive, const uint32_t *items, uint32_t i0, uint32_t i1,
-                      uint64_t groups, const uint32_t *cbase, const uint32_t *cbat, float4 *ops,
-                      float *qv, const SplatArgs &a, hipStream_t s, const uint32_t *dn) {
+// Grid of a kernel that walks the staged batches: at most `batches`; about
+// `per` per wave when there are many, in one round of resident workgroups (a
+// second round would queue behind the 8x8 splat's workgroups, and the chains
+// wait for all of them).
+static unsigned stage_grid(const void *k, int slot, uint64_t batches, unsigned per) {
+  return std::max(1u, static_cast<unsigned>(std::min<uint64_t>(
+                          resident_grid(k, slot), (batches + 4 * per - 1) / (4 * per))));
+}
+
+void launch_stage_rows(const uint32_t *items, uint32_t i0, uint32_t i1, uint64_t batches,
+                       const uint32_t *cbat, uint64_t *masks, uint32_t *rows, const SplatArgs &a,
+                       hipStream_t s, const uint32_t *dn) {
   if (i1 <= i0) return;
-  // batches: at most groups / 16 + lists; about four per wave when there are
-  // many, in one round of resident workgroups (a second round would queue
-  // behind the 8x8 splat's workgroups, and the chains wait for all of them)
-  const uint64_t nbat = groups / 16 + (i1 - i0);
-  const unsigned res = additive ? resident_grid(reinterpret_cast<const void *>(k_stage_ops<1>), 1)
-                                : resident_grid(reinterpret_cast<const void *>(k_stage_ops<0>), 0);
-  const unsigned grid =
-      std::max(1u, static_cast<unsigned>(std::min<uint64_t>(res, (nbat + 15) / 16)));
-  if (additive) k_stage_ops<1><<<grid, 256, 0, s>>>(a, items, i0, i1, cbase, cbat, ops, qv, dn);
-  else k_stage_ops<0><<<grid, 256, 0, s>>>(a, items, i0, i1, cbase, cbat, ops, qv, dn);
+  const unsigned grid = stage_grid(reinterpret_cast<const void *>(k_stage_rows), 2, batches, 4);
+  k_stage_rows<<<grid, 256, 0, s>>>(a, items, i0, i1, cbat, masks, rows, dn);
+  hip_check(hipGetLastError(), "k_stage_rows launch");
+}
+
+void launch_stage_ops(bool additive, const uint32_t *items, uint32_t i0, uint32_t i1,
+                      uint64_t batches, const uint32_t *cbase, const uint32_t *cbat,
+                      const uint64_t *masks, const uint32_t *rows, const uint32_t *gofs,
+                      float4 *ops, uint64_t stride, const SplatArgs &a, hipStream_t s,
+                      const uint32_t *dn) {
+  if (i1 <= i0) return;
+  const void *k = additive ? reinterpret_cast<const void *>(k_stage_ops<1>)
+                           : reinterpret_cast<const void *>(k_stage_ops<0>);
+  const unsigned grid = stage_grid(k, additive ? 1 : 0, batches, 4);
+  if (additive)
+    k_stage_ops<1><<<grid, 256, 0, s>>>(a, items, i0, i1, cbase, cbat, masks, rows, gofs, ops,
+                                        stride, dn);
+  else
+    k_stage_ops<0><<<grid, 256, 0, s>>>(a, items, i0, i1, cbase, cbat, masks, rows, gofs, ops,
+                                        stride, dn);
   hip_check(hipGetLastError(), "k_stage_ops launch");
 }
 
 void launch_stage_chain(bool additive, const uint32_t *items, uint32_t i0, uint32_t i1,
-                        const uint32_t *cbase, const float4 *ops, const float *qv,
+                        const uint32_t *cbase, const uint32_t *cbat, const uint32_t *rows,
+                        const uint32_t *gofs, const float4 *ops, uint64_t stride,
                         const SplatArgs &a, hipStream_t s, const uint32_t *dn) {
   if (i1 <= i0) return;
-  const unsigned grid = 3u * static_cast<unsigned>(additive ? chain_groups<1>() : chain_groups<0>()) *
-                        (i1 - i0);
-  if (additive) k_stage_chain<1><<<grid, 64, 0, s>>>(a, items, i0, cbase, ops, qv, dn);
-  else k_stage_chain<0><<<grid, 64, 0, s>>>(a, items, i0, cbase, ops, qv, dn);
+  const unsigned grid = 24u * (i1 - i0);  // channels x pixel columns
+  if (additive)
+    k_stage_chain<1><<<grid, 64, 0, s>>>(a, items, i0, cbase, cbat, rows, gofs, ops, stride, dn);
+  else
+    k_stage_chain<0><<<grid, 64, 0, s>>>(a, items, i0, cbase, cbat, rows, gofs, ops, stride, dn);
   hip_check(hipGetLastError(), "k_stage_chain launch");
 }
 
 __global__ void k_partition(PartitionArgs a, uint32_t *out) {
   uint32_t ns = 0;
   if (a.len0 != 0xffffffffu) {
-    const int j = stage_rule(a.len0, a.ordered_auto != 0, *a.lmax, *a.etot, a.span, a.ratio,
-                             a.crit);
-    if (j >= 0) {
-      ns = a.stage_cnt[j];
-      if (ns > a.ns_cap || a.stage_grp[j] > a.groups_cap) ns = 0;
-    }
+    int j = stage_rule(a.len0, a.mode, *a.lmax, *a.etot);
+    for (; j >= 0 && j < kStageLevels; ++j)
+      if (a.stage_cnt[j] <= a.ns_cap && a.stage_grp[j] <= a.groups_cap) {
+        ns = a.stage_cnt[j];
+        break;
+      }
   }
   const uint32_t nh = *a.heavy_cnt;
   const uint32_t npc = (a.heavy_max == 0 || nh <= ns) ? 0u : min(nh - ns, a.heavy_max);
