@@ -357,6 +357,7 @@ struct NormArgs {
   const float *r;
   const uint8_t *type;
   int32_t ntypes, norm_int;
+  int32_t vector;  // some type has a vector colour (set by launch_normalize)
   int32_t flags[kMaxTypes][4];
   int32_t ovr_set[kMaxTypes][4];
   float ovr[kMaxTypes][4];

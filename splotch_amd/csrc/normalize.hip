@@ -63,9 +63,52 @@ __device__ __forceinline__ uint32_t wave_max(uint32_t v) {
   return v;
 }
 
-// Pass 1: transforms in place and reduces the extremes of NT types.
-template <int NT>
-__global__ __launch_bounds__(256) void k_norm_reduce(NormArgs a, uint32_t *keys) {
+// W consecutive values at p + m, of n: one 16-byte vector (4 type bytes) where
+// W = 4 (aligned fields) and four are left; those past the end are not touched.
+template <int W, class T, class V>
+__device__ __forceinline__ void load_w(const T *p, int64_t m, int64_t n, T (&v)[W]) {
+  if constexpr (W == 4) {
+    if (m + 4 <= n) {
+      const V w = *reinterpret_cast<const V *>(p + m);
+      v[0] = w.x;
+      v[1] = w.y;
+      v[2] = w.z;
+      v[3] = w.w;
+      return;
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < W; ++j)
+    if (m + j < n) v[j] = p[m + j];
+}
+template <int W>
+__device__ __forceinline__ void store_w(float *p, int64_t m, int64_t n, const float (&v)[W]) {
+  if constexpr (W == 4) {
+    if (m + 4 <= n) {
+      *reinterpret_cast<float4 *>(p + m) = make_float4(v[0], v[1], v[2], v[3]);
+      return;
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < W; ++j)
+    if (m + j < n) p[m + j] = v[j];
+}
+
+constexpr int kNormThreads = 512;
+// Loads per thread, field and step (all issued before the first is used): two
+// vectors of four particles, or four single particles.
+template <int W> constexpr int loads() { return W == 4 ? 2 : 4; }
+
+// Pass 1: transforms in place and reduces the extremes of NT types.  Both
+// passes are bound by HBM (13 B, then 17 B per particle); a thread takes four
+// consecutive particles per 16-byte load.  16M particles of two types: 122 ->
+// 97 us without logs (4.9 TB/s), 198 -> 187 with, 253 -> 168 with a vector
+// colour, against a float per load
+// and four loads in flight per thread and field.
+// GEN: some type has a log10, an asinh or a vector colour (else that code, and
+// its registers, are left out).
+template <int NT, int W, bool GEN>
+__global__ __launch_bounds__(kNormThreads) void k_norm_reduce(NormArgs a, uint32_t *keys) {
   __shared__ int32_t s_flags[NT][4];
   if (threadIdx.x < NT * 4) s_flags[threadIdx.x / 4][threadIdx.x % 4] =
       a.flags[threadIdx.x / 4][threadIdx.x % 4];
@@ -75,105 +118,120 @@ __global__ __launch_bounds__(256) void k_norm_reduce(NormArgs a, uint32_t *keys)
   for (int t = 0; t < NT; ++t)
 #pragma unroll
     for (int q = 0; q < K_N; ++q) k[t][q] = (q % 2 == 0) ? 0xffffffffu : 0u;
-  // four particles per step, their loads issued before any store
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * 256;
-  for (int64_t m0 = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; m0 < a.n;
-       m0 += 4 * stride) {
-    int tv[4];
-    float Iv[4], ev[4], rv[4];
+  constexpr int kV = loads<W>();
+  const int64_t stride = static_cast<int64_t>(gridDim.x) * kNormThreads * W;
+  for (int64_t m0 = (static_cast<int64_t>(blockIdx.x) * kNormThreads + threadIdx.x) * W; m0 < a.n;
+       m0 += kV * stride) {
+    uint8_t tv[kV][W] = {};
+    float Iv[kV][W], ev[kV][W], rv[kV][W], gv[GEN ? kV : 1][W], bv[GEN ? kV : 1][W];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int64_t m = m0 + j * stride;
-      tv[j] = NT;
+    for (int q = 0; q < kV; ++q) {
+      const int64_t m = m0 + q * stride;
       if (m < a.n) {
-        tv[j] = a.type ? a.type[m] : 0;
-        Iv[j] = a.I[m];
-        ev[j] = a.er[m];
-        rv[j] = a.r[m];
+        if (GEN && a.vector) {
+          load_w<W, float, float4>(a.eg, m, a.n, gv[GEN ? q : 0]);
+          load_w<W, float, float4>(a.eb, m, a.n, bv[GEN ? q : 0]);
+        }
+        if (a.type) load_w<W, uint8_t, uchar4>(a.type, m, a.n, tv[q]);
+        load_w<W, float, float4>(a.I, m, a.n, Iv[q]);
+        load_w<W, float, float4>(a.er, m, a.n, ev[q]);
+        load_w<W, float, float4>(a.r, m, a.n, rv[q]);
       }
     }
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int64_t m = m0 + j * stride;
-      const int t = tv[j];
-      if (t >= NT) continue;  // past the end, or a type beyond ptypes (not rendered)
-      const int f_il = s_flags[t][0], f_cl = s_flags[t][1], f_ca = s_flags[t][2],
-                f_cv = s_flags[t][3];
-      // extremes of this particle (min keys start high, max keys low)
-      uint32_t cmin = 0xffffffffu, cmax = 0u, imin = 0xffffffffu, imax = 0u;
-      const float r = rv[j];
-      if (r == r) {
-        const uint32_t kr = fkey(r);
+    for (int q = 0; q < kV; ++q) {
+      const int64_t mq = m0 + q * stride;
+      bool put_I = false, put_e = false, put_v = false;
+#pragma unroll
+      for (int j = 0; j < W; ++j) {
+        const int64_t m = mq + j;
+        const int t = m < a.n ? tv[q][j] : NT;
+        if (t >= NT) continue;  // past the end, or a type beyond ptypes (not rendered)
+        const int f_il = GEN ? s_flags[t][0] : 0, f_cl = GEN ? s_flags[t][1] : 0,
+                  f_ca = GEN ? s_flags[t][2] : 0, f_cv = GEN ? s_flags[t][3] : 0;
+        // extremes of this particle (min keys start high, max keys low)
+        uint32_t cmin = 0xffffffffu, cmax = 0u, imin = 0xffffffffu, imax = 0u;
+        const float r = rv[q][j];
+        if (r == r) {
+          const uint32_t kr = fkey(r);
+#pragma unroll
+          for (int u = 0; u < NT; ++u)
+            if (u == t) {
+              k[u][K_RMIN] = min(k[u][K_RMIN], kr);
+              k[u][K_RMAX] = max(k[u][K_RMAX], kr);
+            }
+        }
+        float I = Iv[q][j];
+        bool icol = true;
+        if (f_il) {
+          if (I > 0) {
+            I = log10_f(I);
+          } else {
+            I = -38.f;
+            icol = false;
+          }
+          Iv[q][j] = I;
+          put_I = true;
+        }
+        if (icol && I == I) imin = imax = fkey(I);
+        float e = ev[q][j];
+        bool ccol = true;
+        if (f_cl) {
+          if (e > 0) {
+            e = log10_f(e);
+          } else {
+            e = -38.f;
+            ccol = false;
+          }
+        } else if (f_ca) {
+          e = asinh_f(e);
+        }
+        if (f_cl || f_ca) {
+          ev[q][j] = e;
+          put_e = true;
+        }
+        if (ccol && e == e) cmin = cmax = fkey(e);
+        if (f_cv) {
+          float &g = gv[GEN ? q : 0][j], &b = bv[GEN ? q : 0][j];
+          if (f_cl) {
+            g = log10_f(g);
+            b = log10_f(b);
+          }
+          if (f_ca) {
+            g = asinh_f(g);
+            b = asinh_f(b);
+          }
+          put_v |= f_cl || f_ca;
+          if (g == g) {
+            cmin = min(cmin, fkey(g));
+            cmax = max(cmax, fkey(g));
+          }
+          if (b == b) {
+            cmin = min(cmin, fkey(b));
+            cmax = max(cmax, fkey(b));
+          }
+        }
 #pragma unroll
         for (int u = 0; u < NT; ++u)
           if (u == t) {
-            k[u][K_RMIN] = min(k[u][K_RMIN], kr);
-            k[u][K_RMAX] = max(k[u][K_RMAX], kr);
+            k[u][K_CMIN] = min(k[u][K_CMIN], cmin);
+            k[u][K_CMAX] = max(k[u][K_CMAX], cmax);
+            k[u][K_IMIN] = min(k[u][K_IMIN], imin);
+            k[u][K_IMAX] = max(k[u][K_IMAX], imax);
           }
       }
-      float I = Iv[j];
-      bool icol = true;
-      if (f_il) {
-        if (I > 0) {
-          I = log10_f(I);
-        } else {
-          I = -38.f;
-          icol = false;
-        }
-        a.I[m] = I;
+      // unchanged particles of the four get their own value back
+      if (put_I) store_w<W>(a.I, mq, a.n, Iv[q]);
+      if (put_e) store_w<W>(a.er, mq, a.n, ev[q]);
+      if (put_v) {
+        store_w<W>(a.eg, mq, a.n, gv[GEN ? q : 0]);
+        store_w<W>(a.eb, mq, a.n, bv[GEN ? q : 0]);
       }
-      if (icol && I == I) imin = imax = fkey(I);
-      float e = ev[j];
-      bool ccol = true;
-      if (f_cl) {
-        if (e > 0) {
-          e = log10_f(e);
-        } else {
-          e = -38.f;
-          ccol = false;
-        }
-        a.er[m] = e;
-      } else if (f_ca) {
-        e = asinh_f(e);
-        a.er[m] = e;
-      }
-      if (ccol && e == e) cmin = cmax = fkey(e);
-      if (f_cv) {
-        float g = a.eg[m], b = a.eb[m];
-        if (f_cl) {
-          g = log10_f(g);
-          b = log10_f(b);
-        }
-        if (f_ca) {
-          g = asinh_f(g);
-          b = asinh_f(b);
-        }
-        if (f_cl || f_ca) {
-          a.eg[m] = g;
-          a.eb[m] = b;
-        }
-        if (g == g) {
-          cmin = min(cmin, fkey(g));
-          cmax = max(cmax, fkey(g));
-        }
-        if (b == b) {
-          cmin = min(cmin, fkey(b));
-          cmax = max(cmax, fkey(b));
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < NT; ++u)
-        if (u == t) {
-          k[u][K_CMIN] = min(k[u][K_CMIN], cmin);
-          k[u][K_CMAX] = max(k[u][K_CMAX], cmax);
-          k[u][K_IMIN] = min(k[u][K_IMIN], imin);
-          k[u][K_IMAX] = max(k[u][K_IMAX], imax);
-        }
     }
   }
   // per wave by shuffles, per block through LDS, then one atomic per block
   // and value (thousands of atomics on a few addresses would serialize)
-  __shared__ uint32_t s_k[4][NT * K_N];
+  __shared__ uint32_t s_k[kNormThreads / 64][NT * K_N];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
   for (int t = 0; t < NT; ++t)
@@ -187,7 +245,7 @@ __global__ __launch_bounds__(256) void k_norm_reduce(NormArgs a, uint32_t *keys)
   if (i < NT * K_N) {
     const bool is_min = (i % K_N) % 2 == 0;
     uint32_t v = s_k[0][i];
-    for (int w = 1; w < 4; ++w) v = is_min ? min(v, s_k[w][i]) : max(v, s_k[w][i]);
+    for (int w = 1; w < kNormThreads / 64; ++w) v = is_min ? min(v, s_k[w][i]) : max(v, s_k[w][i]);
     if (is_min) {
       if (v != 0xffffffffu) atomicMin(&keys[i], v);
     } else {
@@ -212,7 +270,8 @@ struct Range {
 
 // Pass 2: normAndClamp of intensity (unless NO_I_NORM) and colour; the
 // block first stages every type's two ranges and vector flag in LDS.
-__global__ __launch_bounds__(256) void k_norm_clamp(NormArgs a, const uint32_t *keys) {
+template <int W, bool GEN>
+__global__ __launch_bounds__(kNormThreads) void k_norm_clamp(NormArgs a, const uint32_t *keys) {
   __shared__ Range s_int[kMaxTypes], s_col[kMaxTypes];
   __shared__ int32_t s_vec[kMaxTypes];
   const int i = threadIdx.x;
@@ -227,49 +286,70 @@ __global__ __launch_bounds__(256) void k_norm_clamp(NormArgs a, const uint32_t *
     s_vec[i] = a.flags[i][3];
   }
   __syncthreads();
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * 256;
-  for (int64_t m0 = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; m0 < a.n;
-       m0 += 4 * stride) {
-    int tv[4];
-    float Iv[4], ev[4];
+  constexpr int kV = loads<W>();
+  const int64_t stride = static_cast<int64_t>(gridDim.x) * kNormThreads * W;
+  for (int64_t m0 = (static_cast<int64_t>(blockIdx.x) * kNormThreads + threadIdx.x) * W; m0 < a.n;
+       m0 += kV * stride) {
+    uint8_t tv[kV][W] = {};
+    float Iv[kV][W], ev[kV][W], gv[GEN ? kV : 1][W], bv[GEN ? kV : 1][W];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {  // loads first
-      const int64_t m = m0 + j * stride;
-      tv[j] = kMaxTypes;
+    for (int q = 0; q < kV; ++q) {  // loads first
+      const int64_t m = m0 + q * stride;
       if (m < a.n) {
-        tv[j] = a.type ? a.type[m] : 0;
-        Iv[j] = a.I[m];
-        ev[j] = a.er[m];
+        if (GEN && a.vector) {
+          load_w<W, float, float4>(a.eg, m, a.n, gv[GEN ? q : 0]);
+          load_w<W, float, float4>(a.eb, m, a.n, bv[GEN ? q : 0]);
+        }
+        if (a.type) load_w<W, uint8_t, uchar4>(a.type, m, a.n, tv[q]);
+        load_w<W, float, float4>(a.I, m, a.n, Iv[q]);
+        load_w<W, float, float4>(a.er, m, a.n, ev[q]);
       }
     }
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int64_t m = m0 + j * stride;
-      const int t = tv[j];
-      if (t >= a.ntypes) continue;
-      if (a.norm_int) {
-        float I = Iv[j];
-        s_int[t].clamp(I);
-        a.I[m] = I;
+    for (int q = 0; q < kV; ++q) {
+      const int64_t mq = m0 + q * stride;
+      bool put = false, put_v = false;
+#pragma unroll
+      for (int j = 0; j < W; ++j) {
+        const int64_t m = mq + j;
+        const int t = m < a.n ? tv[q][j] : kMaxTypes;
+        if (t >= a.ntypes) continue;
+        put = true;
+        if (a.norm_int) s_int[t].clamp(Iv[q][j]);
+        const Range C = s_col[t];
+        C.clamp(ev[q][j]);
+        if (GEN && s_vec[t]) {
+          put_v = true;
+          C.clamp(gv[GEN ? q : 0][j]);
+          C.clamp(bv[GEN ? q : 0][j]);
+        }
       }
-      const Range C = s_col[t];
-      float e = ev[j];
-      C.clamp(e);
-      a.er[m] = e;
-      if (s_vec[t]) {
-        float g = a.eg[m], b = a.eb[m];
-        C.clamp(g);
-        C.clamp(b);
-        a.eg[m] = g;
-        a.eb[m] = b;
+      if (put) {
+        if (a.norm_int) store_w<W>(a.I, mq, a.n, Iv[q]);
+        store_w<W>(a.er, mq, a.n, ev[q]);
+      }
+      if (put_v) {
+        store_w<W>(a.eg, mq, a.n, gv[GEN ? q : 0]);
+        store_w<W>(a.eb, mq, a.n, bv[GEN ? q : 0]);
       }
     }
   }
 }
 
-template <int NT>
-void launch_reduce(const NormArgs &a, uint32_t *keys, unsigned grid, hipStream_t s) {
-  k_norm_reduce<NT><<<grid, 256, 0, s>>>(a, keys);
+template <int W, bool GEN>
+void launch_passes(const NormArgs &a, uint32_t *keys, hipStream_t s) {
+  const unsigned grid = static_cast<unsigned>(
+      std::min<int64_t>((a.n + W * kNormThreads - 1) / (W * kNormThreads), 1024));
+#define SPLHIP_NORM(N) \
+  case N: k_norm_reduce<N, W, GEN><<<grid, kNormThreads, 0, s>>>(a, keys); break;
+  switch (a.ntypes) {
+    SPLHIP_NORM(1) SPLHIP_NORM(2) SPLHIP_NORM(3) SPLHIP_NORM(4)
+    SPLHIP_NORM(5) SPLHIP_NORM(6) SPLHIP_NORM(7) SPLHIP_NORM(8)
+  }
+#undef SPLHIP_NORM
+  hip_check(hipGetLastError(), "k_norm_reduce launch");
+  k_norm_clamp<W, GEN><<<grid, kNormThreads, 0, s>>>(a, keys);
+  hip_check(hipGetLastError(), "k_norm_clamp launch");
 }
 
 }  // namespace
@@ -277,23 +357,24 @@ void launch_reduce(const NormArgs &a, uint32_t *keys, unsigned grid, hipStream_t
 void launch_normalize(const NormArgs &a, uint32_t *keys, hipStream_t s) {
   k_norm_init<<<1, 256, 0, s>>>(keys, a.ntypes);
   hip_check(hipGetLastError(), "k_norm_init launch");
-  if (a.n > 0) {
-    const unsigned grid =
-        static_cast<unsigned>(std::min<int64_t>(std::max<int64_t>((a.n + 255) / 256, 1), 1024));
-    switch (a.ntypes) {
-      case 1: launch_reduce<1>(a, keys, grid, s); break;
-      case 2: launch_reduce<2>(a, keys, grid, s); break;
-      case 3: launch_reduce<3>(a, keys, grid, s); break;
-      case 4: launch_reduce<4>(a, keys, grid, s); break;
-      case 5: launch_reduce<5>(a, keys, grid, s); break;
-      case 6: launch_reduce<6>(a, keys, grid, s); break;
-      case 7: launch_reduce<7>(a, keys, grid, s); break;
-      default: launch_reduce<8>(a, keys, grid, s); break;
-    }
-    hip_check(hipGetLastError(), "k_norm_reduce launch");
-    k_norm_clamp<<<grid, 256, 0, s>>>(a, keys);
-    hip_check(hipGetLastError(), "k_norm_clamp launch");
+  if (a.n <= 0) return;
+  auto at = [](const void *p, uintptr_t m) { return reinterpret_cast<uintptr_t>(p) % m == 0; };
+  NormArgs b = a;
+  bool gen = false;
+  b.vector = 0;
+  for (int t = 0; t < a.ntypes; ++t) {
+    gen = gen || a.flags[t][0] || a.flags[t][1] || a.flags[t][2] || a.flags[t][3];
+    b.vector |= a.flags[t][3];
   }
+  // four particles per load where the fields are aligned and there are enough
+  // to fill the GPU that way; else one (20k particles with logs: 14.8 us with
+  // one, 16.3 with four, whose logarithms a thread takes in turn)
+  const bool vec = a.n >= (1 << 19) && at(a.I, 16) && at(a.er, 16) && at(a.r, 16) &&
+                   at(a.type, 4) && (!b.vector || (at(a.eg, 16) && at(a.eb, 16)));
+  if (vec && gen) launch_passes<4, true>(b, keys, s);
+  else if (vec) launch_passes<4, false>(b, keys, s);
+  else if (gen) launch_passes<1, true>(b, keys, s);
+  else launch_passes<1, false>(b, keys, s);
 }
 
 }  // namespace splhip
