@@ -438,6 +438,8 @@ struct Plan {
   uint32_t nsplit[2] = {0, 0};
   // staged lists (the first nstage items; nheavy counts them too) and their
   // groups of 4 entries (padded to whole chain loads)
+  bool counted[2] = {false, false};  // work items counted in this frame
+  bool late = false;  // the pass sizes are still on the device (m: capacities)
   uint32_t nstage[2] = {0, 0};
   uint64_t sgroups[2] = {0, 0};
   uint64_t etot[2] = {0, 0};  // (block, particle) entries of each pass (or chunk)
@@ -644,23 +646,49 @@ void make_plan(splhip_ctx *c, int nj, const JobIn *jobs, int G, Plan &pl, hipStr
 }
 
 // Totals slot layout (device u32): [0..1] pass sizes, [2..3] bin entries,
-// [4..5] work items, [6..7] heavy items, [8..11] bin entries as u64,
-// [12..13] region entries, [14] the ordered pass has a non-finite q,
-// [15] capacity overflow bits of a device-count render (bit p: pass p),
-// from T_STAGE on the lists from stage_level(stage_len, j) entries on and from
-// T_SGRP on their groups of 4 entries (at most), kStageLevels per pass, then
-// the longest list of each pass and a device-count render's long-list
-// partition (4 per pass: staged, producer/consumer, both).
+// [4..5] work items, [6] the ordered pass has a non-finite q, [7] capacity
+// overflow bits of a device-count render (bit p: pass p), [8..11] bin entries
+// as u64, [12..13] region entries; from T_LIST on per pass (kListWords each)
+// its lists from heavy_len entries on, its longest list, the lists from
+// stage_level(stage_len, j) entries on and their groups of 4 entries (at
+// most); then a device-count render's long-list partition (4 per pass: staged,
+// producer/consumer, both, by channel).
+constexpr int kListWords = 2 + 2 * kStageLevels;
+enum { L_HEAVY = 0, L_MAX = 1, L_CNT = 2, L_GRP = 2 + kStageLevels };
 enum {
-  T_M = 0, T_E = 2, T_ITEMS = 4, T_HEAVY = 6, T_E64 = 8, T_E16 = 12, T_QBAD = 14, T_OVF = 15,
-  T_STAGE = 16, T_SGRP = T_STAGE + 2 * kStageLevels, T_LMAX = T_SGRP + 2 * kStageLevels,
-  T_PART = T_LMAX + 2, T_N = T_PART + 8
+  T_M = 0, T_E = 2, T_ITEMS = 4, T_QBAD = 6, T_OVF = 7, T_E64 = 8, T_E16 = 12,
+  T_LIST = 16, T_PART = T_LIST + 2 * kListWords, T_N = T_PART + 8
 };
+constexpr int t_list(int p, int k) { return T_LIST + kListWords * p + k; }
 constexpr int kTotalsWords = 256;  // the totals buffer, device and pinned host
 static_assert(T_N <= kTotalsWords, "totals fit their buffers");
 
+// One host sync reads the totals (into c->h_tot), the pass sizes and their job
+// offsets in pass order.
+void read_pass_sizes(splhip_ctx *c, Plan &pl, const uint32_t *tot, hipStream_t s) {
+  uint32_t *h = c->h_tot;
+  const size_t nmo = static_cast<size_t>(pl.nj) + 1;
+  std::vector<uint32_t> &hbv = c->h_mo;  // pageable: read after the sync below
+  hbv.resize(2 * nmo);
+  uint32_t *hb = hbv.data();
+  hip_check(hipMemcpyAsync(h, tot, T_N * 4, hipMemcpyDeviceToHost, s), "read totals");
+  if (pl.nj > 1)  // a single view's offsets are 0 and the pass size
+    for (int p = 0; p < 2; ++p)
+      if (pl.d_mo[p])
+        hip_check(hipMemcpyAsync(hb + p * nmo, pl.d_mo[p], nmo * 4, hipMemcpyDeviceToHost, s),
+                  "read pass offsets");
+  hip_check(hipStreamSynchronize(s), "sync pass sizes");
+  for (int p = 0; p < 2; ++p) {
+    pl.m[p] = pl.d_mo[p] ? h[T_M + p] : 0;
+    if (!pl.d_mo[p]) pl.mo[p].assign(nmo, 0);
+    else if (pl.nj > 1) pl.mo[p].assign(hb + p * nmo, hb + (p + 1) * nmo);
+    else pl.mo[p] = {0u, pl.m[p]};
+  }
+}
+
 // Project all jobs, then the compaction scan of each present pass and its job
-// offsets in pass order; one host sync reads the pass sizes and offsets.
+// offsets in pass order; the pass sizes are read (read_pass_sizes) unless they
+// stay on the device for now.
 void stage_project_compact(splhip_ctx *c, Plan &pl, Rec *rec, uint8_t *act, uint32_t *tot,
                            hipStream_t s) {
   Workspace &ws = *pl.ws;
@@ -678,37 +706,22 @@ void stage_project_compact(splhip_ctx *c, Plan &pl, Rec *rec, uint8_t *act, uint
     launch_pass_offsets(pos, pl.d_pbase, pl.nj, pl.ntot, tot + T_M + p, mo[p], s);
     mark(c, p == 0 ? 1 : 4, false, s);
   }
-  if (pl.dc) {  // the pass sizes stay on the device; capacities: every particle
+  if (pl.dc || pl.late) {  // the pass sizes stay on the device; capacities: every particle
     for (int p = 0; p < 2; ++p) {
       pl.m[p] = mo[p] ? static_cast<uint32_t>(pl.ntot) : 0u;
       pl.d_mo[p] = mo[p];
     }
     return;
   }
-  // sync 1: pass sizes and per-job offsets
-  uint32_t *h = c->h_tot;
-  const size_t nmo = static_cast<size_t>(pl.nj) + 1;
-  std::vector<uint32_t> &hbv = c->h_mo;  // pageable: read after the sync below
-  hbv.resize(2 * nmo);
-  uint32_t *hb = hbv.data();
-  hip_check(hipMemcpyAsync(h, tot, T_N * 4, hipMemcpyDeviceToHost, s), "read totals");
-  for (int p = 0; p < 2; ++p)
-    if (mo[p])
-      hip_check(hipMemcpyAsync(hb + p * nmo, mo[p], nmo * 4, hipMemcpyDeviceToHost, s),
-                "read pass offsets");
-  hip_check(hipStreamSynchronize(s), "sync pass sizes");
-  for (int p = 0; p < 2; ++p) {
-    pl.m[p] = mo[p] ? h[T_M + p] : 0;
-    pl.d_mo[p] = mo[p];
-    if (mo[p]) pl.mo[p].assign(hb + p * nmo, hb + (p + 1) * nmo);
-    else pl.mo[p].assign(nmo, 0);
-  }
+  for (int p = 0; p < 2; ++p) pl.d_mo[p] = mo[p];
+  read_pass_sizes(c, pl, tot, s);  // sync 1
 }
 
 // Per-job pass flags from the pass sizes: the ordered pass writes the image
 // of every job that has ordered particles; the additive pass adds to it there
-// and writes it elsewhere (render_new renders each mode from zero).
-void upload_job_flags(splhip_ctx *c, Plan &pl, hipStream_t s) {
+// and writes it elsewhere (render_new renders each mode from zero).  A late
+// plan's device flags were set from the device's sizes.
+void set_job_flags(splhip_ctx *c, Plan &pl, hipStream_t s) {
   for (int j = 0; j < pl.nj; ++j) {
     const bool w0 = pl.mo[0][j + 1] > pl.mo[0][j];
     const bool w1 = pl.mo[1][j + 1] > pl.mo[1][j];
@@ -718,6 +731,7 @@ void upload_job_flags(splhip_ctx *c, Plan &pl, hipStream_t s) {
     J.need_empty[0] = w0 ? 1 : 0;
     J.need_empty[1] = (w1 && !w0) ? 1 : 0;
   }
+  if (pl.late) return;
   const size_t bytes = pl.nj * sizeof(JobSplat);
   char *h = staging(c, bytes);
   std::memcpy(h, pl.js.data(), bytes);
@@ -733,7 +747,8 @@ void stage_order(splhip_ctx *c, Plan &pl, int p, const Rec *rec, const uint8_t *
   const uint32_t m = pl.m[p];
   const bool do_sort = (p == 0) && pl.sort;
   mark(c, p == 0 ? 1 : 4, true, s);
-  const uint32_t *dm = pl.dc ? pl.tot + T_M + p : nullptr;  // device count (m: capacity)
+  // device count (m: capacity)
+  const uint32_t *dm = pl.dc || pl.late ? pl.tot + T_M + p : nullptr;
   uint32_t *k0 = do_sort ? ws.get_as<uint32_t>(pslot(p, P_K0), m) : nullptr;
   uint32_t *v0 = ws.get_as<uint32_t>(pslot(p, P_V0), m);
   const uint32_t *pos = ws.get_as<uint32_t>(pslot(p, P_POS), static_cast<size_t>(pl.ntot));
@@ -771,20 +786,20 @@ void stage_count(splhip_ctx *c, Plan &pl, int p, const Rec *rec, uint32_t *tot, 
   uint32_t *cnt = ws.get_as<uint32_t>(pslot(p, P_CNT), m);
   uint32_t *off = ws.get_as<uint32_t>(pslot(p, P_OFF), m);
   uint32_t *cnt16 = pl.r16[p] ? ws.get_as<uint32_t>(pslot(p, P_CNT16), m) : nullptr;
-  const uint32_t *dm = pl.dc ? tot + T_M + p : nullptr;  // device count (m: capacity)
+  // device count (m: capacity)
+  const uint32_t *dm = pl.dc || pl.late ? tot + T_M + p : nullptr;
   launch_gather_count(pl.order[p], m, rec, recs, cnt, cnt16, pl.rsh, pl.d_geom, pl.d_mo[p], pl.nj,
                       p == 0 ? tot + T_QBAD : nullptr, s, dm);
   if (p == 0) pl.qbad = tot + T_QBAD;
-  scan_u32(cnt, off, m, tot + T_E + p, ws, s, 0, dm);
-  launch_sum_u64(cnt, m, reinterpret_cast<uint64_t *>(tot + T_E64 + 2 * p), s, dm);
+  uint64_t *e64 = reinterpret_cast<uint64_t *>(tot + T_E64 + 2 * p);
   if (cnt16)
-    scan_u32(cnt16, ws.get_as<uint32_t>(pslot(p, P_OFF16), m), m, tot + T_E16 + p, ws, s, 0,
-             dm);
+    scan_u32_pair(cnt, off, tot + T_E + p, e64, cnt16,
+                  ws.get_as<uint32_t>(pslot(p, P_OFF16), m), tot + T_E16 + p, m, ws, s, dm);
+  else
+    scan_u32(cnt, off, m, tot + T_E + p, ws, s, dm, e64);
   if (pl.dc)  // entries past the reserved capacity: the pass is dropped and flagged
-    launch_cap_check(tot + T_M + p, tot + T_E + p,
-                     reinterpret_cast<const uint64_t *>(tot + T_E64 + 2 * p),
-                     pl.use16[p] ? tot + T_E16 + p : nullptr, pl.e[p], pl.e16[p], 1u << p,
-                     tot + T_OVF, s);
+    launch_cap_check(tot + T_M + p, tot + T_E + p, e64, pl.use16[p] ? tot + T_E16 + p : nullptr,
+                     pl.e[p], pl.e16[p], 1u << p, tot + T_OVF, s);
   pl.recs[p] = recs;
   mark(c, p == 0 ? 2 : 5, false, s);
 }
@@ -940,16 +955,13 @@ void stage_items_count(splhip_ctx *c, Plan &pl, int p, const Tuning &tn, uint32_
   const SplatArgs sa = splat_args(c, pl, p, tn);
   uint32_t *icnt = ws.get_as<uint32_t>(pslot(p, P_ICNT), pl.nunits);
   uint32_t *ioff = ws.get_as<uint32_t>(pslot(p, P_IOFF), pl.nunits);
-  // the count of this call's long-list items only (chunks and autotuning
-  // candidates count again)
-  launch_fill_u32(tot + T_HEAVY + p, 0u, 1, s);
-  launch_fill_u32(tot + T_STAGE + kStageLevels * p, 0u, kStageLevels, s);
-  launch_fill_u32(tot + T_SGRP + kStageLevels * p, 0u, kStageLevels, s);
-  launch_fill_u32(tot + T_LMAX + p, 0u, 1, s);
+  // the counts of this call only (chunks and autotuning candidates count
+  // again; a frame's totals start at zero)
+  if (pl.counted[p]) launch_fill_u32(tot + t_list(p, 0), 0u, kListWords, s);
+  pl.counted[p] = true;
   launch_items_count(pl.bin_off[p], pl.nunits, sa, p == 0 ? 1 : 0, tn.split, icnt,
-                     tot + T_HEAVY + p, s, tot + T_STAGE + kStageLevels * p,
-                     tot + T_SGRP + kStageLevels * p,
-                     tot + T_LMAX + p);
+                     tot + t_list(p, L_HEAVY), s, tot + t_list(p, L_CNT), tot + t_list(p, L_GRP),
+                     tot + t_list(p, L_MAX));
   scan_u32(icnt, ioff, pl.nunits, tot + T_ITEMS + p, wt ? *wt : ws, s);
   mark(c, p == 0 ? 2 : 5, false, s);
 }
@@ -962,11 +974,11 @@ void stage_items_count(splhip_ctx *c, Plan &pl, int p, const Tuning &tn, uint32_
 void take_items(splhip_ctx *c, Plan &pl, int p, const Tuning &tn) {
   const uint32_t *h = c->h_tot;
   pl.nitems[p] = pl.m[p] ? h[T_ITEMS - T_ITEMS + p] : 0u;
-  const uint32_t nheavy_lists = pl.m[p] ? h[T_HEAVY - T_ITEMS + p] : 0u;
-  const uint64_t lmax = h[T_LMAX - T_ITEMS + p];
+  const uint32_t nheavy_lists = pl.m[p] ? h[t_list(p, L_HEAVY) - T_ITEMS] : 0u;
+  const uint64_t lmax = h[t_list(p, L_MAX) - T_ITEMS];
   const uint32_t len0 = p == 1 ? tn.stage : tn.stage_ord;
-  const uint32_t *cnt = h + (T_STAGE - T_ITEMS + kStageLevels * p);
-  const uint32_t *grp = h + (T_SGRP - T_ITEMS + kStageLevels * p);
+  const uint32_t *cnt = h + (t_list(p, L_CNT) - T_ITEMS);
+  const uint32_t *grp = h + (t_list(p, L_GRP) - T_ITEMS);
   uint32_t ns = 0;
   uint64_t groups = 0;
   if (pl.m[p] && len0 != 0xffffffffu)
@@ -1029,10 +1041,10 @@ void stage_splat(splhip_ctx *c, Plan &pl, int p, const Tuning &tn, hipStream_t s
     // the long-list partition from the device counts, as take_items makes it
     part = pl.tot + T_PART + 4 * p;
     PartitionArgs pa;
-    pa.stage_cnt = pl.tot + T_STAGE + kStageLevels * p;
-    pa.stage_grp = pl.tot + T_SGRP + kStageLevels * p;
-    pa.heavy_cnt = pl.tot + T_HEAVY + p;
-    pa.lmax = pl.tot + T_LMAX + p;
+    pa.stage_cnt = pl.tot + t_list(p, L_CNT);
+    pa.stage_grp = pl.tot + t_list(p, L_GRP);
+    pa.heavy_cnt = pl.tot + t_list(p, L_HEAVY);
+    pa.lmax = pl.tot + t_list(p, L_MAX);
     pa.etot = reinterpret_cast<const uint64_t *>(pl.tot + T_E64 + 2 * p);
     pa.len0 = pl.nstage[p] ? (p == 1 ? tn.stage : tn.stage_ord) : 0xffffffffu;
     pa.mode = tn.mode[p];
@@ -1049,7 +1061,7 @@ void stage_splat(splhip_ctx *c, Plan &pl, int p, const Tuning &tn, hipStream_t s
     dc.npc = part + 1;
     dc.nsplit = part + 3;
   }
-  const int rs = radix_sort_pairs(ik0, iv0, ik1, iv1, nitems, 0, 32, wt ? *wt : ws, s, dc.items);
+  const int rs = radix_sort_pairs(ik0, iv0, ik1, iv1, nitems, 0, 8, wt ? *wt : ws, s, dc.items);
   const uint32_t *items = rs ? iv1 : iv0;
   pl.items[p] = items;
   SplatArgs sa = sa0;
@@ -1113,7 +1125,7 @@ void stage_splat(splhip_ctx *c, Plan &pl, int p, const Tuning &tn, hipStream_t s
       auto operands = [&](uint32_t i0, uint32_t i1, uint32_t phase, hipStream_t q) {
         uint32_t *r = rows + phase * nbat * 8, *g = gofs + phase * nbat * 8;
         launch_stage_rows(items, i0, i1, nbat, cbt, masks, r, sa, q, part);
-        scan_u32(r, g, static_cast<int64_t>(nbat * 8), nullptr, tmp, q, 0, nrows + phase);
+        scan_u32(r, g, static_cast<int64_t>(nbat * 8), nullptr, tmp, q, nrows + phase);
         launch_stage_ops(add, items, i0, i1, nbat, cb, cbt, masks, r, g, ops, stride, sa, q, part);
       };
       auto chains = [&](uint32_t i0, uint32_t i1, uint32_t phase, hipStream_t q) {
@@ -1132,9 +1144,12 @@ void stage_splat(splhip_ctx *c, Plan &pl, int p, const Tuning &tn, hipStream_t s
       mark(c, p == 0 ? 11 : 12, false, X.aux3);
       hip_check(hipEventRecord(X.join3, X.aux3), "record join");
     }
-    // The normal items fill every CU; the heavy workgroups (the critical
-    // path) must get their slots first, so the normal launch waits briefly.
-    launch_delay(40, s);
+    // The normal items fill every CU; the producer/consumer workgroups (a CU
+    // each, the critical path) must get theirs first, so the normal launch
+    // waits briefly.  Staged lists need no such start: their operand kernels'
+    // workgroups fit in as the normal ones end (20k ordered at 257 x 193: 0.377
+    // ms with the wait, 0.339 without; larger frames up to 1 % faster without).
+    if (npc > 0) launch_delay(40, s);
     if (placed) hip_check(hipEventRecord(placed, s), "record placed");
     mark(c, p == 0 ? 7 : 9, true, s);
     launch_splat8(p == 1, tn.variant, nit, nn, sn, s, dc, tn.ppw, pl.nsplit[p]);
@@ -1226,9 +1241,11 @@ void render_chunked_pass(splhip_ctx *c, Plan &pl, int p, const Tuning &tn, uint3
     uint32_t e16 = 0;
     uint64_t ec_last = 0;
     for (;;) {  // shrink the range until its entries fit a chunk
-      scan_u32(cnt + s0, off, n, tot + T_E + p, ws, s);
-      launch_sum_u64(cnt + s0, n, e64, s);
-      if (pl.r16[p]) scan_u32(cnt16 + s0, off16, n, tot + T_E16 + p, ws, s);
+      if (pl.r16[p])
+        scan_u32_pair(cnt + s0, off, tot + T_E + p, e64, cnt16 + s0, off16, tot + T_E16 + p, n, ws,
+                      s);
+      else
+        scan_u32(cnt + s0, off, n, tot + T_E + p, ws, s, nullptr, e64);
       read_totals(c, tot, T_N, s);
       uint64_t ec;
       std::memcpy(&ec, c->h_tot + T_E64 + 2 * p, 8);
@@ -1345,6 +1362,10 @@ Tuning autotune(splhip_ctx *c, Plan &pl, const Tuning &base, uint32_t *tot, hipS
 // The frame pipeline over a batch of jobs; three host syncs per batch (pass
 // sizes, bin entries, work items).
 // A choice of the autotuner: work region and the 8x8 splat's decomposition.
+// Frames of at most this many particles (of all views) wait on the host once
+// less (see render_jobs).
+constexpr int64_t kLateParticles = int64_t(1) << 22;
+
 struct Choice {
   int G;
   Tuning tn;
@@ -1371,8 +1392,14 @@ int render_jobs(splhip_ctx *c, int nj, const JobIn *jobs, hipStream_t s, bool ke
   Rec *rec = ws.get_as<Rec>(S_REC, static_cast<size_t>(std::max<int64_t>(pl.ntot, 1)));
   uint8_t *act = ws.get_as<uint8_t>(S_ACT, static_cast<size_t>(std::max<int64_t>(pl.ntot, 1)));
   uint32_t *tot = ws.get_as<uint32_t>(S_TOTALS, kTotalsWords);
+  // Small frames keep the pass sizes on the device until the bin entries are
+  // read, one host wait (about 20 us) less; their launches up to there are
+  // sized for every particle in each pass, which a few million do not notice.
+  pl.late = pl.ntot > 0 && pl.ntot <= kLateParticles;
+  pl.tot = tot;
   stage_project_compact(c, pl, rec, act, tot, s);
-  upload_job_flags(c, pl, s);
+  if (pl.late) launch_job_flags(pl.d_mo[0], pl.d_mo[1], nj, pl.d_js, s);
+  else set_job_flags(c, pl, s);
   for (int p = 0; p < 2; ++p)
     if (pl.m[p]) {
       stage_order(c, pl, p, rec, act, s);
@@ -1380,12 +1407,19 @@ int render_jobs(splhip_ctx *c, int nj, const JobIn *jobs, hipStream_t s, bool ke
     }
   bool chunked[2] = {false, false};
   if (pl.m[0] || pl.m[1]) {
-    read_totals(c, tot + T_E, T_N - T_E, s);  // sync 2
+    // sync 2
+    if (pl.late) {
+      read_pass_sizes(c, pl, tot, s);
+      set_job_flags(c, pl, s);
+      pl.late = false;
+    } else {
+      read_totals(c, tot, T_N, s);
+    }
     uint64_t e64[2];
     for (int p = 0; p < 2; ++p) {
-      std::memcpy(&e64[p], c->h_tot + (T_E64 - T_E) + 2 * p, 8);
-      pl.e[p] = pl.m[p] ? c->h_tot[p] : 0;
-      pl.e16[p] = pl.m[p] ? c->h_tot[(T_E16 - T_E) + p] : 0;
+      std::memcpy(&e64[p], c->h_tot + T_E64 + 2 * p, 8);
+      pl.e[p] = pl.m[p] ? c->h_tot[T_E + p] : 0;
+      pl.e16[p] = pl.m[p] ? c->h_tot[T_E16 + p] : 0;
       chunked[p] = pl.m[p] && e64[p] > tn.chunk;
     }
     // A single unchunked view with both passes: the additive splat runs

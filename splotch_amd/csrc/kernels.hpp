@@ -121,9 +121,6 @@ void launch_map(const uint32_t *idx, const uint32_t *table, uint32_t *out, int64
                 hipStream_t s);
 void launch_fill(float *p, float v, int64_t n, hipStream_t s);
 void launch_fill_u32(uint32_t *p, uint32_t v, int64_t n, hipStream_t s);
-// *out (device, 8 bytes) = sum of v[0..n) in 64 bits.
-void launch_sum_u64(const uint32_t *v, int64_t n, uint64_t *out, hipStream_t s,
-                    const uint32_t *dn = nullptr);
 // Device-count pipeline helpers: per-job pass flags from the pass offsets
 // (null: pass absent), zeros into the images of jobs with no particle in
 // either pass, and the capacity check of a pass (counts zeroed, bit set in
@@ -163,6 +160,8 @@ void launch_items_count(const uint32_t *bin_off, uint32_t nunits, const SplatArg
                         int ordered, uint32_t split, uint32_t *cnt, uint32_t *heavy_cnt,
                         hipStream_t s, uint32_t *stage_cnt = nullptr,
                         uint32_t *stage_grp = nullptr, uint32_t *lmax = nullptr);
+// keys: 8 bits, the longer lists first, by quarter octaves of the length (lists
+// from the long-list length on before the others).
 void launch_items_emit(const uint32_t *bin_off, uint32_t nunits, const SplatArgs &a, int ordered,
                        uint32_t split, const uint32_t *off, uint32_t *keys, uint32_t *vals,
                        hipStream_t s);

@@ -1,17 +1,25 @@
 // Device-wide exclusive scan and stable LSD radix sort for wave64 (gfx950).
 //
-// Scan: reduce-then-scan over 4096-element tiles (256 threads x 16 items).
-// Each thread scans its 16 items serially, the 64 lanes of a wave combine
-// their sums with a log-step shuffle scan, and the 4 wave totals are combined
-// through LDS.  Tile sums are scanned recursively.
+// Frames of up to a few million particles are bound by the number of launches
+// (about 5 us each, most of them scans and sort passes), so both take as few
+// as the size allows.
 //
-// Radix sort: per digit of up to 9 bits, (1) a per-tile digit histogram
-// written digit-major, (2) an exclusive scan of that histogram (digit-major
-// order makes the result stable), (3) a scatter: each wave ranks its keys in
-// input order with a 64-lane "match any" on the digit (one ballot per bit), the
-// rank among equal digits from a popcount under the lane mask, and a
-// wave-private running count per digit; the tile is then staged in LDS in
-// digit order and written out as contiguous per-digit runs.
+// Scan: up to 16384 elements in one workgroup; else reduce-then-scan over
+// 4096-element tiles (256 threads x 16 items), two launches: a tile sums the
+// tile sums before it itself (at most 8192 of them; beyond, they are scanned
+// recursively first).  Each thread scans its 16 items serially, the 64 lanes
+// of a wave combine their sums with a log-step shuffle scan, and the wave
+// totals are combined through LDS.
+//
+// Radix sort: up to 4096 pairs in one workgroup and one launch, digit after
+// digit in LDS.  Else per digit of up to 9 bits, (1) a per-tile digit
+// histogram, (2) for more than 128 tiles an exclusive scan of the histograms
+// in digit-major order (which makes the result stable); up to 128 tiles, the
+// scatter's workgroups sum the histograms themselves, (3) a scatter: each wave
+// ranks its keys in input order with a 64-lane "match any" on the digit (one
+// ballot per bit), the rank among equal digits from a popcount under the lane
+// mask, and a wave-private running count per digit; the tile is then staged in
+// LDS in digit order and written out as contiguous per-digit runs.
 #include "scan_sort.hpp"
 
 #include <algorithm>
@@ -26,6 +34,13 @@ constexpr int kMaxBits = 9;
 struct LoadU32 {
   const uint32_t *p;
   __device__ __forceinline__ uint32_t operator()(int64_t i) const { return p[i]; }
+};
+
+struct LoadLow32 {  // of tile sums
+  const uint64_t *p;
+  __device__ __forceinline__ uint32_t operator()(int64_t i) const {
+    return static_cast<uint32_t>(p[i]);
+  }
 };
 
 struct LoadU8Bit {
@@ -43,13 +58,14 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v, int lane) {
   return v;
 }
 
-__device__ __forceinline__ uint32_t wave_reduce(uint32_t v) {
+__device__ __forceinline__ uint64_t wave_reduce(uint64_t v) {
 #pragma unroll
   for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d, 64);
   return v;
 }
 
-// Exclusive scan of one value per thread over a 256-thread block.
+// Exclusive scan of one value per thread over a block of W waves.
+template <int W = 4>
 __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t *s_w) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const uint32_t inc = wave_incl_scan(v, lane);
@@ -57,7 +73,7 @@ __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t *s_w) {
   __syncthreads();
   uint32_t woff = 0;
 #pragma unroll
-  for (int w = 0; w < 4; ++w)
+  for (int w = 0; w < W; ++w)
     if (w < wave) woff += s_w[w];
   __syncthreads();
   return woff + inc - v;
@@ -69,90 +85,175 @@ __device__ __forceinline__ int64_t count_of(int64_t cap, const uint32_t *dn) {
   return dn ? min(cap, static_cast<int64_t>(*dn)) : cap;
 }
 
+// One or two scans of a launch (blockIdx.y), of the same element count.
 template <class In>
-__global__ __launch_bounds__(256) void k_scan_reduce(In in, int64_t cap, const uint32_t *dn,
-                                                     uint32_t *partial) {
-  __shared__ uint32_t s_w[4];
+struct Job {
+  In in;
+  uint32_t *out;
+  uint32_t *total;    // optional: the sum of all elements ...
+  uint64_t *total64;  // ... and in 64 bits
+  uint64_t *partial;  // tile sums
+  uint32_t *psum;     // their exclusive scan (null: the tiles add them up themselves)
+};
+template <class In>
+struct Jobs {
+  Job<In> j[2];
+};
+
+// Sum of each tile, in 64 bits.
+template <class In>
+__global__ __launch_bounds__(256) void k_scan_reduce(Jobs<In> jobs, int64_t cap,
+                                                     const uint32_t *dn) {
+  __shared__ uint64_t s_w[4];
+  const Job<In> &J = jobs.j[blockIdx.y];
   const int64_t n = count_of(cap, dn);
   const int64_t base = static_cast<int64_t>(blockIdx.x) * kTile;
-  uint32_t s = 0;
+  uint64_t s = 0;
 #pragma unroll
   for (int i = 0; i < kItems; ++i) {
     const int64_t idx = base + i * 256 + threadIdx.x;
-    if (idx < n) s += in(idx);
+    if (idx < n) s += J.in(idx);
   }
   s = wave_reduce(s);
   if ((threadIdx.x & 63) == 0) s_w[threadIdx.x >> 6] = s;
   __syncthreads();
-  if (threadIdx.x == 0) partial[blockIdx.x] = s_w[0] + s_w[1] + s_w[2] + s_w[3];
+  if (threadIdx.x == 0) J.partial[blockIdx.x] = s_w[0] + s_w[1] + s_w[2] + s_w[3];
 }
 
 template <class In>
-__global__ __launch_bounds__(256) void k_scan_apply(In in, uint32_t *out, int64_t cap,
-                                                    const uint32_t *dn, const uint32_t *partial,
-                                                    uint32_t *total) {
+__global__ __launch_bounds__(256) void k_scan_apply(Jobs<In> jobs, int64_t cap,
+                                                    const uint32_t *dn) {
   __shared__ uint32_t s_w[4];
+  __shared__ uint64_t s_p[4];
+  const Job<In> &J = jobs.j[blockIdx.y];
   const int64_t n = count_of(cap, dn);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t base = static_cast<int64_t>(blockIdx.x) * kTile + threadIdx.x * kItems;
+  const bool last = blockIdx.x == gridDim.x - 1;
+  // the elements of the tiles before this one
+  const bool add_up = !J.psum || (last && J.total64);
+  uint64_t before = 0;
+  if (add_up) {
+    for (uint32_t i = threadIdx.x; i < blockIdx.x; i += 256) before += J.partial[i];
+    before = wave_reduce(before);
+    if (lane == 0) s_p[wave] = before;
+  }
   uint32_t v[kItems];
   uint32_t sum = 0;
   if (base + kItems <= n) {
 #pragma unroll
     for (int i = 0; i < kItems; ++i) {
-      v[i] = in(base + i);
+      v[i] = J.in(base + i);
       sum += v[i];
     }
   } else {
 #pragma unroll
     for (int i = 0; i < kItems; ++i) {
-      v[i] = (base + i < n) ? in(base + i) : 0u;
+      v[i] = (base + i < n) ? J.in(base + i) : 0u;
       sum += v[i];
     }
   }
-  const uint32_t inc = wave_incl_scan(sum, lane);
-  if (lane == 63) s_w[wave] = inc;
-  __syncthreads();
-  uint32_t woff = 0;
-#pragma unroll
-  for (int w = 0; w < 4; ++w)
-    if (w < wave) woff += s_w[w];
-  uint32_t prefix = (partial ? partial[blockIdx.x] : 0u) + woff + inc - sum;
+  const uint32_t excl = block_excl_scan(sum, s_w);
+  before = add_up ? s_p[0] + s_p[1] + s_p[2] + s_p[3] : J.psum[blockIdx.x];
+  uint32_t prefix = static_cast<uint32_t>(before) + excl;
 #pragma unroll
   for (int i = 0; i < kItems; ++i) {
-    if (base + i < n) out[base + i] = prefix;
+    if (base + i < n) J.out[base + i] = prefix;
     prefix += v[i];
   }
-  if (total && blockIdx.x == gridDim.x - 1 && threadIdx.x == 255) *total = prefix;
+  if (last && threadIdx.x == 255) {
+    if (J.total) *J.total = prefix;
+    if (J.total64) *J.total64 = before + J.partial[blockIdx.x];
+  }
 }
 
-__global__ void k_set_u32(uint32_t *p, uint32_t v) { *p = v; }
+// The whole scan in one workgroup, for at most kOneScan elements.
+constexpr int kOneThreads = 1024;
+constexpr int64_t kOneScan = kOneThreads * kItems;
+template <class In>
+__global__ __launch_bounds__(kOneThreads) void k_scan_one(Jobs<In> jobs, int64_t cap,
+                                                          const uint32_t *dn) {
+  __shared__ uint32_t s_w[kOneThreads / 64];
+  __shared__ uint64_t s_p[kOneThreads / 64];
+  const Job<In> &J = jobs.j[blockIdx.y];
+  const int64_t n = count_of(cap, dn);
+  const int64_t base = static_cast<int64_t>(threadIdx.x) * kItems;
+  uint32_t v[kItems];
+  uint32_t sum = 0;
+  uint64_t wide = 0;
+#pragma unroll
+  for (int i = 0; i < kItems; ++i) {
+    v[i] = (base + i < n) ? J.in(base + i) : 0u;
+    sum += v[i];
+    wide += v[i];
+  }
+  if (J.total64) {
+    wide = wave_reduce(wide);
+    if ((threadIdx.x & 63) == 0) s_p[threadIdx.x >> 6] = wide;
+  }
+  uint32_t prefix = block_excl_scan<kOneThreads / 64>(sum, s_w);
+#pragma unroll
+  for (int i = 0; i < kItems; ++i) {
+    if (base + i < n) J.out[base + i] = prefix;
+    prefix += v[i];
+  }
+  if (threadIdx.x == kOneThreads - 1) {
+    if (J.total) *J.total = prefix;
+    if (J.total64) {
+      wide = 0;
+      for (int w = 0; w < kOneThreads / 64; ++w) wide += s_p[w];
+      *J.total64 = wide;
+    }
+  }
+}
+
+__global__ void k_set_totals(uint32_t *total, uint64_t *total64) {
+  if (total) *total = 0;
+  if (total64) *total64 = 0;
+}
+
+constexpr int64_t kDirectTiles = 8192;  // tile sums that a tile adds up itself
 
 // n: the element count, or with dn the capacity the launches are sized for
 // (the count itself then read from *dn on the device).
 template <class In>
-void scan_impl(In in, uint32_t *out, int64_t n, uint32_t *total, Workspace &ws, hipStream_t s,
-               int level, const uint32_t *dn) {
+void scan_impl(Jobs<In> jobs, unsigned nj, int64_t n, Workspace &ws, hipStream_t s, int level,
+               const uint32_t *dn) {
   if (n <= 0) {
-    if (total) k_set_u32<<<1, 1, 0, s>>>(total, 0u);
+    for (unsigned y = 0; y < nj; ++y)
+      if (jobs.j[y].total || jobs.j[y].total64)
+        k_set_totals<<<1, 1, 0, s>>>(jobs.j[y].total, jobs.j[y].total64);
+    return;
+  }
+  if (n <= kOneScan) {
+    k_scan_one<In><<<dim3(1, nj), kOneThreads, 0, s>>>(jobs, n, dn);
     return;
   }
   const int64_t nb = (n + kTile - 1) / kTile;
-  if (nb == 1) {
-    k_scan_apply<In><<<1, 256, 0, s>>>(in, out, n, dn, nullptr, total);
-    return;
-  }
   if (level >= 4) throw HipError{hipErrorInvalidValue, "scan too deep"};
-  uint32_t *partial = ws.get_as<uint32_t>(S_SCAN0 + level, static_cast<size_t>(nb));
-  k_scan_reduce<In><<<static_cast<unsigned>(nb), 256, 0, s>>>(in, n, dn, partial);
-  scan_impl(LoadU32{partial}, partial, nb, nullptr, ws, s, level + 1, nullptr);
-  k_scan_apply<In><<<static_cast<unsigned>(nb), 256, 0, s>>>(in, out, n, dn, partial, total);
+  uint64_t *partial = ws.get_as<uint64_t>(S_SCAN0 + level, 4 * static_cast<size_t>(nb));
+  for (unsigned y = 0; y < nj; ++y) {
+    jobs.j[y].partial = partial + 2 * y * nb;
+    jobs.j[y].psum = nullptr;
+  }
+  const dim3 grid(static_cast<unsigned>(nb), nj);
+  k_scan_reduce<In><<<grid, 256, 0, s>>>(jobs, n, dn);
+  if (nb > kDirectTiles) {
+    Jobs<LoadLow32> up{};
+    for (unsigned y = 0; y < nj; ++y) {
+      jobs.j[y].psum = reinterpret_cast<uint32_t *>(partial + (2 * y + 1) * nb);
+      up.j[y].in.p = jobs.j[y].partial;
+      up.j[y].out = jobs.j[y].psum;
+    }
+    scan_impl(up, nj, nb, ws, s, level + 1, nullptr);
+  }
+  k_scan_apply<In><<<grid, 256, 0, s>>>(jobs, n, dn);
 }
 
 template <int BITS>
 __global__ __launch_bounds__(256) void k_rs_hist(const uint32_t *keys, int64_t cap,
                                                  const uint32_t *dn, int shift, uint32_t *hist,
-                                                 int64_t nblocks) {
+                                                 int64_t nblocks, bool tile_major) {
   const int64_t n = count_of(cap, dn);
   constexpr int R = 1 << BITS;
   constexpr uint32_t M = R - 1;
@@ -168,39 +269,24 @@ __global__ __launch_bounds__(256) void k_rs_hist(const uint32_t *keys, int64_t c
   }
   __syncthreads();
   for (int d = threadIdx.x; d < R; d += 256)
-    hist[static_cast<int64_t>(d) * nblocks + blockIdx.x] = h[0][d] + h[1][d] + h[2][d] + h[3][d];
+    hist[tile_major ? static_cast<int64_t>(blockIdx.x) * R + d
+                    : static_cast<int64_t>(d) * nblocks + blockIdx.x] =
+        h[0][d] + h[1][d] + h[2][d] + h[3][d];
 }
 
+// Ranks a wave's kItems keys (striped: item it of lane l is input it * 64 + l)
+// by digit, in input order: rk[it] = rank among the wave's equal digits, counts
+// per digit in wh (zeroed by the caller).
 template <int BITS>
-__global__ __launch_bounds__(256) void k_rs_scatter(const uint32_t *kin, const uint32_t *vin,
-                                                    uint32_t *kout, uint32_t *vout, int64_t cap,
-                                                    const uint32_t *dn, int shift,
-                                                    const uint32_t *hist, int64_t nblocks) {
-  const int64_t n = count_of(cap, dn);
-  constexpr int R = 1 << BITS;
-  constexpr uint32_t M = R - 1;
-  constexpr int DPT = (R + 255) / 256;  // digits per thread in the block scan
-  __shared__ uint32_t wh[4][R];         // per-wave digit counts -> offsets
-  __shared__ uint32_t dstart[R];        // block-local start of each digit run
-  __shared__ uint32_t gbase[R];         // global start of (digit, this tile)
-  __shared__ uint32_t sk[kTile], sv[kTile];
-  __shared__ uint32_t s_w[4];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  for (int i = threadIdx.x; i < 4 * R; i += 256) (&wh[0][0])[i] = 0;
-  for (int d = threadIdx.x; d < R; d += 256)
-    gbase[d] = hist[static_cast<int64_t>(d) * nblocks + blockIdx.x];
-  __syncthreads();
-  const int64_t tbase = static_cast<int64_t>(blockIdx.x) * kTile;
-  const int64_t base = tbase + wave * (kTile / 4);
+__device__ __forceinline__ void wave_rank(const uint32_t (&kk)[kItems], const bool (&ok)[kItems],
+                                          int shift, int lane, uint32_t *wh,
+                                          uint32_t (&rk)[kItems]) {
+  constexpr uint32_t M = (1u << BITS) - 1;
   const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  uint32_t kk[kItems], vv[kItems], rk[kItems];
 #pragma unroll
   for (int it = 0; it < kItems; ++it) {
-    const int64_t idx = base + it * 64 + lane;
-    const bool valid = idx < n;
-    const uint32_t key = valid ? kin[idx] : 0u;
-    const uint32_t d = (key >> shift) & M;
-    uint64_t m = __ballot(valid);
+    const uint32_t d = (kk[it] >> shift) & M;
+    uint64_t m = __ballot(ok[it]);
 #pragma unroll
     for (int b = 0; b < BITS; ++b) {
       const bool bit = (d >> b) & 1u;
@@ -212,14 +298,17 @@ __global__ __launch_bounds__(256) void k_rs_scatter(const uint32_t *kin, const u
     // the lowest lane of each peer group reserves cnt slots; peers read its base
     const int leader = __ffsll(static_cast<long long>(m)) - 1;
     uint32_t old = 0;
-    if (valid && rank_in == 0) old = atomicAdd(&wh[wave][d], cnt);
+    if (ok[it] && rank_in == 0) old = atomicAdd(&wh[d], cnt);
     old = __shfl(old, leader & 63, 64);
-    kk[it] = key;
-    vv[it] = valid ? vin[idx] : 0u;
     rk[it] = old + rank_in;
   }
-  __syncthreads();
-  // digit totals of the tile -> wave offsets within each digit, digit starts
+}
+
+// Digit totals of the block's 4 waves (wh[w][d] counts) to the wave offsets
+// within each digit (wh) and the start of each digit's run (dstart).
+template <int R>
+__device__ __forceinline__ void digit_starts(uint32_t (*wh)[R], uint32_t *dstart, uint32_t *s_w) {
+  constexpr int DPT = (R + 255) / 256;  // digits per thread in the block scan
   uint32_t tot[DPT];
   uint32_t tsum = 0;
 #pragma unroll
@@ -244,11 +333,74 @@ __global__ __launch_bounds__(256) void k_rs_scatter(const uint32_t *kin, const u
     if (d < R) dstart[d] = start;
     start += tot[j];
   }
+}
+
+// DIRECT: hist holds the tiles' own histograms, tile-major, and the workgroup
+// sums them to its digits' global starts; else their digit-major scan.
+template <int BITS, bool DIRECT>
+__global__ __launch_bounds__(256) void k_rs_scatter(const uint32_t *kin, const uint32_t *vin,
+                                                    uint32_t *kout, uint32_t *vout, int64_t cap,
+                                                    const uint32_t *dn, int shift,
+                                                    const uint32_t *hist, int64_t nblocks) {
+  const int64_t n = count_of(cap, dn);
+  constexpr int R = 1 << BITS;
+  constexpr uint32_t M = R - 1;
+  constexpr int DPT = (R + 255) / 256;
+  __shared__ uint32_t wh[4][R];   // per-wave digit counts -> offsets
+  __shared__ uint32_t dstart[R];  // block-local start of each digit run
+  __shared__ uint32_t gbase[R];   // global start of (digit, this tile)
+  __shared__ uint32_t sk[kTile], sv[kTile];
+  __shared__ uint32_t s_w[4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t tbase = static_cast<int64_t>(blockIdx.x) * kTile;
+  if (tbase >= n) return;  // a tile past the device count (uniform)
+  for (int i = threadIdx.x; i < 4 * R; i += 256) (&wh[0][0])[i] = 0;
+  if (DIRECT) {
+    // thread t: digits [t DPT, t DPT + DPT), counts below this tile and in all
+    uint32_t below[DPT], all[DPT], sum = 0;
+#pragma unroll
+    for (int j = 0; j < DPT; ++j) {
+      const int d = threadIdx.x * DPT + j;
+      below[j] = all[j] = 0;
+      if (d < R) {
+#pragma unroll 8
+        for (int b = 0; b < static_cast<int>(nblocks); ++b) {
+          const uint32_t h = hist[static_cast<int64_t>(b) * R + d];
+          all[j] += h;
+          below[j] += b < static_cast<int>(blockIdx.x) ? h : 0u;
+        }
+      }
+      sum += all[j];
+    }
+    uint32_t start = block_excl_scan(sum, s_w);
+#pragma unroll
+    for (int j = 0; j < DPT; ++j) {
+      const int d = threadIdx.x * DPT + j;
+      if (d < R) gbase[d] = start + below[j];
+      start += all[j];
+    }
+  } else {
+    for (int d = threadIdx.x; d < R; d += 256)
+      gbase[d] = hist[static_cast<int64_t>(d) * nblocks + blockIdx.x];
+  }
   __syncthreads();
+  const int64_t base = tbase + wave * (kTile / 4);
+  uint32_t kk[kItems], vv[kItems], rk[kItems];
+  bool ok[kItems];
 #pragma unroll
   for (int it = 0; it < kItems; ++it) {
     const int64_t idx = base + it * 64 + lane;
-    if (idx < n) {
+    ok[it] = idx < n;
+    kk[it] = ok[it] ? kin[idx] : 0u;
+    vv[it] = ok[it] ? vin[idx] : 0u;
+  }
+  wave_rank<BITS>(kk, ok, shift, lane, wh[wave], rk);
+  __syncthreads();
+  digit_starts<R>(wh, dstart, s_w);
+  __syncthreads();
+#pragma unroll
+  for (int it = 0; it < kItems; ++it) {
+    if (ok[it]) {
       const uint32_t d = (kk[it] >> shift) & M;
       const uint32_t lp = dstart[d] + wh[wave][d] + rk[it];
       sk[lp] = kk[it];
@@ -266,28 +418,105 @@ __global__ __launch_bounds__(256) void k_rs_scatter(const uint32_t *kin, const u
   }
 }
 
+// The whole sort in one workgroup, for at most kTile pairs: digits of 8 bits
+// (the last pass's digit is cut at end_bit).
+__global__ __launch_bounds__(256) void k_rs_one(const uint32_t *kin, const uint32_t *vin,
+                                                uint32_t *kout, uint32_t *vout, int64_t cap,
+                                                const uint32_t *dn, int begin_bit, int end_bit) {
+  const int n = static_cast<int>(count_of(cap, dn));
+  constexpr int R = 256;
+  __shared__ uint32_t wh[4][R], dstart[R], sk[kTile], sv[kTile], s_w[4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int base = wave * (kTile / 4);
+  uint32_t kk[kItems], vv[kItems], rk[kItems];
+  bool ok[kItems];
+#pragma unroll
+  for (int it = 0; it < kItems; ++it) {
+    const int idx = base + it * 64 + lane;
+    ok[it] = idx < n;
+    kk[it] = ok[it] ? kin[idx] : 0u;
+    vv[it] = ok[it] ? vin[idx] : 0u;
+  }
+  const uint32_t keep = end_bit < 32 ? (1u << end_bit) - 1u : ~0u;
+  for (int shift = begin_bit; shift < end_bit; shift += 8) {
+    for (int i = threadIdx.x; i < 4 * R; i += 256) (&wh[0][0])[i] = 0;
+    __syncthreads();
+    uint32_t dk[kItems];
+#pragma unroll
+    for (int it = 0; it < kItems; ++it) dk[it] = kk[it] & keep;
+    wave_rank<8>(dk, ok, shift, lane, wh[wave], rk);
+    __syncthreads();
+    digit_starts<R>(wh, dstart, s_w);
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < kItems; ++it) {
+      if (ok[it]) {
+        const uint32_t d = (dk[it] >> shift) & (R - 1);
+        const uint32_t lp = dstart[d] + wh[wave][d] + rk[it];
+        sk[lp] = kk[it];
+        sv[lp] = vv[it];
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < kItems; ++it) {
+      const int idx = base + it * 64 + lane;
+      if (ok[it]) {
+        kk[it] = sk[idx];
+        vv[it] = sv[idx];
+      }
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int it = 0; it < kItems; ++it) {
+    const int idx = base + it * 64 + lane;
+    if (ok[it]) {
+      kout[idx] = kk[it];
+      vout[idx] = vv[it];
+    }
+  }
+}
+
+constexpr int64_t kDirectSort = 128;  // tiles whose histograms a scatter workgroup sums itself
+
 template <int BITS>
 void rs_pass(const uint32_t *sk, const uint32_t *sv, uint32_t *dk, uint32_t *dv, int64_t n,
              const uint32_t *dn, int shift, int64_t nb, uint32_t *hist, Workspace &ws,
              hipStream_t s) {
-  k_rs_hist<BITS><<<static_cast<unsigned>(nb), 256, 0, s>>>(sk, n, dn, shift, hist, nb);
-  scan_u32(hist, hist, (int64_t(1) << BITS) * nb, nullptr, ws, s, 0);
-  k_rs_scatter<BITS><<<static_cast<unsigned>(nb), 256, 0, s>>>(sk, sv, dk, dv, n, dn, shift,
-                                                               hist, nb);
+  const bool direct = nb <= kDirectSort;
+  const unsigned g = static_cast<unsigned>(nb);
+  k_rs_hist<BITS><<<g, 256, 0, s>>>(sk, n, dn, shift, hist, nb, direct);
+  if (direct) {
+    k_rs_scatter<BITS, true><<<g, 256, 0, s>>>(sk, sv, dk, dv, n, dn, shift, hist, nb);
+  } else {
+    scan_u32(hist, hist, (int64_t(1) << BITS) * nb, nullptr, ws, s);
+    k_rs_scatter<BITS, false><<<g, 256, 0, s>>>(sk, sv, dk, dv, n, dn, shift, hist, nb);
+  }
   hip_check(hipGetLastError(), "radix sort launch");
 }
 
 }  // namespace
 
 void scan_u32(const uint32_t *in, uint32_t *out, int64_t n, uint32_t *total, Workspace &ws,
-              hipStream_t s, int level, const uint32_t *dn) {
-  scan_impl(LoadU32{in}, out, n, total, ws, s, level, dn);
+              hipStream_t s, const uint32_t *dn, uint64_t *total64) {
+  scan_impl(Jobs<LoadU32>{{{{in}, out, total, total64, nullptr, nullptr}, {}}}, 1, n, ws, s, 0, dn);
   hip_check(hipGetLastError(), "scan_u32 launch");
+}
+
+void scan_u32_pair(const uint32_t *in0, uint32_t *out0, uint32_t *total0, uint64_t *total64,
+                   const uint32_t *in1, uint32_t *out1, uint32_t *total1, int64_t n, Workspace &ws,
+                   hipStream_t s, const uint32_t *dn) {
+  scan_impl(Jobs<LoadU32>{{{{in0}, out0, total0, total64, nullptr, nullptr},
+                           {{in1}, out1, total1, nullptr, nullptr, nullptr}}},
+            2, n, ws, s, 0, dn);
+  hip_check(hipGetLastError(), "scan_u32_pair launch");
 }
 
 void scan_u8bit(const uint8_t *flags, uint8_t bits, uint32_t *out, int64_t n, uint32_t *total,
                 Workspace &ws, hipStream_t s) {
-  scan_impl(LoadU8Bit{flags, bits}, out, n, total, ws, s, 0, nullptr);
+  scan_impl(Jobs<LoadU8Bit>{{{{flags, bits}, out, total, nullptr, nullptr, nullptr}, {}}}, 1, n, ws,
+            s, 0, nullptr);
   hip_check(hipGetLastError(), "scan_u8bit launch");
 }
 
@@ -295,6 +524,11 @@ int radix_sort_pairs(uint32_t *k0, uint32_t *v0, uint32_t *k1, uint32_t *v1, int
                      int begin_bit, int end_bit, Workspace &ws, hipStream_t s,
                      const uint32_t *dn) {
   if (n <= 1 || end_bit <= begin_bit) return 0;
+  if (n <= kTile) {
+    k_rs_one<<<1, 256, 0, s>>>(k0, v0, k1, v1, n, dn, begin_bit, end_bit);
+    hip_check(hipGetLastError(), "k_rs_one launch");
+    return 1;
+  }
   const int64_t nb = (n + kTile - 1) / kTile;
   const int bits = end_bit - begin_bit;
   const int passes = (bits + kMaxBits - 1) / kMaxBits;

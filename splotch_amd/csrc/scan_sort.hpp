@@ -10,12 +10,17 @@
 
 namespace splhip {
 
-// out[i] = sum_{j<i} in[j] over n elements (in == out allowed).  If total is
-// non-null the grand total is stored there (device).  Scratch: S_SCAN0+level.
-// dn (device, optional): the element count is min(n, *dn), read on the device
-// (launches sized for n elements; no host wait).
+// out[i] = sum_{j<i} in[j] over n elements (in == out allowed).  total /
+// total64 (device, optional): the grand total in 32 and 64 bits.  Scratch:
+// S_SCAN0+level.  dn (device, optional): the element count is min(n, *dn),
+// read on the device (launches sized for n elements; no host wait).
 void scan_u32(const uint32_t *in, uint32_t *out, int64_t n, uint32_t *total, Workspace &ws,
-              hipStream_t s, int level = 0, const uint32_t *dn = nullptr);
+              hipStream_t s, const uint32_t *dn = nullptr, uint64_t *total64 = nullptr);
+
+// Two scans of n elements each in the launches of one (total64: of the first).
+void scan_u32_pair(const uint32_t *in0, uint32_t *out0, uint32_t *total0, uint64_t *total64,
+                   const uint32_t *in1, uint32_t *out1, uint32_t *total1, int64_t n, Workspace &ws,
+                   hipStream_t s, const uint32_t *dn = nullptr);
 
 // Same with in[i] = ((flags[i] & bits) != 0).
 void scan_u8bit(const uint8_t *flags, uint8_t bits, uint32_t *out, int64_t n, uint32_t *total,

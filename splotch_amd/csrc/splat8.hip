@@ -1735,6 +1735,18 @@ __global__ __launch_bounds__(256) void k_items_count(SplatArgs a, uint32_t nunit
   }
 }
 
+// Sort key of a list: the long lists (one item each) first, then by length in
+// quarter octaves, longest first.  8 bits are one radix pass; the splats only
+// need the order of scheduling, not the exact lengths.
+__device__ __forceinline__ uint32_t item_key(uint32_t len, uint32_t long_len) {
+  uint32_t q = 0;
+  if (len > 0) {
+    const uint32_t e = 31u - static_cast<uint32_t>(__clz(static_cast<int>(len)));
+    q = 4u * e + ((e >= 2u ? len >> (e - 2u) : len << (2u - e)) & 3u);
+  }
+  return (len >= long_len ? 0u : 128u) + 127u - q;
+}
+
 __global__ __launch_bounds__(256) void k_items_emit(SplatArgs a, uint32_t nunits, int ordered,
                                                     uint32_t split, const uint32_t *off,
                                                     uint32_t *keys, uint32_t *vals) {
@@ -1743,7 +1755,7 @@ __global__ __launch_bounds__(256) void k_items_emit(SplatArgs a, uint32_t nunits
     const uint32_t k = unit_items(a, static_cast<uint32_t>(u), ordered, split, len);
     const uint32_t o = off[u];
     for (uint32_t c = 0; c < k; ++c) {
-      keys[o + c] = ~len;  // ascending sort of ~len = heaviest first
+      keys[o + c] = item_key(len, long_len_of(a));
       vals[o + c] = (static_cast<uint32_t>(u) << 2) | (k == 3 ? c : 3u);
     }
   }
@@ -1811,20 +1823,19 @@ unsigned resident_grid(const void *k, int slot) {
   return r;
 }
 
-// Grid of a kernel that walks the staged batches: at most `batches`; about
-// `per` per wave when there are many, in one round of resident workgroups (a
-// second round would queue behind the 8x8 splat's workgroups, and the chains
-// wait for all of them).
-static unsigned stage_grid(const void *k, int slot, uint64_t batches, unsigned per) {
-  return std::max(1u, static_cast<unsigned>(std::min<uint64_t>(
-                          resident_grid(k, slot), (batches + 4 * per - 1) / (4 * per))));
+// Grid of a kernel that walks the staged batches (at most `batches`): a wave
+// per batch up to one round of resident workgroups (a second round would queue
+// behind the 8x8 splat's workgroups, and the chains wait for all of them).
+static unsigned stage_grid(const void *k, int slot, uint64_t batches) {
+  return std::max(1u, static_cast<unsigned>(
+                          std::min<uint64_t>(resident_grid(k, slot), (batches + 3) / 4)));
 }
 
 void launch_stage_rows(const uint32_t *items, uint32_t i0, uint32_t i1, uint64_t batches,
                        const uint32_t *cbat, uint64_t *masks, uint32_t *rows, const SplatArgs &a,
                        hipStream_t s, const uint32_t *dn) {
   if (i1 <= i0) return;
-  const unsigned grid = stage_grid(reinterpret_cast<const void *>(k_stage_rows), 2, batches, 4);
+  const unsigned grid = stage_grid(reinterpret_cast<const void *>(k_stage_rows), 2, batches);
   k_stage_rows<<<grid, 256, 0, s>>>(a, items, i0, i1, cbat, masks, rows, dn);
   hip_check(hipGetLastError(), "k_stage_rows launch");
 }
@@ -1837,7 +1848,7 @@ void launch_stage_ops(bool additive, const uint32_t *items, uint32_t i0, uint32_
   if (i1 <= i0) return;
   const void *k = additive ? reinterpret_cast<const void *>(k_stage_ops<1>)
                            : reinterpret_cast<const void *>(k_stage_ops<0>);
-  const unsigned grid = stage_grid(k, additive ? 1 : 0, batches, 4);
+  const unsigned grid = stage_grid(k, additive ? 1 : 0, batches);
   if (additive)
     k_stage_ops<1><<<grid, 256, 0, s>>>(a, items, i0, i1, cbase, cbat, masks, rows, gofs, ops,
                                         stride, dn);
