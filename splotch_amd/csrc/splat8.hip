@@ -120,12 +120,38 @@ __device__ __forceinline__ int xexp_index(float p) {
   return static_cast<int>(ok ? p : 0.f);
 }
 
-// x where row cy of the column mask m is set (the pixel is in the particle's
-// footprint), else +0: the row's bit, sign-extended, masks x's bits.
-__device__ __forceinline__ float in_footprint(float x, uint32_t m, int cy) {
-  const uint32_t all = static_cast<uint32_t>(__builtin_amdgcn_sbfe(static_cast<int>(m), cy, 1));
+// v of the lane j of every group of four lanes (a DPP operand of the
+// instruction that uses it, at no instruction of its own).
+template <int J>
+__device__ __forceinline__ float quad_lane(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), J * 0x55, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float quad_of(float v, int j) {  // j: constant after unrolling
+  switch (j & 3) {
+    case 0: return quad_lane<0>(v);
+    case 1: return quad_lane<1>(v);
+    case 2: return quad_lane<2>(v);
+    default: return quad_lane<3>(v);
+  }
+}
+__device__ __forceinline__ float4 quad_of(const float4 &v, int j) {
+  return make_float4(quad_of(v.x, j), quad_of(v.y, j), quad_of(v.z, j), quad_of(v.w, j));
+}
+// v of lane k (wave-uniform, k < 4) of the wave's first four lanes.
+__device__ __forceinline__ float4 chunk_lane(const float4 &v, int k) {
+  return make_float4(lane_f(v.x, k), lane_f(v.y, k), lane_f(v.z, k), lane_f(v.w, k));
+}
+
+// x where bit 8 (j & 3) of the pixel's coverage word m is set (byte j: particle
+// j of four, shifted down by the pixel's row), else +0: the bit, sign-extended,
+// masks x's bits.
+__device__ __forceinline__ float covered(float x, uint32_t m, int j) {
+  const uint32_t all =
+      static_cast<uint32_t>(__builtin_amdgcn_sbfe(static_cast<int>(m), 8 * (j & 3), 1));
   return __uint_as_float(__float_as_uint(x) & all);
 }
+
+constexpr int kColPad = 68;  // bytes per column of coverage (a word per four particles)
 
 // One fast chunk of the ordered walk (all particles of the chunk have every
 // a_c in [kFastA, 0] and finite q_c) for channel class CH: J particles from
@@ -133,44 +159,67 @@ __device__ __forceinline__ float in_footprint(float x, uint32_t m, int cy) {
 // Taylor branch at every pixel of its footprint in the block, so its update
 // is l += ((l - q) * a) * att (att replaced by +0 outside the footprint) with
 // no table work.
+//
+// The walk is bound by the CU's LDS, which returns 128 B per clock (a b32
+// read of a wave 2 clocks, a b128 read 8, whether or not the lanes share
+// addresses; a random table lookup about 6), before its VALU.  So the
+// constants of four particles are read once, lane l those of particle l % 4,
+// and reach the operations as quad-permuted DPP operands (2 clocks more per
+// use, against 16 LDS clocks per particle), and four particles' coverage of a
+// column is one word: 47 -> 33 LDS clocks per particle in the expm1 branch, 22
+// -> 9 in the Taylor branch.
 template <int CH, int J, uint32_t TB>
-__device__ __forceinline__ void fast_chunk(int k0, int cx, int cy, const uint32_t (*cmask)[kPad],
+__device__ __forceinline__ void fast_chunk(int k0, int cx, int cy, const uint8_t (*col)[kColPad],
                                            const float (*pre2)[kPad],
                                            const float (*pre1)[kPad], const float *tab,
                                            const float4 *cst, float expfac4, float tl,
                                            float &l0, float &l1, float &l2) {
   constexpr bool C0 = (CH == 3 || CH == 0), C1 = (CH == 3 || CH == 1), C2 = (CH == 3 || CH == 2);
-  float m2[J], g0[J], g1[J], g2[J], u0[J], w0[J], u1[J], w1[J], u2[J], w2[J];
-  float4 ca[J], cq[J];
+  constexpr int JQ = (J + 3) / 4;
+  float at[J], m2[J], g0[J], g1[J], g2[J], u0[J], w0[J], u1[J], w1[J], u2[J], w2[J];
+  float4 ca[JQ], cq[JQ];
+  uint32_t cov[JQ];
   bool tay[J];
   // slots past the batch hold finite values of earlier batches (or
   // zeros) and are masked; table offsets are masked into the tables
 #pragma unroll
-  for (int j = 0; j < J; ++j) {
-    const int k = k0 + j;
-    ca[j] = cst[2 * k];
-    cq[j] = cst[2 * k + 1];
+  for (int q = 0; q < JQ; ++q) {
+    const int k = (k0 & ~3) + 4 * q;
+    ca[q] = cst[2 * (k + (cy & 3))];
+    cq[q] = cst[2 * (k + (cy & 3)) + 1];
+    cov[q] = *reinterpret_cast<const uint32_t *>(&col[cx][k]) >> cy;
+    if (J < 4) cov[q] >>= 8 * (k0 & 3);
   }
 #pragma unroll
   for (int j = 0; j < J; ++j) {
     const int k = k0 + j;
-    const float at = pre1[cy][k] * pre2[cx][k];
+    at[j] = covered(pre1[cy][k] * pre2[cx][k], cov[j / 4], j);
+  }
+  // (chunks of fewer than four start inside a group of four: their constants
+  // come by lane from there)
+  auto con = [&](const float4 &v, int j) {
+    return J < 4 ? chunk_lane(v, (k0 & 3) + j) : quad_of(v, j);
+  };
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
     if ((TB >> j) & 1u) {
-      m2[j] = in_footprint(at, cmask[cx][k], cy);
+      m2[j] = at[j];
       continue;
     }
-    tay[j] = (ca[j].w * at) < tl;
-    m2[j] = in_footprint(tay[j] ? at : 1.f, cmask[cx][k], cy);
-    if (C0) { g0[j] = at * ca[j].x; xtab_fast(tab, g0[j], expfac4, u0[j], w0[j]); }
-    if (C1) { g1[j] = at * ca[j].y; xtab_fast(tab, g1[j], expfac4, u1[j], w1[j]); }
-    if (C2) { g2[j] = at * ca[j].z; xtab_fast(tab, g2[j], expfac4, u2[j], w2[j]); }
+    const float4 a4 = con(ca[j / 4], j);
+    tay[j] = (a4.w * at[j]) < tl;
+    m2[j] = tay[j] ? at[j] : 1.f;
+    if (C0) { g0[j] = at[j] * a4.x; xtab_fast(tab, g0[j], expfac4, u0[j], w0[j]); }
+    if (C1) { g1[j] = at[j] * a4.y; xtab_fast(tab, g1[j], expfac4, u1[j], w1[j]); }
+    if (C2) { g2[j] = at[j] * a4.z; xtab_fast(tab, g2[j], expfac4, u2[j], w2[j]); }
   }
 #pragma unroll
   for (int j = 0; j < J; ++j) {
+    const float4 a4 = con(ca[j / 4], j), q4 = con(cq[j / 4], j);
     if ((TB >> j) & 1u) {
-      if (C0) l0 = l0 + ((l0 - cq[j].x) * ca[j].x) * m2[j];
-      if (C1) l1 = l1 + ((l1 - cq[j].y) * ca[j].y) * m2[j];
-      if (C2) l2 = l2 + ((l2 - cq[j].z) * ca[j].z) * m2[j];
+      if (C0) l0 = l0 + ((l0 - q4.x) * a4.x) * m2[j];
+      if (C1) l1 = l1 + ((l1 - q4.y) * a4.y) * m2[j];
+      if (C2) l2 = l2 + ((l2 - q4.z) * a4.z) * m2[j];
       continue;
     }
     // the table product is formed before the select: written inside
@@ -179,20 +228,20 @@ __device__ __forceinline__ void fast_chunk(int k0, int cx, int cy, const uint32_
     if (C0) {
       const float ex = u0[j] * w0[j] - 1.f;
       const float em = (fabsf(g0[j]) < tl) ? g0[j] : ex;
-      const float m1 = tay[j] ? ca[j].x : em;
-      l0 = l0 + ((l0 - cq[j].x) * m1) * m2[j];
+      const float m1 = tay[j] ? a4.x : em;
+      l0 = l0 + ((l0 - q4.x) * m1) * m2[j];
     }
     if (C1) {
       const float ex = u1[j] * w1[j] - 1.f;
       const float em = (fabsf(g1[j]) < tl) ? g1[j] : ex;
-      const float m1 = tay[j] ? ca[j].y : em;
-      l1 = l1 + ((l1 - cq[j].y) * m1) * m2[j];
+      const float m1 = tay[j] ? a4.y : em;
+      l1 = l1 + ((l1 - q4.y) * m1) * m2[j];
     }
     if (C2) {
       const float ex = u2[j] * w2[j] - 1.f;
       const float em = (fabsf(g2[j]) < tl) ? g2[j] : ex;
-      const float m1 = tay[j] ? ca[j].z : em;
-      l2 = l2 + ((l2 - cq[j].z) * m1) * m2[j];
+      const float m1 = tay[j] ? a4.z : em;
+      l2 = l2 + ((l2 - q4.z) * m1) * m2[j];
     }
   }
 }
@@ -208,7 +257,7 @@ __device__ __forceinline__ void fast_chunk(int k0, int cx, int cy, const uint32_
 // are -0, so they never hold -0 and l + 0 == l bit for bit: the result equals
 // the reference's skip.
 template <int ADD, int CH, int J>
-__device__ __forceinline__ void walk_chunks(int nb, int cx, int cy, const uint32_t (*cmask)[kPad],
+__device__ __forceinline__ void walk_chunks(int nb, int cx, int cy, const uint8_t (*col)[kColPad],
                                             const float (*pre2)[kPad], const float (*pre1)[kPad],
                                             const float *tab, float va0, float va1, float va2,
                                             float vq0, float vq1, float vq2, float vmax,
@@ -240,7 +289,7 @@ __device__ __forceinline__ void walk_chunks(int nb, int cx, int cy, const uint32
         const uint32_t tb = static_cast<uint32_t>(taymask >> k0);
         if (CH == 3 && J == 4) {
           switch (tb & 15u) {
-#define SPLHIP_FAST(T) case T: fast_chunk<CH, J, T>(k0, cx, cy, cmask, pre2, pre1, tab, cst, expfac4, tl, l0, l1, l2); break;
+#define SPLHIP_FAST(T) case T: fast_chunk<CH, J, T>(k0, cx, cy, col, pre2, pre1, tab, cst, expfac4, tl, l0, l1, l2); break;
             SPLHIP_FAST(0) SPLHIP_FAST(1) SPLHIP_FAST(2) SPLHIP_FAST(3)
             SPLHIP_FAST(4) SPLHIP_FAST(5) SPLHIP_FAST(6) SPLHIP_FAST(7)
             SPLHIP_FAST(8) SPLHIP_FAST(9) SPLHIP_FAST(10) SPLHIP_FAST(11)
@@ -248,30 +297,33 @@ __device__ __forceinline__ void walk_chunks(int nb, int cx, int cy, const uint32
 #undef SPLHIP_FAST
           }
         } else {
-          fast_chunk<CH, J, 0u>(k0, cx, cy, cmask, pre2, pre1, tab, cst, expfac4, tl, l0, l1, l2);
+          fast_chunk<CH, J, 0u>(k0, cx, cy, col, pre2, pre1, tab, cst, expfac4, tl, l0, l1, l2);
         }
         continue;
       }
     } else {
-      // Additive: the particles' a_c come from LDS (cst: (a0, a1, a2, 0)) as
-      // vector operands, and slots past the batch (stale or uninitialised
-      // values) are read at their own offsets and masked by the select, so
-      // no address or lane read is computed per particle.
+      // Additive: constants and coverage as in the fast chunks (cst: (a0, a1,
+      // a2, 0)); slots past the batch (stale or uninitialised values) are read
+      // at their own offsets and their products masked, as their coverage is 0.
+      constexpr int JQ = (J + 3) / 4;
       float at[J];
-      float4 ca[J];
-      uint32_t mv[J];
+      float4 ca[JQ];
+      uint32_t cov[JQ];
 #pragma unroll
-      for (int j = 0; j < J; ++j) {
-        const int k = k0 + j;
-        ca[j] = cst[k];
-        mv[j] = cmask[cx][k];
-        at[j] = pre1[cy][k] * pre2[cx][k];
+      for (int q = 0; q < JQ; ++q) {
+        const int k = (k0 & ~3) + 4 * q;
+        ca[q] = cst[k + (cy & 3)];
+        cov[q] = *reinterpret_cast<const uint32_t *>(&col[cx][k]) >> cy;
+        if (J < 4) cov[q] >>= 8 * (k0 & 3);
       }
 #pragma unroll
+      for (int j = 0; j < J; ++j) at[j] = pre1[cy][k0 + j] * pre2[cx][k0 + j];
+#pragma unroll
       for (int j = 0; j < J; ++j) {
-        if (C0) l0 = l0 + in_footprint(ca[j].x * at[j], mv[j], cy);
-        if (C1) l1 = l1 + in_footprint(ca[j].y * at[j], mv[j], cy);
-        if (C2) l2 = l2 + in_footprint(ca[j].z * at[j], mv[j], cy);
+        const float4 a4 = J < 4 ? chunk_lane(ca[j / 4], (k0 & 3) + j) : quad_of(ca[j / 4], j);
+        if (C0) l0 = l0 + covered(a4.x * at[j], cov[j / 4], j);
+        if (C1) l1 = l1 + covered(a4.y * at[j], cov[j / 4], j);
+        if (C2) l2 = l2 + covered(a4.z * at[j], cov[j / 4], j);
       }
       continue;
     }
@@ -281,7 +333,7 @@ __device__ __forceinline__ void walk_chunks(int nb, int cx, int cy, const uint32
 #pragma unroll
     for (int j = 0; j < J; ++j) {
       const int k = min(k0 + j, nb - 1);  // uniform; out-of-batch slots masked below
-      const uint32_t mk = cmask[cx][k];
+      const uint32_t mk = col[cx][k];
       msk[j] = (k0 + j < nb) ? mk : 0u;
       att[j] = pre1[cy][k] * pre2[cx][k];
     }
@@ -420,10 +472,10 @@ __device__ __forceinline__ void walk_batch(int nb, int cx, int cy, const uint32_
 // slices.  att_bound: the largest row factor times the largest column factor
 // (+inf if one is NaN); float multiplication being monotone, every pixel's
 // att = pre1 * pre2 is at most it, and vmax * att at most vmax * att_bound.
-template <bool BITS>
+template <bool BITS, class Col>
 __device__ __forceinline__ void tabulate(const SplatArgs &a, const Rec &R, int lane, int x0s,
                                         int y0s, int w, int h, int bxo, int byo,
-                                        const float *s_tab, uint32_t (*col)[kPad],
+                                        const float *s_tab, Col col,
                                         float (*pre2)[kPad], float (*pre1)[kPad],
                                         float expfac, float &att_bound) {
   const float rfacr = R.r * a.rfac;
@@ -555,72 +607,51 @@ __device__ __forceinline__ uint32_t splat_items(const uint32_t *&items, uint32_t
   return tot - nh;
 }
 
-// PPW (variant 4): particles per chunk of the walk (1, 2, 4 or 8; 0: 8 for
-// one channel, 8 additive / 4 ordered for all three).
-template <int ADD, int VAR, int PPW>
-__global__ __launch_bounds__(256) void k_splat8(SplatArgs a, const uint32_t *items,
-                                                uint32_t nitems_, ItemCounts dc,
-                                                uint32_t nsplit_) {
-  constexpr int J1 = PPW ? PPW : 8, J3 = PPW ? PPW : (ADD ? 8 : 4);
-  const uint32_t nreal = splat_items(items, nitems_, dc);
-  // the first nsplit items are long lists served as three one-channel items
-  const uint32_t nsplit = min(dc.nsplit ? *dc.nsplit : nsplit_, nreal);
-  const uint32_t nitems = nreal + 2u * nsplit;
-  __shared__ float s_tab[2048];
-  __shared__ uint32_t s_col[4][8][kPad];
-  __shared__ float s_pre2[4][8][kPad];
-  __shared__ float s_pre1[4][8][kPad];
+// The wave's LDS of the 8x8 splat.  col: per column and particle the row bits
+// (a byte each in variant 4, whose chunks read four particles' at once; row
+// stride kColPad) or, in variants 1 and 2, the row range.
+template <int ADD, int VAR>
+struct SplatLds {
+  typename std::conditional<VAR == 4, uint8_t, uint32_t>::type
+      __attribute__((aligned(16))) col[8][VAR == 4 ? kColPad : kPad];
+  float pre2[8][kPad], pre1[8][kPad];
   // per-particle constants: ordered (a0, a1, a2, max |a|), (q0, q1, q2, 0);
   // additive (a0, a1, a2, 0)
-  __shared__ float4 s_cst[4][64 * (ADD ? 1 : 2)];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  // a workgroup past the items (a grid sized for a capacity) leaves at once
-  if (blockIdx.x * 4u >= nitems) return;
-  for (int i = tid; i < 2048; i += 256) s_tab[i] = a.exptab[i];
-  __syncthreads();
-  const uint32_t it = blockIdx.x * 4u + wave;
-  if (it >= nitems) return;
-  const uint64_t t_start = a.trace ? __builtin_amdgcn_s_memrealtime() : 0;
-  // wave-uniform values are moved to scalar registers so that loop bounds and
-  // channel selection compile to scalar branches
-  const uint32_t item = it < 3u * nsplit ? (uniform(items[it / 3u]) & ~3u) | (it % 3u)
-                                          : uniform(items[it - 2u * nsplit]);
-  const uint32_t u = item >> 2;
-  const int chan = static_cast<int>(item & 3u);  // 3: all channels
-  const UnitGeom ug = unit_geom_uniform(a, u);
-  const int gy = ug.gy, gx = ug.gx, x0s = ug.x0s, y0s = ug.y0s, w = ug.w, h = ug.h;
-  const int bxo = gx * 8, byo = gy * 8;  // tile frame
-  const int cx = lane >> 3, cy = lane & 7;
-  const int lx = bxo + cx, ly = byo + cy;
-  uint32_t(*col)[kPad] = s_col[wave];
-  float(*pre2)[kPad] = s_pre2[wave];
-  float(*pre1)[kPad] = s_pre1[wave];
-  float4 *wcst = s_cst[wave];
-  if (!ADD) {
-    // the fast chunks read every slot of a chunk, also past a short batch
-    // (masked there): start from finite values
-    for (int i = lane; i < 8 * kPad; i += 64) {
-      (&col[0][0])[i] = 0u;
-      (&pre2[0][0])[i] = 0.f;
-      (&pre1[0][0])[i] = 0.f;
-    }
-    wcst[2 * lane] = make_float4(0.f, 0.f, 0.f, 0.f);
-    wcst[2 * lane + 1] = make_float4(0.f, 0.f, 0.f, 0.f);
-  }
-  const float expfac = a.expfac, tl = a.taylorlimit;
+  float4 cst[64 * (ADD ? 1 : 2)];
+};
 
-  float l0 = 0.f, l1 = 0.f, l2 = 0.f;
-  const bool pix_in = lx < min(bxo + 8, w) && ly < min(byo + 8, h);
-  if (ug.accumulate == 2 && pix_in) {  // a later chunk: continue the chain
-    const float *d = ug.pic + (static_cast<int64_t>(x0s + lx) * ug.yres + (y0s + ly)) * 3;
-    l0 = d[0];
-    l1 = d[1];
-    l2 = d[2];
+// Cleared once per wave: the ordered fast chunks read every slot of a chunk,
+// also past a short batch (masked there), and start from finite values.
+template <int ADD, int VAR>
+__device__ __forceinline__ void clear_slots(SplatLds<ADD, VAR> &L, int lane) {
+  if (ADD) return;
+  for (int i = lane; i < static_cast<int>(sizeof(L.col) / 4); i += 64)
+    reinterpret_cast<uint32_t *>(L.col)[i] = 0u;
+  for (int i = lane; i < 8 * kPad; i += 64) {
+    (&L.pre2[0][0])[i] = 0.f;
+    (&L.pre1[0][0])[i] = 0.f;
   }
-  const uint32_t e0 = uniform(a.bin_off[u]), e1 = uniform(a.bin_off[u + 1]);
-  // long lists are near the critical path: let their waves issue ahead of the
-  // rest (priority 2; the producer/consumer workgroups, the critical path, run at 3)
-  if (e1 - e0 >= a.prio_len) __builtin_amdgcn_s_setprio(2);
+  L.cst[2 * lane] = make_float4(0.f, 0.f, 0.f, 0.f);
+  L.cst[2 * lane + 1] = make_float4(0.f, 0.f, 0.f, 0.f);
+}
+
+// Applies list entries [e0, e1) to the lane's pixel (lx, ly) of the unit, in
+// list order, for channel chan (3: all).  PPW (variant 4): particles per chunk
+// of the walk (1, 2, 4 or 8; 0: 8 for one channel, 8 additive / 4 ordered for
+// all three).
+template <int ADD, int VAR, int PPW>
+__device__ __forceinline__ void walk_list(const SplatArgs &a, const UnitGeom &ug, uint32_t e0,
+                                          uint32_t e1, int chan, int lane, const float *s_tab,
+                                          SplatLds<ADD, VAR> &L, float &l0, float &l1, float &l2) {
+  constexpr int J1 = PPW ? PPW : 8, J3 = PPW ? PPW : (ADD ? 8 : 4);
+  const int bxo = ug.gx * 8, byo = ug.gy * 8;  // tile frame
+  const int cx = lane >> 3, cy = lane & 7;
+  const int ly = byo + cy;
+  auto *col = L.col;
+  float(*pre2)[kPad] = L.pre2;
+  float(*pre1)[kPad] = L.pre1;
+  float4 *wcst = L.cst;
+  const float expfac = a.expfac, tl = a.taylorlimit;
   // The records of a batch are gathered one batch ahead and their slots two
   // ahead, so that the walk of a batch covers the latency of the next gather.
   Rec rn{};
@@ -637,8 +668,8 @@ __global__ __launch_bounds__(256) void k_splat8(SplatArgs a, const uint32_t *ite
     bool vfast = false, vtay = false;
     if (lane < nb) {
       float ab;
-      tabulate<VAR >= 3>(a, R, lane, x0s, y0s, w, h, bxo, byo, s_tab, col, pre2, pre1, expfac,
-                         ab);
+      tabulate<VAR >= 3>(a, R, lane, ug.x0s, ug.y0s, ug.w, ug.h, bxo, byo, s_tab, col, pre2, pre1,
+                         expfac, ab);
       va0 = -R.e0;
       va1 = -R.e1;
       va2 = -R.e2;
@@ -670,7 +701,7 @@ __global__ __launch_bounds__(256) void k_splat8(SplatArgs a, const uint32_t *ite
     wave_sync();
     const uint64_t fastmask = __ballot(vfast), taymask = __ballot(vtay);
     // Phase B: lane = pixel, particles in list order.
-    if (VAR == 4) {
+    if constexpr (VAR == 4) {
       switch (chan) {
         case 0: walk_chunks<ADD, 0, J1>(nb, cx, cy, col, pre2, pre1, s_tab, va0, va1, va2, vq0, vq1, vq2, vmax, wcst, fastmask, taymask, expfac, tl, l0, l1, l2); break;
         case 1: walk_chunks<ADD, 1, J1>(nb, cx, cy, col, pre2, pre1, s_tab, va0, va1, va2, vq0, vq1, vq2, vmax, wcst, fastmask, taymask, expfac, tl, l0, l1, l2); break;
@@ -680,7 +711,7 @@ __global__ __launch_bounds__(256) void k_splat8(SplatArgs a, const uint32_t *ite
       wave_sync();
       continue;
     }
-    if (VAR == 3) {
+    if constexpr (VAR == 3) {
       switch (chan) {
         case 0: walk_batch<ADD, 0>(nb, cx, cy, col, pre2, pre1, s_tab, va0, va1, va2, vq0, vq1, vq2, vmax, expfac, tl, l0, l1, l2); break;
         case 1: walk_batch<ADD, 1>(nb, cx, cy, col, pre2, pre1, s_tab, va0, va1, va2, vq0, vq1, vq2, vmax, expfac, tl, l0, l1, l2); break;
@@ -690,7 +721,7 @@ __global__ __launch_bounds__(256) void k_splat8(SplatArgs a, const uint32_t *ite
       wave_sync();
       continue;
     }
-    if (VAR == 1) {
+    if constexpr (VAR == 1) {
       for (int k = 0; k < nb; ++k) {
         const uint32_t lohi = col[cx][k];
         if (ly >= static_cast<int>(lohi & 0xffffu) && ly < static_cast<int>(lohi >> 16)) {
@@ -774,6 +805,53 @@ __global__ __launch_bounds__(256) void k_splat8(SplatArgs a, const uint32_t *ite
     }
     wave_sync();
   }
+}
+
+// Four workgroups per CU (their LDS, 35 KB each, and at most 128 VGPRs a lane):
+// the walk waits on LDS returns, and 16 waves hide more of them than the 12
+// that 142 VGPRs allow (64 views with 137M ordered and 124M additive entries:
+// 31.9 -> 30.6 ms; 32.1 with constants and coverage read per particle).
+template <int ADD, int VAR, int PPW>
+__global__ __launch_bounds__(256, 4) void k_splat8(SplatArgs a, const uint32_t *items,
+                                                uint32_t nitems_, ItemCounts dc,
+                                                uint32_t nsplit_) {
+  const uint32_t nreal = splat_items(items, nitems_, dc);
+  // the first nsplit items are long lists served as three one-channel items
+  const uint32_t nsplit = min(dc.nsplit ? *dc.nsplit : nsplit_, nreal);
+  const uint32_t nitems = nreal + 2u * nsplit;
+  __shared__ float s_tab[2048];
+  __shared__ SplatLds<ADD, VAR> s_wave[4];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  // a workgroup past the items (a grid sized for a capacity) leaves at once
+  if (blockIdx.x * 4u >= nitems) return;
+  for (int i = tid; i < 2048; i += 256) s_tab[i] = a.exptab[i];
+  __syncthreads();
+  const uint32_t it = blockIdx.x * 4u + wave;
+  if (it >= nitems) return;
+  const uint64_t t_start = a.trace ? __builtin_amdgcn_s_memrealtime() : 0;
+  // wave-uniform values are moved to scalar registers so that loop bounds and
+  // channel selection compile to scalar branches
+  const uint32_t item = it < 3u * nsplit ? (uniform(items[it / 3u]) & ~3u) | (it % 3u)
+                                          : uniform(items[it - 2u * nsplit]);
+  const uint32_t u = item >> 2;
+  const int chan = static_cast<int>(item & 3u);  // 3: all channels
+  const UnitGeom ug = unit_geom_uniform(a, u);
+  const int lx = ug.gx * 8 + (lane >> 3), ly = ug.gy * 8 + (lane & 7);
+  clear_slots(s_wave[wave], lane);
+
+  float l0 = 0.f, l1 = 0.f, l2 = 0.f;
+  const bool pix_in = lx < ug.w && ly < ug.h;
+  if (ug.accumulate == 2 && pix_in) {  // a later chunk: continue the chain
+    const float *d = ug.pic + (static_cast<int64_t>(ug.x0s + lx) * ug.yres + (ug.y0s + ly)) * 3;
+    l0 = d[0];
+    l1 = d[1];
+    l2 = d[2];
+  }
+  const uint32_t e0 = uniform(a.bin_off[u]), e1 = uniform(a.bin_off[u + 1]);
+  // long lists are near the critical path: let their waves issue ahead of the
+  // rest (priority 2; the producer/consumer workgroups, the critical path, run at 3)
+  if (e1 - e0 >= a.prio_len) __builtin_amdgcn_s_setprio(2);
+  walk_list<ADD, VAR, PPW>(a, ug, e0, e1, chan, lane, s_tab, s_wave[wave], l0, l1, l2);
   if (a.trace && lane == 0) {
     uint64_t *tr = a.trace + 4 * static_cast<uint64_t>(it);
     tr[0] = t_start;
@@ -782,7 +860,7 @@ __global__ __launch_bounds__(256) void k_splat8(SplatArgs a, const uint32_t *ite
     tr[3] = static_cast<uint64_t>(__smid());
   }
   if (pix_in) {
-    float *d = ug.pic + (static_cast<int64_t>(x0s + lx) * ug.yres + (y0s + ly)) * 3;
+    float *d = ug.pic + (static_cast<int64_t>(ug.x0s + lx) * ug.yres + (ug.y0s + ly)) * 3;
     const bool add = ug.accumulate == 1;
     if (chan == 3 || chan == 0) d[0] = add ? d[0] + l0 : l0;
     if (chan == 3 || chan == 1) d[1] = add ? d[1] + l1 : l1;
