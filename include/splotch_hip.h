@@ -104,11 +104,9 @@ typedef struct {
                                               terms are computed across the GPU first, then
                                               summed in list order by one wave per channel
                                               and pixel column (0 = auto: from entries /
-                                              1300 or the longest list / 64 on, but none for
-                                              a single view with both passes in one chunk,
-                                              whose additive splat runs beside the ordered
-                                              pass, and none where the longest list is below
-                                              1536 entries; < 0 = never) */
+                                              1300 or the longest list / 64 on, none where
+                                              the longest list is below 1536 entries; < 0 =
+                                              never) */
   int32_t hip_stage_ordered;               /* hip_stage_ordered: the same for an ordered pass
                                               (per-pixel operands of the compositing update
                                               computed first; not when a particle's q_c is

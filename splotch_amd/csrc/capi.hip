@@ -1422,13 +1422,6 @@ int render_jobs(splhip_ctx *c, int nj, const JobIn *jobs, hipStream_t s, bool ke
       pl.e16[p] = pl.m[p] ? c->h_tot[T_E16 + p] : 0;
       chunked[p] = pl.m[p] && e64[p] > tn.chunk;
     }
-    // A single unchunked view with both passes: the additive splat runs
-    // beside the ordered pass on a second stream, where its long lists are
-    // off the critical path and staged operands' HBM traffic would slow the
-    // ordered pass's binning: no staging unless hip_stage asks for it.
-    if (nj == 1 && pl.m[0] && pl.m[1] && !chunked[0] && !chunked[1] &&
-        jobs[0].prm->hip_stage == 0)
-      tn.stage = 0xffffffffu;
     for (int p = 0; p < 2; ++p) pl.etot[p] = e64[p];
     if (chunked[0] || chunked[1]) {
       c->split_hint = nj > 1;  // the caller may render the views in smaller groups
@@ -1458,8 +1451,12 @@ int render_jobs(splhip_ctx *c, int nj, const JobIn *jobs, hipStream_t s, bool ke
   // splats; the scratch image is then added to the image: pic + l per pixel,
   // the additive pass's own update (pixels it does not touch add +0, which
   // leaves any value but -0 as it is; the ordered pass never writes -0).
-  // Its longest lists stay in the 8x8 kernel: producer/consumer workgroups
-  // would hold whole CUs beside the ordered pass's.
+  // Its long lists are staged (a list of 1.2M entries takes one wave of the
+  // 8x8 kernel 64 ms, its staged chains 0.3 ms: such a 16M-particle frame 74 ->
+  // 51 ms, others within 1 %), after the ordered pass's and on the same streams
+  // (on streams of their own they delayed its splat: 53 ms); none goes to
+  // producer/consumer workgroups, which would hold whole CUs beside the
+  // ordered pass's.
   const bool sweep = !force && G == 8 && jobs[0].prm->hip_autotune;
   const bool early = !chunked[0] && !chunked[1] && nj == 1 && G == 8 && pl.m[0] && pl.m[1] &&
                      pl.js[0].accumulate[1] == 1 && !sweep;
