@@ -75,7 +75,12 @@ typedef struct {
                                               3 = software pipelined, 4 = chunked branch-free */
   int32_t hip_heavy;                       /* hip_heavy: list length from which an 8x8 block is
                                               splatted by a producer/consumer workgroup
-                                              (0 = auto: 32768, < 0 = never) */
+                                              (0 = auto: 32768, < 0 = never).  With this and
+                                              the other decomposition keys 0, an ordered pass
+                                              of 160M (block, particle) entries or more walks
+                                              its lists of 81920 entries and more in segments
+                                              at once instead, where their optical depth
+                                              allows it; the image is the same */
   int32_t hip_heavy_max;                   /* hip_heavy_max: at most this many such workgroups
                                               per pass, the heaviest (0 = auto: 192) */
   int32_t hip_chunk_entries;               /* hip_chunk_entries: a single-view pass with more

@@ -101,6 +101,7 @@ struct splhip_ctx {
   // launched and given their head start (see stage_splat)
   hipEvent_t ev_placed = nullptr;
   Workspace ws2;
+  bool sizing = false;  // a render that sizes a reservation
   // block-file ingest: two pinned buffers, each freed for reuse by its event
   char *h_ing[2] = {nullptr, nullptr};
   hipEvent_t ev_ing[2] = {nullptr, nullptr};
@@ -442,6 +443,8 @@ struct Plan {
   bool late = false;  // the pass sizes are still on the device (m: capacities)
   uint32_t nstage[2] = {0, 0};
   uint64_t sgroups[2] = {0, 0};
+  uint32_t seglen[2] = {0, 0};  // lists walked in segments: their length (0: none)
+  uint32_t nseglists[2] = {0, 0}, nsegs[2] = {0, 0}, nslots[2] = {0, 0};
   uint64_t etot[2] = {0, 0};  // (block, particle) entries of each pass (or chunk)
   uint32_t e16[2] = {0, 0};         // (region, particle) entries
   bool r16[2] = {false, false};     // the pass's region counts are scanned (e16 valid)
@@ -652,12 +655,14 @@ void make_plan(splhip_ctx *c, int nj, const JobIn *jobs, int G, Plan &pl, hipStr
 // its lists from heavy_len entries on, its longest list, the lists from
 // stage_level(stage_len, j) entries on and their groups of 4 entries (at
 // most); then a device-count render's long-list partition (4 per pass: staged,
-// producer/consumer, both, by channel).
+// producer/consumer, both, by channel); from T_SEG on the ordered pass's lists
+// walked in segments (SC_*).
 constexpr int kListWords = 2 + 2 * kStageLevels;
 enum { L_HEAVY = 0, L_MAX = 1, L_CNT = 2, L_GRP = 2 + kStageLevels };
 enum {
   T_M = 0, T_E = 2, T_ITEMS = 4, T_QBAD = 6, T_OVF = 7, T_E64 = 8, T_E16 = 12,
-  T_LIST = 16, T_PART = T_LIST + 2 * kListWords, T_N = T_PART + 8
+  T_LIST = 16, T_PART = T_LIST + 2 * kListWords, T_SEG = T_PART + 8,
+  T_N = T_SEG + SC_N
 };
 constexpr int t_list(int p, int k) { return T_LIST + kListWords * p + k; }
 constexpr int kTotalsWords = 256;  // the totals buffer, device and pinned host
@@ -880,7 +885,23 @@ struct Tuning {
   uint32_t stage, stage_ord;  // lists from this length on are staged, additive / ordered
                               // pass (0xffffffff: none)
   StageMode mode[2];          // the staging length's rule, ordered / additive pass
+  bool seg;                   // long ordered lists may be walked in segments
 };
+
+// Length of the segments that a pass's ordered lists are walked in (0: none),
+// those of twice this length on.  In a pass of hundreds of millions of entries
+// the long lists are too many to stage and take a producer/consumer workgroup 48
+// ns and a whole CU per entry, where the 8x8 walk of all CUs takes 15 ns of one;
+// in segments they cost that and the warm-ups (16M-particle frames at 2048^2,
+// 195M to 322M entries: 33.9 -> 27.4, 37.8 -> 28.3, 53.0 -> 31.0, 51.0 -> 23.4
+// ms).  The length is that of a walk of about half such a pass: 24576 entries
+// 31.1, 30.4, 42.2, 27.6 ms (warm-ups), 56000 the first and third 35.6, 36.4 (the
+// last segments outlast the pass).  In smaller passes they outlast it at any
+// length that pays for its warm-ups (64 views, 137M entries: 30.6 ms without,
+// 32.2 from lists of 33k on).
+constexpr uint64_t kSegEntries = 160000000;
+constexpr uint32_t kSegLen = 40960;
+uint32_t seg_length(uint64_t etot) { return etot < kSegEntries ? 0u : kSegLen; }
 
 // Staged operands of a pass: room for 3 KiB per group of 4 entries additive, 7
 // KiB ordered (what is written depends on the entries' coverage); of a pass
@@ -922,6 +943,10 @@ Tuning tuning_of(const splhip_params *prm) {
   };
   stage(prm->hip_stage, 1, t.stage);
   stage(prm->hip_stage_ordered, 0, t.stage_ord);
+  // only where nothing asks for another decomposition
+  t.seg = prm->hip_variant <= 0 && prm->hip_ppw == 0 && prm->hip_split <= 0 &&
+          prm->hip_heavy == 0 && prm->hip_heavy_max <= 0 && prm->hip_stage_ordered == 0 &&
+          !prm->hip_autotune;
   return t;
 }
 
@@ -940,11 +965,28 @@ SplatArgs splat_args(splhip_ctx *c, const Plan &pl, int p, const Tuning &tn) {
   sa.expfac = c->consts.expfac;
   sa.taylorlimit = c->consts.taylorlimit;
   sa.prio_len = tn.split;
-  sa.heavy_len = tn.heavy;
+  // lists of one segment stay in the 8x8 splat
+  sa.heavy_len = pl.seglen[p] ? std::max(tn.heavy, 2u * pl.seglen[p]) : tn.heavy;
   // device counts: staging only where the reservation holds room for it
   sa.stage_len = (pl.dc && pl.nstage[p] == 0) ? 0xffffffffu : p == 1 ? tn.stage : tn.stage_ord;
   sa.qbad = p == 0 ? pl.qbad : nullptr;
   return sa;
+}
+
+// The segments' buffers of pass p (pl.seglen set).
+SegArgs seg_args(const Plan &pl, int p, uint32_t *tot) {
+  Workspace &ws = *pl.ws;
+  SegArgs g{};
+  seg_caps(pl.etot[p], pl.seglen[p], g);
+  g.cnt = tot + T_SEG;
+  g.flag = ws.get_as<uint32_t>(pslot(p, P_SEGF), pl.nunits);
+  g.cand = ws.get_as<SegCand>(pslot(p, P_SEGC), g.candcap);
+  g.chunk = ws.get_as<uint32_t>(pslot(p, P_SEGK), 2 * static_cast<size_t>(g.chunkcap));
+  g.sample = ws.get_as<float>(pslot(p, P_SEGX), static_cast<size_t>(g.samplecap) * 192u);
+  g.win = ws.get_as<uint32_t>(pslot(p, P_SEGW), g.samplecap);
+  g.lists = ws.get_as<SegList>(pslot(p, P_SEGL), g.candcap);
+  g.segs = ws.get_as<Seg>(pslot(p, P_SEGI), g.segcap);
+  return g;
 }
 
 // Work items of pass p: count per unit (heavy units counted too), scan.
@@ -952,7 +994,14 @@ void stage_items_count(splhip_ctx *c, Plan &pl, int p, const Tuning &tn, uint32_
                        hipStream_t s, Workspace *wt = nullptr) {
   Workspace &ws = *pl.ws;
   mark(c, p == 0 ? 2 : 5, true, s);
-  const SplatArgs sa = splat_args(c, pl, p, tn);
+  pl.seglen[p] = p == 0 && tn.seg && !pl.dc && !c->sizing ? seg_length(pl.etot[p]) : 0u;
+  SplatArgs sa = splat_args(c, pl, p, tn);
+  if (pl.seglen[p]) {
+    const SegArgs g = seg_args(pl, p, tot);
+    if (pl.counted[p]) launch_fill_u32(g.cnt, 0u, SC_N, s);
+    launch_seg_pick(pl.nunits, g, sa, s);
+    sa.seg = g.flag;
+  }
   uint32_t *icnt = ws.get_as<uint32_t>(pslot(p, P_ICNT), pl.nunits);
   uint32_t *ioff = ws.get_as<uint32_t>(pslot(p, P_IOFF), pl.nunits);
   // the counts of this call only (chunks and autotuning candidates count
@@ -974,6 +1023,9 @@ void stage_items_count(splhip_ctx *c, Plan &pl, int p, const Tuning &tn, uint32_
 void take_items(splhip_ctx *c, Plan &pl, int p, const Tuning &tn) {
   const uint32_t *h = c->h_tot;
   pl.nitems[p] = pl.m[p] ? h[T_ITEMS - T_ITEMS + p] : 0u;
+  pl.nseglists[p] = pl.seglen[p] ? h[T_SEG + SC_LIST - T_ITEMS] : 0u;
+  pl.nsegs[p] = pl.seglen[p] ? h[T_SEG + SC_SEG - T_ITEMS] : 0u;
+  pl.nslots[p] = pl.seglen[p] ? h[T_SEG + SC_SLOT - T_ITEMS] : 0u;
   const uint32_t nheavy_lists = pl.m[p] ? h[t_list(p, L_HEAVY) - T_ITEMS] : 0u;
   const uint64_t lmax = h[t_list(p, L_MAX) - T_ITEMS];
   const uint32_t len0 = p == 1 ? tn.stage : tn.stage_ord;
@@ -1026,6 +1078,8 @@ void stage_splat(splhip_ctx *c, Plan &pl, int p, const Tuning &tn, hipStream_t s
     mark(c, p == 0 ? 3 : 6, false, s);
     return;
   }
+  if (pl.seglen[p]) sa0.seg = ws.get_as<uint32_t>(pslot(p, P_SEGF), pl.nunits);
+  const uint32_t nseg = pl.nseglists[p];
   const uint32_t nitems = pl.nitems[p], nheavy = std::min(pl.nheavy[p], nitems);
   const uint32_t *ioff = ws.get_as<uint32_t>(pslot(p, P_IOFF), pl.nunits);
   uint32_t *ik0 = ws.get_as<uint32_t>(pslot(p, P_IK0), nitems);
@@ -1065,8 +1119,10 @@ void stage_splat(splhip_ctx *c, Plan &pl, int p, const Tuning &tn, hipStream_t s
   const uint32_t *items = rs ? iv1 : iv0;
   pl.items[p] = items;
   SplatArgs sa = sa0;
-  // the trace holds a record per item, the long lists served by channel three
-  const size_t ntrace = static_cast<size_t>(nitems) + 2 * static_cast<size_t>(pl.nsplit[p]);
+  // the trace holds a record per item, the long lists served by channel three,
+  // then one per list walked in segments
+  const size_t nitrace = static_cast<size_t>(nitems) + 2 * static_cast<size_t>(pl.nsplit[p]);
+  const size_t ntrace = nitrace + nseg;
   if (c->trace && !pl.dc)
     sa.trace = ws.get_as<uint64_t>(pslot(p, P_TRACE), ntrace * 4);
   SplatArgs sn = sa;  // normal items follow the heavy ones
@@ -1081,7 +1137,7 @@ void stage_splat(splhip_ctx *c, Plan &pl, int p, const Tuning &tn, hipStream_t s
   SplatArgs sp = sa;
   if (sp.trace) sp.trace += 4 * static_cast<size_t>(nstage);
   const uint32_t *pit = pl.dc ? items : items + nstage;
-  if (nstage > 0 || (npc > 0 && fork)) {
+  if (nseg > 0 || nstage > 0 || (npc > 0 && fork)) {
     // heavy blocks run on second streams, beside the normal items: the
     // producer/consumer workgroups at once, the staged chains after the
     // operand kernel (on s, across the GPU)
@@ -1097,6 +1153,27 @@ void stage_splat(splhip_ctx *c, Plan &pl, int p, const Tuning &tn, hipStream_t s
       mark(c, p == 0 ? 8 : 10, true, s);
       launch_splat_pc(p == 1, pit, npc, sp, s, dc);
       mark(c, p == 0 ? 8 : 10, false, s);
+    }
+    if (nseg > 0) {
+      // before the normal items, as their longest walks; where there are
+      // producer/consumer workgroups, after their head start and on the third
+      // stream
+      if (npc > 0)
+        ensure_aux3(c, set);
+      else
+        ensure_aux(c, set);
+      const hipStream_t q = npc > 0 ? X.aux3 : X.aux;
+      const hipEvent_t fk = npc > 0 ? X.fork3 : X.fork;
+      const SegArgs g = seg_args(pl, p, pl.tot);
+      SplatArgs ss = sa;
+      if (ss.trace) ss.trace += 4 * nitrace;
+      float *st = ws.get_as<float>(pslot(p, P_SEGS), static_cast<size_t>(pl.nslots[p]) * 192u);
+      if (npc > 0) launch_delay(40, s);
+      hip_check(hipEventRecord(fk, s), "record fork");
+      hip_check(hipStreamWaitEvent(q, fk, 0), "wait fork");
+      launch_seg_walk(g, pl.nsegs[p], st, ss, q);
+      launch_seg_join(g, nseg, st, ss, q);
+      hip_check(hipEventRecord(npc > 0 ? X.join3 : X.join, q), "record join");
     }
     if (nstage > 0) {
       // the operand kernel and then the chains on a third stream, beside the
@@ -1149,13 +1226,13 @@ void stage_splat(splhip_ctx *c, Plan &pl, int p, const Tuning &tn, hipStream_t s
     // waits briefly.  Staged lists need no such start: their operand kernels'
     // workgroups fit in as the normal ones end (20k ordered at 257 x 193: 0.377
     // ms with the wait, 0.339 without; larger frames up to 1 % faster without).
-    if (npc > 0) launch_delay(40, s);
+    if (npc > 0 || nseg > 0) launch_delay(40, s);
     if (placed) hip_check(hipEventRecord(placed, s), "record placed");
     mark(c, p == 0 ? 7 : 9, true, s);
     launch_splat8(p == 1, tn.variant, nit, nn, sn, s, dc, tn.ppw, pl.nsplit[p]);
     mark(c, p == 0 ? 7 : 9, false, s);
-    if (npc > 0 && fork) hip_check(hipStreamWaitEvent(s, X.join, 0), "wait join");
-    if (nstage > 0) hip_check(hipStreamWaitEvent(s, X.join3, 0), "wait join");
+    if ((npc > 0 && fork) || (nseg > 0 && npc == 0)) hip_check(hipStreamWaitEvent(s, X.join, 0), "wait join");
+    if (nstage > 0 || (nseg > 0 && npc > 0)) hip_check(hipStreamWaitEvent(s, X.join3, 0), "wait join");
     if (nstage > kStagePhase1) hip_check(hipStreamWaitEvent(s, X.join4, 0), "wait join");
   } else if (npc > 0) {
     mark(c, p == 0 ? 8 : 10, true, s);
@@ -1175,7 +1252,7 @@ void stage_splat(splhip_ctx *c, Plan &pl, int p, const Tuning &tn, hipStream_t s
   if (c->trace && !pl.dc) {
     std::vector<uint64_t> &tv = c->trace_items[p];
     tv.resize(ntrace * 4);
-    if (nitems)
+    if (ntrace)
       hip_check(hipMemcpyAsync(tv.data(), sa.trace, tv.size() * 8, hipMemcpyDeviceToHost, s),
                 "D2H trace");
     hip_check(hipStreamSynchronize(s), "sync trace");
@@ -1839,7 +1916,17 @@ int capture_reserve(splhip_ctx *c, int nj, const JobIn *jobs, float headroom, hi
   if (!(headroom >= 1.f)) return fail(c, SPLHIP_E_ARG, "headroom must be at least 1");
   delete c->rv;
   c->rv = nullptr;
-  if (int rc = render_tuned(c, nj, jobs, s, false, true)) return rc;
+  // the sizing render makes the long lists' decomposition as the reserved ones
+  // will (which walk no list in segments)
+  struct Sizing {
+    splhip_ctx *c;
+    explicit Sizing(splhip_ctx *x) : c(x) { c->sizing = true; }
+    ~Sizing() { c->sizing = false; }
+  };
+  {
+    Sizing sizing(c);
+    if (int rc = render_tuned(c, nj, jobs, s, false, true)) return rc;
+  }
   Tuning tn = tuning_of(jobs[0].prm);
   if (c->last_entries[0] > static_cast<int64_t>(tn.chunk) ||
       c->last_entries[1] > static_cast<int64_t>(tn.chunk))

@@ -56,6 +56,7 @@ struct SplatArgs {
   // so no list goes to the producer/consumer kernel (it applies every particle
   // to the whole block with zero operands, and (l - q) * 0 is NaN there)
   const uint32_t *qbad;
+  const uint32_t *seg;  // (optional) per unit: nonzero = walked in segments, no items
 };
 
 void launch_project(const ProjectArgs *jobs, const uint32_t *blk, int nj, uint32_t nblocks,
@@ -186,6 +187,44 @@ struct ItemCounts {
 void launch_splat8(bool additive, int variant, const uint32_t *items, uint32_t nitems,
                    const SplatArgs &a, hipStream_t s, const ItemCounts &dc = ItemCounts{},
                    int ppw = 0, uint32_t nsplit = 0);
+// Ordered lists walked in segments (splat8.hip): lists of at least 2 * seglen
+// entries, cut where the sampled entries before the cut make every pixel's chain
+// forget its start.  flag[u] says per unit whether its list is (the item kernels
+// skip those: SplatArgs::seg).
+struct SegCand {
+  uint32_t unit, samples;  // first sample (192 floats each)
+  uint32_t on;             // bit c: the list absorbs in channel c
+};
+struct SegList {
+  uint32_t unit, first, n;  // first segment, segments
+};
+struct Seg {
+  uint32_t list, e0, e1, warm, slot;  // entries, warm-up entries before e0, first kept state
+  uint32_t chan;                      // 3: all
+};
+constexpr uint32_t kSegCheck = 1024;    // entries between a segment's kept states (192 floats)
+constexpr uint32_t kSegSample = 2048;   // one batch of 64 is sampled in this many entries
+constexpr uint32_t kSegWarm = 32;       // samples of the longest warm-up
+// Device counts (zeroed before launch_seg_pick).
+enum { SC_CAND, SC_CHUNK, SC_SAMPLE, SC_LIST, SC_SEG, SC_SLOT, SC_N };
+struct SegArgs {
+  uint32_t seglen, candcap, chunkcap, samplecap, segcap;
+  uint32_t *flag, *cnt;
+  SegCand *cand;      // [candcap]
+  uint32_t *chunk;    // [chunkcap * 2]
+  float *sample;      // [samplecap * 192]
+  uint32_t *win;      // [samplecap]
+  SegList *lists;     // [candcap]
+  Seg *segs;          // [segcap]
+};
+// The capacities that a pass of etot entries cannot exceed.
+void seg_caps(uint64_t etot, uint32_t seglen, SegArgs &g);
+void launch_seg_pick(uint32_t nunits, const SegArgs &g, const SplatArgs &a, hipStream_t s);
+// The segments (states: the slots counted, 192 floats each), then the lists' blocks.
+void launch_seg_walk(const SegArgs &g, uint32_t nseg, float *states, const SplatArgs &a,
+                     hipStream_t s);
+void launch_seg_join(const SegArgs &g, uint32_t nlists, const float *states, const SplatArgs &a,
+                     hipStream_t s);
 // Staged lists (splat8.hip), the first n items of a pass (groups: an upper
 // bound of their groups of 4 entries): list offsets into cbase / cbat ([n + 1]
 // each); then, for lists [i0, i1) (called in two phases, [0, n1) and [n1, n)),
