@@ -36,7 +36,6 @@ namespace splhip {
 namespace {
 
 constexpr int kPadA = 65;
-constexpr uint32_t kSeg = kAdjSeg;  // entries per backward work item (list segment)
 
 __device__ __forceinline__ int64_t gtid_() {
   return static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -45,23 +44,40 @@ __device__ __forceinline__ int64_t gstride_() {
   return static_cast<int64_t>(gridDim.x) * blockDim.x;
 }
 
-// Sum over the wave's 64 lanes with DPP row operations (quad permutes,
-// half-row and row mirrors, then row broadcasts 15 and 31); the total ends in
-// lane 63 and is returned to every lane.
-template <int CTRL, int ROWS>
-__device__ __forceinline__ float dpp_add(float v) {
-  const int s = __builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROWS, 0xf, false);
-  return v + __int_as_float(s);
+// The lane keeps a (sel clear) or b (sel set) and adds its DPP partner's share
+// of the value it keeps (the partner's sel differs).
+template <int CTRL>
+__device__ __forceinline__ float dpp_fold(bool sel, float a, float b) {
+  const float keep = sel ? b : a, give = sel ? a : b;
+  const int s = __builtin_amdgcn_mov_dpp(__float_as_int(give), CTRL, 0xf, 0xf, true);
+  return keep + __int_as_float(s);
 }
 
-__device__ __forceinline__ float wave_sum(float v) {
-  v = dpp_add<0xb1, 0xf>(v);   // quad_perm [1,0,3,2]
-  v = dpp_add<0x4e, 0xf>(v);   // quad_perm [2,3,0,1]
-  v = dpp_add<0x141, 0xf>(v);  // row_half_mirror
-  v = dpp_add<0x140, 0xf>(v);  // row_mirror: every lane of a row holds the row sum
-  v = dpp_add<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
-  v = dpp_add<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+// Sums of six values over the wave's 64 lanes: sum i in lane i (i < 6).  The
+// first three levels of the trees fold pairs of values into one register, as
+// half of the lanes suffice for each: 23 operations, where six separate trees
+// take 36 and their totals 11 more.
+__device__ __forceinline__ float wave_sum6(int lane, float v0, float v1, float v2, float v3,
+                                           float v4, float v5) {
+  const bool b0 = lane & 1, b1 = lane & 2, b2 = lane & 4;
+  const float a0 = dpp_fold<0xb1>(b0, v0, v1);  // quad_perm [1,0,3,2]: lanes l ^ 1
+  const float a1 = dpp_fold<0xb1>(b0, v2, v3);
+  const float a2 = dpp_fold<0xb1>(b0, v4, v5);
+  const float c0 = dpp_fold<0x4e>(b1, a0, a1);  // quad_perm [2,3,0,1]: l ^ 2
+  const float c1 = dpp_fold<0x4e>(false, a2, a2);
+  // l ^ 4: row_shl:4 into the even quads, row_shr:4 into the odd ones
+  const int give = __float_as_int(b2 ? c0 : c1);
+  int s = __builtin_amdgcn_update_dpp(0, give, 0x104, 0xf, 0x5, false);
+  s = __builtin_amdgcn_update_dpp(s, give, 0x114, 0xf, 0xa, false);
+  float d = (b2 ? c1 : c0) + __int_as_float(s);
+  // row_ror:8, then rows 0 + 1 and 2 + 3, then the halves
+  d += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(d), 0x128, 0xf, 0xf, true));
+  const unsigned u = __float_as_uint(d);
+  const auto r16 = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  d = __uint_as_float(r16[0]) + __uint_as_float(r16[1]);
+  const unsigned t = __float_as_uint(d);
+  const auto r32 = __builtin_amdgcn_permlane32_swap(t, t, false, false);
+  return __uint_as_float(r32[0]) + __uint_as_float(r32[1]);
 }
 
 // Additive adjoint, one lane per particle: the additive gradient of a particle
@@ -70,7 +86,8 @@ __device__ __forceinline__ float wave_sum(float v) {
 // cross-lane reduction.
 __global__ __launch_bounds__(256) void k_adjoint_add(SplatArgs a, const uint32_t *seg_unit,
                                                      const uint32_t *seg_first, uint32_t nseg,
-                                                     const float *grad, float *part) {
+                                                     uint32_t seglen, const float *grad,
+                                                     float *part) {
   __shared__ float s_g[4][3][64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const uint32_t sg = blockIdx.x * 4u + wave;
@@ -91,7 +108,7 @@ __global__ __launch_bounds__(256) void k_adjoint_add(SplatArgs a, const uint32_t
   wave_sync();
   const float(*G)[64] = s_g[wave];
   const uint32_t e0 = uniform(seg_first[sg]);
-  const uint32_t e1 = uniform(min(e0 + kSeg, a.bin_off[u + 1]));
+  const uint32_t e1 = uniform(min(e0 + seglen, a.bin_off[u + 1]));
   for (uint32_t base = e0; base < e1; base += 64) {
     if (base + lane >= e1) break;
     const uint32_t s = a.ent[base + lane];
@@ -147,7 +164,7 @@ __global__ __launch_bounds__(256) void k_adjoint_add(SplatArgs a, const uint32_t
   }
 }
 
-// Backward work items are list segments of at most kSeg entries: (unit,
+// Backward work items are list segments of at most seglen entries: (unit,
 // first entry).  Additive segments are independent; ordered segments are
 // joined per pixel by the affine composite map of each segment (passes A, B).
 
@@ -165,32 +182,52 @@ struct SegView {
 };
 
 __global__ __launch_bounds__(256) void k_seg_count(const uint32_t *bin_off, uint32_t nunits,
-                                                   uint32_t *cnt) {
+                                                   uint32_t seglen, uint32_t *cnt) {
   for (int64_t u = gtid_(); u < nunits; u += gstride_())
-    cnt[u] = (bin_off[u + 1] - bin_off[u] + kSeg - 1) / kSeg;
+    cnt[u] = (bin_off[u + 1] - bin_off[u] + seglen - 1) / seglen;
 }
 
 __global__ __launch_bounds__(256) void k_seg_emit(const uint32_t *bin_off, uint32_t nunits,
-                                                  const uint32_t *soff, uint32_t *seg_unit,
+                                                  uint32_t seglen, const uint32_t *soff, uint32_t *seg_unit,
                                                   uint32_t *seg_first) {
   for (int64_t u = gtid_(); u < nunits; u += gstride_()) {
     const uint32_t b = bin_off[u], e = bin_off[u + 1];
     uint32_t o = soff[u];
-    for (uint32_t f = b; f < e; f += kSeg, ++o) {
+    for (uint32_t f = b; f < e; f += seglen, ++o) {
       seg_unit[o] = static_cast<uint32_t>(u);
       seg_first[o] = f;
     }
   }
 }
 
-// One wave per ordered segment, lane = pixel of the 8x8 block.
+// exp(-x) - 1 for 0 <= x <= kSmallX, by its series to x^8 (the next term is
+// below 2^-32 of the result): over all floats there at most 0.695 ulp off, mean
+// 0.25; the library's 0.735 and 0.25, at 25 instructions to these 9.
+constexpr float kSmallX = 0.3f;
+__device__ __forceinline__ float expm1_small(float x) {
+  float p = 1.f / 40320.f;
+  p = fmaf(p, x, -1.f / 5040.f);
+  p = fmaf(p, x, 1.f / 720.f);
+  p = fmaf(p, x, -1.f / 120.f);
+  p = fmaf(p, x, 1.f / 24.f);
+  p = fmaf(p, x, -1.f / 6.f);
+  p = fmaf(p, x, 0.5f);
+  return fmaf(x * x, p, -x);
+}
+
+// One wave per ordered segment, lane = pixel of the 8x8 block: bound by its VALU
+// issue (about 85 and 190 instructions per entry) at 5 waves per SIMD.  500k
+// particles at 512^2, 1.46M entries: 353 -> 250 us (pass A) and 945 -> 560 us (C)
+// with the series for exp - 1, the six sums in one tree, q's derivative once per
+// particle and segments of 128 entries.
 //   PASS 0 (A): the segment's composite map and optical depth per pixel.
 //   PASS 2 (C): gradients, from the segment's start value and the depth
 //               behind it (pass B), particles in render order.
 template <int PASS>
 __global__ __launch_bounds__(256) void k_adjoint_ord(SplatArgs a, const uint32_t *seg_unit,
                                                      const uint32_t *seg_first, uint32_t nseg,
-                                                     const float *grad, float *part, SegView sv) {
+                                                     uint32_t seglen, const float *grad,
+                                                     float *part, SegView sv) {
   __shared__ uint32_t s_col[4][8][kPadA];
   __shared__ float s_ex[4][8][kPadA];
   __shared__ float s_ey[4][8][kPadA];
@@ -217,14 +254,16 @@ __global__ __launch_bounds__(256) void k_adjoint_ord(SplatArgs a, const uint32_t
   const float gray = ug.grayabsorb;
   const float lxf = static_cast<float>(lx), lyf = static_cast<float>(ly);
   const uint32_t e0 = uniform(seg_first[sg]);
-  const uint32_t e1 = uniform(min(e0 + kSeg, a.bin_off[u + 1]));
+  const uint32_t e1 = uniform(min(e0 + seglen, a.bin_off[u + 1]));
 
   // per-lane particle state of the current batch (lane = particle)
-  float pe[3], pq[3], ppx, ppy, pstp, pdstp;
+  float pe[3], pq[3], pdq[3], ppx, ppy, pstp, pdstp;
+  uint64_t small = 0;  // batch particles with every e_c (so e_c * att too, att <= 1) small
   // Phase A (lane = particle): the forward's footprint masks of this block's
   // columns (same float rules as the splat), smooth column / row factors.
   auto phase_a = [&](uint32_t base, int nb) {
     pe[0] = pe[1] = pe[2] = pq[0] = pq[1] = pq[2] = 0.f;
+    pdq[0] = pdq[1] = pdq[2] = 0.f;
     ppx = ppy = pstp = pdstp = 0.f;
     if (lane < nb) {
       const uint32_t s = a.ent[base + lane];
@@ -264,14 +303,27 @@ __global__ __launch_bounds__(256) void k_adjoint_ord(SplatArgs a, const uint32_t
       pq[0] = R.e0 / (R.e0 + gray);
       pq[1] = R.e1 / (R.e1 + gray);
       pq[2] = R.e2 / (R.e2 + gray);
+      for (int c = 0; c < 3; ++c) pdq[c] = gray / ((pe[c] + gray) * (pe[c] + gray));  // d q / d e
       ppx = posx;
       ppy = posy;
       pstp = stp;
       // d stp / d r = 2 / (h2sigma^2 r^3)
       pdstp = 2.f / (a.h2sigma * a.h2sigma * R.r * R.r * R.r);
     }
+    auto fits = [](float e) { return e >= 0.f && e <= kSmallX; };
+    small = __ballot(fits(pe[0]) && fits(pe[1]) && fits(pe[2]));
   };
 
+  // exp(-e_c att) - 1 of the batch's particle k
+  auto exp_minus_1 = [&](int k, float att, float *em) {
+    if ((small >> k) & 1u) {
+#pragma unroll
+      for (int c = 0; c < 3; ++c) em[c] = expm1_small(lane_f(pe[c], k) * att);
+    } else {
+#pragma unroll
+      for (int c = 0; c < 3; ++c) em[c] = expm1f(-(lane_f(pe[c], k) * att));
+    }
+  };
   // running state in double: P - q and depth differences cancel for opaque pixels
   double P[3], D[3], Dseg[3], Dafter[3];
 #pragma unroll
@@ -295,11 +347,13 @@ __global__ __launch_bounds__(256) void k_adjoint_ord(SplatArgs a, const uint32_t
       if (PASS == 0) {
         if (in) {
           const float att = ey[cy][k] * ex[cx][k];
+          float em[3];
+          exp_minus_1(k, att, em);
 #pragma unroll
           for (int c = 0; c < 3; ++c) {
             const float ea = lane_f(pe[c], k) * att;
             const double q = lane_f(pq[c], k);
-            const double T = 1.0 + static_cast<double>(expm1f(-ea));
+            const double T = 1.0 + static_cast<double>(em[c]);
             P[c] = q + (P[c] - q) * T;
             D[c] += static_cast<double>(ea);
           }
@@ -316,31 +370,30 @@ __global__ __launch_bounds__(256) void k_adjoint_ord(SplatArgs a, const uint32_t
       const float dx = lxf - lane_f(ppx, k), dy = lyf - lane_f(ppy, k);
       const float stp = lane_f(pstp, k);
       float gatt = 0.f, ge[3] = {0.f, 0.f, 0.f};
+      if (in) {
+        float em[3];
+        exp_minus_1(k, att, em);
 #pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        if (!in) continue;
-        const float e = lane_f(pe[c], k);
-        const float q = lane_f(pq[c], k);
-        const float ea = e * att;
-        const float omt = -expm1f(-ea);  // 1 - T without cancellation for small e*att
-        const float T = 1.f - omt;
-        D[c] += static_cast<double>(ea);
-        // transmittance behind particle k: the rest of this segment and the later ones
-        const float S = __expf(static_cast<float>(-((Dseg[c] - D[c]) + Dafter[c])));
-        const float gk = G[c] * S;  // dL/dP_k
-        const float dPdT = static_cast<float>(P[c] - static_cast<double>(q));
-        const float dqde = gray / ((e + gray) * (e + gray));
-        gatt += gk * dPdT * (-e * T);
-        ge[c] = gk * (dPdT * (-att * T) + omt * dqde);
-        P[c] = static_cast<double>(q) + (P[c] - static_cast<double>(q)) * static_cast<double>(T);
+        for (int c = 0; c < 3; ++c) {
+          const float e = lane_f(pe[c], k);
+          const float q = lane_f(pq[c], k);
+          const float ea = e * att;
+          const float omt = -em[c];  // 1 - T without cancellation for small e*att
+          const float T = 1.f - omt;
+          D[c] += static_cast<double>(ea);
+          // transmittance behind particle k: the rest of this segment and the later ones
+          const float S = __expf(static_cast<float>(-((Dseg[c] - D[c]) + Dafter[c])));
+          const float gk = G[c] * S;  // dL/dP_k
+          const float dPdT = static_cast<float>(P[c] - static_cast<double>(q));
+          gatt += gk * dPdT * (-e * T);
+          ge[c] = gk * (dPdT * (-att * T) + omt * lane_f(pdq[c], k));
+          P[c] = static_cast<double>(q) + (P[c] - static_cast<double>(q)) * static_cast<double>(T);
+        }
       }
       const float gsx = gatt * (-2.f * stp * dx * att);
       const float gsy = gatt * (-2.f * stp * dy * att);
       const float gr = gatt * att * (dx * dx + dy * dy) * lane_f(pdstp, k);
-      const float s0 = wave_sum(gsx), s1 = wave_sum(gsy), s2 = wave_sum(gr);
-      const float s3 = wave_sum(ge[0]), s4 = wave_sum(ge[1]), s5 = wave_sum(ge[2]);
-      const float v = lane == 0 ? s0 : lane == 1 ? s1 : lane == 2 ? s2 :
-                      lane == 3 ? s3 : lane == 4 ? s4 : s5;
+      const float v = wave_sum6(lane, gsx, gsy, gr, ge[0], ge[1], ge[2]);
       if (lane < 6) pp[lane] = v;
     }
     wave_sync();
@@ -363,19 +416,38 @@ __global__ __launch_bounds__(192) void k_adjoint_join(const uint32_t *soff, uint
   const uint32_t u = blockIdx.x;
   if (u >= nunits) return;
   const int c = threadIdx.x >> 6, px = threadIdx.x & 63;
-  const uint32_t j0 = soff[u], j1 = soff[u + 1];
+  const uint32_t j0 = uniform(soff[u]), j1 = uniform(soff[u + 1]);
+  // kJ segments' states are loaded at once (the last one's again past the end),
+  // as a step that waits for its own loads takes two memory latencies per 256
+  // entries of the longest list
+  constexpr uint32_t kJ = 16;
   double Pst = 0.0;
-  for (uint32_t j = j0; j < j1; ++j) {
-    const size_t i = sv.at(j, c, px);
-    const double A = sv.s0[i], B = sv.s1[i];
-    sv.s0[i] = Pst;
-    Pst = A * Pst + B;
+  for (uint32_t j = j0; j < j1; j += kJ) {
+    double A[kJ], B[kJ];
+#pragma unroll
+    for (uint32_t t = 0; t < kJ; ++t) {
+      const size_t i = sv.at(min(j + t, j1 - 1u), c, px);
+      A[t] = sv.s0[i];
+      B[t] = sv.s1[i];
+    }
+#pragma unroll
+    for (uint32_t t = 0; t < kJ; ++t) {
+      if (j + t >= j1) break;
+      sv.s0[sv.at(j + t, c, px)] = Pst;
+      Pst = A[t] * Pst + B[t];
+    }
   }
   double Da = 0.0;
-  for (uint32_t j = j1; j > j0; --j) {
-    const size_t i = sv.at(j - 1, c, px);
-    sv.s1[i] = Da;
-    Da += sv.s2[i];
+  for (uint32_t j = j1; j > j0; j -= min(kJ, j - j0)) {
+    double D[kJ];
+#pragma unroll
+    for (uint32_t t = 0; t < kJ; ++t) D[t] = sv.s2[sv.at(max(j, j0 + 1u + t) - 1u - t, c, px)];
+#pragma unroll
+    for (uint32_t t = 0; t < kJ; ++t) {
+      if (j - j0 <= t) break;
+      sv.s1[sv.at(j - 1u - t, c, px)] = Da;
+      Da += D[t];
+    }
   }
 }
 
@@ -525,34 +597,37 @@ __global__ __launch_bounds__(256) void k_reduce_parts(const uint32_t *poff, cons
 }
 }  // namespace
 
-void launch_seg_count(const uint32_t *bin_off, uint32_t nunits, uint32_t *cnt, hipStream_t s) {
-  k_seg_count<<<grid_of(nunits), 256, 0, s>>>(bin_off, nunits, cnt);
+void launch_seg_count(const uint32_t *bin_off, uint32_t nunits, uint32_t seglen, uint32_t *cnt,
+                      hipStream_t s) {
+  k_seg_count<<<grid_of(nunits), 256, 0, s>>>(bin_off, nunits, seglen, cnt);
   hip_check(hipGetLastError(), "k_seg_count launch");
 }
 
-void launch_seg_emit(const uint32_t *bin_off, uint32_t nunits, const uint32_t *soff,
-                     uint32_t *seg_unit, uint32_t *seg_first, hipStream_t s) {
-  k_seg_emit<<<grid_of(nunits), 256, 0, s>>>(bin_off, nunits, soff, seg_unit, seg_first);
+void launch_seg_emit(const uint32_t *bin_off, uint32_t nunits, uint32_t seglen,
+                     const uint32_t *soff, uint32_t *seg_unit, uint32_t *seg_first,
+                     hipStream_t s) {
+  k_seg_emit<<<grid_of(nunits), 256, 0, s>>>(bin_off, nunits, seglen, soff, seg_unit, seg_first);
   hip_check(hipGetLastError(), "k_seg_emit launch");
 }
 
 void launch_adjoint(bool additive, const uint32_t *seg_unit, const uint32_t *seg_first,
-                    uint32_t nseg, const uint32_t *soff, uint32_t nunits, const SplatArgs &a,
-                    const float *grad, float *part, double *segstate, hipStream_t s) {
+                    uint32_t nseg, uint32_t seglen, const uint32_t *soff, uint32_t nunits,
+                    const SplatArgs &a, const float *grad, float *part, double *segstate,
+                    hipStream_t s) {
   if (nseg == 0) return;
   const unsigned grid = (nseg + 3) / 4;
   if (additive) {
-    k_adjoint_add<<<grid, 256, 0, s>>>(a, seg_unit, seg_first, nseg, grad, part);
+    k_adjoint_add<<<grid, 256, 0, s>>>(a, seg_unit, seg_first, nseg, seglen, grad, part);
     hip_check(hipGetLastError(), "k_adjoint_add launch");
     return;
   }
   const size_t per = static_cast<size_t>(nseg) * 3 * 64;
   const SegView sv{segstate, segstate + per, segstate + 2 * per};
-  k_adjoint_ord<0><<<grid, 256, 0, s>>>(a, seg_unit, seg_first, nseg, grad, part, sv);
+  k_adjoint_ord<0><<<grid, 256, 0, s>>>(a, seg_unit, seg_first, nseg, seglen, grad, part, sv);
   hip_check(hipGetLastError(), "k_adjoint_ord (segment maps) launch");
   k_adjoint_join<<<nunits, 192, 0, s>>>(soff, nunits, sv);
   hip_check(hipGetLastError(), "k_adjoint_join launch");
-  k_adjoint_ord<2><<<grid, 256, 0, s>>>(a, seg_unit, seg_first, nseg, grad, part, sv);
+  k_adjoint_ord<2><<<grid, 256, 0, s>>>(a, seg_unit, seg_first, nseg, seglen, grad, part, sv);
   hip_check(hipGetLastError(), "k_adjoint_ord (gradients) launch");
 }
 

@@ -2006,11 +2006,12 @@ int backward_impl(splhip_ctx *c, const float *grad, const splhip_grads *out, hip
   uint32_t *tot = ws.get_as<uint32_t>(S_TOTALS, kTotalsWords);
   for (int p = 0; p < 2; ++p) {
     if (!pl.m[p]) continue;
-    // work items: list segments of at most kAdjSeg entries
+    // work items: list segments
+    const uint32_t seglen = adjoint_seglen(p == 1, pl.etot[p]);
     const uint32_t nu = pl.nunits;
     uint32_t *cnt = ws.get_as<uint32_t>(S_GRAD1, 2 * (static_cast<size_t>(nu) + 1));
     uint32_t *soff = cnt + nu + 1;
-    launch_seg_count(pl.bin_off[p], nu, cnt, s);
+    launch_seg_count(pl.bin_off[p], nu, seglen, cnt, s);
     scan_u32(cnt, soff, nu, soff + nu, ws, s);
     hip_check(hipMemcpyAsync(tot, soff + nu, 4, hipMemcpyDeviceToDevice, s), "segment total");
     hip_check(hipMemcpyAsync(tot + 1, pl.bin_off[p] + nu, 4, hipMemcpyDeviceToDevice, s),
@@ -2019,14 +2020,14 @@ int backward_impl(splhip_ctx *c, const float *grad, const splhip_grads *out, hip
     const uint32_t nseg = c->h_tot[0], ne = c->h_tot[1];
     if (nseg == 0) continue;
     uint32_t *seg = ws.get_as<uint32_t>(S_GRAD3, 2 * static_cast<size_t>(nseg));
-    launch_seg_emit(pl.bin_off[p], nu, soff, seg, seg + nseg, s);
+    launch_seg_emit(pl.bin_off[p], nu, seglen, soff, seg, seg + nseg, s);
     double *state = p == 0 ? ws.get_as<double>(S_GRAD4, static_cast<size_t>(nseg) * 3 * 64 * 3)
                            : nullptr;
     // per-entry partials, then per particle their sum in a fixed order: the
     // entries sorted stably by particle (render position), summed in FP64
     float *part = ws.get_as<float>(S_GRAD2, static_cast<size_t>(ne) * 6);
     const SplatArgs sa = splat_args(c, pl, p, F.tn);
-    launch_adjoint(p == 1, seg, seg + nseg, nseg, soff, nu, sa, grad, part, state, s);
+    launch_adjoint(p == 1, seg, seg + nseg, nseg, seglen, soff, nu, sa, grad, part, state, s);
     uint32_t *k0 = ws.get_as<uint32_t>(S_GRAD5, ne), *v0 = ws.get_as<uint32_t>(S_GRAD6, ne);
     uint32_t *k1 = ws.get_as<uint32_t>(S_GRAD7, ne), *v1 = ws.get_as<uint32_t>(S_GRAD8, ne);
     uint32_t *poff = ws.get_as<uint32_t>(S_GRAD9, static_cast<size_t>(pl.m[p]) + 1);

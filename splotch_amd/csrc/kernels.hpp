@@ -338,20 +338,30 @@ void launch_splat_pc(bool additive, const uint32_t *items, uint32_t npc, const S
 // Differentiable form (adjoint.hip): screen-space gradient accumulation over
 // the forward's work items (gscr: n x 6 doubles, zeroed by the caller), the
 // chain to the particle fields of job 0, and an FP64 fill.
-// Backward work items: list segments of at most kAdjSeg entries per unit
+// Backward work items: list segments of at most seglen entries per unit
 // (cnt[u] segments; soff = exclusive scan of cnt).  A segment is one wave's
-// serial walk, so short segments shorten the backward's critical path (500k
-// ordered particles at 512^2, forward + backward: 8.41 ms with 2048 entries,
-// 4.80 with 512, 4.50 with 256) for 18 B of FP64 segment state per entry.
-constexpr uint32_t kAdjSeg = 256;
-void launch_seg_count(const uint32_t *bin_off, uint32_t nunits, uint32_t *cnt, hipStream_t s);
-void launch_seg_emit(const uint32_t *bin_off, uint32_t nunits, const uint32_t *soff,
-                     uint32_t *seg_unit, uint32_t *seg_first, hipStream_t s);
+// serial walk, so short segments shorten the backward's critical path and its
+// last, partly filled round of waves; an ordered one has 4.6 KB of FP64 state
+// (500k ordered particles at 512^2, forward + backward: 2.97 ms with 512 entries,
+// 2.41 with 256, 2.29 with 128, 2.39 with 64; 2M additive ones 2.15 ms with 256,
+// 2.20 with 128).  Ordered passes past kAdjShort entries, which fill the GPU many
+// times over, keep 256 and half the state.
+constexpr uint32_t kAdjSeg = 256, kAdjSegOrdered = 128;
+constexpr uint64_t kAdjShort = uint64_t(1) << 26;
+inline uint32_t adjoint_seglen(bool additive, uint64_t entries) {
+  return additive || entries > kAdjShort ? kAdjSeg : kAdjSegOrdered;
+}
+void launch_seg_count(const uint32_t *bin_off, uint32_t nunits, uint32_t seglen, uint32_t *cnt,
+                      hipStream_t s);
+void launch_seg_emit(const uint32_t *bin_off, uint32_t nunits, uint32_t seglen,
+                     const uint32_t *soff, uint32_t *seg_unit, uint32_t *seg_first,
+                     hipStream_t s);
 // part: 6 floats per list entry (the particle's screen-space partials over
 // the entry's block); segstate: ordered mode only, nseg * 3 * 64 * 3 doubles.
 void launch_adjoint(bool additive, const uint32_t *seg_unit, const uint32_t *seg_first,
-                    uint32_t nseg, const uint32_t *soff, uint32_t nunits, const SplatArgs &a,
-                    const float *grad, float *part, double *segstate, hipStream_t s);
+                    uint32_t nseg, uint32_t seglen, const uint32_t *soff, uint32_t nunits,
+                    const SplatArgs &a, const float *grad, float *part, double *segstate,
+                    hipStream_t s);
 // v[i] = i
 void launch_iota(uint32_t *v, uint32_t n, hipStream_t s);
 // gscr[order[s]] += sum over t in [poff[s], poff[s+1]) of part[jv[t]] (FP64,
