@@ -353,9 +353,9 @@ inline uint32_t adjoint_seglen(bool additive, uint64_t entries) {
 }
 void launch_seg_count(const uint32_t *bin_off, uint32_t nunits, uint32_t seglen, uint32_t *cnt,
                       hipStream_t s);
-void launch_seg_emit(const uint32_t *bin_off, uint32_t nunits, uint32_t seglen,
-                     const uint32_t *soff, uint32_t *seg_unit, uint32_t *seg_first,
-                     hipStream_t s);
+void launch_seg_emit(const uint32_t *bin_off, uint32_t nunits, uint32_t nseg,
+                     uint32_t seglen, const uint32_t *soff, uint32_t *seg_unit,
+                     uint32_t *seg_first, hipStream_t s);
 // part: 6 floats per list entry (the particle's screen-space partials over
 // the entry's block); segstate: ordered mode only, nseg * 3 * 64 * 3 doubles.
 void launch_adjoint(bool additive, const uint32_t *seg_unit, const uint32_t *seg_first,
