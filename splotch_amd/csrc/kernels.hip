@@ -503,6 +503,20 @@ __device__ __forceinline__ uint32_t lane_pick(const uint32_t (&v)[NB], int lane)
   return x;
 }
 
+// The masks of entries [i0, i1) of a chunk, 0 past i1; one wait for all loads
+// (a load per step of 64 entries waits 16 times).
+constexpr int kSplitSteps = kSplitChunk / 64;
+__device__ __forceinline__ void chunk_masks(const uint32_t *keys, uint32_t i0, uint32_t i1,
+                                            int rbits, int lane, uint32_t (&mk)[kSplitSteps]) {
+#pragma unroll
+  for (int j = 0; j < kSplitSteps; ++j) {
+    const uint32_t i = i0 + 64u * j + lane;
+    mk[j] = i < i1 ? keys[i] : 0u;
+  }
+#pragma unroll
+  for (int j = 0; j < kSplitSteps; ++j) mk[j] >>= rbits;
+}
+
 template <int NB>
 __global__ __launch_bounds__(256) void k_split_chunks(const uint32_t *keys, uint32_t ecap,
                                                       const uint32_t *de, uint32_t nchunks,
@@ -517,11 +531,14 @@ __global__ __launch_bounds__(256) void k_split_chunks(const uint32_t *keys, uint
     uint32_t n[NB];
 #pragma unroll
     for (int b = 0; b < NB; ++b) n[b] = 0;
-    for (uint32_t i = i0; i < i1; i += 64) {
-      const uint32_t mk = (i + lane < i1) ? (keys[i + lane] >> rbits) : 0u;
+    uint32_t mk[kSplitSteps];
+    chunk_masks(keys, i0, i1, rbits, lane, mk);
+#pragma unroll
+    for (int j = 0; j < kSplitSteps; ++j) {
+      if (i0 + 64u * j >= i1) break;
 #pragma unroll
       for (int b = 0; b < NB; ++b)
-        n[b] += static_cast<uint32_t>(__popcll(__ballot((mk >> b) & 1u)));
+        n[b] += static_cast<uint32_t>(__popcll(__ballot((mk[j] >> b) & 1u)));
     }
     const uint32_t v = lane_pick<NB>(n, lane);
     if (lane < NB) ccnt[static_cast<int64_t>(lane) * nchunks + c] = v;
@@ -536,11 +553,14 @@ __device__ __forceinline__ void split_prefix(const uint32_t *keys, const uint32_
   const uint32_t c = x / kSplitChunk;
 #pragma unroll
   for (int b = 0; b < NB; ++b) n[b] = cpre[static_cast<int64_t>(b) * nchunks + c];
-  for (uint32_t i = c * kSplitChunk; i < x; i += 64) {
-    const uint32_t mk = (i + lane < x) ? (keys[i + lane] >> rbits) : 0u;
+  uint32_t mk[kSplitSteps];
+  chunk_masks(keys, c * kSplitChunk, x, rbits, lane, mk);
+#pragma unroll
+  for (int j = 0; j < kSplitSteps; ++j) {
+    if (c * kSplitChunk + 64u * j >= x) break;
 #pragma unroll
     for (int b = 0; b < NB; ++b)
-      n[b] += static_cast<uint32_t>(__popcll(__ballot((mk >> b) & 1u)));
+      n[b] += static_cast<uint32_t>(__popcll(__ballot((mk[j] >> b) & 1u)));
   }
 }
 
@@ -597,7 +617,9 @@ __global__ __launch_bounds__(256) void k_split_base(uint32_t nregions, const uin
   }
 }
 
-// One wave per chunk: every entry to its blocks' lists.
+// One wave per chunk: every entry to its blocks' lists.  The lists' starts of
+// an entry's region are loaded whole, ahead of the stores: read one by one, each
+// store waited for its own (26k region entries: 35 -> 20 us; 1.8M: 43 -> 23 us).
 template <int S>
 __global__ __launch_bounds__(256) void k_split_scatter(const uint32_t *keys, const uint32_t *vals,
                                                        uint32_t ecap, const uint32_t *de,
@@ -621,7 +643,7 @@ __global__ __launch_bounds__(256) void k_split_scatter(const uint32_t *keys, con
     // they reach L2 as whole lines rather than 16 interleaved partial ones
     for (uint32_t i = i0; i < i1; i += 4 * 64) {
       uint32_t mk[4], idx[4];
-      const uint32_t *bs[4];
+      uint4 bs[4][NB / 4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const uint32_t t = i + 64u * j + lane;
@@ -629,7 +651,10 @@ __global__ __launch_bounds__(256) void k_split_scatter(const uint32_t *keys, con
         const uint32_t k = in ? keys[t] : 0u;
         idx[j] = in ? vals[t] : 0u;
         mk[j] = in ? k >> rbits : 0u;  // no block for entries past the chunk
-        bs[j] = base + static_cast<int64_t>(NB) * (k & rmask);
+        const uint4 *bp = reinterpret_cast<const uint4 *>(base) +
+                          static_cast<int64_t>(NB / 4) * (k & rmask);
+#pragma unroll
+        for (int q = 0; q < NB / 4; ++q) bs[j][q] = bp[q];
       }
 #pragma unroll
       for (int b = 0; b < NB; ++b) {
@@ -637,7 +662,9 @@ __global__ __launch_bounds__(256) void k_split_scatter(const uint32_t *keys, con
         for (int j = 0; j < 4; ++j) {
           const bool on = (mk[j] >> b) & 1u;
           const uint64_t bal = __ballot(on);
-          if (on) ent[bs[j][b] + n[b] + mbcnt64(bal)] = idx[j];
+          const uint4 &v = bs[j][b / 4];
+          const uint32_t at = (b & 3) == 0 ? v.x : (b & 3) == 1 ? v.y : (b & 3) == 2 ? v.z : v.w;
+          if (on) ent[at + n[b] + mbcnt64(bal)] = idx[j];
           n[b] += static_cast<uint32_t>(__popcll(bal));
         }
       }
