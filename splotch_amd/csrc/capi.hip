@@ -1226,7 +1226,7 @@ void stage_splat(splhip_ctx *c, Plan &pl, int p, const Tuning &tn, hipStream_t s
     // waits briefly.  Staged lists need no such start: their operand kernels'
     // workgroups fit in as the normal ones end (20k ordered at 257 x 193: 0.377
     // ms with the wait, 0.339 without; larger frames up to 1 % faster without).
-    if (npc > 0 || nseg > 0) launch_delay(40, s);
+    if (npc > 0 || nseg > 0) launch_delay(40, s, dc.npc);
     if (placed) hip_check(hipEventRecord(placed, s), "record placed");
     mark(c, p == 0 ? 7 : 9, true, s);
     launch_splat8(p == 1, tn.variant, nit, nn, sn, s, dc, tn.ppw, pl.nsplit[p]);

@@ -701,7 +701,8 @@ __global__ __launch_bounds__(256) void k_add_images(float *pic, const float *add
 }
 
 // Bounded wait of `ticks` s_memrealtime ticks (100 MHz): one wave, then exit.
-__global__ __launch_bounds__(64) void k_delay(uint32_t ticks) {
+__global__ __launch_bounds__(64) void k_delay(uint32_t ticks, const uint32_t *n) {
+  if (n && *n == 0) return;
   const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
   while (__builtin_amdgcn_s_memrealtime() - t0 < ticks) __builtin_amdgcn_s_sleep(8);
 }
@@ -1070,8 +1071,8 @@ void launch_add_images(float *pic, const float *add, int64_t n, hipStream_t s) {
   hip_check(hipGetLastError(), "k_add_images launch");
 }
 
-void launch_delay(uint32_t us, hipStream_t s) {
-  k_delay<<<1, 64, 0, s>>>(us * 100u);
+void launch_delay(uint32_t us, hipStream_t s, const uint32_t *n) {
+  k_delay<<<1, 64, 0, s>>>(us * 100u, n);
   hip_check(hipGetLastError(), "k_delay launch");
 }
 

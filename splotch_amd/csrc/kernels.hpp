@@ -135,8 +135,9 @@ void launch_cap_check(uint32_t *m, uint32_t *e, const uint64_t *e64, uint32_t *e
                       hipStream_t s);
 // pic[i] += add[i]
 void launch_add_images(float *pic, const float *add, int64_t n, hipStream_t s);
-// A one-wave kernel that returns after `us` microseconds (bounded wait).
-void launch_delay(uint32_t us, hipStream_t s);
+// A one-wave kernel that returns after `us` microseconds (bounded wait); at once
+// where a device count n is given and is 0.
+void launch_delay(uint32_t us, hipStream_t s, const uint32_t *n = nullptr);
 // Host records staged chunk-major (chunk k: records [k C, k C + cnt_k), its
 // ncol float columns of cnt_k values back to back, then cnt_k type bytes)
 // into the SoA columns soa[q nn + i] and type[i].
