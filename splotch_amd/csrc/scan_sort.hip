@@ -281,7 +281,8 @@ void scan_impl(Jobs<In> jobs, unsigned nj, int64_t n, Workspace &ws, hipStream_t
   k_scan_apply<In><<<grid, 256, 0, s>>>(jobs, n, dn);
 }
 
-template <int BITS>
+// ITEMS: keys per thread; a tile is 256 ITEMS keys.
+template <int BITS, int ITEMS>
 __global__ __launch_bounds__(256) void k_rs_hist(const uint32_t *keys, int64_t cap,
                                                  const uint32_t *dn, int shift, uint32_t *hist,
                                                  int64_t nblocks, bool tile_major) {
@@ -292,9 +293,9 @@ __global__ __launch_bounds__(256) void k_rs_hist(const uint32_t *keys, int64_t c
   for (int i = threadIdx.x; i < 4 * R; i += 256) (&h[0][0])[i] = 0;
   __syncthreads();
   const int wave = threadIdx.x >> 6;
-  const int64_t base = static_cast<int64_t>(blockIdx.x) * kTile;
+  const int64_t base = static_cast<int64_t>(blockIdx.x) * (256 * ITEMS);
 #pragma unroll 4
-  for (int i = 0; i < kItems; ++i) {
+  for (int i = 0; i < ITEMS; ++i) {
     const int64_t idx = base + i * 256 + threadIdx.x;
     if (idx < n) atomicAdd(&h[wave][(keys[idx] >> shift) & M], 1u);
   }
@@ -305,17 +306,17 @@ __global__ __launch_bounds__(256) void k_rs_hist(const uint32_t *keys, int64_t c
         h[0][d] + h[1][d] + h[2][d] + h[3][d];
 }
 
-// Ranks a wave's kItems keys (striped: item it of lane l is input it * 64 + l)
+// Ranks a wave's ITEMS keys (striped: item it of lane l is input it * 64 + l)
 // by digit, in input order: rk[it] = rank among the wave's equal digits, counts
 // per digit in wh (zeroed by the caller).
-template <int BITS>
-__device__ __forceinline__ void wave_rank(const uint32_t (&kk)[kItems], const bool (&ok)[kItems],
+template <int BITS, int ITEMS>
+__device__ __forceinline__ void wave_rank(const uint32_t (&kk)[ITEMS], const bool (&ok)[ITEMS],
                                           int shift, int lane, uint32_t *wh,
-                                          uint32_t (&rk)[kItems]) {
+                                          uint32_t (&rk)[ITEMS]) {
   constexpr uint32_t M = (1u << BITS) - 1;
   const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
 #pragma unroll
-  for (int it = 0; it < kItems; ++it) {
+  for (int it = 0; it < ITEMS; ++it) {
     const uint32_t d = (kk[it] >> shift) & M;
     uint64_t m = __ballot(ok[it]);
 #pragma unroll
@@ -335,11 +336,11 @@ __device__ __forceinline__ void wave_rank(const uint32_t (&kk)[kItems], const bo
   }
 }
 
-// Digit totals of the block's 4 waves (wh[w][d] counts) to the wave offsets
+// Digit totals of the block's W waves (wh[w][d] counts) to the wave offsets
 // within each digit (wh) and the start of each digit's run (dstart).
-template <int R>
+template <int R, int W = 4>
 __device__ __forceinline__ void digit_starts(uint32_t (*wh)[R], uint32_t *dstart, uint32_t *s_w) {
-  constexpr int DPT = (R + 255) / 256;  // digits per thread in the block scan
+  constexpr int DPT = (R + 64 * W - 1) / (64 * W);  // digits per thread in the block scan
   uint32_t tot[DPT];
   uint32_t tsum = 0;
 #pragma unroll
@@ -348,7 +349,7 @@ __device__ __forceinline__ void digit_starts(uint32_t (*wh)[R], uint32_t *dstart
     uint32_t acc = 0;
     if (d < R) {
 #pragma unroll
-      for (int w = 0; w < 4; ++w) {
+      for (int w = 0; w < W; ++w) {
         const uint32_t t = wh[w][d];
         wh[w][d] = acc;
         acc += t;
@@ -357,7 +358,7 @@ __device__ __forceinline__ void digit_starts(uint32_t (*wh)[R], uint32_t *dstart
     tot[j] = acc;
     tsum += acc;
   }
-  uint32_t start = block_excl_scan(tsum, s_w);
+  uint32_t start = block_excl_scan<W>(tsum, s_w);
 #pragma unroll
   for (int j = 0; j < DPT; ++j) {
     const int d = threadIdx.x * DPT + j;
@@ -368,22 +369,22 @@ __device__ __forceinline__ void digit_starts(uint32_t (*wh)[R], uint32_t *dstart
 
 // DIRECT: hist holds the tiles' own histograms, tile-major, and the workgroup
 // sums them to its digits' global starts; else their digit-major scan.
-template <int BITS, bool DIRECT>
+template <int BITS, bool DIRECT, int ITEMS>
 __global__ __launch_bounds__(256) void k_rs_scatter(const uint32_t *kin, const uint32_t *vin,
                                                     uint32_t *kout, uint32_t *vout, int64_t cap,
                                                     const uint32_t *dn, int shift,
                                                     const uint32_t *hist, int64_t nblocks) {
   const int64_t n = count_of(cap, dn);
-  constexpr int R = 1 << BITS;
+  constexpr int R = 1 << BITS, TILE = 256 * ITEMS;
   constexpr uint32_t M = R - 1;
   constexpr int DPT = (R + 255) / 256;
   __shared__ uint32_t wh[4][R];   // per-wave digit counts -> offsets
   __shared__ uint32_t dstart[R];  // block-local start of each digit run
   __shared__ uint32_t gbase[R];   // global start of (digit, this tile)
-  __shared__ uint32_t sk[kTile], sv[kTile];
+  __shared__ uint32_t sk[TILE], sv[TILE];
   __shared__ uint32_t s_w[4];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int64_t tbase = static_cast<int64_t>(blockIdx.x) * kTile;
+  const int64_t tbase = static_cast<int64_t>(blockIdx.x) * TILE;
   if (tbase >= n) return;  // a tile past the device count (uniform)
   for (int i = threadIdx.x; i < 4 * R; i += 256) (&wh[0][0])[i] = 0;
   if (DIRECT) {
@@ -415,22 +416,22 @@ __global__ __launch_bounds__(256) void k_rs_scatter(const uint32_t *kin, const u
       gbase[d] = hist[static_cast<int64_t>(d) * nblocks + blockIdx.x];
   }
   __syncthreads();
-  const int64_t base = tbase + wave * (kTile / 4);
-  uint32_t kk[kItems], vv[kItems], rk[kItems];
-  bool ok[kItems];
+  const int64_t base = tbase + wave * (TILE / 4);
+  uint32_t kk[ITEMS], vv[ITEMS], rk[ITEMS];
+  bool ok[ITEMS];
 #pragma unroll
-  for (int it = 0; it < kItems; ++it) {
+  for (int it = 0; it < ITEMS; ++it) {
     const int64_t idx = base + it * 64 + lane;
     ok[it] = idx < n;
     kk[it] = ok[it] ? kin[idx] : 0u;
     vv[it] = ok[it] ? vin[idx] : 0u;
   }
-  wave_rank<BITS>(kk, ok, shift, lane, wh[wave], rk);
+  wave_rank<BITS, ITEMS>(kk, ok, shift, lane, wh[wave], rk);
   __syncthreads();
   digit_starts<R>(wh, dstart, s_w);
   __syncthreads();
 #pragma unroll
-  for (int it = 0; it < kItems; ++it) {
+  for (int it = 0; it < ITEMS; ++it) {
     if (ok[it]) {
       const uint32_t d = (kk[it] >> shift) & M;
       const uint32_t lp = dstart[d] + wh[wave][d] + rk[it];
@@ -439,7 +440,7 @@ __global__ __launch_bounds__(256) void k_rs_scatter(const uint32_t *kin, const u
     }
   }
   __syncthreads();
-  const int cnt = static_cast<int>(min<int64_t>(kTile, n - tbase));
+  const int cnt = static_cast<int>(min<int64_t>(TILE, n - tbase));
   for (int i = threadIdx.x; i < cnt; i += 256) {
     const uint32_t key = sk[i];
     const uint32_t d = (key >> shift) & M;
@@ -450,19 +451,22 @@ __global__ __launch_bounds__(256) void k_rs_scatter(const uint32_t *kin, const u
 }
 
 // The whole sort in one workgroup, for at most kTile pairs: digits of 8 bits
-// (the last pass's digit is cut at end_bit).
-__global__ __launch_bounds__(256) void k_rs_one(const uint32_t *kin, const uint32_t *vin,
+// (the last pass's digit is cut at end_bit).  1024 threads with 4 pairs each: a
+// wave ranks its keys 64 at a time (256 threads with 16 pairs: 8.4 us for one
+// digit of 1000 keys, 5 with 1024).
+constexpr int kOneItems = kTile / kOneThreads;
+__global__ __launch_bounds__(kOneThreads) void k_rs_one(const uint32_t *kin, const uint32_t *vin,
                                                 uint32_t *kout, uint32_t *vout, int64_t cap,
                                                 const uint32_t *dn, int begin_bit, int end_bit) {
   const int n = static_cast<int>(count_of(cap, dn));
-  constexpr int R = 256;
-  __shared__ uint32_t wh[4][R], dstart[R], sk[kTile], sv[kTile], s_w[4];
+  constexpr int R = 256, W = kOneThreads / 64;
+  __shared__ uint32_t wh[W][R], dstart[R], sk[kTile], sv[kTile], s_w[W];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int base = wave * (kTile / 4);
-  uint32_t kk[kItems], vv[kItems], rk[kItems];
-  bool ok[kItems];
+  const int base = wave * (kTile / W);
+  uint32_t kk[kOneItems], vv[kOneItems], rk[kOneItems];
+  bool ok[kOneItems];
 #pragma unroll
-  for (int it = 0; it < kItems; ++it) {
+  for (int it = 0; it < kOneItems; ++it) {
     const int idx = base + it * 64 + lane;
     ok[it] = idx < n;
     kk[it] = ok[it] ? kin[idx] : 0u;
@@ -470,17 +474,17 @@ __global__ __launch_bounds__(256) void k_rs_one(const uint32_t *kin, const uint3
   }
   const uint32_t keep = end_bit < 32 ? (1u << end_bit) - 1u : ~0u;
   for (int shift = begin_bit; shift < end_bit; shift += 8) {
-    for (int i = threadIdx.x; i < 4 * R; i += 256) (&wh[0][0])[i] = 0;
+    for (int i = threadIdx.x; i < W * R; i += kOneThreads) (&wh[0][0])[i] = 0;
     __syncthreads();
-    uint32_t dk[kItems];
+    uint32_t dk[kOneItems];
 #pragma unroll
-    for (int it = 0; it < kItems; ++it) dk[it] = kk[it] & keep;
-    wave_rank<8>(dk, ok, shift, lane, wh[wave], rk);
+    for (int it = 0; it < kOneItems; ++it) dk[it] = kk[it] & keep;
+    wave_rank<8, kOneItems>(dk, ok, shift, lane, wh[wave], rk);
     __syncthreads();
-    digit_starts<R>(wh, dstart, s_w);
+    digit_starts<R, W>(wh, dstart, s_w);
     __syncthreads();
 #pragma unroll
-    for (int it = 0; it < kItems; ++it) {
+    for (int it = 0; it < kOneItems; ++it) {
       if (ok[it]) {
         const uint32_t d = (dk[it] >> shift) & (R - 1);
         const uint32_t lp = dstart[d] + wh[wave][d] + rk[it];
@@ -490,7 +494,7 @@ __global__ __launch_bounds__(256) void k_rs_one(const uint32_t *kin, const uint3
     }
     __syncthreads();
 #pragma unroll
-    for (int it = 0; it < kItems; ++it) {
+    for (int it = 0; it < kOneItems; ++it) {
       const int idx = base + it * 64 + lane;
       if (ok[it]) {
         kk[it] = sk[idx];
@@ -500,7 +504,7 @@ __global__ __launch_bounds__(256) void k_rs_one(const uint32_t *kin, const uint3
     __syncthreads();
   }
 #pragma unroll
-  for (int it = 0; it < kItems; ++it) {
+  for (int it = 0; it < kOneItems; ++it) {
     const int idx = base + it * 64 + lane;
     if (ok[it]) {
       kout[idx] = kk[it];
@@ -511,20 +515,62 @@ __global__ __launch_bounds__(256) void k_rs_one(const uint32_t *kin, const uint3
 
 constexpr int64_t kDirectSort = 128;  // tiles whose histograms a scatter workgroup sums itself
 
-template <int BITS>
+template <int BITS, int ITEMS>
 void rs_pass(const uint32_t *sk, const uint32_t *sv, uint32_t *dk, uint32_t *dv, int64_t n,
              const uint32_t *dn, int shift, int64_t nb, uint32_t *hist, Workspace &ws,
              hipStream_t s) {
   const bool direct = nb <= kDirectSort;
   const unsigned g = static_cast<unsigned>(nb);
-  k_rs_hist<BITS><<<g, 256, 0, s>>>(sk, n, dn, shift, hist, nb, direct);
+  k_rs_hist<BITS, ITEMS><<<g, 256, 0, s>>>(sk, n, dn, shift, hist, nb, direct);
   if (direct) {
-    k_rs_scatter<BITS, true><<<g, 256, 0, s>>>(sk, sv, dk, dv, n, dn, shift, hist, nb);
+    k_rs_scatter<BITS, true, ITEMS><<<g, 256, 0, s>>>(sk, sv, dk, dv, n, dn, shift, hist, nb);
   } else {
     scan_u32(hist, hist, (int64_t(1) << BITS) * nb, nullptr, ws, s);
-    k_rs_scatter<BITS, false><<<g, 256, 0, s>>>(sk, sv, dk, dv, n, dn, shift, hist, nb);
+    k_rs_scatter<BITS, false, ITEMS><<<g, 256, 0, s>>>(sk, sv, dk, dv, n, dn, shift, hist, nb);
   }
   hip_check(hipGetLastError(), "radix sort launch");
+}
+
+// Sorts of up to kSmallSort pairs take tiles of 1024 (128 of them, as many as a
+// scatter sums the histograms of): a wave ranks its keys 64 at a time, one LDS
+// update after another, which is a pass's time where the tiles do not fill the
+// GPU (20k ordered at 257 x 193: 325 -> 295 us; 16 captured thumbnails 861 -> 842
+// us, 851 up to 65536 pairs only).
+constexpr int64_t kSmallSort = 131072;
+constexpr int kSmallItems = 4;
+
+template <int ITEMS>
+int radix_sort_tiled(uint32_t *k0, uint32_t *v0, uint32_t *k1, uint32_t *v1, int64_t n,
+                     int begin_bit, int end_bit, Workspace &ws, hipStream_t s,
+                     const uint32_t *dn) {
+  const int64_t nb = (n + 256 * ITEMS - 1) / (256 * ITEMS);
+  const int bits = end_bit - begin_bit;
+  const int passes = (bits + kMaxBits - 1) / kMaxBits;
+  const int width = (bits + passes - 1) / passes;  // <= 9
+  uint32_t *hist = ws.get_as<uint32_t>(S_HIST, (size_t(1) << width) * static_cast<size_t>(nb));
+  int cur = 0;
+  for (int shift = begin_bit; shift < end_bit; shift += width) {
+    const int w = std::min(width, end_bit - shift);
+    const uint32_t *sk = cur ? k1 : k0;
+    const uint32_t *sv = cur ? v1 : v0;
+    uint32_t *dk = cur ? k0 : k1;
+    uint32_t *dv = cur ? v0 : v1;
+    switch (w) {
+#define SPLHIP_PASS(B) rs_pass<B, ITEMS>(sk, sv, dk, dv, n, dn, shift, nb, hist, ws, s)
+      case 1: SPLHIP_PASS(1); break;
+      case 2: SPLHIP_PASS(2); break;
+      case 3: SPLHIP_PASS(3); break;
+      case 4: SPLHIP_PASS(4); break;
+      case 5: SPLHIP_PASS(5); break;
+      case 6: SPLHIP_PASS(6); break;
+      case 7: SPLHIP_PASS(7); break;
+      case 8: SPLHIP_PASS(8); break;
+      default: SPLHIP_PASS(9); break;
+#undef SPLHIP_PASS
+    }
+    cur ^= 1;
+  }
+  return cur;
 }
 
 }  // namespace
@@ -556,36 +602,13 @@ int radix_sort_pairs(uint32_t *k0, uint32_t *v0, uint32_t *k1, uint32_t *v1, int
                      const uint32_t *dn) {
   if (n <= 1 || end_bit <= begin_bit) return 0;
   if (n <= kTile) {
-    k_rs_one<<<1, 256, 0, s>>>(k0, v0, k1, v1, n, dn, begin_bit, end_bit);
+    k_rs_one<<<1, kOneThreads, 0, s>>>(k0, v0, k1, v1, n, dn, begin_bit, end_bit);
     hip_check(hipGetLastError(), "k_rs_one launch");
     return 1;
   }
-  const int64_t nb = (n + kTile - 1) / kTile;
-  const int bits = end_bit - begin_bit;
-  const int passes = (bits + kMaxBits - 1) / kMaxBits;
-  const int width = (bits + passes - 1) / passes;  // <= 9
-  uint32_t *hist = ws.get_as<uint32_t>(S_HIST, (size_t(1) << width) * static_cast<size_t>(nb));
-  int cur = 0;
-  for (int shift = begin_bit; shift < end_bit; shift += width) {
-    const int w = std::min(width, end_bit - shift);
-    const uint32_t *sk = cur ? k1 : k0;
-    const uint32_t *sv = cur ? v1 : v0;
-    uint32_t *dk = cur ? k0 : k1;
-    uint32_t *dv = cur ? v0 : v1;
-    switch (w) {
-      case 1: rs_pass<1>(sk, sv, dk, dv, n, dn, shift, nb, hist, ws, s); break;
-      case 2: rs_pass<2>(sk, sv, dk, dv, n, dn, shift, nb, hist, ws, s); break;
-      case 3: rs_pass<3>(sk, sv, dk, dv, n, dn, shift, nb, hist, ws, s); break;
-      case 4: rs_pass<4>(sk, sv, dk, dv, n, dn, shift, nb, hist, ws, s); break;
-      case 5: rs_pass<5>(sk, sv, dk, dv, n, dn, shift, nb, hist, ws, s); break;
-      case 6: rs_pass<6>(sk, sv, dk, dv, n, dn, shift, nb, hist, ws, s); break;
-      case 7: rs_pass<7>(sk, sv, dk, dv, n, dn, shift, nb, hist, ws, s); break;
-      case 8: rs_pass<8>(sk, sv, dk, dv, n, dn, shift, nb, hist, ws, s); break;
-      default: rs_pass<9>(sk, sv, dk, dv, n, dn, shift, nb, hist, ws, s); break;
-    }
-    cur ^= 1;
-  }
-  return cur;
+  return n <= kSmallSort
+             ? radix_sort_tiled<kSmallItems>(k0, v0, k1, v1, n, begin_bit, end_bit, ws, s, dn)
+             : radix_sort_tiled<kItems>(k0, v0, k1, v1, n, begin_bit, end_bit, ws, s, dn);
 }
 
 }  // namespace splhip

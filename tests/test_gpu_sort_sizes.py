@@ -1,5 +1,6 @@
 """GPU parity of binning and depth sort around the sizes where the scans and
-radix sorts change form: one workgroup up to 4096 pairs / 16384 elements, the
+radix sorts change form: one workgroup up to 4096 pairs / 16384 elements, tiles of
+1024 pairs up to 131072, the
 tiles' histograms summed by the scatter up to 128 tiles (524288 pairs), then
 scanned; the pass sizes read late or early.  Bar: the reference-tile lists and
 the render order equal the oracle's, and an ordered image (for the sizes it is
@@ -28,7 +29,8 @@ def R():
     r.close()
 
 
-@pytest.mark.parametrize("n", [1, 2, 63, 4095, 4096, 4097, 16384, 16385, 70001, 524288, 540000])
+@pytest.mark.parametrize("n", [1, 2, 63, 4095, 4096, 4097, 16384, 16385, 70001, 131072,
+                               131073, 140000, 524288, 540000])
 def test_sort_sizes(R, n):
     import splotch_amd as S
     print("case sort sizes n", n, flush=True)
