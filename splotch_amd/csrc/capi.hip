@@ -896,9 +896,10 @@ struct Tuning {
 // 195M to 322M entries: 33.9 -> 27.4, 37.8 -> 28.3, 53.0 -> 31.0, 51.0 -> 23.4
 // ms).  The length is that of a walk of about half such a pass: 24576 entries
 // 31.1, 30.4, 42.2, 27.6 ms (warm-ups), 56000 the first and third 35.6, 36.4 (the
-// last segments outlast the pass).  In smaller passes they outlast it at any
-// length that pays for its warm-ups (64 views, 137M entries: 30.6 ms without,
-// 32.2 from lists of 33k on).
+// last segments outlast the pass).  Batches of 64 views: 160M and 169M entries
+// 37.3 and 38.1 ms without, 33.9 and 34.6 with; 137M to 149M 29.7, 33.7, 33.4 and
+// 34.3 without, 30.9, 35.9, 30.3 and 36.1 with; passes of 4M to 10M entries are
+// slower at any length (a segment and its warm-up outlast them).
 constexpr uint64_t kSegEntries = 160000000;
 constexpr uint32_t kSegLen = 40960;
 uint32_t seg_length(uint64_t etot) { return etot < kSegEntries ? 0u : kSegLen; }

@@ -212,6 +212,7 @@ constexpr uint32_t kSegWarm = 32;       // samples of the longest warm-up
 enum { SC_CAND, SC_CHUNK, SC_SAMPLE, SC_LIST, SC_SEG, SC_SLOT, SC_N };
 struct SegArgs {
   uint32_t seglen, candcap, chunkcap, samplecap, segcap;
+  uint32_t split, longest;  // samples from which a walk goes by channel / is not made
   uint32_t *flag, *cnt;
   SegCand *cand;      // [candcap]
   uint32_t *chunk;    // [chunkcap * 2]

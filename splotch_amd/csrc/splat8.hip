@@ -950,7 +950,6 @@ __global__ __launch_bounds__(256) void k_seg_sample(SplatArgs a, SegArgs g) {
 // sum; the rest is for the bits to meet, and for the samples' error.)
 constexpr float kSegDepth = 24.f;
 constexpr uint32_t kSegCuts = 2048;  // per list at most
-constexpr uint32_t kSegSplit = 3, kSegLongest = 5;  // in seglen: see k_seg_cut
 
 // A wave per chunk of samples, lane = pixel: per sample the shortest window of
 // samples up to it that holds kSegDepth in every pixel (0: none of kSegWarm).
@@ -1021,12 +1020,12 @@ __global__ __launch_bounds__(64) void k_seg_cut(SplatArgs a, SegArgs g) {
     }
   }
   longest = max(longest, ns - cut + extra);
-  if (n == 0 || longest > kSegLongest * smin) return;
+  if (n == 0 || longest > g.longest) return;
   if (lane == 0) {
     uint32_t m = 0, slots = 0, e = 0, x = 0;  // walks (three per long segment), kept states
     for (uint32_t k = 0; k <= n; ++k) {
       const uint32_t hi = k < n ? s_cut[k] : ns;
-      m += hi - e + x > kSegSplit * smin ? 3u : 1u;
+      m += hi - e + x > g.split ? 3u : 1u;
       slots += 1u + ((k < n ? hi * kSegSample : len) - e * kSegSample + kSegCheck - 1u) / kSegCheck;
       e = hi;
       x = k < n ? s_warm[k] : 0u;
@@ -1039,7 +1038,7 @@ __global__ __launch_bounds__(64) void k_seg_cut(SplatArgs a, SegArgs g) {
     for (uint32_t k = 0; k <= n; ++k) {
       const uint32_t hi = k < n ? s_cut[k] : ns;
       Seg S{li, b0 + e * kSegSample, k < n ? b0 + hi * kSegSample : b0 + len, x * kSegSample, slot, 3u};
-      if (hi - e + x > kSegSplit * smin)
+      if (hi - e + x > g.split)
         for (uint32_t c = 0; c < 3u; ++c) {
           S.chan = c;
           g.segs[first++] = S;
@@ -2168,6 +2167,11 @@ void launch_items_emit(const uint32_t *bin_off, uint32_t nunits, const SplatArgs
 // it is its list's last, and the lists have etot entries or fewer.
 void seg_caps(uint64_t etot, uint32_t seglen, SegArgs &g) {
   g.seglen = seglen;
+  // a pass takes about 0.07 ns per entry, one wave's walk 200 ns (by channel half
+  // of that): longer walks would outlast it (64 views, 160M and 169M entries: 33.9
+  // and 34.6 ms; 42.9 and 42.0 with 123k and 205k entries whatever the pass)
+  g.split = static_cast<uint32_t>(etot / 2700u / kSegSample);
+  g.longest = static_cast<uint32_t>(etot / 1500u / kSegSample);
   g.candcap = static_cast<uint32_t>(etot / (2u * seglen)) + 1u;
   g.samplecap = static_cast<uint32_t>(etot / kSegSample) + 1u;
   g.chunkcap = g.samplecap / kSegChunk + g.candcap;
