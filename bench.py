@@ -18,15 +18,16 @@ The JSON line also carries:
                 records around it on its own stream (average of the profiled
                 frames); traffic from rocprofv3 FETCH_SIZE + WRITE_SIZE (KiB
                 per dispatch, scaled by a known-size copy kernel's counts);
-  valu          the limit the splat actually meets: VALU instructions of the
-                ordered splat per frame (rocprofv3 SQ_INSTS_VALU, committed
+  valu          VALU instructions of the ordered splat per frame (rocprofv3
+                SQ_INSTS_VALU, committed summary) over the ordered splat
+                stage's live duration, against the issue peak of the simplest
+                operations (256 CUs x 4 SIMDs x one wave64 instruction per 2
+                clocks at 2.4 GHz; others take 4);
+  lds           the limit the splat meets: the LDS read peak measured by a
+                microbenchmark on this GPU (libmembench), and the splats' busy
+                LDS cycles per frame (rocprofv3 LDS counters, committed
                 summary) over the ordered splat stage's live duration, against
-                the issue peak (256 CUs x 4 SIMDs x one wave64 instruction per
-                4 clocks at 2.4 GHz);
-  lds           the LDS read peak measured by a microbenchmark on this GPU
-                (libmembench), and the splat kernels' LDS bytes per dispatch
-                (rocprofv3 LDS counters, scaled by the microbenchmark's own
-                counts; committed summary) over their event durations;
+                the microbenchmark's busy cycles;
   parity        per workload, the max per-channel relative error of the GPU
                 image (denominator max(|ref|, 1e-6 max|ref|)) against the
                 oracle (stable depth order), the genuine reference renderer
@@ -74,7 +75,7 @@ if int(os.environ.get("GPU_MAX_HW_QUEUES") or 4) < 8:
 
 METRIC = "ms/frame & Mparticles/s (16M, 2048²); batched and fwd+bwd vs plain"
 HBM_PEAK_GBS = 8000.0
-VALU_PEAK = 256 * 4 * 2.4e9 / 4  # wave64 VALU instructions per second (one per SIMD per 4 clocks)
+VALU_PEAK = 256 * 4 * 2.4e9 / 2  # wave64 VALU instructions per second (one per SIMD per 2 clocks)
 LDS_SPEC_GBS = 256 * 128 * 2.4e9 / 1e9  # 128 B per clock per CU (32 banks x 4 B)
 
 
@@ -780,8 +781,7 @@ def main():
                           "valu_instructions_per_frame ordered_splat") if default else None
     if ninst is not None:
         rate = ninst / (stages["ordered_splat"] * 1e-3)
-        valu = {"kernels": "k_splat8<ordered> + k_splat_pc<ordered> + k_stage_ops<ordered> + "
-                           "k_stage_chain<ordered> (concurrent)",
+        valu = {"kernels": "k_splat8<ordered> + k_seg_sample + k_seg_walk + k_seg_join",
                 "instructions": int(ninst), "stage_ms": stages["ordered_splat"],
                 "achieved": round(rate / 1e9, 2), "peak": VALU_PEAK / 1e9,
                 "unit": "G wave64 instr/s", "frac": round(rate / VALU_PEAK, 4),
@@ -818,24 +818,21 @@ def main():
                      "frac": round(achieved / HBM_PEAK_GBS, 6), "traffic": traffic,
                      "traffic_source": traffic_src,
                      "bytes_per_launch": splat_bytes, "launch_ms": splat_ms,
-                     "note": "the splat is VALU-issue-bound (see valu); HBM is not its "
-                             "limit"},
+                     "note": "the splat is LDS-bound (see lds); HBM is not its limit"},
         "valu": valu,
     }
-    # LDS: measured peak; the splat kernels' LDS bytes from the committed profile
+    # LDS: measured peak; the splats' busy LDS cycles from the committed profile
     lp = lds_peak()
     lds = {"peak_measured_GBs": lp["GBs"], "peak_spec_GBs": LDS_SPEC_GBS,
            "microbenchmark": lp}
-    for kname, stage in (("k_splat8<0, 4>", "ordered_k_splat8"),
-                         ("k_splat_pc<0>", "ordered_k_splat_heavy")):
-        b = profile_value("pmc_lds_gas_stars_16M_2048.md",
-                          "lds_bytes_per_dispatch " + kname) if default else None
-        if b is not None and stages.get(stage):
-            gbs = b / (stages[stage] * 1e-3) / 1e9
-            lds[kname] = {"bytes_per_dispatch": int(b), "ms": stages[stage],
-                          "achieved_GBs": round(gbs, 1),
-                          "frac_of_measured_peak": round(gbs / lp["GBs"], 4),
-                          "source": "profiles/pmc_lds_gas_stars_16M_2048.md"}
+    busy = profile_value("pmc_lds_gas_stars_16M_2048.md",
+                         "lds_active_cycles_per_frame splats") if default else None
+    per_ms = profile_value("pmc_lds_gas_stars_16M_2048.md",
+                           "lds_active_cycles_per_ms peak_stream") if default else None
+    if busy is not None and per_ms is not None:
+        lds["splats"] = {"active_cycles_per_frame": int(busy), "stage_ms": stages["ordered_splat"],
+                         "frac_of_peak_stream": round(busy / stages["ordered_splat"] / per_ms, 4),
+                         "source": "profiles/pmc_lds_gas_stars_16M_2048.md"}
     out["lds"] = lds
     fo = profile_value("fragments_gas_stars_16M_2048.md", "fragments_ordered") if default else None
     fa = profile_value("fragments_gas_stars_16M_2048.md", "fragments_additive") if default else None
