@@ -711,6 +711,16 @@ __global__ __launch_bounds__(256) void k_fill_u32(uint32_t *p, uint32_t v, int64
   for (int64_t i = gtid(); i < n; i += gstride()) p[i] = v;
 }
 
+// One workgroup: n <= 256 words to host memory, then flag = seq.
+__global__ __launch_bounds__(256) void k_publish(const uint32_t *src, uint32_t n, uint32_t *dst,
+                                                 uint32_t *flag, uint32_t seq) {
+  if (threadIdx.x < n) dst[threadIdx.x] = src[threadIdx.x];
+  __threadfence_system();
+  __syncthreads();
+  if (threadIdx.x == 0)
+    __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // Per-job pass flags from the pass offsets mo0 / mo1 (null: pass absent):
 // the ordered pass writes the image of a job that has ordered particles; the
 // additive pass adds to it there and writes the image elsewhere.
@@ -1074,6 +1084,12 @@ void launch_add_images(float *pic, const float *add, int64_t n, hipStream_t s) {
 void launch_delay(uint32_t us, hipStream_t s, const uint32_t *n) {
   k_delay<<<1, 64, 0, s>>>(us * 100u, n);
   hip_check(hipGetLastError(), "k_delay launch");
+}
+
+void launch_publish(const uint32_t *src, uint32_t n, uint32_t *dst, uint32_t *flag, uint32_t seq,
+                    hipStream_t s) {
+  k_publish<<<1, 256, 0, s>>>(src, n, dst, flag, seq);
+  hip_check(hipGetLastError(), "k_publish launch");
 }
 
 void launch_fill_u32(uint32_t *p, uint32_t v, int64_t n, hipStream_t s) {

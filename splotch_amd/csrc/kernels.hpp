@@ -137,6 +137,9 @@ void launch_cap_check(uint32_t *m, uint32_t *e, const uint64_t *e64, uint32_t *e
                       hipStream_t s);
 // pic[i] += add[i]
 void launch_add_images(float *pic, const float *add, int64_t n, hipStream_t s);
+// n <= 256 words from src to dst in host memory, then *flag = seq there.
+void launch_publish(const uint32_t *src, uint32_t n, uint32_t *dst, uint32_t *flag, uint32_t seq,
+                    hipStream_t s);
 // A one-wave kernel that returns after `us` microseconds (bounded wait); at once
 // where a device count n is given and is 0.
 void launch_delay(uint32_t us, hipStream_t s, const uint32_t *n = nullptr);
