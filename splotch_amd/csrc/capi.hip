@@ -722,19 +722,23 @@ void stage_project_compact(splhip_ctx *c, Plan &pl, Rec *rec, uint8_t *act, uint
                            hipStream_t s) {
   Workspace &ws = *pl.ws;
   mark(c, 0, true, s);
-  launch_project(pl.d_pa, pl.d_blk, pl.nj, pl.nblocks, rec, act, s);
+  launch_project(pl.d_pa, pl.d_blk, pl.nj, pl.nblocks, rec, act, tot, T_N, s);
   mark(c, 0, false, s);
-  launch_fill_u32(tot, 0, T_N, s);
-  uint32_t *mo[2] = {nullptr, nullptr};
+  PassOffsets po{};
+  auto &mo = po.mo;
   for (int p = 0; p < 2; ++p) {
     if (!pl.present[p] || pl.ntot == 0) continue;
     mark(c, p == 0 ? 1 : 4, true, s);
     uint32_t *pos = ws.get_as<uint32_t>(pslot(p, P_POS), static_cast<size_t>(pl.ntot));
     scan_u8bit(act, static_cast<uint8_t>(p + 1), pos, pl.ntot, tot + T_M + p, ws, s);
     mo[p] = ws.get_as<uint32_t>(pslot(p, P_MO), pl.nj + 1);
-    launch_pass_offsets(pos, pl.d_pbase, pl.nj, pl.ntot, tot + T_M + p, mo[p], s);
+    po.pos[p] = pos;
+    po.total[p] = tot + T_M + p;
     mark(c, p == 0 ? 1 : 4, false, s);
   }
+  // with the pass sizes on the device, the jobs' flags too
+  JobSplat *js = pl.dc || pl.late ? pl.d_js : nullptr;
+  if (js || mo[0] || mo[1]) launch_pass_offsets(po, pl.d_pbase, pl.nj, pl.ntot, js, s);
   if (pl.dc || pl.late) {  // the pass sizes stay on the device; capacities: every particle
     for (int p = 0; p < 2; ++p) {
       pl.m[p] = mo[p] ? static_cast<uint32_t>(pl.ntot) : 0u;
@@ -1495,8 +1499,7 @@ int render_jobs(splhip_ctx *c, int nj, const JobIn *jobs, hipStream_t s, bool ke
   pl.late = pl.ntot > 0 && pl.ntot <= kLateParticles;
   pl.tot = tot;
   stage_project_compact(c, pl, rec, act, tot, s);
-  if (pl.late) launch_job_flags(pl.d_mo[0], pl.d_mo[1], nj, pl.d_js, s);
-  else set_job_flags(c, pl, s);
+  if (!pl.late) set_job_flags(c, pl, s);
   for (int p = 0; p < 2; ++p)
     if (pl.m[p]) {
       stage_order(c, pl, p, rec, act, s);
@@ -1895,7 +1898,6 @@ int render_jobs_dc(splhip_ctx *c, int nj, const JobIn *jobs, hipStream_t s) {
     pl.e16[p] = rv.e16cap[p];
   }
   stage_project_compact(c, pl, rec, act, tot, s);
-  launch_job_flags(pl.d_mo[0], pl.d_mo[1], nj, pl.d_js, s);
   for (int p = 0; p < 2; ++p) {
     pl.nstage[p] = rv.ns_cap[p];
     pl.sgroups[p] = rv.groups_cap[p];
@@ -2907,7 +2909,7 @@ int splhip_project(splhip_ctx *c, const splhip_particles *P, const splhip_camera
     Plan pl;
     make_plan(c, 1, &job, 0, pl, s);
     launch_project(pl.d_pa, pl.d_blk, 1, pl.nblocks, reinterpret_cast<Rec *>(rec_out), active_out,
-                   s);
+                   nullptr, 0u, s);
   } catch (const HipError &e) {
     return hip_fail(c, e);
   }

@@ -51,7 +51,10 @@ unsigned grid_for(int64_t n, int per_block = 256, int64_t cap = 1 << 20) {
 __global__ __launch_bounds__(256) void k_project(const ProjectArgs *__restrict__ jobs,
                                                  const uint32_t *__restrict__ blk, int nj,
                                                  Rec *__restrict__ rec,
-                                                 uint8_t *__restrict__ act) {
+                                                 uint8_t *__restrict__ act,
+                                                 uint32_t *__restrict__ tot, uint32_t ntot) {
+  if (blockIdx.x == 0)  // the frame's totals, counted by the kernels after this one
+    for (uint32_t k = threadIdx.x; k < ntot; k += 256) tot[k] = 0u;
   const int j = __builtin_amdgcn_readfirstlane(find_job(blk, nj, blockIdx.x));
   const ProjectArgs &a = jobs[j];
   const int64_t i0 = static_cast<int64_t>(blockIdx.x - blk[j]) * kPerBlock;
@@ -170,11 +173,28 @@ __global__ __launch_bounds__(256) void k_compact(const ProjectArgs *__restrict__
   }
 }
 
-__global__ __launch_bounds__(256) void k_pass_offsets(const uint32_t *pos, const uint32_t *pbase,
-                                                      int nj, int64_t n, const uint32_t *total,
-                                                      uint32_t *mo) {
-  for (int64_t j = gtid(); j <= nj; j += gstride())
-    mo[j] = (j < nj && pbase[j] < n) ? pos[pbase[j]] : *total;
+// mo[j]: the particles of jobs before j in the pass (j <= nj), for both passes
+// (mo null: pass absent); then, with js, the jobs' pass flags: the ordered pass
+// writes the image of a job that has ordered particles; the additive pass adds
+// to it there and writes the image elsewhere.
+__global__ __launch_bounds__(256) void k_pass_offsets(PassOffsets a, const uint32_t *pbase, int nj,
+                                                      int64_t n, JobSplat *js) {
+  auto at = [&](int p, int64_t j) {
+    return (j < nj && pbase[j] < n) ? a.pos[p][pbase[j]] : *a.total[p];
+  };
+  for (int64_t j = gtid(); j <= nj; j += gstride()) {
+    uint32_t o[2] = {0u, 0u};
+    for (int p = 0; p < 2; ++p)
+      if (a.mo[p]) a.mo[p][j] = o[p] = at(p, j);
+    if (!js || j == nj) continue;
+    const bool w0 = a.mo[0] && at(0, j + 1) > o[0];
+    const bool w1 = a.mo[1] && at(1, j + 1) > o[1];
+    JobSplat &J = js[j];
+    J.accumulate[0] = 0;
+    J.accumulate[1] = w0 ? 1 : 0;
+    J.need_empty[0] = w0 ? 1 : 0;
+    J.need_empty[1] = (w1 && !w0) ? 1 : 0;
+  }
 }
 
 // The count of a launch sized for `cap` items: cap, or the device count *dn
@@ -721,22 +741,6 @@ __global__ __launch_bounds__(256) void k_publish(const uint32_t *src, uint32_t n
     __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// Per-job pass flags from the pass offsets mo0 / mo1 (null: pass absent):
-// the ordered pass writes the image of a job that has ordered particles; the
-// additive pass adds to it there and writes the image elsewhere.
-__global__ __launch_bounds__(64) void k_job_flags(const uint32_t *mo0, const uint32_t *mo1,
-                                                  int nj, JobSplat *js) {
-  for (int64_t j = gtid(); j < nj; j += gstride()) {
-    const bool w0 = mo0 && mo0[j + 1] > mo0[j];
-    const bool w1 = mo1 && mo1[j + 1] > mo1[j];
-    JobSplat &J = js[j];
-    J.accumulate[0] = 0;
-    J.accumulate[1] = w0 ? 1 : 0;
-    J.need_empty[0] = w0 ? 1 : 0;
-    J.need_empty[1] = (w1 && !w0) ? 1 : 0;
-  }
-}
-
 // Zeros into the image of every job with no particle in either pass
 // (grid.y = job).
 __global__ __launch_bounds__(256) void k_fill_empty_jobs(const uint32_t *mo0, const uint32_t *mo1,
@@ -954,9 +958,12 @@ __global__ __launch_bounds__(256) void k_splat(SplatArgs a) {
 }  // namespace
 
 void launch_project(const ProjectArgs *jobs, const uint32_t *blk, int nj, uint32_t nblocks,
-                    Rec *rec, uint8_t *act, hipStream_t s) {
-  if (nblocks == 0) return;
-  k_project<<<nblocks, 256, 0, s>>>(jobs, blk, nj, rec, act);
+                    Rec *rec, uint8_t *act, uint32_t *tot, uint32_t ntot, hipStream_t s) {
+  if (nblocks == 0) {
+    if (ntot) launch_fill_u32(tot, 0u, ntot, s);
+    return;
+  }
+  k_project<<<nblocks, 256, 0, s>>>(jobs, blk, nj, rec, act, tot, ntot);
   hip_check(hipGetLastError(), "k_project launch");
 }
 
@@ -968,9 +975,9 @@ void launch_compact(const ProjectArgs *jobs, const uint32_t *blk, int nj, uint32
   hip_check(hipGetLastError(), "k_compact launch");
 }
 
-void launch_pass_offsets(const uint32_t *pos, const uint32_t *pbase, int nj, int64_t n,
-                         const uint32_t *total, uint32_t *mo, hipStream_t s) {
-  k_pass_offsets<<<grid_for(nj + 1), 256, 0, s>>>(pos, pbase, nj, n, total, mo);
+void launch_pass_offsets(const PassOffsets &a, const uint32_t *pbase, int nj, int64_t n,
+                         JobSplat *js, hipStream_t s) {
+  k_pass_offsets<<<grid_for(nj + 1), 256, 0, s>>>(a, pbase, nj, n, js);
   hip_check(hipGetLastError(), "k_pass_offsets launch");
 }
 
@@ -1095,12 +1102,6 @@ void launch_publish(const uint32_t *src, uint32_t n, uint32_t *dst, uint32_t *fl
 void launch_fill_u32(uint32_t *p, uint32_t v, int64_t n, hipStream_t s) {
   k_fill_u32<<<grid_for(n), 256, 0, s>>>(p, v, n);
   hip_check(hipGetLastError(), "k_fill_u32 launch");
-}
-
-void launch_job_flags(const uint32_t *mo0, const uint32_t *mo1, int nj, JobSplat *js,
-                      hipStream_t s) {
-  k_job_flags<<<(nj + 63) / 64, 64, 0, s>>>(mo0, mo1, nj, js);
-  hip_check(hipGetLastError(), "k_job_flags launch");
 }
 
 void launch_fill_empty_jobs(const uint32_t *mo0, const uint32_t *mo1, int nj, const JobSplat *js,

@@ -61,8 +61,9 @@ struct SplatArgs {
   const uint32_t *seg;  // (optional) per unit: nonzero = walked in segments, no items
 };
 
+// tot: ntot words set to 0 beside.
 void launch_project(const ProjectArgs *jobs, const uint32_t *blk, int nj, uint32_t nblocks,
-                    Rec *rec, uint8_t *act, hipStream_t s);
+                    Rec *rec, uint8_t *act, uint32_t *tot, uint32_t ntot, hipStream_t s);
 // Compaction of one pass (act & code) into pass order; keys (optional): the
 // depth-sort key of each job's sort_type.
 void launch_compact(const ProjectArgs *jobs, const uint32_t *blk, int nj, uint32_t nblocks,
@@ -73,9 +74,14 @@ void launch_compact(const ProjectArgs *jobs, const uint32_t *blk, int nj, uint32
 // count from that device word (at most the capacity), so that no host wait
 // is needed between the stage that counts and the stage that consumes.
 //
-// mo[j] = pos[pbase[j]] (pass particles before job j), mo[nj] = *total.
-void launch_pass_offsets(const uint32_t *pos, const uint32_t *pbase, int nj, int64_t n,
-                         const uint32_t *total, uint32_t *mo, hipStream_t s);
+// Per pass mo[j] = pos[pbase[j]] (pass particles before job j), mo[nj] = *total;
+// with js also the jobs' pass flags from them.
+struct PassOffsets {
+  const uint32_t *pos[2], *total[2];
+  uint32_t *mo[2];  // null: pass absent
+};
+void launch_pass_offsets(const PassOffsets &a, const uint32_t *pbase, int nj, int64_t n,
+                         JobSplat *js, hipStream_t s);
 // keys[i] = job of global particle index vals[i].
 void launch_job_of_index(const uint32_t *vals, uint32_t m, const uint32_t *pbase, int nj,
                          uint32_t *keys, hipStream_t s, const uint32_t *dm = nullptr);
@@ -124,12 +130,9 @@ void launch_map(const uint32_t *idx, const uint32_t *table, uint32_t *out, int64
                 hipStream_t s);
 void launch_fill(float *p, float v, int64_t n, hipStream_t s);
 void launch_fill_u32(uint32_t *p, uint32_t v, int64_t n, hipStream_t s);
-// Device-count pipeline helpers: per-job pass flags from the pass offsets
-// (null: pass absent), zeros into the images of jobs with no particle in
-// either pass, and the capacity check of a pass (counts zeroed, bit set in
+// Device-count pipeline helpers: zeros into the images of jobs with no particle
+// in either pass (mo null: pass absent), and the capacity check of a pass (counts zeroed, bit set in
 // *ovf when e64 > ecap or *e16 > e16cap).
-void launch_job_flags(const uint32_t *mo0, const uint32_t *mo1, int nj, JobSplat *js,
-                      hipStream_t s);
 void launch_fill_empty_jobs(const uint32_t *mo0, const uint32_t *mo1, int nj, const JobSplat *js,
                             hipStream_t s);
 void launch_cap_check(uint32_t *m, uint32_t *e, const uint64_t *e64, uint32_t *e16,
