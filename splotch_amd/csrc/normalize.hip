@@ -15,6 +15,7 @@
 #include "kernels.hpp"
 
 #include <algorithm>
+#include <type_traits>
 
 #include "workspace.hpp"
 
@@ -94,7 +95,6 @@ __device__ __forceinline__ void store_w(float *p, int64_t m, int64_t n, const fl
     if (m + j < n) p[m + j] = v[j];
 }
 
-constexpr int kNormThreads = 512;
 // Loads per thread, field and step (all issued before the first is used): two
 // vectors of four particles, or four single particles.
 template <int W> constexpr int loads() { return W == 4 ? 2 : 4; }
@@ -102,13 +102,12 @@ template <int W> constexpr int loads() { return W == 4 ? 2 : 4; }
 // Pass 1: transforms in place and reduces the extremes of NT types.  Both
 // passes are bound by HBM (13 B, then 17 B per particle); a thread takes four
 // consecutive particles per 16-byte load.  16M particles of two types: 122 ->
-// 97 us without logs (4.9 TB/s), 198 -> 187 with, 253 -> 168 with a vector
-// colour, against a float per load
-// and four loads in flight per thread and field.
-// GEN: some type has a log10, an asinh or a vector colour (else that code, and
-// its registers, are left out).
-template <int NT, int W, bool GEN>
-__global__ __launch_bounds__(kNormThreads) void k_norm_reduce(NormArgs a, uint32_t *keys) {
+// 97 us without logs (4.9 TB/s), against a float per load and four loads in flight
+// per thread and field.
+// GEN: some type has a log10, an asinh or a vector colour, VEC: some type has a
+// vector colour (else that code, and its registers, are left out).
+template <int NT, int W, bool GEN, bool VEC, int kT>
+__global__ __launch_bounds__(kT) void k_norm_reduce(NormArgs a, uint32_t *keys) {
   __shared__ int32_t s_flags[NT][4];
   if (threadIdx.x < NT * 4) s_flags[threadIdx.x / 4][threadIdx.x % 4] =
       a.flags[threadIdx.x / 4][threadIdx.x % 4];
@@ -119,18 +118,18 @@ __global__ __launch_bounds__(kNormThreads) void k_norm_reduce(NormArgs a, uint32
 #pragma unroll
     for (int q = 0; q < K_N; ++q) k[t][q] = (q % 2 == 0) ? 0xffffffffu : 0u;
   constexpr int kV = loads<W>();
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * kNormThreads * W;
-  for (int64_t m0 = (static_cast<int64_t>(blockIdx.x) * kNormThreads + threadIdx.x) * W; m0 < a.n;
+  const int64_t stride = static_cast<int64_t>(gridDim.x) * kT * W;
+  for (int64_t m0 = (static_cast<int64_t>(blockIdx.x) * kT + threadIdx.x) * W; m0 < a.n;
        m0 += kV * stride) {
     uint8_t tv[kV][W] = {};
-    float Iv[kV][W], ev[kV][W], rv[kV][W], gv[GEN ? kV : 1][W], bv[GEN ? kV : 1][W];
+    float Iv[kV][W], ev[kV][W], rv[kV][W], gv[VEC ? kV : 1][W], bv[VEC ? kV : 1][W];
 #pragma unroll
     for (int q = 0; q < kV; ++q) {
       const int64_t m = m0 + q * stride;
       if (m < a.n) {
-        if (GEN && a.vector) {
-          load_w<W, float, float4>(a.eg, m, a.n, gv[GEN ? q : 0]);
-          load_w<W, float, float4>(a.eb, m, a.n, bv[GEN ? q : 0]);
+        if (VEC) {
+          load_w<W, float, float4>(a.eg, m, a.n, gv[VEC ? q : 0]);
+          load_w<W, float, float4>(a.eb, m, a.n, bv[VEC ? q : 0]);
         }
         if (a.type) load_w<W, uint8_t, uchar4>(a.type, m, a.n, tv[q]);
         load_w<W, float, float4>(a.I, m, a.n, Iv[q]);
@@ -148,7 +147,7 @@ __global__ __launch_bounds__(kNormThreads) void k_norm_reduce(NormArgs a, uint32
         const int t = m < a.n ? tv[q][j] : NT;
         if (t >= NT) continue;  // past the end, or a type beyond ptypes (not rendered)
         const int f_il = GEN ? s_flags[t][0] : 0, f_cl = GEN ? s_flags[t][1] : 0,
-                  f_ca = GEN ? s_flags[t][2] : 0, f_cv = GEN ? s_flags[t][3] : 0;
+                  f_ca = GEN ? s_flags[t][2] : 0, f_cv = VEC ? s_flags[t][3] : 0;
         // extremes of this particle (min keys start high, max keys low)
         uint32_t cmin = 0xffffffffu, cmax = 0u, imin = 0xffffffffu, imax = 0u;
         const float r = rv[q][j];
@@ -192,7 +191,7 @@ __global__ __launch_bounds__(kNormThreads) void k_norm_reduce(NormArgs a, uint32
         }
         if (ccol && e == e) cmin = cmax = fkey(e);
         if (f_cv) {
-          float &g = gv[GEN ? q : 0][j], &b = bv[GEN ? q : 0][j];
+          float &g = gv[VEC ? q : 0][j], &b = bv[VEC ? q : 0][j];
           if (f_cl) {
             g = log10_f(g);
             b = log10_f(b);
@@ -224,14 +223,14 @@ __global__ __launch_bounds__(kNormThreads) void k_norm_reduce(NormArgs a, uint32
       if (put_I) store_w<W>(a.I, mq, a.n, Iv[q]);
       if (put_e) store_w<W>(a.er, mq, a.n, ev[q]);
       if (put_v) {
-        store_w<W>(a.eg, mq, a.n, gv[GEN ? q : 0]);
-        store_w<W>(a.eb, mq, a.n, bv[GEN ? q : 0]);
+        store_w<W>(a.eg, mq, a.n, gv[VEC ? q : 0]);
+        store_w<W>(a.eb, mq, a.n, bv[VEC ? q : 0]);
       }
     }
   }
   // per wave by shuffles, per block through LDS, then one atomic per block
   // and value (thousands of atomics on a few addresses would serialize)
-  __shared__ uint32_t s_k[kNormThreads / 64][NT * K_N];
+  __shared__ uint32_t s_k[kT / 64][NT * K_N];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
   for (int t = 0; t < NT; ++t)
@@ -245,7 +244,7 @@ __global__ __launch_bounds__(kNormThreads) void k_norm_reduce(NormArgs a, uint32
   if (i < NT * K_N) {
     const bool is_min = (i % K_N) % 2 == 0;
     uint32_t v = s_k[0][i];
-    for (int w = 1; w < kNormThreads / 64; ++w) v = is_min ? min(v, s_k[w][i]) : max(v, s_k[w][i]);
+    for (int w = 1; w < kT / 64; ++w) v = is_min ? min(v, s_k[w][i]) : max(v, s_k[w][i]);
     if (is_min) {
       if (v != 0xffffffffu) atomicMin(&keys[i], v);
     } else {
@@ -270,8 +269,8 @@ struct Range {
 
 // Pass 2: normAndClamp of intensity (unless NO_I_NORM) and colour; the
 // block first stages every type's two ranges and vector flag in LDS.
-template <int W, bool GEN>
-__global__ __launch_bounds__(kNormThreads) void k_norm_clamp(NormArgs a, const uint32_t *keys) {
+template <int W, bool GEN, bool VEC, int kT>
+__global__ __launch_bounds__(kT) void k_norm_clamp(NormArgs a, const uint32_t *keys) {
   __shared__ Range s_int[kMaxTypes], s_col[kMaxTypes];
   __shared__ int32_t s_vec[kMaxTypes];
   const int i = threadIdx.x;
@@ -287,18 +286,18 @@ __global__ __launch_bounds__(kNormThreads) void k_norm_clamp(NormArgs a, const u
   }
   __syncthreads();
   constexpr int kV = loads<W>();
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * kNormThreads * W;
-  for (int64_t m0 = (static_cast<int64_t>(blockIdx.x) * kNormThreads + threadIdx.x) * W; m0 < a.n;
+  const int64_t stride = static_cast<int64_t>(gridDim.x) * kT * W;
+  for (int64_t m0 = (static_cast<int64_t>(blockIdx.x) * kT + threadIdx.x) * W; m0 < a.n;
        m0 += kV * stride) {
     uint8_t tv[kV][W] = {};
-    float Iv[kV][W], ev[kV][W], gv[GEN ? kV : 1][W], bv[GEN ? kV : 1][W];
+    float Iv[kV][W], ev[kV][W], gv[VEC ? kV : 1][W], bv[VEC ? kV : 1][W];
 #pragma unroll
     for (int q = 0; q < kV; ++q) {  // loads first
       const int64_t m = m0 + q * stride;
       if (m < a.n) {
-        if (GEN && a.vector) {
-          load_w<W, float, float4>(a.eg, m, a.n, gv[GEN ? q : 0]);
-          load_w<W, float, float4>(a.eb, m, a.n, bv[GEN ? q : 0]);
+        if (VEC) {
+          load_w<W, float, float4>(a.eg, m, a.n, gv[VEC ? q : 0]);
+          load_w<W, float, float4>(a.eb, m, a.n, bv[VEC ? q : 0]);
         }
         if (a.type) load_w<W, uint8_t, uchar4>(a.type, m, a.n, tv[q]);
         load_w<W, float, float4>(a.I, m, a.n, Iv[q]);
@@ -318,10 +317,10 @@ __global__ __launch_bounds__(kNormThreads) void k_norm_clamp(NormArgs a, const u
         if (a.norm_int) s_int[t].clamp(Iv[q][j]);
         const Range C = s_col[t];
         C.clamp(ev[q][j]);
-        if (GEN && s_vec[t]) {
+        if (VEC && s_vec[t]) {
           put_v = true;
-          C.clamp(gv[GEN ? q : 0][j]);
-          C.clamp(bv[GEN ? q : 0][j]);
+          C.clamp(gv[VEC ? q : 0][j]);
+          C.clamp(bv[VEC ? q : 0][j]);
         }
       }
       if (put) {
@@ -329,26 +328,26 @@ __global__ __launch_bounds__(kNormThreads) void k_norm_clamp(NormArgs a, const u
         store_w<W>(a.er, mq, a.n, ev[q]);
       }
       if (put_v) {
-        store_w<W>(a.eg, mq, a.n, gv[GEN ? q : 0]);
-        store_w<W>(a.eb, mq, a.n, bv[GEN ? q : 0]);
+        store_w<W>(a.eg, mq, a.n, gv[VEC ? q : 0]);
+        store_w<W>(a.eb, mq, a.n, bv[VEC ? q : 0]);
       }
     }
   }
 }
 
-template <int W, bool GEN>
+template <int W, bool GEN, bool VEC, int kT>
 void launch_passes(const NormArgs &a, uint32_t *keys, hipStream_t s) {
   const unsigned grid = static_cast<unsigned>(
-      std::min<int64_t>((a.n + W * kNormThreads - 1) / (W * kNormThreads), 1024));
+      std::min<int64_t>((a.n + W * kT - 1) / (W * kT), 1024));
 #define SPLHIP_NORM(N) \
-  case N: k_norm_reduce<N, W, GEN><<<grid, kNormThreads, 0, s>>>(a, keys); break;
+  case N: k_norm_reduce<N, W, GEN, VEC, kT><<<grid, kT, 0, s>>>(a, keys); break;
   switch (a.ntypes) {
     SPLHIP_NORM(1) SPLHIP_NORM(2) SPLHIP_NORM(3) SPLHIP_NORM(4)
     SPLHIP_NORM(5) SPLHIP_NORM(6) SPLHIP_NORM(7) SPLHIP_NORM(8)
   }
 #undef SPLHIP_NORM
   hip_check(hipGetLastError(), "k_norm_reduce launch");
-  k_norm_clamp<W, GEN><<<grid, kNormThreads, 0, s>>>(a, keys);
+  k_norm_clamp<W, GEN, VEC, kT><<<grid, kT, 0, s>>>(a, keys);
   hip_check(hipGetLastError(), "k_norm_clamp launch");
 }
 
@@ -371,10 +370,23 @@ void launch_normalize(const NormArgs &a, uint32_t *keys, hipStream_t s) {
   // one, 16.3 with four, whose logarithms a thread takes in turn)
   const bool vec = a.n >= (1 << 19) && at(a.I, 16) && at(a.er, 16) && at(a.r, 16) &&
                    at(a.type, 4) && (!b.vector || (at(a.eg, 16) && at(a.eb, 16)));
-  if (vec && gen) launch_passes<4, true>(b, keys, s);
-  else if (vec) launch_passes<4, false>(b, keys, s);
-  else if (gen) launch_passes<1, true>(b, keys, s);
-  else launch_passes<1, false>(b, keys, s);
+  // Logs and vector colours hold the passes at 3 waves per SIMD, where workgroups
+  // of 512 threads fit a CU once, two waves per SIMD, and those of 256 three times
+  // (16M particles, logs, fields not aligned: 204 us with 512, 144 with 256; 4M
+  // aligned, four types in random order: 118 and 85); small fields have a workgroup
+  // per CU at most, and fewer of them end in fewer atomics (600k, two types: 30 us
+  // with 512, 37 with 256).
+  auto go = [&](auto w) {
+    constexpr int W = decltype(w)::value;
+    const bool small = a.n < (b.vector ? 1 << 21 : 1 << 20);
+    if (b.vector && small) launch_passes<W, true, true, 512>(b, keys, s);
+    else if (b.vector) launch_passes<W, true, true, 256>(b, keys, s);
+    else if (gen && small) launch_passes<W, true, false, 512>(b, keys, s);
+    else if (gen) launch_passes<W, true, false, 256>(b, keys, s);
+    else launch_passes<W, false, false, 512>(b, keys, s);
+  };
+  if (vec) go(std::integral_constant<int, 4>{});
+  else go(std::integral_constant<int, 1>{});
 }
 
 }  // namespace splhip
