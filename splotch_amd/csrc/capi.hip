@@ -140,6 +140,7 @@ int fail(splhip_ctx *c, int code, const std::string &msg) {
 }
 
 int hip_fail(splhip_ctx *c, const HipError &e) {
+  (void)hipGetLastError();  // reported here, not by the next call's launches
   std::string m = std::string(e.what) + ": " + hipGetErrorString(e.code);
   return fail(c, SPLHIP_E_HIP, m);
 }
@@ -333,7 +334,10 @@ void upload_palettes(splhip_ctx *c) {
   const size_t need = static_cast<size_t>(stride) * kMaxTypes;
   if (need > c->pal_cap) {
     if (c->d_palx) hip_check(hipFree(c->d_palx), "hipFree palette");
+    c->d_palx = nullptr;
     if (c->d_palrgb) hip_check(hipFree(c->d_palrgb), "hipFree palette");
+    c->d_palrgb = nullptr;
+    c->pal_cap = 0;
     hip_check(hipMalloc(&c->d_palx, need * sizeof(double)), "hipMalloc palette");
     hip_check(hipMalloc(&c->d_palrgb, need * 3 * sizeof(float)), "hipMalloc palette");
     c->pal_cap = need;
@@ -480,6 +484,7 @@ char *staging(splhip_ctx *c, size_t bytes) {
   if (c->h_stage_cap < bytes) {
     if (c->h_stage) hip_check(hipHostFree(c->h_stage), "hipHostFree");
     c->h_stage = nullptr;
+    c->h_stage_cap = 0;
     hip_check(hipHostMalloc(reinterpret_cast<void **>(&c->h_stage), bytes, hipHostMallocDefault),
               "hipHostMalloc");
     c->h_stage_cap = bytes;

@@ -54,7 +54,9 @@ class Workspace {
       if (ptr_[slot]) {
         hip_check(hipDeviceSynchronize(), "sync before workspace growth");
         hip_check(hipFree(ptr_[slot]), "hipFree");
+        // nothing is held from here on, also if the allocation below fails
         ptr_[slot] = nullptr;
+        cap_[slot] = 0;
       }
       size_t c = bytes + bytes / 8;  // headroom against small growth steps
       c = (c + 4095) & ~size_t(4095);
