@@ -939,7 +939,8 @@ uint32_t seg_length(uint64_t etot) { return etot < kSegEntries ? 0u : kSegLen; }
 
 // Staged operands of a pass: room for 3 KiB per group of 4 entries additive, 7
 // KiB ordered (what is written depends on the entries' coverage); of a pass
-// whose staged lists need more, fewer are staged (the longest).
+// whose staged lists need more, or more than the device memory has to spare,
+// fewer are staged (the longest).
 constexpr uint64_t kStageBudget = uint64_t(32) << 30;
 // Long lists left to the 8x8 splat that would outlast the pass, walked by
 // one wave at about 230 ns per entry against about 0.1 ns per entry of the
@@ -1007,6 +1008,17 @@ SplatArgs splat_args(splhip_ctx *c, const Plan &pl, int p, const Tuning &tn) {
   return sa;
 }
 
+// Room for ns staged lists of `groups` groups of pass p, if there is: the buffers
+// that stage_splat takes.
+bool stage_room(Workspace &ws, int p, uint32_t ns, uint64_t groups) {
+  const uint64_t bytes = 4 * stage_floats(p == 1, groups), nbat = stage_batches(groups, ns);
+  return bytes <= kStageBudget &&
+         ws.optional({{pslot(p, P_SOPS), bytes},
+                      {pslot(p, P_SMASK), nbat * 64 * 8},
+                      {pslot(p, P_SROWS), nbat * 16 * 4},
+                      {pslot(p, P_SGOFS), nbat * 16 * 4}});
+}
+
 // The segments' buffers of pass p (pl.seglen set).
 SegArgs seg_args(const Plan &pl, int p, uint32_t *tot) {
   Workspace &ws = *pl.ws;
@@ -1023,12 +1035,23 @@ SegArgs seg_args(const Plan &pl, int p, uint32_t *tot) {
   return g;
 }
 
+// Room for the segments of pass p, their kept states included, if there is (1 to 2
+// B per entry, beside some 25 of the lists).
+bool seg_room(const Plan &pl, int p) {
+  SegArgs g{};
+  seg_caps(pl.etot[p], pl.seglen[p], g);
+  const size_t slots = static_cast<size_t>(pl.etot[p] / kSegCheck) + 2u * g.segcap;
+  return pl.ws->optional({{pslot(p, P_SEGX), static_cast<size_t>(g.samplecap) * 768u},
+                          {pslot(p, P_SEGS), slots * 768u}});
+}
+
 // Work items of pass p: count per unit (heavy units counted too), scan.
 void stage_items_count(splhip_ctx *c, Plan &pl, int p, const Tuning &tn, uint32_t *tot,
                        hipStream_t s, Workspace *wt = nullptr) {
   Workspace &ws = *pl.ws;
   mark(c, p == 0 ? 2 : 5, true, s);
   pl.seglen[p] = p == 0 && tn.seg && !pl.dc && !c->sizing ? seg_length(pl.etot[p]) : 0u;
+  if (pl.seglen[p] && !seg_room(pl, p)) pl.seglen[p] = 0u;
   SplatArgs sa = splat_args(c, pl, p, tn);
   if (pl.seglen[p]) {
     const SegArgs g = seg_args(pl, p, tot);
@@ -1051,8 +1074,8 @@ void stage_items_count(splhip_ctx *c, Plan &pl, int p, const Tuning &tn, uint32_
 
 // Item counts of pass p from c->h_tot read from tot + T_ITEMS on (T_N -
 // T_ITEMS words): work items; long lists (one item each, sorted first) = the
-// staged ones (from stage_rule's level on, raised until their operands fit
-// kStageBudget), then at most heavy_max of the others from heavy_len on for
+// staged ones (from stage_rule's level on, raised until there is room for their
+// operands), then at most heavy_max of the others from heavy_len on for
 // the producer/consumer kernel; the rest go to the 8x8 splat.
 void take_items(splhip_ctx *c, Plan &pl, int p, const Tuning &tn) {
   const uint32_t *h = c->h_tot;
@@ -1069,7 +1092,7 @@ void take_items(splhip_ctx *c, Plan &pl, int p, const Tuning &tn) {
   uint64_t groups = 0;
   if (pl.m[p] && len0 != 0xffffffffu)
     for (int j = stage_rule(len0, tn.mode[p], lmax, pl.etot[p]); j >= 0 && j < kStageLevels; ++j)
-      if (4 * stage_floats(p == 1, grp[j]) <= kStageBudget) {
+      if (cnt[j] == 0u || stage_room(*pl.ws, p, cnt[j], grp[j])) {
         ns = cnt[j];
         groups = grp[j];
         break;
@@ -1914,6 +1937,15 @@ int render_jobs_dc(splhip_ctx *c, int nj, const JobIn *jobs, hipStream_t s) {
     }
   for (int p = 0; p < 2; ++p)
     if (pl.m[p]) stage_bins(c, pl, p, s);
+  // the first render sizes the workspace: staging takes what there is room for
+  if (!ws.frozen())
+    for (int p = 0; p < 2; ++p) {
+      while (pl.m[p] && rv.groups_cap[p] && !stage_room(ws, p, rv.ns_cap[p], rv.groups_cap[p]))
+        rv.groups_cap[p] /= 2;
+      if (rv.groups_cap[p] == 0) rv.ns_cap[p] = 0;
+      pl.nstage[p] = rv.ns_cap[p];
+      pl.sgroups[p] = rv.groups_cap[p];
+    }
   for (int p = 0; p < 2; ++p)
     if (pl.m[p]) {
       stage_items_count(c, pl, p, tn, tot, s);
@@ -1983,13 +2015,10 @@ int capture_reserve(splhip_ctx *c, int nj, const JobIn *jobs, float headroom, hi
     if (c->last_stage_n[p] > 0) {
       rv->ns_cap[p] = static_cast<uint32_t>(std::min(
           static_cast<double>(c->last_stage_n[p]) * headroom + 16.0, 1048576.0));
-      const double g = static_cast<double>(c->last_stage_groups[p]) * headroom + 1024.0;
-      const uint64_t gc = static_cast<uint64_t>(g);
-      if (4 * stage_floats(p == 1, gc) <= kStageBudget) {
-        rv->groups_cap[p] = gc;
-      } else {
-        rv->ns_cap[p] = 0;
-      }
+      // (at most what the budget holds: k_partition then stages the longest)
+      rv->groups_cap[p] = std::min<uint64_t>(
+          static_cast<uint64_t>(static_cast<double>(c->last_stage_groups[p]) * headroom + 1024.0),
+          stage_groups_in(p == 1, kStageBudget));
     }
   }
   Plan pl;

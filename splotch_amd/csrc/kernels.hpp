@@ -250,6 +250,7 @@ void launch_seg_join(const SegArgs &g, uint32_t nlists, const float *states, con
 // (read ahead, never applied).
 constexpr uint32_t kStagePad = 512;
 uint64_t stage_floats(bool additive, uint64_t groups);
+uint64_t stage_groups_in(bool additive, uint64_t bytes);  // the most with operands of `bytes`
 uint64_t stage_stride(uint64_t groups);
 uint64_t stage_batches(uint64_t groups, uint32_t n);
 void launch_stage_base(const uint32_t *items, uint32_t n, uint32_t n1, uint32_t *cbase,

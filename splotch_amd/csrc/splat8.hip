@@ -2210,6 +2210,10 @@ uint64_t stage_floats(bool additive, uint64_t groups) {
   return (additive ? stage_planes<1>() : stage_planes<0>()) * stage_stride(groups) * 32u;
 }
 
+uint64_t stage_groups_in(bool additive, uint64_t bytes) {
+  return (bytes / (128u * (additive ? stage_planes<1>() : stage_planes<0>())) - kStagePad) / 8u;
+}
+
 uint64_t stage_batches(uint64_t groups, uint32_t n) { return groups / 16u + n; }
 
 void launch_stage_base(const uint32_t *items, uint32_t n, uint32_t n1, uint32_t *cbase,

@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 #include <cstddef>
 #include <cstdint>
+#include <initializer_list>
 #include <string>
 
 namespace splhip {
@@ -46,6 +47,7 @@ class Workspace {
   // A frozen workspace never grows: a request past a slot's capacity throws
   // (no allocation or device synchronisation, e.g. under stream capture).
   void freeze(bool f) { frozen_ = f; }
+  bool frozen() const { return frozen_; }
   void *get(int slot, size_t bytes) {
     if (bytes == 0) bytes = 256;
     if (cap_[slot] < bytes && frozen_)
@@ -58,8 +60,7 @@ class Workspace {
         ptr_[slot] = nullptr;
         cap_[slot] = 0;
       }
-      size_t c = bytes + bytes / 8;  // headroom against small growth steps
-      c = (c + 4095) & ~size_t(4095);
+      const size_t c = grown(bytes);
       hip_check(hipMalloc(&ptr_[slot], c), "hipMalloc workspace");
       cap_[slot] = c;
     }
@@ -68,6 +69,25 @@ class Workspace {
   template <class T>
   T *get_as(int slot, size_t count) {
     return static_cast<T *>(get(slot, count * sizeof(T)));
+  }
+  // Buffers that a pass can do without: true, and the slots hold them, where
+  // they need at most half of the free device memory beyond what the slots hold
+  // already (the rest is for what the call cannot do without).
+  struct Request {
+    int slot;
+    size_t bytes;
+  };
+  bool optional(std::initializer_list<Request> rs) {
+    size_t more = 0;
+    for (const Request &r : rs)
+      if (cap_[r.slot] < r.bytes) more += grown(r.bytes) - cap_[r.slot];
+    if (more > 0) {
+      size_t free = 0, total = 0;
+      hip_check(hipMemGetInfo(&free, &total), "hipMemGetInfo");
+      if (more > free / 2) return false;
+      for (const Request &r : rs) (void)get(r.slot, r.bytes);
+    }
+    return true;
   }
   size_t total_bytes() const {
     size_t s = 0;
@@ -83,6 +103,9 @@ class Workspace {
   }
 
  private:
+  static size_t grown(size_t bytes) {  // headroom against small growth steps
+    return (bytes + bytes / 8 + 4095) & ~size_t(4095);
+  }
   void *ptr_[S_NSLOTS] = {};
   size_t cap_[S_NSLOTS] = {};
   bool frozen_ = false;

@@ -2,7 +2,8 @@
 to grow holds nothing, so a later, smaller request gets memory of its own rather
 than the address it had before with the capacity of then.  Runs on the CPU:
 splotch_amd/csrc/workspace.hpp is compiled against a stand-in for the HIP
-allocator that fails past a limit.
+allocator that fails past a limit.  Buffers that a pass can do without are taken
+only where they leave half of the free memory.
 """
 import os
 import subprocess
@@ -51,14 +52,42 @@ int main() {
 """
 
 
-def test_slot_after_failed_growth(tmp_path):
+OPTIONAL = r"""
+#include "workspace.hpp"
+using namespace splhip;
+int main() {
+  Workspace w;
+  limit() = 16 << 20;  // free
+  if (w.optional({{S_REC, 5 << 20}, {S_ACT, 4 << 20}})) return 1;  // more than half
+  if (w.total_bytes() != 0) return 2;
+  if (!w.optional({{S_REC, 5 << 20}, {S_ACT, 2 << 20}})) return 3;
+  const size_t held = w.total_bytes();
+  if (held < (7 << 20) || held > (8 << 20)) return 4;
+  limit() = 0;  // held already: nothing more is needed
+  if (!w.optional({{S_REC, 5 << 20}, {S_ACT, 1 << 20}})) return 5;
+  limit() = 4 << 20;  // growth beyond what is held counts
+  if (w.optional({{S_REC, 5 << 20}, {S_ACT, 5 << 20}})) return 6;
+  if (w.total_bytes() != held) return 7;
+  return 0;
+}
+"""
+
+
+def compiled(tmp_path, main):
     (tmp_path / "hip").mkdir()
     (tmp_path / "hip" / "hip_runtime.h").write_text(HIP)
-    (tmp_path / "main.cpp").write_text(MAIN)
+    (tmp_path / "main.cpp").write_text(main)
     exe = str(tmp_path / "main")
     subprocess.run(["g++", "-std=c++17", "-O1", "-g", "-I", str(tmp_path), "-I",
                     os.path.join(ROOT, "splotch_amd", "csrc"), str(tmp_path / "main.cpp"),
                     "-o", exe], check=True)
-    r = subprocess.run([exe])
-    assert r.returncode == 0, {3: "a null pointer for a slot that failed to grow"}.get(
-        r.returncode, r.returncode)
+    return subprocess.run([exe]).returncode
+
+
+def test_slot_after_failed_growth(tmp_path):
+    rc = compiled(tmp_path, MAIN)
+    assert rc == 0, {3: "a null pointer for a slot that failed to grow"}.get(rc, rc)
+
+
+def test_optional_buffers(tmp_path):
+    assert compiled(tmp_path, OPTIONAL) == 0
