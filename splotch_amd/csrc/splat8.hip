@@ -137,11 +137,6 @@ __device__ __forceinline__ float quad_of(float v, int j) {  // j: constant after
 __device__ __forceinline__ float4 quad_of(const float4 &v, int j) {
   return make_float4(quad_of(v.x, j), quad_of(v.y, j), quad_of(v.z, j), quad_of(v.w, j));
 }
-// v of lane k (wave-uniform, k < 4) of the wave's first four lanes.
-__device__ __forceinline__ float4 chunk_lane(const float4 &v, int k) {
-  return make_float4(lane_f(v.x, k), lane_f(v.y, k), lane_f(v.z, k), lane_f(v.w, k));
-}
-
 // x where bit 8 (j & 3) of the pixel's coverage word m is set (byte j: particle
 // j of four, shifted down by the pixel's row), else +0: the bit, sign-extended,
 // masks x's bits.
@@ -175,7 +170,11 @@ __device__ __forceinline__ void fast_chunk(int k0, int cx, int cy, const uint8_t
                                            const float4 *cst, float expfac4, float tl,
                                            float &l0, float &l1, float &l2) {
   constexpr bool C0 = (CH == 3 || CH == 0), C1 = (CH == 3 || CH == 1), C2 = (CH == 3 || CH == 2);
-  constexpr int JQ = (J + 3) / 4;
+  // constants and coverage of four particles, or where a chunk has fewer, of one
+  // (by lane from the four's: 100k additive particles at 512^2, hip_ppw 1, nothing
+  // staged, 2.15 ms; so 1.39)
+  constexpr bool kQuads = J >= 4;
+  constexpr int JQ = kQuads ? J / 4 : J;
   float at[J], m2[J], g0[J], g1[J], g2[J], u0[J], w0[J], u1[J], w1[J], u2[J], w2[J];
   float4 ca[JQ], cq[JQ];
   uint32_t cov[JQ];
@@ -184,29 +183,24 @@ __device__ __forceinline__ void fast_chunk(int k0, int cx, int cy, const uint8_t
   // zeros) and are masked; table offsets are masked into the tables
 #pragma unroll
   for (int q = 0; q < JQ; ++q) {
-    const int k = (k0 & ~3) + 4 * q;
-    ca[q] = cst[2 * (k + (cy & 3))];
-    cq[q] = cst[2 * (k + (cy & 3)) + 1];
-    cov[q] = *reinterpret_cast<const uint32_t *>(&col[cx][k]) >> cy;
-    if (J < 4) cov[q] >>= 8 * (k0 & 3);
+    const int k = kQuads ? k0 + 4 * q : k0 + q, kl = kQuads ? k + (cy & 3) : k;
+    ca[q] = cst[2 * kl];
+    cq[q] = cst[2 * kl + 1];
+    cov[q] = (kQuads ? *reinterpret_cast<const uint32_t *>(&col[cx][k]) : col[cx][k]) >> cy;
   }
 #pragma unroll
   for (int j = 0; j < J; ++j) {
     const int k = k0 + j;
-    at[j] = covered(pre1[cy][k] * pre2[cx][k], cov[j / 4], j);
+    at[j] = covered(pre1[cy][k] * pre2[cx][k], kQuads ? cov[j / 4] : cov[j], kQuads ? j : 0);
   }
-  // (chunks of fewer than four start inside a group of four: their constants
-  // come by lane from there)
-  auto con = [&](const float4 &v, int j) {
-    return J < 4 ? chunk_lane(v, (k0 & 3) + j) : quad_of(v, j);
-  };
+  auto con = [&](const float4 (&v)[JQ], int j) { return kQuads ? quad_of(v[j / 4], j) : v[j]; };
 #pragma unroll
   for (int j = 0; j < J; ++j) {
     if ((TB >> j) & 1u) {
       m2[j] = at[j];
       continue;
     }
-    const float4 a4 = con(ca[j / 4], j);
+    const float4 a4 = con(ca, j);
     tay[j] = (a4.w * at[j]) < tl;
     m2[j] = tay[j] ? at[j] : 1.f;
     if (C0) { g0[j] = at[j] * a4.x; xtab_fast(tab, g0[j], expfac4, u0[j], w0[j]); }
@@ -215,7 +209,7 @@ __device__ __forceinline__ void fast_chunk(int k0, int cx, int cy, const uint8_t
   }
 #pragma unroll
   for (int j = 0; j < J; ++j) {
-    const float4 a4 = con(ca[j / 4], j), q4 = con(cq[j / 4], j);
+    const float4 a4 = con(ca, j), q4 = con(cq, j);
     if ((TB >> j) & 1u) {
       if (C0) l0 = l0 + ((l0 - q4.x) * a4.x) * m2[j];
       if (C1) l1 = l1 + ((l1 - q4.y) * a4.y) * m2[j];
@@ -305,25 +299,26 @@ __device__ __forceinline__ void walk_chunks(int nb, int cx, int cy, const uint8_
       // Additive: constants and coverage as in the fast chunks (cst: (a0, a1,
       // a2, 0)); slots past the batch (stale or uninitialised values) are read
       // at their own offsets and their products masked, as their coverage is 0.
-      constexpr int JQ = (J + 3) / 4;
+      constexpr bool kQuads = J >= 4;
+      constexpr int JQ = kQuads ? J / 4 : J;
       float at[J];
       float4 ca[JQ];
       uint32_t cov[JQ];
 #pragma unroll
       for (int q = 0; q < JQ; ++q) {
-        const int k = (k0 & ~3) + 4 * q;
-        ca[q] = cst[k + (cy & 3)];
-        cov[q] = *reinterpret_cast<const uint32_t *>(&col[cx][k]) >> cy;
-        if (J < 4) cov[q] >>= 8 * (k0 & 3);
+        const int k = kQuads ? k0 + 4 * q : k0 + q;
+        ca[q] = cst[kQuads ? k + (cy & 3) : k];
+        cov[q] = (kQuads ? *reinterpret_cast<const uint32_t *>(&col[cx][k]) : col[cx][k]) >> cy;
       }
 #pragma unroll
       for (int j = 0; j < J; ++j) at[j] = pre1[cy][k0 + j] * pre2[cx][k0 + j];
 #pragma unroll
       for (int j = 0; j < J; ++j) {
-        const float4 a4 = J < 4 ? chunk_lane(ca[j / 4], (k0 & 3) + j) : quad_of(ca[j / 4], j);
-        if (C0) l0 = l0 + covered(a4.x * at[j], cov[j / 4], j);
-        if (C1) l1 = l1 + covered(a4.y * at[j], cov[j / 4], j);
-        if (C2) l2 = l2 + covered(a4.z * at[j], cov[j / 4], j);
+        const float4 a4 = kQuads ? quad_of(ca[j / 4], j) : ca[j];
+        const uint32_t m = kQuads ? cov[j / 4] : cov[j];
+        if (C0) l0 = l0 + covered(a4.x * at[j], m, kQuads ? j : 0);
+        if (C1) l1 = l1 + covered(a4.y * at[j], m, kQuads ? j : 0);
+        if (C2) l2 = l2 + covered(a4.z * at[j], m, kQuads ? j : 0);
       }
       continue;
     }
@@ -810,11 +805,16 @@ __device__ __forceinline__ void walk_list(const SplatArgs &a, const UnitGeom &ug
 // Four workgroups per CU (their LDS, 35 KB each, and at most 128 VGPRs a lane):
 // the walk waits on LDS returns, and 16 waves hide more of them than the 12
 // that 142 VGPRs allow (64 views with 137M ordered and 124M additive entries:
-// 31.9 -> 30.6 ms; 32.1 with constants and coverage read per particle).
+// 31.9 -> 30.6 ms; 32.1 with constants and coverage read per particle).  Ordered
+// chunks of 8 (hip_ppw 8) hold 181 VGPRs: two (1M particles at 1024^2, nothing
+// staged: 6.4 ms; 7.9 with 128 VGPRs and the rest in scratch).
+template <int ADD, int PPW>
+constexpr int splat_waves() {
+  return !ADD && PPW == 8 ? 2 : 4;
+}
 template <int ADD, int VAR, int PPW>
-__global__ __launch_bounds__(256, 4) void k_splat8(SplatArgs a, const uint32_t *items,
-                                                uint32_t nitems_, ItemCounts dc,
-                                                uint32_t nsplit_) {
+__global__ __launch_bounds__(256, (splat_waves<ADD, PPW>())) void k_splat8(
+    SplatArgs a, const uint32_t *items, uint32_t nitems_, ItemCounts dc, uint32_t nsplit_) {
   const uint32_t nreal = splat_items(items, nitems_, dc);
   // the first nsplit items are long lists served as three one-channel items
   const uint32_t nsplit = min(dc.nsplit ? *dc.nsplit : nsplit_, nreal);
@@ -834,7 +834,8 @@ __global__ __launch_bounds__(256, 4) void k_splat8(SplatArgs a, const uint32_t *
   const uint32_t item = it < 3u * nsplit ? (uniform(items[it / 3u]) & ~3u) | (it % 3u)
                                           : uniform(items[it - 2u * nsplit]);
   const uint32_t u = item >> 2;
-  const int chan = static_cast<int>(item & 3u);  // 3: all channels
+  // 3: all channels (variant 1 looks at it per particle)
+  const int chan = static_cast<int>(VAR == 1 ? uniform(item & 3u) : item & 3u);
   const UnitGeom ug = unit_geom_uniform(a, u);
   const int lx = ug.gx * 8 + (lane >> 3), ly = ug.gy * 8 + (lane & 7);
   clear_slots(s_wave[wave], lane);
