@@ -322,6 +322,7 @@ __device__ __forceinline__ void walk_chunks(int nb, int cx, int cy, const uint8_
       }
       continue;
     }
+    // ordered, with a particle in the chunk that is not fast
     float att[J], g0[J], g1[J], g2[J], p0[J], p1[J], p2[J];
     float u0[J], w0[J], u1[J], w1[J], u2[J], w2[J];
     uint32_t msk[J];
@@ -332,44 +333,36 @@ __device__ __forceinline__ void walk_chunks(int nb, int cx, int cy, const uint8_
       msk[j] = (k0 + j < nb) ? mk : 0u;
       att[j] = pre1[cy][k] * pre2[cx][k];
     }
-    if (!ADD) {
 #pragma unroll
-      for (int j = 0; j < J; ++j) {
-        const int k = min(k0 + j, nb - 1);
-        if (C0) { g0[j] = att[j] * lane_f(va0, k); p0[j] = g0[j] * expfac; const int i = xexp_index(p0[j]); u0[j] = tab[i >> 10]; w0[j] = tab[1024 + (i & 1023)]; }
-        if (C1) { g1[j] = att[j] * lane_f(va1, k); p1[j] = g1[j] * expfac; const int i = xexp_index(p1[j]); u1[j] = tab[i >> 10]; w1[j] = tab[1024 + (i & 1023)]; }
-        if (C2) { g2[j] = att[j] * lane_f(va2, k); p2[j] = g2[j] * expfac; const int i = xexp_index(p2[j]); u2[j] = tab[i >> 10]; w2[j] = tab[1024 + (i & 1023)]; }
-      }
+    for (int j = 0; j < J; ++j) {
+      const int k = min(k0 + j, nb - 1);
+      if (C0) { g0[j] = att[j] * lane_f(va0, k); p0[j] = g0[j] * expfac; const int i = xexp_index(p0[j]); u0[j] = tab[i >> 10]; w0[j] = tab[1024 + (i & 1023)]; }
+      if (C1) { g1[j] = att[j] * lane_f(va1, k); p1[j] = g1[j] * expfac; const int i = xexp_index(p1[j]); u1[j] = tab[i >> 10]; w1[j] = tab[1024 + (i & 1023)]; }
+      if (C2) { g2[j] = att[j] * lane_f(va2, k); p2[j] = g2[j] * expfac; const int i = xexp_index(p2[j]); u2[j] = tab[i >> 10]; w2[j] = tab[1024 + (i & 1023)]; }
     }
 #pragma unroll
     for (int j = 0; j < J; ++j) {
       const int k = min(k0 + j, nb - 1);
       const bool in = (msk[j] >> cy) & 1u;
       const float at = att[j];
-      if (ADD) {
-        if (C0) { const float t = lane_f(va0, k) * at; l0 = l0 + (in ? t : 0.f); }
-        if (C1) { const float t = lane_f(va1, k) * at; l1 = l1 + (in ? t : 0.f); }
-        if (C2) { const float t = lane_f(va2, k) * at; l2 = l2 + (in ? t : 0.f); }
-      } else {
-        const bool tay = (lane_f(vmax, k) * at) < tl;
-        if (C0) {
-          const float em = xexpm1_finish(g0[j], p0[j], u0[j], w0[j], tl);
-          const float d = l0 - lane_f(vq0, k);
-          const float ta = (d * lane_f(va0, k)) * at, te = em * d;
-          l0 = l0 + (in ? (tay ? ta : te) : 0.f);
-        }
-        if (C1) {
-          const float em = xexpm1_finish(g1[j], p1[j], u1[j], w1[j], tl);
-          const float d = l1 - lane_f(vq1, k);
-          const float ta = (d * lane_f(va1, k)) * at, te = em * d;
-          l1 = l1 + (in ? (tay ? ta : te) : 0.f);
-        }
-        if (C2) {
-          const float em = xexpm1_finish(g2[j], p2[j], u2[j], w2[j], tl);
-          const float d = l2 - lane_f(vq2, k);
-          const float ta = (d * lane_f(va2, k)) * at, te = em * d;
-          l2 = l2 + (in ? (tay ? ta : te) : 0.f);
-        }
+      const bool tay = (lane_f(vmax, k) * at) < tl;
+      if (C0) {
+        const float em = xexpm1_finish(g0[j], p0[j], u0[j], w0[j], tl);
+        const float d = l0 - lane_f(vq0, k);
+        const float ta = (d * lane_f(va0, k)) * at, te = em * d;
+        l0 = l0 + (in ? (tay ? ta : te) : 0.f);
+      }
+      if (C1) {
+        const float em = xexpm1_finish(g1[j], p1[j], u1[j], w1[j], tl);
+        const float d = l1 - lane_f(vq1, k);
+        const float ta = (d * lane_f(va1, k)) * at, te = em * d;
+        l1 = l1 + (in ? (tay ? ta : te) : 0.f);
+      }
+      if (C2) {
+        const float em = xexpm1_finish(g2[j], p2[j], u2[j], w2[j], tl);
+        const float d = l2 - lane_f(vq2, k);
+        const float ta = (d * lane_f(va2, k)) * at, te = em * d;
+        l2 = l2 + (in ? (tay ? ta : te) : 0.f);
       }
     }
   }
