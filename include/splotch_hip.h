@@ -67,9 +67,14 @@ typedef struct {
   float gray_absorption;                   /* gray_absorption (0.2) */
   int32_t tile_size;                       /* tile_size_cpu (50): reference tile */
   int32_t hip_region;                      /* hip_region: GPU work region, px: 8, 16, 32, 64 (0 = auto) */
-  int32_t hip_split;                       /* hip_split: list length from which an 8x8 block is
-                                              splatted as one work item per channel
-                                              (0 = auto: 32768) */
+  int32_t hip_split;                       /* hip_split: list length from which an 8x8 block that
+                                              is neither staged nor a producer/consumer
+                                              workgroup's is splatted as one work item per
+                                              channel (twice it in an additive pass; from the
+                                              staging base length on, lengths are rounded
+                                              down to a level of it, see hip_stage_ordered)
+                                              (0 = auto: 32768; below, lists from the pass's
+                                              entries / 2048 on are in any case) */
   int32_t hip_variant;                     /* hip_variant: 8x8 splat inner loop, 0 = auto (4),
                                               1 = per particle, 2 = 4-particle groups,
                                               3 = software pipelined, 4 = chunked branch-free */

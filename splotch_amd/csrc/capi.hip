@@ -40,7 +40,7 @@ struct splhip_ctx {
   bool split_hint = false;  // the last capacity error can be avoided by smaller groups
   // the 8x8 splat decomposition found by the last inner autotuner sweep:
   // variant, ppw, split, heavy, heavy_max
-  uint32_t inner_choice[5] = {4, 0, 32768, 32768, 192};
+  uint32_t inner_choice[5] = {4, 0, kSplitAuto, 32768, 192};
   int device = 0;
   std::string err;
   Workspace ws;
@@ -942,14 +942,6 @@ uint32_t seg_length(uint64_t etot) { return etot < kSegEntries ? 0u : kSegLen; }
 // whose staged lists need more, or more than the device memory has to spare,
 // fewer are staged (the longest).
 constexpr uint64_t kStageBudget = uint64_t(32) << 30;
-// Long lists left to the 8x8 splat that would outlast the pass, walked by
-// one wave at about 230 ns per entry against about 0.1 ns per entry of the
-// pass over all CUs (16M particles at 2048^2), are served by channel, three
-// waves each: those from entries / kSplitRatio on (rounded down to a level).
-// Serving every such list by channel costs more than it saves (41.2 ->
-// 48.2 ms at 16M / 2048^2): three one-channel walks take more VALU work than
-// one three-channel walk.
-constexpr uint32_t kSplitRatio = 2048;
 // Staged lists whose chains start right after their own operands (the
 // longest; the others' operands and chains follow beside them).  The 64-view
 // batch: 34.9 ms with 64, 33.7 with 16, 34.1 with 4; the 1M / 800^2 frame and
@@ -961,7 +953,7 @@ Tuning tuning_of(const splhip_params *prm) {
   t.ppw = prm->hip_ppw;
   // lists from hip_heavy on go to producer/consumer workgroups (up to the cap)
   // or stay whole: splitting by channel pays only without those workgroups
-  t.split = prm->hip_split > 0 ? static_cast<uint32_t>(prm->hip_split) : 32768u;
+  t.split = prm->hip_split > 0 ? static_cast<uint32_t>(prm->hip_split) : kSplitAuto;
   t.heavy = prm->hip_heavy < 0 ? 0xffffffffu
             : prm->hip_heavy > 0 ? static_cast<uint32_t>(prm->hip_heavy) : 32768u;
   // a producer/consumer workgroup occupies a CU: leave the splat8 items
@@ -1113,7 +1105,7 @@ void take_items(splhip_ctx *c, Plan &pl, int p, const Tuning &tn) {
   const uint32_t nlong = !pl.m[p] ? 0u : len0s <= tn.heavy ? cnt[0] : nheavy_lists;
   pl.nsplit[p] = pl.m[p] ? split_lists(len0s, cnt,
                                        std::min(nlong, pl.nitems[p]), pl.nheavy[p], pl.etot[p],
-                                       kSplitRatio)
+                                       p == 1, tn.split)
                          : 0u;
 }
 
@@ -1163,7 +1155,8 @@ void stage_splat(splhip_ctx *c, Plan &pl, int p, const Tuning &tn, hipStream_t s
     pa.groups_cap = pl.sgroups[p];
     pa.heavy_max = tn.heavy == 0xffffffffu ? 0u : tn.heavy_max;
     pa.heavy_len = tn.heavy;
-    pa.split = kSplitRatio;
+    pa.additive = p == 1;
+    pa.split = tn.split;
     launch_partition(pa, part, s);
     dc.items = pl.tot + T_ITEMS + p;
     dc.heavy = part + 2;
@@ -1468,7 +1461,7 @@ Tuning autotune(splhip_ctx *c, Plan &pl, const Tuning &base, uint32_t *tot, hipS
     if (ms < best_ms) { best_ms = ms; best = t; }
   }
   const Tuning b1 = best;
-  for (uint32_t split : {4096u, 8192u, 32768u}) {
+  for (uint32_t split : {4096u, 8192u, kSplitAuto}) {
     Tuning t = b1;
     t.split = split;
     const float ms = time_of(t);

@@ -286,18 +286,31 @@ struct PartitionArgs {
   uint64_t groups_cap;
   uint32_t heavy_max;  // 0: no producer/consumer workgroups
   uint32_t heavy_len;  // lists from this length on go to producer/consumer workgroups
-  uint32_t split;
+  bool additive;
+  uint32_t split;  // hip_split
 };
 // The long lists after the first nheavy items that the 8x8 splat serves by
-// channel: those from the greatest level of len0 with level * split <= etot
-// on (level 0 when none is; none without a stage length), of the nlong long
-// lists; count[j]: the lists from level j on.
+// channel, of the nlong long lists: those from entries / kSplitRatio on, or from a
+// given hip_split on where that is less (twice it in an additive pass), rounded
+// down to a level of len0 (level 0 when none is; none without a stage length);
+// count[j]: the lists from level j on.
+//
+// Left to one wave, such a list would outlast the pass: about 200 ns per entry (by
+// channel half of it, see stage_rule) against about 0.1 ns per entry of the pass
+// over all CUs (16M particles at 2048^2).  Serving every such list by channel costs
+// more than it saves (41.2 -> 48.2 ms at 16M / 2048^2): three one-channel walks take
+// more VALU work than one three-channel walk.
+constexpr uint32_t kSplitRatio = 2048;
+constexpr uint32_t kSplitAuto = 32768;  // hip_split by default: the rule alone
 __host__ __device__ inline uint32_t split_lists(uint32_t len0, const uint32_t *count,
                                                 uint32_t nlong, uint32_t nheavy, uint64_t etot,
-                                                uint32_t split) {
+                                                bool additive, uint32_t split) {
   if (len0 == 0xffffffffu) return 0u;
+  uint64_t from = etot / kSplitRatio;
+  const uint64_t given = static_cast<uint64_t>(split) * (additive ? 2u : 1u);
+  if (split < kSplitAuto && given < from) from = given;
   int j = 0;
-  while (j < kStageLevels - 1 && stage_level(len0, j + 1) * split <= etot) ++j;
+  while (j < kStageLevels - 1 && stage_level(len0, j + 1) <= from) ++j;
   const uint32_t n = count[j] < nlong ? count[j] : nlong;
   return n > nheavy ? n - nheavy : 0u;
 }

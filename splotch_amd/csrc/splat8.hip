@@ -2297,7 +2297,7 @@ __global__ void k_partition(PartitionArgs a, uint32_t *out) {
   out[0] = ns;
   out[1] = npc;
   out[2] = ns + npc;
-  out[3] = split_lists(a.len0, a.stage_cnt, nlong, ns + npc, *a.etot, a.split);
+  out[3] = split_lists(a.len0, a.stage_cnt, nlong, ns + npc, *a.etot, a.additive, a.split);
 }
 
 void launch_partition(const PartitionArgs &pa, uint32_t *out, hipStream_t s) {
