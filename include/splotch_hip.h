@@ -331,7 +331,8 @@ int splhip_stage_times(splhip_ctx *ctx, float *ms, int64_t *counts);
 /* Work-item trace of the 8x8-block splat (no reference counterpart; the
    reference's tstack timers stop at stage granularity).  With tracing on, each
    render records per work item {start, end} (s_memrealtime, 100 MHz), the list
-   length | channel << 32 (channel 3 = all) and the hardware CU id;
+   length | channel << 32 (channel 3 = all; 4 = a list walked in segments, 5 =
+   some of those by channel) and the hardware CU id;
    splhip_trace_items copies the last frame's items of one pass (4 uint64 each;
    call with out=NULL to get the count in *n). */
 int splhip_set_trace(splhip_ctx *ctx, int32_t enable);

@@ -387,7 +387,7 @@ class Renderer:
 
     def trace_items(self, ordered: bool = True):
         """Last frame's splat work items: array (n, 4) of start, end (100 MHz
-        ticks), list length | channel << 32, CU id."""
+        ticks), list length | channel << 32 (3: all, 4 and more: in segments), CU id."""
         n = C.c_int64()
         L = lib()
         L.splhip_trace_items(self._c, C.c_int32(int(ordered)), None, C.c_int64(0), C.byref(n))

@@ -1121,9 +1121,11 @@ __global__ __launch_bounds__(64) void k_seg_join(SplatArgs a, SegArgs g, const f
   const UnitGeom ug = unit_geom_uniform(a, u);
   clear_slots(s_wave, lane);
   float l0 = 0.f, l1 = 0.f, l2 = 0.f;
+  uint64_t code = 4;  // the trace's channel code
   for (uint32_t k = 0; k < n; ++k) {
     const Seg *S = g.segs + first + k;
     const uint32_t chan = uniform(S->chan);
+    if (chan != 3u) code |= 1u;
     if (chan == 1u || chan == 2u) continue;  // (walks of the segment before)
     const uint32_t e0 = uniform(S->e0), e1 = uniform(S->e1);
     const float *c = states + static_cast<uint64_t>(uniform(S->slot)) * 192u;
@@ -1141,7 +1143,7 @@ __global__ __launch_bounds__(64) void k_seg_join(SplatArgs a, SegArgs g, const f
   if (a.trace && lane == 0) {
     uint64_t *tr = a.trace + 4 * static_cast<uint64_t>(blockIdx.x);
     tr[1] = __builtin_amdgcn_s_memrealtime();
-    tr[2] = static_cast<uint64_t>(a.bin_off[u + 1] - a.bin_off[u]) | (uint64_t(3) << 32);
+    tr[2] = static_cast<uint64_t>(a.bin_off[u + 1] - a.bin_off[u]) | (code << 32);
     tr[3] = static_cast<uint64_t>(__smid());
   }
   const int lx = ug.gx * 8 + (lane >> 3), ly = ug.gy * 8 + (lane & 7);
