@@ -970,10 +970,10 @@ Tuning tuning_of(const splhip_params *prm) {
   };
   stage(prm->hip_stage, 1, t.stage);
   stage(prm->hip_stage_ordered, 0, t.stage_ord);
-  // only where nothing asks for another decomposition
+  // only where nothing asks for another decomposition (the autotuner's choice is
+  // for the lists that are not walked in segments)
   t.seg = prm->hip_variant <= 0 && prm->hip_ppw == 0 && prm->hip_split <= 0 &&
-          prm->hip_heavy == 0 && prm->hip_heavy_max <= 0 && prm->hip_stage_ordered == 0 &&
-          !prm->hip_autotune;
+          prm->hip_heavy == 0 && prm->hip_heavy_max <= 0 && prm->hip_stage_ordered == 0;
   return t;
 }
 
@@ -1767,8 +1767,10 @@ int render_tuned(splhip_ctx *c, int nj, const JobIn *jobs, hipStream_t s, bool k
                  bool region8 = false) {
   const splhip_params *prm = jobs[0].prm;
   if (!prm->hip_autotune) return render_jobs(c, nj, jobs, s, keep_fwd, nullptr);
+  // (the render that sizes a reservation walks no list in segments)
   const uint64_t key = bucket_of(nj, jobs) | ((keep_fwd || region8) ? uint64_t(1) << 40 : 0) |
-                       (static_cast<uint64_t>(prm->hip_region & 0x7f) << 41);
+                       (static_cast<uint64_t>(prm->hip_region & 0x7f) << 41) |
+                       (c->sizing ? uint64_t(1) << 48 : 0);
   auto decode = [](const std::vector<uint32_t> &v, Choice &ch) {
     ch.G = static_cast<int>(v[0]);
     ch.tn.variant = static_cast<int>(v[1]);

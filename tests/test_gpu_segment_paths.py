@@ -119,3 +119,28 @@ def test_segment_paths(R, kind):
         assert stages["ordered_staged"] > 0.0
     if kind == "beside_workgroups":
         assert stages["ordered_k_splat_heavy"] > 0.0
+
+
+def test_autotuned_frame_keeps_its_segments(R):
+    """The autotuner chooses the decomposition of the other lists; tuning a frame must
+    not put its long lists back into producer/consumer workgroups."""
+    import splotch_amd as S
+    dev = S.to_device(frame("deep")[0])
+    cam = S.camera_setup(synth.default_view(SIDE))
+    pics = []
+    for tune in (0, 1):
+        print("case segments autotuned", tune, flush=True)
+        prm = S.params(a_eq_e=False, brightness=[100.0], hip_autotune=tune, hip_region=8)
+        pic = torch.empty(SIDE * SIDE * 3, dtype=torch.float32, device="cuda")
+        R.render(dev, cam, prm, pic)  # (tunes)
+        R.set_trace(True)
+        try:
+            R.render(dev, cam, prm, pic)
+            codes = R.trace_items(True)[:, 2] >> 32
+        finally:
+            R.set_trace(False)
+        torch.cuda.synchronize()
+        assert R.tuning()["autotuned"] == bool(tune)
+        assert (codes == 4).all() and codes.size == BLOCKS
+        pics.append(pic.cpu().numpy())
+    assert np.array_equal(pics[0].view(np.uint32), pics[1].view(np.uint32))
