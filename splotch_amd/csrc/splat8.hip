@@ -1052,19 +1052,6 @@ __device__ __forceinline__ void keep_state(float *st, int lane, uint32_t chan, f
   if (chan == 3u || chan == 1u) st[64 + lane] = l1;
   if (chan == 3u || chan == 2u) st[128 + lane] = l2;
 }
-__device__ __forceinline__ void take_state(const float *st, int lane, float &l0, float &l1,
-                                           float &l2) {
-  l0 = st[lane];
-  l1 = st[64 + lane];
-  l2 = st[128 + lane];
-}
-// The wave's states are the kept ones in all bits.
-__device__ __forceinline__ bool is_state(const float *st, int lane, float l0, float l1, float l2) {
-  return __all(__float_as_uint(st[lane]) == __float_as_uint(l0) &&
-               __float_as_uint(st[64 + lane]) == __float_as_uint(l1) &&
-               __float_as_uint(st[128 + lane]) == __float_as_uint(l2));
-}
-
 // One wave per segment.  Kept states: slot 0 at its first entry, slot j after j
 // * kSegCheck entries, the last after its last entry.
 __global__ __launch_bounds__(256, 4) void k_seg_walk(SplatArgs a, SegArgs g, uint32_t nseg,
@@ -1109,18 +1096,28 @@ __global__ __launch_bounds__(256, 4) void k_seg_walk(SplatArgs a, SegArgs g, uin
   }
 }
 
-// One wave per list: the segments' states joined, then the block's pixels.
+// Three waves per list, one a channel: the segments' states joined, then the block's
+// pixels.  A channel walks a segment again until it meets a kept state, at about 100
+// ns per entry (one wave for all channels: 200), so where the samples do not represent
+// the lists at all a pass ends at worst 100 ns per entry of its longest cut list
+// after its other work, twice a producer/consumer workgroup's 48.  (Absorption in the
+// sampled batch of 64 in 2048 only: four such lists of 1M in 273M entries 65 ms
+// without segments, 93 here, 105 with one wave; 23 of 1.2M in 229M 53, 122 and 140;
+// 1296 of 160k 39, 40 and 32.  Handing such lists to those workgroups after all
+// measured 101, 95 and 39, and a launch of them that finds none delays a batch by 8 %,
+// as each waits for a whole CU.)
 __global__ __launch_bounds__(64) void k_seg_join(SplatArgs a, SegArgs g, const float *states) {
   __shared__ float s_tab[2048];
   __shared__ SplatLds<0, 4> s_wave;
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x, c = static_cast<int>(blockIdx.x % 3u);
   for (int i = lane; i < 2048; i += 64) s_tab[i] = a.exptab[i];
   __syncthreads();
-  const SegList &L = g.lists[blockIdx.x];
+  const SegList &L = g.lists[blockIdx.x / 3u];
   const uint32_t u = uniform(L.unit), n = uniform(L.n), first = uniform(L.first);
   const UnitGeom ug = unit_geom_uniform(a, u);
   clear_slots(s_wave, lane);
-  float l0 = 0.f, l1 = 0.f, l2 = 0.f;
+  float l[3] = {0.f, 0.f, 0.f};
+  auto chain = [&]() -> float & { return c == 0 ? l[0] : c == 1 ? l[1] : l[2]; };
   uint64_t code = 4;  // the trace's channel code
   for (uint32_t k = 0; k < n; ++k) {
     const Seg *S = g.segs + first + k;
@@ -1128,31 +1125,32 @@ __global__ __launch_bounds__(64) void k_seg_join(SplatArgs a, SegArgs g, const f
     if (chan != 3u) code |= 1u;
     if (chan == 1u || chan == 2u) continue;  // (walks of the segment before)
     const uint32_t e0 = uniform(S->e0), e1 = uniform(S->e1);
-    const float *c = states + static_cast<uint64_t>(uniform(S->slot)) * 192u;
-    const float *end = c + 192u * ((e1 - e0 + kSegCheck - 1u) / kSegCheck);
-    bool met = k == 0 || is_state(c, lane, l0, l1, l2);
+    const float *st = states + static_cast<uint64_t>(uniform(S->slot)) * 192u + 64 * c + lane;
+    const float *end = st + 192u * ((e1 - e0 + kSegCheck - 1u) / kSegCheck);
+    // the wave's state is the kept one in all bits
+    auto is_state = [&]() {
+      return __all(__float_as_uint(*st) == __float_as_uint(chain())) != 0;
+    };
+    bool met = k == 0 || is_state();
     for (uint32_t pos = e0; !met && pos < e1;) {
       const uint32_t next = min(pos + kSegCheck, e1);
-      walk_list<0, 4, 0>(a, ug, pos, next, 3, lane, s_tab, s_wave, l0, l1, l2);
+      walk_list<0, 4, 0>(a, ug, pos, next, c, lane, s_tab, s_wave, l[0], l[1], l[2]);
       pos = next;
-      c += 192;
-      met = is_state(c, lane, l0, l1, l2);
+      st += 192;
+      met = is_state();
     }
-    if (met) take_state(end, lane, l0, l1, l2);
+    if (met) chain() = *end;
   }
-  if (a.trace && lane == 0) {
-    uint64_t *tr = a.trace + 4 * static_cast<uint64_t>(blockIdx.x);
+  if (a.trace && c == 0 && lane == 0) {
+    uint64_t *tr = a.trace + 4 * static_cast<uint64_t>(blockIdx.x / 3u);
     tr[1] = __builtin_amdgcn_s_memrealtime();
     tr[2] = static_cast<uint64_t>(a.bin_off[u + 1] - a.bin_off[u]) | (code << 32);
     tr[3] = static_cast<uint64_t>(__smid());
   }
   const int lx = ug.gx * 8 + (lane >> 3), ly = ug.gy * 8 + (lane & 7);
   if (lx < ug.w && ly < ug.h) {
-    float *d = ug.pic + (static_cast<int64_t>(ug.x0s + lx) * ug.yres + (ug.y0s + ly)) * 3;
-    const bool add = ug.accumulate == 1;
-    d[0] = add ? d[0] + l0 : l0;
-    d[1] = add ? d[1] + l1 : l1;
-    d[2] = add ? d[2] + l2 : l2;
+    float *d = ug.pic + (static_cast<int64_t>(ug.x0s + lx) * ug.yres + (ug.y0s + ly)) * 3 + c;
+    *d = ug.accumulate == 1 ? *d + chain() : chain();
   }
 }
 
@@ -2196,7 +2194,7 @@ void launch_seg_walk(const SegArgs &g, uint32_t nseg, float *states, const Splat
 void launch_seg_join(const SegArgs &g, uint32_t nlists, const float *states, const SplatArgs &a,
                      hipStream_t s) {
   if (nlists == 0) return;
-  k_seg_join<<<nlists, 64, 0, s>>>(a, g, states);
+  k_seg_join<<<3u * nlists, 64, 0, s>>>(a, g, states);
   hip_check(hipGetLastError(), "k_seg_join launch");
 }
 

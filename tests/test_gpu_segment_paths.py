@@ -3,7 +3,8 @@
 The work-item trace has a record per such list (channel code 4, 5 where some of its
 segments are walked by channel), which shows that a frame took the path it is meant
 to test: lists cut or not by their absorption, walks by channel, two chunks of which
-the second continues cut lists from the image, cut lists beside producer/consumer
+the second continues cut lists from the image, lists whose samples do not represent them (walked
+again by channel), cut lists beside producer/consumer
 workgroups, beside staged lists, and beside an additive pass.  Bar: bit-exact against
 the walk of whole lists (no producer/consumer workgroups, no staging).
 
@@ -53,6 +54,12 @@ def late(n):
     return np.where((s >= 33) & (s < 40), 1.0, 1e-4)
 
 
+def sampled(n):
+    """Absorption almost only where the lists are sampled."""
+    s = np.arange(n) % 2048
+    return np.where((s >= 992) & (s < 1056), 1.0, 1e-4)
+
+
 # kind: (field, render keys, check of the ordered trace's lengths and channel codes)
 def frame(kind):
     if kind == "deep":
@@ -64,6 +71,14 @@ def frame(kind):
     if kind == "chunked":  # two chunks of 168.7M and 174.7M entries; the trace is the second's
         return (cluster(265_000, 50.0, 90.0, 1.0), dict(hip_chunk_entries=180_000_000),
                 lambda ln, ch: (ch == 4).all() and (ln > 130_000).all() and (ln < 136_000).all())
+    if kind == "sampled":  # a few long lists
+        a, b = cluster(240_000, 30.0, 35.0, 1.0), cluster(500_000, 92.0, 4.0, sampled(500_000), 0.02)
+        return (synth.concat(a, b), {},
+                lambda ln, ch: ((ch >= 4) & (ln == 500_000)).sum() > 2 and (ch >= 4).sum() > 50)
+    if kind == "sampled_chunked":  # in both chunks, the second from the image
+        inten = np.concatenate([sampled(130_207), sampled(134_793)])  # the chunks' particles
+        return (cluster(265_000, 50.0, 90.0, inten), dict(hip_chunk_entries=180_000_000),
+                lambda ln, ch: (ln == 134_793).all() and (ch >= 4).all())
     if kind == "beside_workgroups":  # a disc of cut lists, and one of lists that cannot be
         a, b = cluster(230_000, 80.0, 20.0, 1.0), cluster(230_000, 20.0, 20.0, 1e-5)
         return (synth.concat(a, b), {},
@@ -80,8 +95,9 @@ def frame(kind):
             lambda ln, ch: (ch == 4).all())
 
 
-@pytest.mark.parametrize("kind", ["deep", "thin", "by_channel", "chunked", "beside_workgroups",
-                                  "beside_staged", "beside_additive"])
+@pytest.mark.parametrize("kind", ["deep", "thin", "by_channel", "chunked", "sampled",
+                                  "sampled_chunked", "beside_workgroups", "beside_staged",
+                                  "beside_additive"])
 def test_segment_paths(R, kind):
     import splotch_amd as S
     fld, keys, check = frame(kind)
@@ -108,7 +124,7 @@ def test_segment_paths(R, kind):
     stages, counts = R.stage_times()
     entries = counts["ordered_entries"]
     assert entries >= LEAST
-    if kind == "chunked":
+    if kind in ("chunked", "sampled_chunked"):
         assert entries - 180_000_000 * 15 // 16 >= LEAST
     ln, ch = (tr[:, 2] & 0xffffffff).astype(np.int64), (tr[:, 2] >> 32).astype(np.int64)
     print("%s: %d entries, codes %s, longest %d" % (
