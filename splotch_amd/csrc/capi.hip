@@ -977,6 +977,12 @@ Tuning tuning_of(const splhip_params *prm) {
   return t;
 }
 
+// Lists from this length on may go to producer/consumer workgroups (beside segments,
+// those of one segment stay in the 8x8 splat).
+uint32_t heavy_length(const Plan &pl, int p, const Tuning &tn) {
+  return pl.seglen[p] ? std::max(tn.heavy, 2u * pl.seglen[p]) : tn.heavy;
+}
+
 SplatArgs splat_args(splhip_ctx *c, const Plan &pl, int p, const Tuning &tn) {
   SplatArgs sa{};
   sa.bin_off = pl.bin_off[p];
@@ -992,8 +998,7 @@ SplatArgs splat_args(splhip_ctx *c, const Plan &pl, int p, const Tuning &tn) {
   sa.expfac = c->consts.expfac;
   sa.taylorlimit = c->consts.taylorlimit;
   sa.prio_len = tn.split;
-  // lists of one segment stay in the 8x8 splat
-  sa.heavy_len = pl.seglen[p] ? std::max(tn.heavy, 2u * pl.seglen[p]) : tn.heavy;
+  sa.heavy_len = heavy_length(pl, p, tn);
   // device counts: staging only where the reservation holds room for it
   sa.stage_len = (pl.dc && pl.nstage[p] == 0) ? 0xffffffffu : p == 1 ? tn.stage : tn.stage_ord;
   sa.qbad = p == 0 ? pl.qbad : nullptr;
@@ -1076,17 +1081,22 @@ void take_items(splhip_ctx *c, Plan &pl, int p, const Tuning &tn) {
   pl.nsegs[p] = pl.seglen[p] ? h[T_SEG + SC_SEG - T_ITEMS] : 0u;
   pl.nslots[p] = pl.seglen[p] ? h[T_SEG + SC_SLOT - T_ITEMS] : 0u;
   const uint32_t nheavy_lists = pl.m[p] ? h[t_list(p, L_HEAVY) - T_ITEMS] : 0u;
-  const uint64_t lmax = h[t_list(p, L_MAX) - T_ITEMS];
   const uint32_t len0 = p == 1 ? tn.stage : tn.stage_ord;
   const uint32_t *cnt = h + (t_list(p, L_CNT) - T_ITEMS);
   const uint32_t *grp = h + (t_list(p, L_GRP) - T_ITEMS);
+  const uint32_t heavy_max = tn.heavy == 0xffffffffu ? 0u : tn.heavy_max;
+  const uint32_t heavy_len = heavy_length(pl, p, tn);
+  const ListCounts lc{cnt, grp, len0, nheavy_lists, heavy_max, heavy_len,
+                      h[t_list(p, L_MAX) - T_ITEMS], pl.etot[p]};
   uint32_t ns = 0;
   uint64_t groups = 0;
+  float longest = static_cast<float>(lc.lmax);  // of the lists that are not staged
   if (pl.m[p] && len0 != 0xffffffffu)
-    for (int j = stage_rule(len0, tn.mode[p], lmax, pl.etot[p]); j >= 0 && j < kStageLevels; ++j)
+    for (int j = stage_rule(lc, tn.mode[p]); j >= 0 && j < kStageLevels; ++j)
       if (cnt[j] == 0u || stage_room(*pl.ws, p, cnt[j], grp[j])) {
         ns = cnt[j];
         groups = grp[j];
+        if (ns) longest = static_cast<float>(stage_level(len0, j));
         break;
       }
   pl.nstage[p] = ns;
@@ -1095,17 +1105,18 @@ void take_items(splhip_ctx *c, Plan &pl, int p, const Tuning &tn) {
   c->last_stage_groups[p] = pl.sgroups[p];
   // staged lists from a threshold at least heavy_len are all among those
   // from heavy_len on; from a lower one they include all of those
-  const uint32_t npc = tn.heavy == 0xffffffffu || nheavy_lists <= ns
-                           ? 0u : std::min(nheavy_lists - ns, tn.heavy_max);
+  const uint32_t npc =
+      heavy_max == 0u || nheavy_lists <= ns ? 0u : std::min(nheavy_lists - ns, heavy_max);
+  if (npc > 0 && npc == nheavy_lists - ns)
+    longest = std::min(longest, static_cast<float>(heavy_len));
   // the heaviest items (sorted first); a unit's channel items are
   // independent, so the cut may fall between them
   pl.nheavy[p] = std::min(ns + npc, pl.nitems[p]);
   // lists from min(stage length, heavy_len) entries on have one item each
-  const uint32_t len0s = p == 1 ? tn.stage : tn.stage_ord;
-  const uint32_t nlong = !pl.m[p] ? 0u : len0s <= tn.heavy ? cnt[0] : nheavy_lists;
-  pl.nsplit[p] = pl.m[p] ? split_lists(len0s, cnt,
-                                       std::min(nlong, pl.nitems[p]), pl.nheavy[p], pl.etot[p],
-                                       p == 1, tn.split)
+  const uint32_t nlong = !pl.m[p] ? 0u : len0 <= heavy_len ? cnt[0] : nheavy_lists;
+  pl.nsplit[p] = pl.m[p] ? split_lists(lc, std::min(nlong, pl.nitems[p]), pl.nheavy[p],
+                                       static_cast<uint32_t>(pl.sgroups[p]), longest, p == 1,
+                                       tn.split)
                          : 0u;
 }
 
@@ -1279,7 +1290,7 @@ void stage_splat(splhip_ctx *c, Plan &pl, int p, const Tuning &tn, hipStream_t s
     if (npc > 0 || nseg > 0) launch_delay(40, s, dc.npc);
     if (placed) hip_check(hipEventRecord(placed, s), "record placed");
     mark(c, p == 0 ? 7 : 9, true, s);
-    launch_splat8(p == 1, tn.variant, nit, nn, sn, s, dc, tn.ppw, pl.nsplit[p]);
+    launch_splat8(p == 1, tn.variant, nit, nn, sn, s, dc, tn.ppw, pl.nsplit[p], npc > 0);
     mark(c, p == 0 ? 7 : 9, false, s);
     if ((npc > 0 && fork) || (nseg > 0 && npc == 0)) hip_check(hipStreamWaitEvent(s, X.join, 0), "wait join");
     if (nstage > 0 || (nseg > 0 && npc > 0)) hip_check(hipStreamWaitEvent(s, X.join3, 0), "wait join");

@@ -192,10 +192,11 @@ struct ItemCounts {
 // *dc.nsplit): the first nsplit of the 8x8 splat's items are long lists (one
 // all-channel item each) left over by the staged and producer/consumer
 // kernels; the 8x8 splat serves each as three one-channel items, so that
-// three waves share its chain (a grid for nitems + 2 nsplit items).
+// three waves share its chain (a grid for nitems + 2 nsplit items).  beside: producer/
+// consumer workgroups run at the same time.
 void launch_splat8(bool additive, int variant, const uint32_t *items, uint32_t nitems,
                    const SplatArgs &a, hipStream_t s, const ItemCounts &dc = ItemCounts{},
-                   int ppw = 0, uint32_t nsplit = 0);
+                   int ppw = 0, uint32_t nsplit = 0, bool beside = false);
 // Ordered lists walked in segments (splat8.hip): lists of at least 2 * seglen
 // entries, cut where the sampled entries before the cut make every pixel's chain
 // forget its start.  flag[u] says per unit whether its list is (the item kernels
@@ -289,38 +290,67 @@ struct PartitionArgs {
   bool additive;
   uint32_t split;  // hip_split
 };
-// The long lists after the first nheavy items that the 8x8 splat serves by
-// channel, of the nlong long lists: those from entries / kSplitRatio on, or from a
-// given hip_split on where that is less (twice it in an additive pass), rounded
-// down to a level of len0 (level 0 when none is; none without a stage length);
-// count[j]: the lists from level j on.
-//
-// Left to one wave, such a list would outlast the pass: about 200 ns per entry (by
-// channel half of it, see stage_rule) against about 0.1 ns per entry of the pass
-// over all CUs (16M particles at 2048^2).  Serving every such list by channel costs
-// more than it saves (41.2 -> 48.2 ms at 16M / 2048^2): three one-channel walks take
-// more VALU work than one three-channel walk.
+// What an entry of a list costs, in ns (MI355X; a lone wave's walk 140 to 230 ordered,
+// by absorption, 62 additive; by channel 100 to 118 and 54; in a producer/consumer
+// workgroup 44 to 54 and 30).
+struct ListRates {
+  float walk, heavy;    // its walk by one wave, and in a producer/consumer workgroup
+  float channels;       // the GPU's time for one walked by channel
+  float staged, full;   // and for a staged one: typically covered, and in full
+};
+__host__ __device__ inline ListRates list_rates(bool additive) {
+  return additive ? ListRates{62.f, 30.f, 0.15f, 0.165f, 0.28f}
+                  : ListRates{190.f, 50.f, 0.16f, 0.2f, 0.65f};
+}
+// A pass's lists: count[j] and groups[j] (of 4 entries) of those from level j of
+// len0 on, nheavy of those from heavy_len on.
+struct ListCounts {
+  const uint32_t *count, *groups;
+  uint32_t len0, nheavy, heavy_max, heavy_len;
+  uint64_t lmax, etot;
+  __host__ __device__ float entries(int j) const { return 4.f * static_cast<float>(groups[j]); }
+  __host__ __device__ bool enough_heavy() const { return heavy_max != 0u && nheavy <= heavy_max; }
+  // Time of a list of `len` entries on its own, and of the longest shorter ones.
+  __host__ __device__ float walk(float len, const ListRates &r) const {
+    const float h = static_cast<float>(heavy_len);
+    if (!enough_heavy() || len <= h) return len * r.walk;
+    return len * r.heavy > h * r.walk ? len * r.heavy : h * r.walk;
+  }
+};
+// The long lists after the first nheavy items (the staged ones, of `staged` groups,
+// first) that the 8x8 splat serves by channel, of the nlong long lists: with
+// hip_split given below its default (twice it in an additive pass), those from it on
+// rounded down to a level of len0; else those from entries / kSplitRatio on.  Left to
+// one wave, such a list (190 ns per entry ordered, by channel 105; additive 62 and 54)
+// would outlast the pass (about 0.1 ns per entry over all CUs).  But walking a list by
+// channel takes the GPU about twice the work: so not where that takes longer than the
+// longest of these lists (16M particles at 2048^2, every leftover list by channel:
+// 41.2 -> 48.2 ms; 1296 lists of 8000 ordered entries 1.6 and 2.5 ms, by absorption,
+// 2.2 by channel, of 30k 5.0 and 8.3, and 7.1; 5184 of up to 30k additive ones 2.6, and
+// 3.3), unless lists that producer/consumer workgroups have no room for wait beside
+// them (1104 of 100k ordered: 28 ms by channel, 43 not).
 constexpr uint32_t kSplitRatio = 2048;
-constexpr uint32_t kSplitAuto = 32768;  // hip_split by default: the rule alone
-__host__ __device__ inline uint32_t split_lists(uint32_t len0, const uint32_t *count,
-                                                uint32_t nlong, uint32_t nheavy, uint64_t etot,
+constexpr uint32_t kSplitAuto = 32768;  // hip_split by default: the rule
+__host__ __device__ inline uint32_t split_lists(const ListCounts &c, uint32_t nlong,
+                                                uint32_t nheavy, uint32_t staged, float longest,
                                                 bool additive, uint32_t split) {
-  if (len0 == 0xffffffffu) return 0u;
-  uint64_t from = etot / kSplitRatio;
-  const uint64_t given = static_cast<uint64_t>(split) * (additive ? 2u : 1u);
-  if (split < kSplitAuto && given < from) from = given;
+  if (c.len0 == 0xffffffffu) return 0u;
+  const bool given = split < kSplitAuto;
+  const uint64_t from = given ? static_cast<uint64_t>(split) * (additive ? 2u : 1u)
+                              : c.etot / kSplitRatio;
   int j = 0;
-  while (j < kStageLevels - 1 && stage_level(len0, j + 1) <= from) ++j;
-  const uint32_t n = count[j] < nlong ? count[j] : nlong;
+  while (j < kStageLevels - 1 && stage_level(c.len0, j + 1) <= from) ++j;
+  const ListRates r = list_rates(additive);
+  if (!given && c.nheavy <= c.heavy_max &&
+      (c.entries(j) - 4.f * static_cast<float>(staged)) * r.channels >= longest * r.walk)
+    return 0u;
+  const uint32_t n = c.count[j] < nlong ? c.count[j] : nlong;
   return n > nheavy ? n - nheavy : 0u;
 }
 // The staging level of a pass (-1: none): level 0 with a given length, else by
-// the pass's entries and its longest list.  A staged entry costs the GPU about
-// 1.5 times an entry of the 8x8 splat, whose lone wave walks a list at about
-// 75 (additive) or 200 (ordered; by channel about 100) ns per entry against
-// 0.1 ns per entry of the pass over all CUs.  So lists are staged from the
-// length on whose walk would outlast the pass, and not below a share of the
-// longest list, whose chain bounds the pass anyway:
+// the pass's entries and its longest list.  Lists are staged from the length on whose
+// walk would outlast the pass, and not below a share of the longest list, whose chain
+// bounds the pass anyway:
 //   additive  from entries / 1300 (rounded down to a level) or the longest
 //             list / 64 on (1M at 800^2, 5.2M entries, longest 165k: 1.23 ms
 //             from 4096, 1.32 from 8192, 1.36 from 1024; 2M at 512^2: 2.35 ms
@@ -338,21 +368,35 @@ __host__ __device__ inline uint32_t split_lists(uint32_t len0, const uint32_t *c
 //             the rest; else none
 // and none where the longest list is short: its walk costs less than the
 // staged kernels' launches (20k ordered at 257 x 193, longest 1345 entries:
-// 0.54 ms staged, 0.67 not).
-__host__ __device__ inline int stage_rule(uint32_t len0, StageMode mode, uint64_t lmax,
-                                          uint64_t etot) {
+// 0.54 ms staged, 0.67 not).  From there the level rises while staging takes the GPU
+// longer than the lists just below the next level take to walk, and past the longest
+// list (none) where staging its like takes longer than its walk: a view in which every
+// particle covers every block has hundreds of lists as long as the longest (1296 of
+// 8000 additive entries: 3.5 ms staged, 0.97 not; 324 of 30k 3.2 and 2.1, ordered 7.1
+// and 4.4).
+__host__ __device__ inline int stage_rule(const ListCounts &c, StageMode mode) {
   if (mode == kStageGiven) return 0;
   const bool add = mode == kStageAutoAdditive;
+  const uint64_t lmax = c.lmax, etot = c.etot;
+  const uint32_t len0 = c.len0;
   if (lmax < (add ? 1536u : 512u)) return -1;
   int j = 0;
   if (add || lmax * 216u >= etot) {
     while (j < kStageLevels - 1 && stage_level(len0, j) * (add ? 64u : 16u) < lmax) ++j;
     while (j < kStageLevels - 1 && stage_level(len0, j + 1) * (add ? 1300u : 700u) <= etot) ++j;
-    return j;
+  } else {
+    if (lmax * 432u < etot || stage_level(len0, kStageLevels - 1) * 432u < etot) return -1;
+    while (j < kStageLevels - 1 && stage_level(len0, j + 1) * 432u <= etot) ++j;
   }
-  if (lmax * 432u < etot || stage_level(len0, kStageLevels - 1) * 432u < etot) return -1;
-  while (j < kStageLevels - 1 && stage_level(len0, j + 1) * 432u <= etot) ++j;
-  return j;
+  const ListRates r = list_rates(add);
+  for (; j < kStageLevels && c.count[j] != 0u; ++j) {
+    while (j < kStageLevels - 1 && c.count[j + 1] == c.count[j]) ++j;  // the same lists
+    const uint64_t next = j < kStageLevels - 1 ? stage_level(len0, j + 1) : lmax;
+    const bool last = next >= lmax;
+    const float cost = c.entries(j) * (last ? r.full : r.staged);
+    if (cost <= c.walk(static_cast<float>(last ? lmax : next), r)) return j;
+  }
+  return -1;
 }
 void launch_partition(const PartitionArgs &pa, uint32_t *out, hipStream_t s);
 // Producer/consumer workgroups (splat8.hip), one per item: the first npc

@@ -2281,27 +2281,37 @@ void launch_stage_chain(bool additive, const uint32_t *items, uint32_t i0, uint3
   hip_check(hipGetLastError(), "k_stage_chain launch");
 }
 
-__global__ void k_partition(PartitionArgs a, uint32_t *out) {
-  uint32_t ns = 0;
-  if (a.len0 != 0xffffffffu) {
-    int j = stage_rule(a.len0, a.mode, *a.lmax, *a.etot);
-    for (; j >= 0 && j < kStageLevels; ++j)
-      if (a.stage_cnt[j] <= a.ns_cap && a.stage_grp[j] <= a.groups_cap) {
-        ns = a.stage_cnt[j];
+__global__ __launch_bounds__(64) void k_partition(PartitionArgs a, uint32_t *out) {
+  __shared__ uint32_t s_cnt[kStageLevels], s_grp[kStageLevels];  // (read at once)
+  if (threadIdx.x < kStageLevels) {
+    s_cnt[threadIdx.x] = a.stage_cnt[threadIdx.x];
+    s_grp[threadIdx.x] = a.stage_grp[threadIdx.x];
+  }
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  const uint32_t nh = *a.heavy_cnt;
+  const ListCounts c{s_cnt, s_grp, a.len0, nh, a.heavy_max, a.heavy_len, *a.lmax, *a.etot};
+  uint32_t ns = 0, staged = 0;
+  float longest = static_cast<float>(c.lmax);
+  if (a.len0 != 0xffffffffu)
+    for (int j = stage_rule(c, a.mode); j >= 0 && j < kStageLevels; ++j)
+      if (s_cnt[j] <= a.ns_cap && s_grp[j] <= a.groups_cap) {
+        ns = s_cnt[j];
+        staged = s_grp[j];
+        if (ns) longest = static_cast<float>(stage_level(a.len0, j));
         break;
       }
-  }
-  const uint32_t nh = *a.heavy_cnt;
   const uint32_t npc = (a.heavy_max == 0 || nh <= ns) ? 0u : min(nh - ns, a.heavy_max);
-  const uint32_t nlong = a.len0 <= a.heavy_len ? a.stage_cnt[0] : nh;
+  if (npc && npc == nh - ns) longest = fminf(longest, static_cast<float>(a.heavy_len));
+  const uint32_t nlong = a.len0 <= a.heavy_len ? s_cnt[0] : nh;
   out[0] = ns;
   out[1] = npc;
   out[2] = ns + npc;
-  out[3] = split_lists(a.len0, a.stage_cnt, nlong, ns + npc, *a.etot, a.additive, a.split);
+  out[3] = split_lists(c, nlong, ns + npc, staged, longest, a.additive, a.split);
 }
 
 void launch_partition(const PartitionArgs &pa, uint32_t *out, hipStream_t s) {
-  k_partition<<<1, 1, 0, s>>>(pa, out);
+  k_partition<<<1, 64, 0, s>>>(pa, out);
   hip_check(hipGetLastError(), "k_partition launch");
 }
 
@@ -2315,13 +2325,19 @@ void launch_splat_pc(bool additive, const uint32_t *items, uint32_t npc, const S
 
 void launch_splat8(bool additive, int variant, const uint32_t *items, uint32_t nitems,
                    const SplatArgs &a, hipStream_t s, const ItemCounts &dc, int ppw,
-                   uint32_t nsplit) {
+                   uint32_t nsplit, bool beside) {
   if (nitems == 0) return;
   // device counts: nitems, a capacity of three items per unit, also bounds
   // the items with the long lists served by channel
   if (dc.items) nsplit = 0;
   const unsigned grid = static_cast<unsigned>((uint64_t(nitems) + 2u * uint64_t(nsplit) + 3) / 4);
-#define SPLAT8(ADDV, VARV, PPWV) k_splat8<ADDV, VARV, PPWV><<<grid, 256, 0, s>>>(a, items, nitems, dc, nsplit)
+  // Beside producer/consumer workgroups a small grid would fit whole on the CUs that
+  // they leave, four workgroups each, and stay there when the others are free: three
+  // (by LDS) leave some for those (1296 lists of 100k ordered entries, 192 of them in
+  // such workgroups: 27.9 ms with four, 24.9 with three; grids of tens of thousands
+  // are 3 % slower with three).
+  const unsigned spread = beside && grid <= 2048u ? 6144u : 0u;
+#define SPLAT8(ADDV, VARV, PPWV) k_splat8<ADDV, VARV, PPWV><<<grid, 256, spread, s>>>(a, items, nitems, dc, nsplit)
   if (variant == 4) {
     switch (ppw) {
       case 1: if (additive) SPLAT8(1, 4, 1); else SPLAT8(0, 4, 1); break;
