@@ -23,11 +23,12 @@ The JSON line also carries:
                 stage's live duration, against the issue peak of the simplest
                 operations (256 CUs x 4 SIMDs x one wave64 instruction per 2
                 clocks at 2.4 GHz; others take 4);
-  lds           the limit the splat meets: the LDS read peak measured by a
-                microbenchmark on this GPU (libmembench), and the splats' busy
-                LDS cycles per frame (rocprofv3 LDS counters, committed
-                summary) over the ordered splat stage's live duration, against
-                the microbenchmark's busy cycles;
+  lds           LDS reads measured by a microbenchmark on this GPU (libmembench:
+                bandwidth, and clocks per instruction and CU), and the splats'
+                LDS instructions and busy cycles per frame (rocprofv3 LDS
+                counters, committed summary) over the ordered splat stage's live
+                duration: the share of the CUs' clocks (256 at 2.4 GHz) in which
+                the LDS works, and the clocks per instruction;
   parity        per workload, the max per-channel relative error of the GPU
                 image (denominator max(|ref|, 1e-6 max|ref|)) against the
                 oracle (stable depth order), the genuine reference renderer
@@ -76,7 +77,7 @@ if int(os.environ.get("GPU_MAX_HW_QUEUES") or 4) < 8:
 METRIC = "ms/frame & Mparticles/s (16M, 2048²); batched and fwd+bwd vs plain"
 HBM_PEAK_GBS = 8000.0
 VALU_PEAK = 256 * 4 * 2.4e9 / 2  # wave64 VALU instructions per second (one per SIMD per 2 clocks)
-LDS_SPEC_GBS = 256 * 128 * 2.4e9 / 1e9  # 128 B per clock per CU (32 banks x 4 B)
+CU_CLOCKS_PER_MS = 256 * 2.4e6  # 256 CUs at 2.4 GHz
 
 
 def log(*a):
@@ -249,27 +250,32 @@ def gpu_time(torch, fn, steps, warmup):
 
 def membench():
     lib = ctypes.CDLL(os.path.join(ROOT, "splotch_amd", "libmembench.so"))
-    lib.lds_peak_run.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
-                                 ctypes.POINTER(ctypes.c_float), ctypes.POINTER(ctypes.c_double)]
+    lib.lds_peak_run.argtypes = [ctypes.c_int] * 5 + [ctypes.POINTER(ctypes.c_float),
+                                                      ctypes.POINTER(ctypes.c_double)]
     lib.hbm_copy_run.argtypes = [ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_int,
                                  ctypes.POINTER(ctypes.c_float)]
     return lib
 
 
-def lds_peak(grid=2048, iters=12000):
-    """LDS read bandwidth of conflict-free ds_read_b32 / b64 / b128 streams;
-    the best is the measured peak."""
+def lds_peak(grid=2048, iters=6000):
+    """LDS reads of all CUs at once (ds_read_b32 / b64 / b128, no bank conflict):
+    bandwidth of linear reads, and the clocks (2.4 GHz) that an instruction takes its
+    CU; also with 4 distinct words per wave.  The best bandwidth is the measured peak."""
     runs = {}
     for words, name in ((1, "b32"), (2, "b64"), (4, "b128")):
-        ms, nbytes = ctypes.c_float(), ctypes.c_double()
-        it = iters * 4 // words  # about the same time per variant
-        rc = membench().lds_peak_run(0, grid, it, words, ctypes.byref(ms), ctypes.byref(nbytes))
-        if rc != 0:
-            raise RuntimeError("lds_peak_run failed (%d)" % rc)
-        runs[name] = {"ms": round(ms.value, 4), "bytes": nbytes.value,
-                      "GBs": round(nbytes.value / (ms.value * 1e-3) / 1e9, 1)}
-    best = max(runs, key=lambda k: runs[k]["GBs"])
-    return {"kernel": "k_lds_read<words> (conflict-free ds_read_%s)" % best,
+        for four in (0, 1):
+            ms, ninst = ctypes.c_float(), ctypes.c_double()
+            rc = membench().lds_peak_run(0, grid, iters, words, four, ctypes.byref(ms),
+                                         ctypes.byref(ninst))
+            if rc != 0:
+                raise RuntimeError("lds_peak_run failed (%d)" % rc)
+            run = {"ms": round(ms.value, 4),
+                   "clocks_per_instruction": round(ms.value * CU_CLOCKS_PER_MS / ninst.value, 3)}
+            if not four:
+                run["GBs"] = round(ninst.value * 256 * words / (ms.value * 1e-3) / 1e9, 1)
+            runs[name + ("_four" if four else "")] = run
+    best = max((k for k in runs if "GBs" in runs[k]), key=lambda k: runs[k]["GBs"])
+    return {"kernel": "k_lds_read (linear ds_read_%s)" % best,
             "GBs": runs[best]["GBs"], "variants": runs}
 
 
@@ -818,21 +824,21 @@ def main():
                      "frac": round(achieved / HBM_PEAK_GBS, 6), "traffic": traffic,
                      "traffic_source": traffic_src,
                      "bytes_per_launch": splat_bytes, "launch_ms": splat_ms,
-                     "note": "the splat is LDS-bound (see lds); HBM is not its limit"},
+                     "note": "HBM is not the splat's limit: see valu and lds"},
         "valu": valu,
     }
-    # LDS: measured peak; the splats' busy LDS cycles from the committed profile
+    # LDS: measured peak; the splats' LDS instructions and busy cycles from the committed profile
     lp = lds_peak()
-    lds = {"peak_measured_GBs": lp["GBs"], "peak_spec_GBs": LDS_SPEC_GBS,
-           "microbenchmark": lp}
-    busy = profile_value("pmc_lds_gas_stars_16M_2048.md",
-                         "lds_active_cycles_per_frame splats") if default else None
-    per_ms = profile_value("pmc_lds_gas_stars_16M_2048.md",
-                           "lds_active_cycles_per_ms peak_stream") if default else None
-    if busy is not None and per_ms is not None:
+    lds = {"peak_measured_GBs": lp["GBs"], "microbenchmark": lp}
+    lds_md = "pmc_lds_gas_stars_16M_2048.md"
+    busy = profile_value(lds_md, "lds_active_cycles_per_frame splats") if default else None
+    ninst = profile_value(lds_md, "lds_instructions_per_frame splats") if default else None
+    if busy is not None and ninst is not None:
+        clocks = stages["ordered_splat"] * CU_CLOCKS_PER_MS
         lds["splats"] = {"active_cycles_per_frame": int(busy), "stage_ms": stages["ordered_splat"],
-                         "frac_of_peak_stream": round(busy / stages["ordered_splat"] / per_ms, 4),
-                         "source": "profiles/pmc_lds_gas_stars_16M_2048.md"}
+                         "active_share": round(busy / clocks, 4),
+                         "clocks_per_instruction": round(clocks / ninst, 3),
+                         "source": "profiles/" + lds_md}
     out["lds"] = lds
     fo = profile_value("fragments_gas_stars_16M_2048.md", "fragments_ordered") if default else None
     fa = profile_value("fragments_gas_stars_16M_2048.md", "fragments_additive") if default else None

@@ -2,13 +2,14 @@
 // library): the chip's practical peaks that the bench sets kernels against,
 // and known-size kernels for scaling profiler counters.
 //
-// LDS read bandwidth: every workgroup fills 32 KiB of LDS, then each lane
-// reads 4-, 8- or 16-byte words (ds_read_b32 / b64 / b128) at conflict-free
-// addresses: a wave's 64 lanes read consecutive bytes per instruction.  The
-// reads are folded into an integer checksum (at most two VALU operations per
-// read, below the VALU issue limit), which is written once per lane so that
-// no read can be removed.  Bytes per launch = grid * 256 lanes * iters * 8
-// reads * the word size.
+// LDS reads: every workgroup fills 33 KiB of LDS (4 workgroups, 16 waves per
+// CU), then each wave reads 4-, 8- or 16-byte words (ds_read_b32 / b64 / b128)
+// from 16 places 1 KiB apart, by immediate offsets from one address per lane:
+// linear (64 lanes, consecutive words: no bank conflict), or 4 distinct words
+// (lane l that of l % 4, as a splat reads the constants of 4 particles).  Every
+// word that is read goes into a checksum (one VALU operation, below the issue
+// limit) that is written at the end: a part of a vector that nothing uses would
+// be left out of the read.  Reads per launch and wave = iters * 16.
 //
 // HBM copy: dst[i] = src[i] over n 16-byte vectors, grid-stride, each lane
 // moving four vectors per step with all four loads issued before the stores.
@@ -19,34 +20,29 @@
 
 namespace {
 
-constexpr int kWords = 2048;  // uint4 slots: 32 KiB
+constexpr int kLdsBytes = 33 * 1024;
+constexpr int kReads = 16;  // per iteration, 1 KiB apart
 
-// V: 32-bit words per lane and read (1: ds_read_b32, 2: b64, 4: b128).
-template <int V>
-__global__ __launch_bounds__(256) void k_lds_read(uint32_t *out, int iters) {
-  __shared__ uint4 buf[kWords];
-  const int t = threadIdx.x;
-  for (int i = t; i < kWords; i += 256)
+template <typename T, bool FOUR>
+__global__ __launch_bounds__(256, 4) void k_lds_read(uint32_t *out, int iters) {
+  __shared__ uint4 buf[kLdsBytes / 16];
+  const int t = threadIdx.x, lane = t & 63;
+  for (int i = t; i < kLdsBytes / 16; i += 256)
     buf[i] = make_uint4(i, i * 3u + 1u, i * 5u + 2u, i * 7u + 3u);
   __syncthreads();
   uint32_t acc = 0;
-  int base = t;
-  constexpr int kSlots = kWords * 4 / V;  // V-word slots in the buffer
+  uint32_t x = FOUR ? lane & 3 : lane;  // the lane's word: at most 1 KiB, then 2 KiB on and back
   for (int k = 0; k < iters; ++k) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int slot = (base + j * 256) & (kSlots - 1);
-      if (V == 4) {
-        const uint4 v = buf[slot];
-        acc ^= v.x + v.w;
-      } else if (V == 2) {
-        const uint2 v = reinterpret_cast<const uint2 *>(buf)[slot];
-        acc ^= v.x + v.y;
-      } else {
-        acc += reinterpret_cast<const uint32_t *>(buf)[slot];
-      }
+    for (int j = 0; j < kReads; ++j) {
+      const T v = reinterpret_cast<const T *>(buf)[x + j * (1024 / sizeof(T))];
+      if constexpr (sizeof(T) == 16) acc ^= v.x ^ v.y ^ v.z ^ v.w;
+      else if constexpr (sizeof(T) == 8) acc ^= v.x ^ v.y;
+      else acc ^= v.x;
+      asm volatile("" ::: "memory");  // one read each: not joined, not kept
     }
-    base = (base + 64) & (kSlots - 1);  // the next reads start a wave further on
+    x ^= 2048 / sizeof(T);
+    asm volatile("" : "+v"(x));
   }
   out[static_cast<int64_t>(blockIdx.x) * 256 + t] = acc;
 }
@@ -74,11 +70,13 @@ __global__ __launch_bounds__(256) void k_copy(const uint4 *__restrict__ src,
 extern "C" {
 
 // Times one launch of `grid` workgroups x `iters` iterations of reads of
-// `words` 32-bit words per lane (1, 2 or 4), after one warm-up launch, with
-// HIP events on a stream of its own.  Returns 0 and writes the milliseconds
-// and the bytes read from LDS; a HIP error code otherwise.
-int lds_peak_run(int device, int grid, int iters, int words, float *ms, double *bytes) {
-  if (grid < 1 || iters < 1 || !ms || !bytes || (words != 1 && words != 2 && words != 4))
+// `words` 32-bit words per lane (1, 2 or 4; four != 0: 4 distinct ones per wave),
+// after one warm-up launch, with HIP events on a stream of its own.  Returns 0
+// and writes the milliseconds and the read instructions (of a wave each); a
+// HIP error code otherwise.
+int lds_peak_run(int device, int grid, int iters, int words, int four, float *ms,
+                 double *instructions) {
+  if (grid < 1 || iters < 1 || !ms || !instructions || (words != 1 && words != 2 && words != 4))
     return -1;
   if (hipSetDevice(device) != hipSuccess) return -2;
   uint32_t *out = nullptr;
@@ -91,9 +89,11 @@ int lds_peak_run(int device, int grid, int iters, int words, float *ms, double *
     rc = -2;
   } else {
     auto launch = [&]() {
-      if (words == 4) k_lds_read<4><<<grid, 256, 0, s>>>(out, iters);
-      else if (words == 2) k_lds_read<2><<<grid, 256, 0, s>>>(out, iters);
-      else k_lds_read<1><<<grid, 256, 0, s>>>(out, iters);
+      void (*kernel)(uint32_t *, int) =
+          words == 4   ? (four ? k_lds_read<uint4, true> : k_lds_read<uint4, false>)
+          : words == 2 ? (four ? k_lds_read<uint2, true> : k_lds_read<uint2, false>)
+                       : (four ? k_lds_read<uint1, true> : k_lds_read<uint1, false>);
+      kernel<<<grid, 256, 0, s>>>(out, iters);
     };
     launch();
     (void)hipEventRecord(e0, s);
@@ -103,7 +103,7 @@ int lds_peak_run(int device, int grid, int iters, int words, float *ms, double *
       rc = -2;
     } else {
       (void)hipEventElapsedTime(ms, e0, e1);
-      *bytes = static_cast<double>(grid) * 256.0 * iters * 8.0 * 4.0 * words;
+      *instructions = static_cast<double>(grid) * 4.0 * iters * kReads;
     }
   }
   if (e0) (void)hipEventDestroy(e0);

@@ -155,14 +155,15 @@ constexpr int kColPad = 68;  // bytes per column of coverage (a word per four pa
 // is l += ((l - q) * a) * att (att replaced by +0 outside the footprint) with
 // no table work.
 //
-// The walk is bound by the CU's LDS, which returns 128 B per clock (a b32
-// read of a wave 2 clocks, a b128 read 8, whether or not the lanes share
-// addresses; a random table lookup about 6), before its VALU.  So the
-// constants of four particles are read once, lane l those of particle l % 4,
-// and reach the operations as quad-permuted DPP operands (2 clocks more per
-// use, against 16 LDS clocks per particle), and four particles' coverage of a
-// column is one word: 47 -> 33 LDS clocks per particle in the expm1 branch, 22
-// -> 9 in the Taylor branch.
+// The walk issues VALU work most of the time and keeps the CU's LDS busy half
+// of it, and waits on the LDS's returns where 16 waves do not hide them (at
+// 2.4 GHz a linear or broadcast b32 read of a wave takes its CU 2.5 clocks, a
+// b128 one 4.3, whether or not the lanes share addresses; a random table lookup
+// 6).  So the constants of four particles are read once, lane l those of
+// particle l % 4, and reach the operations as quad-permuted DPP operands (2
+// VALU clocks more per use), and four particles' coverage of a column is one
+// word: 52 -> 44 LDS clocks per particle in the expm1 branch, 16 -> 8 in the
+// Taylor branch.
 template <int CH, int J, uint32_t TB>
 __device__ __forceinline__ void fast_chunk(int k0, int cx, int cy, const uint8_t (*col)[kColPad],
                                            const float (*pre2)[kPad],
