@@ -73,8 +73,10 @@ typedef struct {
                                               channel (twice it in an additive pass; from the
                                               staging base length on, lengths are rounded
                                               down to a level of it, see hip_stage_ordered)
-                                              (0 = auto: 32768; below, lists from the pass's
-                                              entries / 2048 on are in any case) */
+                                              (0 = auto, and from 32768 on: from the pass's
+                                              entries / 2048 on, unless walking these lists
+                                              by channel takes the GPU longer than the
+                                              longest of them one wave) */
   int32_t hip_variant;                     /* hip_variant: 8x8 splat inner loop, 0 = auto (4),
                                               1 = per particle, 2 = 4-particle groups,
                                               3 = software pipelined, 4 = chunked branch-free */
@@ -98,8 +100,9 @@ typedef struct {
                                               work region hip_region (8, 16, 32, 64 px) and,
                                               for 8 px, the 8x8 splat's decomposition
                                               (hip_heavy_max, hip_split, hip_variant and
-                                              hip_ppw), and reuse the fastest for the bucket
-                                              (0 = off) */
+                                              hip_ppw), and reuse the fastest for the bucket;
+                                              passes that walk their long lists in segments
+                                              (see hip_heavy) still do (0 = off) */
   int32_t hip_bin_group;                   /* hip_bin_group: 8 px units are binned through
                                               regions of g x g units, then split: 4, 2, or
                                               1 = sort the unit entries directly (0 = auto: the
@@ -115,8 +118,12 @@ typedef struct {
                                               summed in list order by one wave per channel
                                               and pixel column (0 = auto: from entries /
                                               1300 or the longest list / 64 on, none where
-                                              the longest list is below 1536 entries; < 0 =
-                                              never) */
+                                              the longest list is below 1536 entries, and
+                                              only so many that staging them takes no longer
+                                              than walking the longest of the others; < 0 =
+                                              never).  Staged operands use device memory that
+                                              is free then, at most: without it the lists are
+                                              splatted otherwise, with the same image */
   int32_t hip_stage_ordered;               /* hip_stage_ordered: the same for an ordered pass
                                               (per-pixel operands of the compositing update
                                               computed first; not when a particle's q_c is
@@ -125,8 +132,9 @@ typedef struct {
                                               lists from the longest / 16 or entries / 700
                                               on; else, when it x 432 does, the lists from
                                               entries / 432 on; else, and where the longest
-                                              list is below 512 entries, none; thresholds
-                                              are levels 256 x 2^(j/2); < 0 = never) */
+                                              list is below 512 entries, none; of these only
+                                              so many as for hip_stage; thresholds are levels
+                                              256 x 2^(j/2); < 0 = never) */
 } splhip_params;
 
 /* SoA particle fields (device pointers), post particle_normalize:

@@ -444,10 +444,10 @@ struct Plan {
   // long lists after the first nheavy items (one item each), which the 8x8
   // splat serves by channel
   uint32_t nsplit[2] = {0, 0};
-  // staged lists (the first nstage items; nheavy counts them too) and their
-  // groups of 4 entries (padded to whole chain loads)
   bool counted[2] = {false, false};  // work items counted in this frame
   bool late = false;  // the pass sizes are still on the device (m: capacities)
+  // staged lists (the first nstage items; nheavy counts them too) and their
+  // groups of 4 entries (padded to whole chain loads)
   uint32_t nstage[2] = {0, 0};
   uint64_t sgroups[2] = {0, 0};
   uint32_t seglen[2] = {0, 0};  // lists walked in segments: their length (0: none)
@@ -1492,18 +1492,18 @@ Tuning autotune(splhip_ctx *c, Plan &pl, const Tuning &base, uint32_t *tot, hipS
   return best;
 }
 
-// The frame pipeline over a batch of jobs; three host syncs per batch (pass
-// sizes, bin entries, work items).
-// A choice of the autotuner: work region and the 8x8 splat's decomposition.
 // Frames of at most this many particles (of all views) wait on the host once
 // less (see render_jobs).
 constexpr int64_t kLateParticles = int64_t(1) << 22;
 
+// A choice of the autotuner: work region and the 8x8 splat's decomposition.
 struct Choice {
   int G;
   Tuning tn;
 };
 
+// The frame pipeline over a batch of jobs; three host syncs per batch (pass
+// sizes, bin entries, work items), two up to kLateParticles.
 // force: a tuning chosen by the autotuner (null: the params' keys; with
 // hip_autotune and 8 px regions the splat's decomposition is then swept on
 // this frame, and the choice left in c->inner_choice).
@@ -1539,7 +1539,7 @@ int render_jobs(splhip_ctx *c, int nj, const JobIn *jobs, hipStream_t s, bool ke
     }
   bool chunked[2] = {false, false};
   if (pl.m[0] || pl.m[1]) {
-    // sync 2
+    // sync 2 (the first where pl.late)
     if (pl.late) {
       read_pass_sizes(c, pl, tot, s);
       set_job_flags(c, pl, s);

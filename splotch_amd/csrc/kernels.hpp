@@ -131,8 +131,8 @@ void launch_map(const uint32_t *idx, const uint32_t *table, uint32_t *out, int64
 void launch_fill(float *p, float v, int64_t n, hipStream_t s);
 void launch_fill_u32(uint32_t *p, uint32_t v, int64_t n, hipStream_t s);
 // Device-count pipeline helpers: zeros into the images of jobs with no particle
-// in either pass (mo null: pass absent), and the capacity check of a pass (counts zeroed, bit set in
-// *ovf when e64 > ecap or *e16 > e16cap).
+// in either pass (mo null: pass absent), and the capacity check of a pass (counts
+// zeroed, bit set in *ovf when e64 > ecap or *e16 > e16cap).
 void launch_fill_empty_jobs(const uint32_t *mo0, const uint32_t *mo1, int nj, const JobSplat *js,
                             hipStream_t s);
 void launch_cap_check(uint32_t *m, uint32_t *e, const uint64_t *e64, uint32_t *e16,
@@ -164,8 +164,8 @@ __host__ __device__ inline uint64_t stage_level(uint32_t sl, int j) {
 // channel 3 = all), heaviest first.  heavy_cnt (device, optional): incremented
 // once per unit whose list reaches a.heavy_len (one item); stage_cnt /
 // stage_grp (optional, [kStageLevels] each): [j] once per unit whose list
-// reaches stage_level(a.stage_len, j), and by its groups of 4 entries (at most); lmax (optional): the longest list of a unit with
-// items.
+// reaches stage_level(a.stage_len, j), and by its groups of 4 entries (at most); lmax
+// (optional): the longest list of a unit with items.
 void launch_items_count(const uint32_t *bin_off, uint32_t nunits, const SplatArgs &a,
                         int ordered, uint32_t split, uint32_t *cnt, uint32_t *heavy_cnt,
                         hipStream_t s, uint32_t *stage_cnt = nullptr,

@@ -1,6 +1,7 @@
 // Device-wide exclusive scan and stable LSD radix sort (key/value u32 pairs),
 // written for wave64: wave-level scans over 64 lanes, wave-local digit
-// ranking with ballots, 4096-element tiles per 256-thread workgroup.
+// ranking with ballots; tiles of 1024 elements (small inputs) or 4096 per 256-thread
+// workgroup, and inputs of one tile in one workgroup.
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -2162,8 +2162,8 @@ void launch_items_emit(const uint32_t *bin_off, uint32_t nunits, const SplatArgs
 // it is its list's last, and the lists have etot entries or fewer.
 void seg_caps(uint64_t etot, uint32_t seglen, SegArgs &g) {
   g.seglen = seglen;
-  // a pass takes about 0.07 ns per entry, one wave's walk 200 ns (by channel half
-  // of that): longer walks would outlast it (64 views, 160M and 169M entries: 33.9
+  // a pass takes about 0.07 ns per entry, a lone wave's walk up to 200 ns (ListRates;
+  // by channel half): longer walks would outlast it (64 views, 160M and 169M entries: 33.9
   // and 34.6 ms; 42.9 and 42.0 with 123k and 205k entries whatever the pass)
   g.split = static_cast<uint32_t>(etot / 2700u / kSegSample);
   g.longest = static_cast<uint32_t>(etot / 1500u / kSegSample);
@@ -2338,7 +2338,8 @@ void launch_splat8(bool additive, int variant, const uint32_t *items, uint32_t n
   // such workgroups: 27.9 ms with four, 24.9 with three; grids of tens of thousands
   // are 3 % slower with three).
   const unsigned spread = beside && grid <= 2048u ? 6144u : 0u;
-#define SPLAT8(ADDV, VARV, PPWV) k_splat8<ADDV, VARV, PPWV><<<grid, 256, spread, s>>>(a, items, nitems, dc, nsplit)
+#define SPLAT8(ADDV, VARV, PPWV) \
+  k_splat8<ADDV, VARV, PPWV><<<grid, 256, spread, s>>>(a, items, nitems, dc, nsplit)
   if (variant == 4) {
     switch (ppw) {
       case 1: if (additive) SPLAT8(1, 4, 1); else SPLAT8(0, 4, 1); break;
