@@ -327,8 +327,9 @@ struct ListCounts {
 // longest of these lists (16M particles at 2048^2, every leftover list by channel:
 // 41.2 -> 48.2 ms; 1296 lists of 8000 ordered entries 1.6 and 2.5 ms, by absorption,
 // 2.2 by channel, of 30k 5.0 and 8.3, and 7.1; 5184 of up to 30k additive ones 2.6, and
-// 3.3), unless lists that producer/consumer workgroups have no room for wait beside
-// them (1104 of 100k ordered: 28 ms by channel, 43 not).
+// 3.3), unless ordered lists that producer/consumer workgroups have no room for wait
+// beside them (1104 of 100k: 28 ms by channel, 43 not; additive ones 14.6 and 14.0,
+// 762 of 66k to 95k beside 4200 shorter 12.5 and 11.7).
 constexpr uint32_t kSplitRatio = 2048;
 constexpr uint32_t kSplitAuto = 32768;  // hip_split by default: the rule
 __host__ __device__ inline uint32_t split_lists(const ListCounts &c, uint32_t nlong,
@@ -341,7 +342,7 @@ __host__ __device__ inline uint32_t split_lists(const ListCounts &c, uint32_t nl
   int j = 0;
   while (j < kStageLevels - 1 && stage_level(c.len0, j + 1) <= from) ++j;
   const ListRates r = list_rates(additive);
-  if (!given && c.nheavy <= c.heavy_max &&
+  if (!given && (additive || c.nheavy <= c.heavy_max) &&
       (c.entries(j) - 4.f * static_cast<float>(staged)) * r.channels >= longest * r.walk)
     return 0u;
   const uint32_t n = c.count[j] < nlong ? c.count[j] : nlong;

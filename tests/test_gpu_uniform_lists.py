@@ -69,3 +69,30 @@ def test_uniform_lists(R, kind, n, hsml, spread, side, additive):
     R.capture_reserve([(dev, cam, prm, pic)], 1.25)
     torch.cuda.synchronize()
     assert_bitexact(pic.cpu().numpy().reshape(side, side, 3), want, kind + " reserved")
+
+
+@pytest.mark.parametrize("additive", [True, False])
+def test_more_than_the_workgroups_serve(R, additive):
+    """1296 lists for 192 producer/consumer workgroups: the ordered ones that are
+    left go by channel, the additive ones do not."""
+    import splotch_amd as S
+    side = 256
+    fld, view = field(6000, 90.0, 0.3), synth.default_view(side)
+    print("case left lists additive", additive, flush=True)
+    want, _ = O.host_rendering(fld, view, [synth.default_palette()], a_eq_e=additive, stable=True)
+    dev, cam = S.to_device(fld), S.camera_setup(view)
+    prm = S.params(a_eq_e=additive, hip_heavy=4096)
+    pic = torch.empty(side * side * 3, dtype=torch.float32, device="cuda")
+    R.set_trace(True)
+    try:
+        R.render(dev, cam, prm, pic)
+        tr = R.trace_items(not additive)
+    finally:
+        R.set_trace(False)
+    torch.cuda.synchronize()
+    assert ((tr[:, 2] >> 32) < 3).any() == (not additive)
+    assert_bitexact(pic.cpu().numpy().reshape(side, side, 3), want, "left lists")
+    pic.fill_(7.0)
+    R.capture_reserve([(dev, cam, prm, pic)], 1.25)
+    torch.cuda.synchronize()
+    assert_bitexact(pic.cpu().numpy().reshape(side, side, 3), want, "left lists reserved")
